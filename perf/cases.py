@@ -219,21 +219,21 @@ def run(s):
             v = node.v
             functional.reset_net(node)
             return [packed, v, bit_spike_decompress(packed, spikes.shape, dtype=x.dtype)]
-    # Blocks of convolutions, batch norms and neurons.  Their spikes are handed out as truth values: a neuron within
-    # rounding of its threshold may fire or not with the order in which a convolution's products are added.
+    # Blocks of convolutions, batch norms and neurons.  Their spikes leave as bits, as a program that keeps them for later
+    # stores them.
     block = s["block"]
     if kind == "attention" and not s["case"]["train"]:
         with torch.no_grad():
             spikes = block(x)
         functional.reset_net(block)
-        return [spikes.bool()]
+        return [bit_spike_compress(spikes)]
     x.grad = None
     for p in block.parameters():
         p.grad = None
     spikes = block(x)
     spikes.backward(s["grad"])
     functional.reset_net(block)
-    return [spikes.detach().bool(), x.grad] + [p.grad for p in block.parameters()]
+    return [bit_spike_compress(spikes.detach()), x.grad] + [p.grad for p in block.parameters()]
 
 
 def work(case):
@@ -270,11 +270,12 @@ def tolerance(case):
     Measured with this framework's own alternatives, stated about four times that: fp32 gradients with the sums of the
     parametric neuron's dL/dk in another order 2e-6; 16-bit gradients whose membrane potentials were stored in the 16-bit
     type between forward and backward instead of recomputed in fp32, bf16: 2.9e-3 (largest single difference 0.05), dL/dk
-    2.5e-2 (its terms cancel); blocks with convolutions split into other terms, or run by the library: up to 5.9e-3 with
-    1.4e-5 of the spikes on the other side of their threshold (and single gradients behind such a spike off by 0.76)."""
+    2.5e-2 (its terms cancel); blocks with convolutions split into other terms, or run by the library: up to 5.9e-3, because
+    1.4e-5 of the spikes (1.1e-4 of their bytes) fall on the other side of their threshold with another order of a
+    convolution's sums, and single gradients behind such a spike are off by 0.76."""
     kind = case["kind"]
     if kind in ("attention", "conv"):
-        return {"rel": 2.4e-2, "max": 0.99, "differ": 1e-4}
+        return {"rel": 2.4e-2, "max": 0.99, "differ": 5e-4}
     if kind != "train":
         return "exact"
     plif = case["node"] == "plif"
