@@ -149,8 +149,8 @@ const char *sjhip_last_error(void);
  *   rtau_device  PLIF only (required there, SJHIP_ERR_INVALID without it; NULL for the other neurons): device
  *             address of one fp32 holding k = sigmoid(w), read by the kernel in place of p->tau so that no host
  *             synchronisation is needed to fetch it
- * T >= 1, N >= 1, T*N < 2^62.  128-bit accesses are used when N is a multiple of 16/sizeof(dtype)
- * and every pointer is 16-byte aligned; otherwise an element-wise kernel runs.
+ * T >= 1, N >= 1, T*N < 2^62.  128-bit accesses are used when N is at least 16/sizeof(dtype), at any alignment of
+ * the rows; shorter rows run an element-wise kernel.  No output may overlap an input.
  */
 int sjhip_neuron_forward(int neuron, int dtype, const sjhip_neuron_params *p,
                          int64_t T, int64_t N,
@@ -229,8 +229,9 @@ int sjhip_neuron_backward_static(int neuron, int dtype, const sjhip_neuron_param
  * in LDS) and then runs the same BPTT.  A forward whose backward will use this entry point can be
  * called with h_seq = NULL, which saves its largest write.  Same argument meaning as
  * sjhip_neuron_backward with (x_seq, v_init) in place of h_seq; `p` carries the forward flags too
- * (SJHIP_FLAG_FP32_STATE, SJHIP_FLAG_RECIPROCAL_TAU).  Requires sjhip_recompute_supported() and
- * 16-byte aligned tensors; returns SJHIP_ERR_UNSUPPORTED / SJHIP_ERR_INVALID otherwise.
+ * (SJHIP_FLAG_FP32_STATE, SJHIP_FLAG_RECIPROCAL_TAU).  Requires N of at least one 128-bit vector, the T of
+ * sjhip_recompute_supported() and tensors that begin on 16 bytes; returns SJHIP_ERR_UNSUPPORTED / SJHIP_ERR_INVALID
+ * otherwise.
  * Stands in for the same reference backward ops as sjhip_neuron_backward; the reference has no
  * recomputing variant (its kernels always read the saved h_seq, multi_step/base.py:137-409).
  */
@@ -252,8 +253,8 @@ int sjhip_neuron_backward_recompute(int neuron, int dtype, const sjhip_neuron_pa
  * back; the gradient of a piece's initial state stays in registers (fp32) for the piece before it.  Results: spikes,
  * states and checkpoints are bit-identical to sjhip_neuron_forward's; gradients are those of the walk over the whole
  * sequence (in fp32 storage also those of sjhip_neuron_backward_recompute applied piece by piece with grad_v_init
- * handed on as grad_v_last).  N must be a multiple of the 128-bit
- * vector width and every tensor 16-byte aligned.  With 16-bit storage and SJHIP_FLAG_FP32_STATE the checkpoints are
+ * handed on as grad_v_last).  N must be at least one 128-bit
+ * vector and every tensor 16-byte aligned.  With 16-bit storage and SJHIP_FLAG_FP32_STATE the checkpoints are
  * fp32 rows ([pieces - 1][N] floats: a checkpoint in the storage dtype would round the state).  The saved state per
  * neuron is 1 / chunk of an h_seq; chunk = 16 keeps
  * five or more blocks resident per compute unit, which is where the single-piece kernel runs fastest.  No counterpart
@@ -274,8 +275,8 @@ int sjhip_neuron_backward_recompute_pieces(int neuron, int dtype, const sjhip_ne
                                            float *grad_rtau, float *workspace,
                                            void *stream);
 
-/* 1 if sjhip_neuron_backward_recompute can serve [T,N] of `dtype` (N a multiple of the 128-bit vector
- * width and T steps of h fitting in LDS: T <= 159), else 0. */
+/* 1 if sjhip_neuron_backward_recompute can serve [T,N] of `dtype` on whole vectors (N a multiple of the 128-bit vector
+ * width and T steps of h fitting in LDS: T <= 159), else 0.  (A longer row that is no such multiple is served as well.) */
 int sjhip_recompute_supported(int dtype, int64_t T, int64_t N);
 
 /* 1 if, beyond being supported, the replay is expected to beat a saved h_seq: its LDS footprint grows with T and

@@ -238,6 +238,15 @@ def _hip_recompute(x2: torch.Tensor) -> bool:
     return width > 0 and x2.shape[1] % width == 0 and x2.shape[0] <= steps
 
 
+def _hip_replays(x2: torch.Tensor) -> bool:
+    """The same for the kernels of IF, LIF, PLIF, QIF, EIF and ILIF, which also take rows that the vector width does not
+    divide (``whole_group`` of ``csrc/sjhip_common.h``): only rows shorter than one vector keep the saved ``h_seq``."""
+    if not configure.hip_backward_recompute:
+        return False
+    width, steps = _replay_limits(x2.dtype, _hip_mode_flags(x2))
+    return width > 0 and x2.shape[1] >= width and x2.shape[0] <= steps
+
+
 def _use_eager_entry() -> bool:
     """The direct ``autograd.Function`` entry serves ordinary eager calls; a tracing compiler needs the operators
     (schema, fake kernels)."""
@@ -273,10 +282,10 @@ def if_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, v_threshold: float, 
     if _use_eager_entry():
         s, v_seq, v_last = K.eager_multistep(L.NEURON_IF, x2, v1, None, 0.0, v_threshold, vr,
                                              K._flags(soft, detach_reset, False, flags), sg_id, sg_alpha, store_v_seq,
-                                             need_grad and _hip_recompute(x2), need_grad)
+                                             need_grad and _hip_replays(x2), need_grad)
     elif need_grad:
         s, v_seq, v_last, _ = K.hip_multistep_if_forward(x2, v1, v_threshold, vr, soft, detach_reset, sg_id,
-                                                         sg_alpha, store_v_seq, flags, _hip_recompute(x2))
+                                                         sg_alpha, store_v_seq, flags, _hip_replays(x2))
     else:
         s, v_seq, v_last = K.hip_multistep_if_inference(x2, v1, v_threshold, vr, soft, store_v_seq, flags)
     return _finish(x_seq, s, v_seq, v_last, store_v_seq)
@@ -300,11 +309,11 @@ def lif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, tau: float, decay_i
     if _use_eager_entry():
         s, v_seq, v_last = K.eager_multistep(L.NEURON_LIF, x2, v1, None, float(tau), v_threshold, vr,
                                              K._flags(soft, detach_reset, decay_input, flags), sg_id, sg_alpha,
-                                             store_v_seq, need_grad and _hip_recompute(x2), need_grad)
+                                             store_v_seq, need_grad and _hip_replays(x2), need_grad)
     elif need_grad:
         s, v_seq, v_last, _ = K.hip_multistep_lif_forward(x2, v1, v_threshold, vr, soft, detach_reset,
                                                           float(tau), decay_input, sg_id, sg_alpha,
-                                                          store_v_seq, flags, _hip_recompute(x2))
+                                                          store_v_seq, flags, _hip_replays(x2))
     else:
         s, v_seq, v_last = K.hip_multistep_lif_inference(x2, v1, v_threshold, vr, soft, float(tau),
                                                          decay_input, store_v_seq, flags)
@@ -331,11 +340,11 @@ def plif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, w: torch.Tensor, d
     if _use_eager_entry():
         s, v_seq, v_last = K.eager_multistep(L.NEURON_PLIF, x2, v1, k, 0.0, v_threshold, vr,
                                              K._flags(soft, detach_reset, decay_input, flags), sg_id, sg_alpha,
-                                             store_v_seq, need_grad and _hip_recompute(x2), need_grad)
+                                             store_v_seq, need_grad and _hip_replays(x2), need_grad)
     elif need_grad:
         s, v_seq, v_last, _ = K.hip_multistep_plif_forward(x2, v1, k, v_threshold, vr, soft, detach_reset,
                                                            decay_input, sg_id, sg_alpha, store_v_seq, flags,
-                                                           _hip_recompute(x2))
+                                                           _hip_replays(x2))
     else:
         s, v_seq, v_last = K.hip_multistep_plif_inference(x2, v1, k, v_threshold, vr, soft, decay_input,
                                                           store_v_seq, flags)
@@ -360,12 +369,12 @@ def qif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, tau: float, v_thres
     if _use_eager_entry():
         s, v_seq, v_last = K.eager_multistep(L.NEURON_QIF, x2, v1, None, float(tau), v_threshold, vr,
                                              K._flags(soft, detach_reset, True, flags), sg_id, sg_alpha, store_v_seq,
-                                             need_grad and _hip_recompute(x2), need_grad,
+                                             need_grad and _hip_replays(x2), need_grad,
                                              qif=(float(v_rest), float(v_c), float(a0)))
     elif need_grad:
         s, v_seq, v_last, _ = K.hip_multistep_qif_forward(x2, v1, v_threshold, vr, soft, detach_reset, float(tau),
                                                           float(v_rest), float(v_c), float(a0), sg_id, sg_alpha,
-                                                          store_v_seq, flags, _hip_recompute(x2))
+                                                          store_v_seq, flags, _hip_replays(x2))
     else:
         s, v_seq, v_last = K.hip_multistep_qif_inference(x2, v1, v_threshold, vr, soft, float(tau), float(v_rest),
                                                          float(v_c), float(a0), store_v_seq, flags)
@@ -390,12 +399,12 @@ def eif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, tau: float, v_thres
     if _use_eager_entry():
         s, v_seq, v_last = K.eager_multistep(L.NEURON_EIF, x2, v1, None, float(tau), v_threshold, vr,
                                              K._flags(soft, detach_reset, True, flags), sg_id, sg_alpha, store_v_seq,
-                                             need_grad and _hip_recompute(x2), need_grad,
+                                             need_grad and _hip_replays(x2), need_grad,
                                              qif=(float(v_rest), float(theta_rh), float(delta_t)))
     elif need_grad:
         s, v_seq, v_last, _ = K.hip_multistep_eif_forward(x2, v1, v_threshold, vr, soft, detach_reset, float(tau),
                                                           float(v_rest), float(theta_rh), float(delta_t), sg_id, sg_alpha,
-                                                          store_v_seq, flags, _hip_recompute(x2))
+                                                          store_v_seq, flags, _hip_replays(x2))
     else:
         s, v_seq, v_last = K.hip_multistep_eif_inference(x2, v1, v_threshold, vr, soft, float(tau), float(v_rest),
                                                          float(theta_rh), float(delta_t), store_v_seq, flags)
@@ -450,12 +459,12 @@ def ilif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, tau: float, v_thre
     if _use_eager_entry():
         s, v_seq, v_last = K.eager_multistep(
             L.NEURON_ILIF, x2, v1, None, float(tau), float(v_threshold), 0.0, K._flags(True, detach_reset, False, flags),
-            L.SG_MULTI_LEVEL, 0.0, store_v_seq, need_grad and _hip_recompute(x2), need_grad,
+            L.SG_MULTI_LEVEL, 0.0, store_v_seq, need_grad and _hip_replays(x2), need_grad,
             levels=(float(levels), float(surrogate_function.grad_min), float(surrogate_function.grad_max)))
     elif need_grad:
         s, v_seq, v_last, _ = K.hip_multistep_ilif_forward(
             x2, v1, float(tau), float(v_threshold), levels, float(surrogate_function.grad_min),
-            float(surrogate_function.grad_max), detach_reset, store_v_seq, flags, _hip_recompute(x2))
+            float(surrogate_function.grad_max), detach_reset, store_v_seq, flags, _hip_replays(x2))
     else:
         s, v_seq, v_last = K.hip_multistep_ilif_inference(x2, v1, float(tau), float(v_threshold), levels,
                                                           store_v_seq, flags)

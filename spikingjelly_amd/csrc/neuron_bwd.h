@@ -350,11 +350,13 @@ __device__ __forceinline__ float backward_body(const BwdArgs &a, bool active, in
   if (PLIF) {
     float v0[V];
     load_state_from<S, VECTOR, SJHIP_BWD_NT != 0>(a.v_init, col, a.v_init_broadcast, v0);
+    // neurons that the work-item shares with its neighbour (whole_group) are counted there
+    const int64_t shared = ((int64_t)column_block(a.spread) * blockDim.x + threadIdx.x) * V - col;
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       const float dh_dk = a.decay_input ? (h_next[j] - v0[j]) : (a.v_reset - v0[j]);
       acc[j] += g_next[j] * dh_dk;
-      acc_total += acc[j];
+      if (j >= shared) acc_total += acc[j];
     }
   }
   return acc_total;
@@ -412,8 +414,9 @@ __device__ __forceinline__ void plif_block_reduce(const BwdArgs &a, float part, 
 template <typename S, bool VECTOR, int MODE>
 __global__ void __launch_bounds__(SJHIP_MAX_BLOCK) backward_kernel(const BwdArgs a) {
   constexpr int V = Acc<S, VECTOR, true>::V;
-  const int64_t col = ((int64_t)column_block(a.spread) * blockDim.x + threadIdx.x) * V;
+  int64_t col = ((int64_t)column_block(a.spread) * blockDim.x + threadIdx.x) * V;
   const bool active = col < a.N;
+  col = whole_group<V>(col, a.N);
   const float k = a.k_device ? *a.k_device : a.k;
   const float part = backward_sg_dispatch<S, VECTOR, MODE, 0>(a, active, col, k, nullptr);
   if (BwdModeOf<MODE>::BASE == BWD_PLIF) plif_block_reduce(a, part, k);

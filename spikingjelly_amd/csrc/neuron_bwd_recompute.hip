@@ -53,8 +53,10 @@ int launch_replay(int neuron, int dtype, const sjhip_neuron_params &p, int64_t T
                   void *grad_x_seq, void *grad_v_init, float *grad_rtau, float *workspace,
                   hipStream_t stream) {
   const int64_t lds_steps = chunk > 0 ? chunk : T;
-  if (!recompute_supported(dtype, lds_steps, N))
-    return fail(SJHIP_ERR_UNSUPPORTED, "backward(recompute): T=%lld N=%lld does not fit (N %% %d != 0 or T too large for LDS)",
+  // (a row that the vector width does not divide runs as well, see whole_group(); the policy functions, which callers
+  // of the saved-h route rely on, speak for whole rows)
+  if (N < (dtype == SJHIP_F32 ? 4 : 8) || recompute_block(dtype, lds_steps, false) == 0)
+    return fail(SJHIP_ERR_UNSUPPORTED, "backward(recompute): T=%lld N=%lld does not fit (N < %d or T too large for LDS)",
                 (long long)T, (long long)N, dtype == SJHIP_F32 ? 4 : 8);
   const bool broadcast = (p.flags & SJHIP_FLAG_V_INIT_BROADCAST) != 0;
   if (!aligned16(x_seq) || (!broadcast && !aligned16(v_init)) || !aligned16(grad_spike_seq) || !aligned16(grad_x_seq) ||
@@ -88,7 +90,7 @@ int launch_replay(int neuron, int dtype, const sjhip_neuron_params &p, int64_t T
     const int want = several ? kSpreadBlock : spread_block(N * (dtype == SJHIP_F32 ? 4 : 2));
     if (want > block && want <= SJHIP_MAX_BLOCK && 2 * lds_steps * want * kHBytesPerItem <= (int64_t)kMaxLds) block = want;
   }
-  const int64_t items = N / V;
+  const int64_t items = (N + V - 1) / V;
   const int64_t blocks = (items + block - 1) / block;
   if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "backward(recompute): N=%lld", (long long)N);
   unsigned lds = (unsigned)(lds_steps * block * kHBytesPerItem);

@@ -1,6 +1,7 @@
 // Multi-step forward (charge -> fire -> reset over T steps) for IF / LIF / PLIF / QIF / ILIF.
 //
-// One work-item owns V consecutive neurons (one 128-bit access per row) and walks the T rows in
+// One work-item owns V consecutive neurons (one 128-bit access per row, whatever the row's alignment; see
+// whole_group() for rows that V does not divide) and walks the T rows in
 // order with the membrane potential in registers.  Rows of x are requested SJHIP_FWD_PF steps ahead
 // of their use so several 128-bit loads per lane are always in flight; every tensor is touched
 // exactly once (default cache policy: the write-dominated forward measured slower with
@@ -265,8 +266,9 @@ __device__ __forceinline__ void forward_body(const FwdArgs &a) {
   constexpr int PF = (OUT & FWD_OUT_SHORT) ? 2 : (sizeof(S) == 2 ? SJHIP_FWD_PF16 : SJHIP_FWD_PF);
 
   const int64_t N = a.N, T = a.T;
-  const int64_t col = ((int64_t)column_block(a.spread) * blockDim.x + threadIdx.x) * V;
+  int64_t col = ((int64_t)column_block(a.spread) * blockDim.x + threadIdx.x) * V;
   if (col >= N) return;
+  col = whole_group<V>(col, N);
 
   const E *xp = (const E *)a.x + col;
   E *sp = (E *)a.spike + col;
@@ -317,7 +319,7 @@ __device__ __forceinline__ void forward_body(const FwdArgs &a) {
 #pragma unroll
             for (int q = 0; q < V / 4; ++q) {
               f32x4 w; w.x = v[4 * q]; w.y = v[4 * q + 1]; w.z = v[4 * q + 2]; w.w = v[4 * q + 3];
-              stream_store<NT>(reinterpret_cast<f32x4 *>(cpf) + q, w);
+              stream_store_any<NT>(cpf + 4 * q, w);
             }
           } else {
             A::store(cp, v);

@@ -61,7 +61,7 @@ template <typename S, bool ROUND_EACH> int launch_pieces_typed(const FwdArgs &a,
   // (2^29 neuron-steps, fp32, T = 64 / 128 / 512: 1.198 / 1.234 / 1.327 ms against 1.231 / 1.283 / 1.398 with 128
   // lanes; T = 48: 1.304 against 1.283).
   const int block = a.T >= 64 && tuning().fwd_block > 64 ? 64 : tuning().fwd_block;
-  const int64_t items = a.N / Acc<S, true, true>::V;
+  const int64_t items = (a.N + Acc<S, true, true>::V - 1) / Acc<S, true, true>::V;
   const int64_t blocks = (items + block - 1) / block;
   if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "forward(pieces): N=%lld", (long long)a.N);
   const unsigned lds = (sizeof(S) == 4 && a.v_seq != nullptr) ? occupancy_cap_lds(tuning().fwd_blocks_per_cu) : 0u;
@@ -80,9 +80,9 @@ int launch_forward_pieces(int neuron, int dtype, const sjhip_neuron_params &p, i
   int rc = build_fwd_args(a, round_each, neuron, dtype, p, T, N, x_seq, v_init, k_device, spike_seq, v_seq, v_last, nullptr);
   if (rc != SJHIP_OK) return rc;
   const int V = dtype == SJHIP_F32 ? 4 : 8;
-  if (N % V != 0 || !aligned16(x_seq) || !(a.v_init_broadcast || aligned16(v_init)) || !aligned16(spike_seq) || !aligned16(v_seq) ||
+  if (N < V || !aligned16(x_seq) || !(a.v_init_broadcast || aligned16(v_init)) || !aligned16(spike_seq) || !aligned16(v_seq) ||
       !aligned16(v_last) || !aligned16(checkpoints))
-    return fail(SJHIP_ERR_UNSUPPORTED, "forward(pieces): N=%lld must be a multiple of %d and every tensor 16-byte aligned", (long long)N, V);
+    return fail(SJHIP_ERR_UNSUPPORTED, "forward(pieces): N=%lld must be at least %d and every tensor 16-byte aligned", (long long)N, V);
   a.checkpoints = checkpoints; a.chunk = chunk;
   switch (dtype) {
     case SJHIP_F32: return launch_pieces_typed<float, false>(a, stream);
@@ -101,8 +101,7 @@ int launch_forward_packed(int neuron, int dtype, const sjhip_neuron_params &p, i
   bool round_each = false;
   int rc = build_fwd_args(a, round_each, neuron, dtype, p, T, N, x_seq, v_init, k_device, spike_bits, v_seq, v_last, nullptr);
   if (rc != SJHIP_OK) return rc;
-  const bool vector = aligned16(x_seq) && (a.v_init_broadcast || aligned16(v_init)) && (v_seq == nullptr || aligned16(v_seq)) &&
-                      (v_last == nullptr || aligned16(v_last));
+  const bool vector = true;  // (N is a multiple of 8: no work-item is left with part of a group)
   switch (dtype) {
     case SJHIP_F32: return launch_typed<float, false, true>(a, vector, stream);
     case SJHIP_F16: return round_each ? launch_typed<f16_t, true, true>(a, vector, stream) : launch_typed<f16_t, false, true>(a, vector, stream);
@@ -119,11 +118,7 @@ int launch_forward(int neuron, int dtype, const sjhip_neuron_params &p, int64_t 
   int rc = build_fwd_args(a, round_each, neuron, dtype, p, T, N, x_seq, v_init, k_device, spike_seq, v_seq, v_last, h_seq);
   if (rc != SJHIP_OK) return rc;
 
-  const int esize = dtype == SJHIP_F32 ? 4 : 2;
-  const int V = 16 / esize;
-  const bool vector = (N % V == 0) && aligned16(x_seq) && (a.v_init_broadcast || aligned16(v_init)) && aligned16(spike_seq) &&
-                      (v_seq == nullptr || aligned16(v_seq)) && (v_last == nullptr || aligned16(v_last)) &&
-                      (h_seq == nullptr || aligned16(h_seq));
+  const bool vector = N >= (dtype == SJHIP_F32 ? 4 : 8);  // any N and any alignment: see whole_group()
 
   switch (dtype) {
     case SJHIP_F32: return launch_typed<float, false>(a, vector, stream);

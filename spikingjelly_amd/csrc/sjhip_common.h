@@ -26,6 +26,12 @@ struct bf16n_t { uint16_t bits; };
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// The same vectors at the alignment of their elements: rows of [T, N] start anywhere when N is not a multiple of the
+// vector width.  The hardware takes such global accesses as they are (one instruction, one more cache line where a
+// wavefront's run straddles one), so the compiler emits the same instruction for either type.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+typedef u32x4 u32x4_any16 __attribute__((aligned(2)));
+typedef u32x2 u32x2_any16 __attribute__((aligned(2)));
 
 template <typename S> struct Cvt;
 
@@ -88,6 +94,22 @@ template <bool NT, typename T> __device__ __forceinline__ void stream_store(T *p
   if (NT) __builtin_nontemporal_store(v, p);
   else *p = v;
 }
+// (spelled out per type: a template argument would lose the alignment of the typedef)
+#define SJHIP_ANY_ALIGNMENT(VEC, ANY, ELEM)                                                  \
+  template <bool NT> __device__ __forceinline__ VEC stream_load_any(const ELEM *p, VEC) {     \
+    const ANY *q = reinterpret_cast<const ANY *>(p);                                          \
+    if (NT) return __builtin_nontemporal_load(q);                                             \
+    return *q;                                                                                \
+  }                                                                                           \
+  template <bool NT> __device__ __forceinline__ void stream_store_any(ELEM *p, VEC v) {       \
+    ANY *q = reinterpret_cast<ANY *>(p);                                                      \
+    if (NT) __builtin_nontemporal_store(v, q);                                                \
+    else *q = v;                                                                              \
+  }
+SJHIP_ANY_ALIGNMENT(f32x4, f32x4_any, float)
+SJHIP_ANY_ALIGNMENT(u32x4, u32x4_any16, uint16_t)
+SJHIP_ANY_ALIGNMENT(u32x2, u32x2_any16, uint16_t)
+#undef SJHIP_ANY_ALIGNMENT
 
 // Accessor: how one work-item reads/writes its V consecutive neurons of one row.
 // raw_t is what stays in registers between the (early) load and the (late) use.
@@ -97,14 +119,14 @@ template <bool NT> struct Acc<float, true, NT> {
   static constexpr int V = 4;
   typedef float elem_t;
   typedef f32x4 raw_t;
-  static __device__ __forceinline__ raw_t load(const elem_t *p) { return stream_load<NT>((const raw_t *)p); }
+  static __device__ __forceinline__ raw_t load(const elem_t *p) { return stream_load_any<NT>(p, raw_t()); }
   static __device__ __forceinline__ raw_t zero() { return (raw_t)(0.f); }
   static __device__ __forceinline__ void unpack(raw_t r, float (&f)[V]) {
     f[0] = r.x; f[1] = r.y; f[2] = r.z; f[3] = r.w;
   }
   static __device__ __forceinline__ void store(elem_t *p, const float (&f)[V]) {
     raw_t r; r.x = f[0]; r.y = f[1]; r.z = f[2]; r.w = f[3];
-    stream_store<NT>((raw_t *)p, r);
+    stream_store_any<NT>(p, r);
   }
   // spikes are exactly 0 or 1: in 16-bit storage the bit pattern is selected instead of converted
   static __device__ __forceinline__ void store_spikes(elem_t *p, const float (&f)[V]) { store(p, f); }
@@ -123,7 +145,7 @@ template <typename H, bool NT> struct Acc16v {
   static constexpr int V = 8;
   typedef uint16_t elem_t;
   typedef u32x4 raw_t;
-  static __device__ __forceinline__ raw_t load(const elem_t *p) { return stream_load<NT>((const raw_t *)p); }
+  static __device__ __forceinline__ raw_t load(const elem_t *p) { return stream_load_any<NT>(p, raw_t()); }
   static __device__ __forceinline__ raw_t zero() { return (raw_t)(0u); }
   static __device__ __forceinline__ void unpack(raw_t r, float (&f)[V]) {
     uint32_t w[4] = {r.x, r.y, r.z, r.w};
@@ -139,7 +161,7 @@ template <typename H, bool NT> struct Acc16v {
     for (int i = 0; i < 4; ++i)
       w[i] = (uint32_t)Cvt<H>::from_float(f[2 * i]) | ((uint32_t)Cvt<H>::from_float(f[2 * i + 1]) << 16);
     raw_t r; r.x = w[0]; r.y = w[1]; r.z = w[2]; r.w = w[3];
-    stream_store<NT>((raw_t *)p, r);
+    stream_store_any<NT>(p, r);
   }
   static __device__ __forceinline__ void store_spikes(elem_t *p, const float (&f)[V]) {
     uint32_t w[4];
@@ -147,7 +169,7 @@ template <typename H, bool NT> struct Acc16v {
     for (int i = 0; i < 4; ++i)
       w[i] = (f[2 * i] != 0.0f ? (uint32_t)Cvt<H>::kOne : 0u) | (f[2 * i + 1] != 0.0f ? (uint32_t)Cvt<H>::kOne << 16 : 0u);
     raw_t r; r.x = w[0]; r.y = w[1]; r.z = w[2]; r.w = w[3];
-    stream_store<NT>((raw_t *)p, r);
+    stream_store_any<NT>(p, r);
   }
   // fp16 values kept as fp16 in registers (native half arithmetic): the stored bits are the register bits
   static __device__ __forceinline__ void unpack(raw_t r, _Float16 (&f)[V]) {
@@ -166,7 +188,7 @@ template <typename H, bool NT> struct Acc16v {
     for (int i = 0; i < 4; ++i)
       w[i] = (uint32_t)__builtin_bit_cast(uint16_t, f[2 * i]) | ((uint32_t)__builtin_bit_cast(uint16_t, f[2 * i + 1]) << 16);
     raw_t r; r.x = w[0]; r.y = w[1]; r.z = w[2]; r.w = w[3];
-    stream_store<NT>((raw_t *)p, r);
+    stream_store_any<NT>(p, r);
   }
   static __device__ __forceinline__ void store_spikes(elem_t *p, const _Float16 (&f)[V]) { store(p, f); }
 };
@@ -175,7 +197,7 @@ template <typename H, bool NT> struct Acc16n {
   static constexpr int V = 4;
   typedef uint16_t elem_t;
   typedef u32x2 raw_t;
-  static __device__ __forceinline__ raw_t load(const elem_t *p) { return stream_load<NT>((const raw_t *)p); }
+  static __device__ __forceinline__ raw_t load(const elem_t *p) { return stream_load_any<NT>(p, raw_t()); }
   static __device__ __forceinline__ raw_t zero() { return (raw_t)(0u); }
   static __device__ __forceinline__ void unpack(raw_t r, float (&f)[V]) {
     f[0] = Cvt<H>::to_float((uint16_t)(r.x & 0xffffu)); f[1] = Cvt<H>::to_float((uint16_t)(r.x >> 16));
@@ -185,7 +207,7 @@ template <typename H, bool NT> struct Acc16n {
     raw_t r;
     r.x = (uint32_t)Cvt<H>::from_float(f[0]) | ((uint32_t)Cvt<H>::from_float(f[1]) << 16);
     r.y = (uint32_t)Cvt<H>::from_float(f[2]) | ((uint32_t)Cvt<H>::from_float(f[3]) << 16);
-    stream_store<NT>((raw_t *)p, r);
+    stream_store_any<NT>(p, r);
   }
 };
 template <typename H, bool NT> struct Acc16s {
@@ -247,7 +269,7 @@ __device__ __forceinline__ void load_state_from(const void *p, int64_t col, int 
     if constexpr (VECTOR && V % 4 == 0) {
 #pragma unroll
       for (int i = 0; i < V / 4; ++i) {
-        const f32x4 w = stream_load<NT>(reinterpret_cast<const f32x4 *>(q) + i);
+        const f32x4 w = stream_load_any<NT>(q + 4 * i, f32x4());
         v[4 * i] = (NUM)w.x; v[4 * i + 1] = (NUM)w.y; v[4 * i + 2] = (NUM)w.z; v[4 * i + 3] = (NUM)w.w;
       }
     } else {
@@ -360,6 +382,20 @@ __device__ __forceinline__ unsigned column_block(int spread) {
   }
   const unsigned per = gridDim.x / 8u;
   return b < per * 8u ? (b % 8u) * per + b / 8u : b;
+}
+#endif
+
+// First of the V neurons of the work-item whose share of a row begins at `col`: the last work-item of a row that V does
+// not divide takes the row's last V neurons, the first of which its neighbour has too (both compute and store the same
+// bits; nothing they read is written by the kernel).  So a row of any N >= V runs on V-wide accesses; shorter ones on the
+// element-wise kernels, which such rows had to take before: one 2- or 4-byte access per lane and row keeps too few bytes in
+// flight, and without the replay h_seq is written and read as well.  Measured (forward / backward, us; element-wise and
+// saved h -> this and the replay): fp32 [8, 2979423] 78 / 157 -> 35 / 53 (5.4 TB/s; a row of whole vectors takes the same),
+// fp16 with every op rounded [6, 3580137] 35 / 264 -> 20 / 34.
+#ifdef __HIPCC__
+template <int V> __device__ __forceinline__ int64_t whole_group(int64_t col, int64_t N) {
+  if (V == 1) return col;
+  return col + V <= N ? col : N - V;
 }
 #endif
 
