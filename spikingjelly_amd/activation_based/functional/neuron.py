@@ -247,6 +247,58 @@ def _hip_replays(x2: torch.Tensor) -> bool:
     return width > 0 and x2.shape[1] >= width and x2.shape[0] <= steps
 
 
+_native = None  # (extension module, resolver of surrogate ids), imported at the first call of a hip functional
+_NO_EXTRA = (0.0,) * 6
+_IF, _LIF, _PLIF, _QIF, _ILIF, _EIF = 0, 1, 2, 3, 4, 5  # sjhip_neuron
+_MULTI_LEVEL = 7  # sjhip_surrogate
+
+
+def _native_sequence(neuron: int, x_seq: torch.Tensor, v: torch.Tensor, k: Optional[torch.Tensor], tau: float, v_threshold: float,
+                     v_reset: Optional[float], detach_reset: bool, decay_input: bool, surrogate_function: Optional[SurrogateFunction],
+                     store_v_seq: bool, single: bool = False, extra: tuple = _NO_EXTRA):
+    """One eager call through the native host path (``csrc/torch_binding.cpp``): ``(spike_seq, v_next, v_seq or None)`` in the
+    shapes of ``x_seq``, or ``None`` when it does not serve the call (the general path below then does: layouts that need a
+    copy, a saved ``h_seq``, a sequence replayed in pieces, function transforms).  ``single``: ``x_seq`` is one step.
+    ``surrogate_function`` ``None``: the windowed gradient of the integer-valued neuron, whose limits are in ``extra``."""
+    global _native
+    if _native is None:
+        from ..hip_kernel import native
+        from ..hip_kernel.surrogate_registry import resolve_sg_hip_id_and_alpha
+
+        _native = (native.load(), resolve_sg_hip_id_and_alpha)
+    module, resolve = _native
+    dtype = x_seq.dtype
+    flags = 0 if dtype is torch.float32 and not configure.hip_lif_reciprocal_tau and not configure.hip_plif_atomic_reduce else (
+        _hip_mode_flags(x_seq))
+    mode = flags
+    if v_reset is None:
+        flags, v_reset = flags | 0x02, 0.0  # FLAG_SOFT_RESET
+    if detach_reset:
+        flags |= 0x04  # FLAG_DETACH_RESET
+    if decay_input:
+        flags |= 0x01  # FLAG_DECAY_INPUT
+    sg_id, sg_alpha, steps = 0, 0.0, 0
+    if torch.is_grad_enabled() and (x_seq.requires_grad or v.requires_grad or (k is not None and k.requires_grad)):
+        sg_id, sg_alpha = (_MULTI_LEVEL, 0.0) if surrogate_function is None else resolve(surrogate_function)
+        if configure.hip_backward_recompute and dtype in _FLOAT_DTYPES:
+            steps = _replay_limits(dtype, mode)[1]
+    return module.neuron_sequence(x_seq, v, k, single, neuron, tau, v_threshold, float(v_reset), flags, sg_id, sg_alpha, store_v_seq,
+                                  steps, extra)
+
+
+_FLOAT_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
+
+
+def _native_packed(neuron: int, x_seq: torch.Tensor, v: torch.Tensor, k: Optional[torch.Tensor], tau: float, v_threshold: float,
+                   v_reset: Optional[float], decay_input: bool, store_v_seq: bool):
+    """The same for inference with bit-packed spikes: ``(spike_bits, v_next, v_seq or None)`` or ``None``."""
+    from ..hip_kernel import native
+
+    flags = _hip_mode_flags(x_seq) | (0x02 if v_reset is None else 0) | (0x01 if decay_input else 0)
+    return native.load().neuron_sequence_packed(x_seq, v, k, neuron, tau, v_threshold, 0.0 if v_reset is None else float(v_reset),
+                                                flags, store_v_seq)
+
+
 def _use_eager_entry() -> bool:
     """The direct ``autograd.Function`` entry serves ordinary eager calls; a tracing compiler needs the operators
     (schema, fake kernels)."""
@@ -269,6 +321,10 @@ def if_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, v_threshold: float, 
                       store_v_seq: bool = False
                       ) -> tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """Multi-step IF on the hip backend.  ``x_seq`` is ``[T, *]``, ``v`` has the shape of ``x_seq[0]``."""
+    if _use_eager_entry():
+        out = _native_sequence(_IF, x_seq, v, None, 0.0, v_threshold, v_reset, detach_reset, False, surrogate_function, store_v_seq)
+        if out is not None:
+            return out
     from ..hip_kernel import library as L
     from ..hip_kernel import neuron_kernel as K
     from ..hip_kernel.surrogate_registry import resolve_sg_hip_id_and_alpha
@@ -296,6 +352,11 @@ def lif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, tau: float, decay_i
                        detach_reset: bool = False, store_v_seq: bool = False
                        ) -> tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """Multi-step LIF on the hip backend."""
+    if _use_eager_entry():
+        out = _native_sequence(_LIF, x_seq, v, None, tau, v_threshold, v_reset, detach_reset, decay_input, surrogate_function,
+                               store_v_seq)
+        if out is not None:
+            return out
     from ..hip_kernel import library as L
     from ..hip_kernel import neuron_kernel as K
     from ..hip_kernel.surrogate_registry import resolve_sg_hip_id_and_alpha
@@ -326,6 +387,12 @@ def plif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, w: torch.Tensor, d
                         ) -> tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """Multi-step parametric LIF on the hip backend.  ``w`` is the pre-sigmoid parameter; the
     sigmoid stays outside the operator so autograd supplies ``dk/dw`` (reference :2173-2182)."""
+    k = w.sigmoid().to(device=x_seq.device, dtype=torch.float32)
+    if _use_eager_entry():
+        out = _native_sequence(_PLIF, x_seq, v, k, 0.0, v_threshold, v_reset, detach_reset, decay_input, surrogate_function,
+                               store_v_seq)
+        if out is not None:
+            return out
     from ..hip_kernel import library as L
     from ..hip_kernel import neuron_kernel as K
     from ..hip_kernel.surrogate_registry import resolve_sg_hip_id_and_alpha
@@ -334,7 +401,6 @@ def plif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, w: torch.Tensor, d
     vr = 0.0 if soft else float(v_reset)
     flags = _hip_mode_flags(x_seq)
     x2, v1 = x_seq.flatten(1), v.flatten()
-    k = w.sigmoid().to(device=x_seq.device, dtype=torch.float32)
     need_grad = _needs_grad(x_seq, v, w)
     sg_id, sg_alpha = resolve_sg_hip_id_and_alpha(surrogate_function) if need_grad else (0, 0.0)
     if _use_eager_entry():
@@ -356,6 +422,11 @@ def qif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, tau: float, v_thres
                        surrogate_function: SurrogateFunction, store_v_seq: bool = False
                        ) -> tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """Multi-step QIF on the hip backend; argument order of the reference's ``qif_multi_step_cupy`` (:2188-2200)."""
+    if _use_eager_entry():
+        out = _native_sequence(_QIF, x_seq, v, None, tau, v_threshold, v_reset, detach_reset, True, surrogate_function, store_v_seq,
+                               extra=(float(v_rest), float(v_c), float(a0), 0.0, 0.0, 0.0))
+        if out is not None:
+            return out
     from ..hip_kernel import library as L
     from ..hip_kernel import neuron_kernel as K
     from ..hip_kernel.surrogate_registry import resolve_sg_hip_id_and_alpha
@@ -386,6 +457,11 @@ def eif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, tau: float, v_thres
                        surrogate_function: SurrogateFunction, store_v_seq: bool = False
                        ) -> tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """Multi-step EIF on the hip backend; argument order of the reference's ``eif_multi_step_cupy`` (:2296-2308)."""
+    if _use_eager_entry():
+        out = _native_sequence(_EIF, x_seq, v, None, tau, v_threshold, v_reset, detach_reset, True, surrogate_function, store_v_seq,
+                               extra=(float(v_rest), float(theta_rh), float(delta_t), 0.0, 0.0, 0.0))
+        if out is not None:
+            return out
     from ..hip_kernel import library as L
     from ..hip_kernel import neuron_kernel as K
     from ..hip_kernel.surrogate_registry import resolve_sg_hip_id_and_alpha
@@ -453,6 +529,12 @@ def ilif_multi_step_hip(x_seq: torch.Tensor, v: torch.Tensor, tau: float, v_thre
     if not isinstance(surrogate_function, surrogate.MultiLevelSpikeCount) or not surrogate_function.spiking:
         raise ValueError("surrogate_function must be a spiking MultiLevelSpikeCount.")
     levels = int(surrogate_function.max_spike_count)
+    if _use_eager_entry():
+        out = _native_sequence(_ILIF, x_seq, v, None, tau, v_threshold, None, detach_reset, False, None, store_v_seq,
+                               extra=(0.0, 0.0, 0.0, float(levels), float(surrogate_function.grad_min),
+                                      float(surrogate_function.grad_max)))
+        if out is not None:
+            return out
     flags = _hip_mode_flags(x_seq)
     x2, v1 = x_seq.flatten(1), v.flatten()
     need_grad = _needs_grad(x_seq, v)
@@ -520,6 +602,10 @@ def if_step_hip(x: torch.Tensor, v: torch.Tensor, v_threshold: float, v_reset: O
                 surrogate_function: SurrogateFunction, detach_reset: bool = False
                 ) -> tuple[torch.Tensor, torch.Tensor]:
     """One IF step on the hip backend: the multi-step kernel on a sequence of length one."""
+    if _use_eager_entry():
+        out = _native_sequence(_IF, x, v, None, 0.0, v_threshold, v_reset, detach_reset, False, surrogate_function, False, single=True)
+        if out is not None:
+            return out[0], out[1]
     spike_seq, v_next, _ = if_multi_step_hip(x.unsqueeze(0), v, v_threshold, v_reset, surrogate_function,
                                              detach_reset, False)
     return spike_seq[0], v_next
@@ -529,6 +615,10 @@ def lif_step_hip(x: torch.Tensor, v: torch.Tensor, tau: float, decay_input: bool
                  v_reset: Optional[float], surrogate_function: SurrogateFunction, detach_reset: bool = False
                  ) -> tuple[torch.Tensor, torch.Tensor]:
     """One LIF step on the hip backend."""
+    if _use_eager_entry():
+        out = _native_sequence(_LIF, x, v, None, tau, v_threshold, v_reset, detach_reset, decay_input, surrogate_function, False, single=True)
+        if out is not None:
+            return out[0], out[1]
     spike_seq, v_next, _ = lif_multi_step_hip(x.unsqueeze(0), v, tau, decay_input, v_threshold, v_reset,
                                               surrogate_function, detach_reset, False)
     return spike_seq[0], v_next
@@ -538,6 +628,11 @@ def plif_step_hip(x: torch.Tensor, v: torch.Tensor, w: torch.Tensor, decay_input
                   v_reset: Optional[float], surrogate_function: SurrogateFunction, detach_reset: bool = False
                   ) -> tuple[torch.Tensor, torch.Tensor]:
     """One parametric-LIF step on the hip backend."""
+    if _use_eager_entry():
+        out = _native_sequence(_PLIF, x, v, w.sigmoid().to(device=x.device, dtype=torch.float32), 0.0, v_threshold, v_reset,
+                               detach_reset, decay_input, surrogate_function, False, single=True)
+        if out is not None:
+            return out[0], out[1]
     spike_seq, v_next, _ = plif_multi_step_hip(x.unsqueeze(0), v, w, decay_input, v_threshold, v_reset,
                                                surrogate_function, detach_reset, False)
     return spike_seq[0], v_next
@@ -563,6 +658,10 @@ def if_multi_step_hip_packed(x_seq: torch.Tensor, v: torch.Tensor, v_threshold: 
                              store_v_seq: bool = False
                              ) -> tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """Multi-step IF inference on the hip backend with bit-packed spike output."""
+    if _use_eager_entry():
+        out = _native_packed(_IF, x_seq, v, None, 0.0, v_threshold, v_reset, False, store_v_seq)
+        if out is not None:
+            return out
     from ..hip_kernel import neuron_kernel as K
 
     soft = v_reset is None
@@ -581,6 +680,10 @@ def lif_multi_step_hip_packed(x_seq: torch.Tensor, v: torch.Tensor, tau: float, 
                               v_threshold: float, v_reset: Optional[float], store_v_seq: bool = False
                               ) -> tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """Multi-step LIF inference on the hip backend with bit-packed spike output."""
+    if _use_eager_entry():
+        out = _native_packed(_LIF, x_seq, v, None, tau, v_threshold, v_reset, decay_input, store_v_seq)
+        if out is not None:
+            return out
     from ..hip_kernel import neuron_kernel as K
 
     soft = v_reset is None
@@ -601,13 +704,17 @@ def plif_multi_step_hip_packed(x_seq: torch.Tensor, v: torch.Tensor, w: torch.Te
                                v_threshold: float, v_reset: Optional[float], store_v_seq: bool = False
                                ) -> tuple[torch.Tensor, torch.Tensor, Optional[torch.Tensor]]:
     """Multi-step parametric-LIF inference on the hip backend with bit-packed spike output."""
+    k = w.sigmoid().to(device=x_seq.device, dtype=torch.float32)
+    if _use_eager_entry():
+        out = _native_packed(_PLIF, x_seq, v, k, 0.0, v_threshold, v_reset, decay_input, store_v_seq)
+        if out is not None:
+            return out
     from ..hip_kernel import neuron_kernel as K
 
     soft = v_reset is None
     vr = 0.0 if soft else float(v_reset)
     flags = _hip_mode_flags(x_seq)
     x2, v1 = x_seq.flatten(1), v.flatten()
-    k = w.sigmoid().to(device=x_seq.device, dtype=torch.float32)
     if K.packed_supported(x2.shape[1]):
         out = K.hip_multistep_plif_inference_packed(x2, v1, k, v_threshold, vr, soft, decay_input, store_v_seq, flags)
     else:

@@ -118,26 +118,38 @@ class BaseNode(base.MemoryModule):
         backend it is a one-element tensor expanded to the shape (read-only, never written back: the next
         state is the kernel's own output) and no ``[N]`` tensor is filled or read."""
         if self.backend == "hip" and x.is_cuda and x.numel() > 1:
-            if torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing():
-                # (memory allocated while a graph is being captured belongs to that graph: not kept)
-                return x.new_full((1,) * x.dim(), value).expand(x.shape)
-            # one element per (device, dtype, value), made once: a fill launch per neuron and call otherwise
-            key = (x.device, x.dtype, float(value), math.copysign(1.0, float(value)))
-            one = _CONSTANT_STATES.get(key)
-            if one is None:
-                # The element outlives this call: it must be an ordinary tensor even when the first call comes under
-                # torch.inference_mode() (an inference tensor could not be saved for a later training backward), and
-                # its fill must have finished before a call on another stream reads it (made once: the wait is free).
-                with torch.inference_mode(False):
-                    one = torch.full((1,), value, dtype=x.dtype, device=x.device)
-                torch.cuda.current_stream(x.device).synchronize()
-                _CONSTANT_STATES[key] = one
-            return one.view((1,) * x.dim()).expand(x.shape)
+            return self._one_element_state(x, value, x.shape)
         return torch.full_like(x, value, requires_grad=False)
 
+    @staticmethod
+    def _one_element_state(x: torch.Tensor, value: float, shape: torch.Size) -> torch.Tensor:
+        if torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing():
+            # (memory allocated while a graph is being captured belongs to that graph: not kept)
+            return x.new_full((1,) * len(shape), value).expand(shape)
+        # one element per (device, dtype, value), made once: a fill launch per neuron and call otherwise
+        key = (x.device, x.dtype, float(value), math.copysign(1.0, value))
+        one = _CONSTANT_STATES.get(key)
+        if one is None:
+            # The element outlives this call: it must be an ordinary tensor even when the first call comes under
+            # torch.inference_mode() (an inference tensor could not be saved for a later training backward), and
+            # its fill must have finished before a call on another stream reads it (made once: the wait is free).
+            with torch.inference_mode(False):
+                one = torch.full((1,), value, dtype=x.dtype, device=x.device)
+            torch.cuda.current_stream(x.device).synchronize()
+            _CONSTANT_STATES[key] = one
+        return one.expand(shape)
+
     def materialize_states(self, inputs, states, step_mode: str):
-        x = inputs[0][0] if step_mode == "m" else inputs[0]
-        v = states[0]
+        x_seq, v = inputs[0], states[0]
+        if self._backend == "hip" and isinstance(x_seq, torch.Tensor) and x_seq.is_cuda and not torch.compiler.is_compiling():
+            # (without a view of the first step where nothing but its shape is needed)
+            shape = x_seq.shape[1:] if step_mode == "m" else x_seq.shape
+            if x_seq.numel() > 0 and shape.numel() > 1:
+                if isinstance(v, float):
+                    return (self._one_element_state(x_seq, v, shape), *states[1:])
+                if isinstance(v, torch.Tensor) and v.shape == shape and v.dtype == x_seq.dtype and v.device == x_seq.device:
+                    return states
+        x = x_seq[0] if step_mode == "m" else x_seq
         if isinstance(v, float):
             v = self._constant_state(x, v)
         elif isinstance(v, torch.Tensor):

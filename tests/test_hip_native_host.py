@@ -1,0 +1,144 @@
+"""The native host path (``csrc/torch_binding.cpp``) against the general Python path: same kernels, so the same bits, for the
+states, layouts and gradients where the two could part; and the calls it must leave to the general path."""
+
+import pytest
+import torch
+
+from spikingjelly_amd import configure
+from spikingjelly_amd.activation_based import functional, neuron, surrogate
+from spikingjelly_amd.activation_based.functional import neuron as F
+from spikingjelly_amd.activation_based.hip_kernel import native
+from spikingjelly_amd.activation_based.hip_kernel.surrogate_registry import resolve_sg_hip_id_and_alpha
+
+pytestmark = pytest.mark.gpu
+
+EXTRA = (0.0,) * 6
+
+
+def _both(monkeypatch, fn):
+    served = []
+    module = native.load()
+
+    class Spy:
+        def __getattr__(self, name):
+            def call(*a):
+                out = getattr(module, name)(*a)
+                served.append(out is not None)
+                return out
+
+            return call
+
+    monkeypatch.setattr(F, "_native", (Spy(), resolve_sg_hip_id_and_alpha))
+    got = fn()
+    monkeypatch.setattr(F, "_native_sequence", lambda *a, **k: None)
+    return got, fn(), served
+
+
+def _equal(a, b):
+    assert len(a) == len(b)
+    for x, y in zip(a, b):
+        assert (x is None) == (y is None) and (x is None or (x.dtype == y.dtype and x.shape == y.shape and torch.equal(x, y)))
+
+
+@pytest.mark.parametrize("shape", [(4, 8, 16, 1, 1), (3, 1, 40), (2, 5, 1), (1, 64)])
+@pytest.mark.parametrize("kind", ["if", "lif", "plif"])
+@pytest.mark.parametrize("state", ["fresh", "dense", "needs_grad"])
+def test_native_and_general_path_give_the_same_bits(kind, shape, state, monkeypatch):
+    g = torch.Generator().manual_seed(sum(shape))
+    x0 = (torch.randn(shape, generator=g) + 0.4).cuda()
+    gs = torch.randn(shape, generator=g).cuda()
+    v0 = (torch.randn(shape[1:], generator=g) * 0.2).cuda()
+    cls = {"if": neuron.IFNode, "lif": neuron.LIFNode, "plif": neuron.ParametricLIFNode}[kind]
+
+    def run():
+        node = cls(step_mode="m", backend="hip", surrogate_function=surrogate.ATan(), store_v_seq=True).cuda()
+        x = x0.clone().requires_grad_()
+        v = v0.clone().requires_grad_(state == "needs_grad")
+        if state != "fresh":
+            node.v = v
+        s = node(x)
+        (s * gs).sum().backward(retain_graph=True)
+        (node.v_seq.sum() + 2.0 * node.v.sum()).backward()  # a second backward through the same node: gradients add up
+        return [s.detach(), node.v.detach(), node.v_seq.detach(), x.grad, v.grad] + [p.grad for p in node.parameters()]
+
+    got, want, served = _both(monkeypatch, run)
+    N = x0.numel() // shape[0]
+    assert served == [N >= 4]  # shorter rows than a vector save h: the general path's business
+    _equal(got, want)
+
+
+def test_truncated_backpropagation_crosses_calls(monkeypatch):
+    x0 = (torch.randn(2, 3, 64, generator=torch.Generator().manual_seed(5)) + 0.4).cuda()
+
+    def run():
+        node = neuron.LIFNode(step_mode="m", backend="hip", surrogate_function=surrogate.ATan()).cuda()
+        x = x0.clone().requires_grad_()
+        first = node(x)
+        second = node(x * 0.5)  # its state is the first call's
+        (second.sum() + 0.1 * first.sum()).backward()
+        return [second.detach(), x.grad]
+
+    got, want, served = _both(monkeypatch, run)
+    assert served == [True, True]
+    _equal(got, want)
+
+
+def test_single_steps(monkeypatch):
+    x0 = (torch.randn(5, 7, 33, generator=torch.Generator().manual_seed(6)) + 0.4).cuda()
+
+    def run():
+        node = neuron.LIFNode(step_mode="s", backend="hip", surrogate_function=surrogate.ATan()).cuda()
+        x = x0.clone().requires_grad_()
+        out = torch.stack([node(x[t]) for t in range(5)])
+        (out * torch.arange(5, device="cuda").view(5, 1, 1)).sum().backward()
+        return [out.detach(), x.grad, node.v.detach()]
+
+    got, want, served = _both(monkeypatch, run)
+    assert served == [True] * 5
+    _equal(got, want)
+
+
+def test_what_the_native_path_leaves_alone(monkeypatch):
+    m = native.load()
+    call = lambda x, v, steps=39: m.neuron_sequence(x, v, None, False, 1, 2.0, 1.0, 0.0, 1, 1, 2.0, False, steps, EXTRA)
+    x = torch.randn(4, 64, device="cuda")
+    v = torch.zeros(64, device="cuda")
+    assert call(x, v) is not None
+    assert call(x.double(), v.double()) is None                          # a dtype without kernels: the general path raises
+    assert call(torch.randn(64, 4, device="cuda").t(), v) is None        # a layout that needs a copy
+    assert call(x, v[:32]) is None and call(x, v.half()) is None
+    assert call(x.cpu(), v.cpu()) is None
+    xg = x.clone().requires_grad_()
+    assert call(xg, v, steps=3) is None                                  # too long to replay in one piece
+    assert call(xg, v, steps=4) is not None
+    with torch.no_grad():
+        assert call(xg, v, steps=0) is not None                          # inference replays nothing
+    seen = []
+    torch.func.vmap(lambda t: (seen.append(call(t, v) is None), t)[1])(torch.randn(2, 4, 64, device="cuda"))
+    assert seen == [True]
+
+
+def test_saved_tensors_go_through_hooks_and_are_freed():
+    packed = []
+    x = torch.randn(4, 64, device="cuda").requires_grad_()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t.cpu())[1], lambda t: t.cuda()):
+        s, _, _ = functional.lif_multi_step_hip(x, torch.zeros(64, device="cuda"), 2.0, True, 1.0, 0.0, surrogate.ATan())
+    s.sum().backward()
+    assert torch.Size((4, 64)) in packed
+    with pytest.raises(RuntimeError, match="backward through the graph a second time"):
+        s.sum().backward()
+    x2 = torch.randn(4, 64, device="cuda").requires_grad_()
+    y = x2 * 1.0
+    s, _, _ = functional.lif_multi_step_hip(y, torch.zeros(64, device="cuda"), 2.0, True, 1.0, 0.0, surrogate.ATan())
+    y.add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        s.sum().backward()
+
+
+def test_packed_inference_equals_the_operator():
+    x = (torch.rand(6, 5, 16, device="cuda") * 0.6).half()
+    v = torch.zeros(5, 16, dtype=torch.float16, device="cuda")
+    bits, v1, v_seq = functional.if_multi_step_hip_packed(x, v, 1.0, None, True)
+    want = torch.ops.sj.hip_multistep_if_inference_packed(x.flatten(1), v.flatten(), 1.0, 0.0, True, True, F._hip_mode_flags(x))
+    assert torch.equal(bits, want[0]) and torch.equal(v_seq.flatten(1), want[1]) and torch.equal(v1.flatten(), want[2])
+    assert configure.hip_half_precision_mode == "torch"
