@@ -4,7 +4,7 @@ The block ``SeqToANNContainer(Conv1d(k=1, bias=False), BatchNorm1d) -> LIFNode``
 ``SpikingSelfAttention`` (layer/attention.py:310-329, 370-384) and, with ``Conv2d`` / ``BatchNorm2d``, in
 ``SpikformerConv2dBNLIF`` (model/spikformer.py:107-212); there torch runs the convolution (MIOpen / hipBLASLt, with
 layout transposes around them), batch norm and the neuron as separate operators.  Here, for fp32 ``[T, B, C, L]``
-tensors (``L`` the flattened positions, a multiple of 4):
+tensors (``L`` the flattened positions, at least 4 of them; what ``supported`` asks beyond that):
 
 * the convolution and its two gradients are GEMMs on the 16-bit matrix cores with the fp32 operands split into terms
   (``csrc/pwconv.hip``): two fp16 terms of power-of-two scaled operands (``configure.hip_conv_split = "f16"``, the
@@ -77,11 +77,17 @@ def _exact(terms: int) -> int:
     return (terms & F16) | 1
 
 
-def supported(x_seq: torch.Tensor, need_grad: bool) -> bool:
-    """fp32 device tensor ``[T, B, C, L]`` whose rows of ``L`` elements start on 16 bytes; at most ``MAX_REPLAY_STEPS`` steps when a
-    backward will follow."""
-    return (x_seq.is_cuda and x_seq.dtype == torch.float32 and x_seq.dim() == 4 and x_seq.shape[-1] % 4 == 0
-            and x_seq.numel() > 0 and (not need_grad or x_seq.shape[0] <= MAX_REPLAY_STEPS))
+def supported(x_seq: torch.Tensor, need_grad: bool, channels: Optional[int] = None) -> bool:
+    """fp32 device tensor ``[T, B, C, L]`` whose ``L`` is a multiple of 4 or, on the fp16 split (whose GEMM takes rows at any
+    4-byte address), at least 4 with samples of ``channels`` (default ``C``) rows a multiple of 4 elements long; at most
+    ``MAX_REPLAY_STEPS`` steps when a backward will follow."""
+    if not (x_seq.is_cuda and x_seq.dtype == torch.float32 and x_seq.dim() == 4 and x_seq.numel() > 0
+            and (not need_grad or x_seq.shape[0] <= MAX_REPLAY_STEPS)):
+        return False
+    Lp = x_seq.shape[-1]
+    if Lp % 4 == 0:
+        return True
+    return Lp >= 4 and (x_seq.shape[2] if channels is None else channels) * Lp % 4 == 0 and bool(_terms() & F16)
 
 
 def _stream(t: torch.Tensor) -> int:
@@ -708,12 +714,12 @@ def lif_conv_bn_lif(pre_seq: torch.Tensor, pre_v_init: torch.Tensor, weight: tor
 
 
 def lif_conv_bn_lif_supported(pre_seq: torch.Tensor, need_grad: bool) -> bool:
-    """What ``supported`` asks, the fp16 split of the GEMM operands (the kernels that read bits belong to it) and a
-    spike tensor whose samples start on a byte."""
+    """What ``supported`` asks, the fp16 split of the GEMM operands (the kernels that read bits belong to it), rows of a
+    multiple of 4 and a spike tensor whose samples start on a byte."""
     if not supported(pre_seq, need_grad) or not (_terms() & F16):
         return False
     T, B, Cin, Lp = pre_seq.shape
-    return (Cin * Lp) % 8 == 0
+    return Lp % 4 == 0 and (Cin * Lp) % 8 == 0
 
 
 def bn_lif(y_seq: torch.Tensor, gamma, beta, v_init: torch.Tensor, bn, spec, k: Optional[torch.Tensor] = None):

@@ -2,8 +2,8 @@
 
 ``Conv1d+BN -> LIF -> scale * (V K^T) Q -> LIF(v_threshold=0.5) -> Conv1d+BN -> LIF`` on ``[T, N, C, L]``
 input.  With ``backend='hip'`` the three LIF nodes run the HIP neuron kernels and the contraction runs on
-the matrix cores (int8 / bf16 MFMA, fp32 accumulation; exact because Q/K/V are binary).  For fp32 device tensors whose
-token count is a multiple of 4 the two ``Conv1d(k=1) -> BatchNorm1d -> LIF`` chains run fused as well (``layer/fused.py``:
+the matrix cores (int8 / bf16 MFMA, fp32 accumulation; exact because Q/K/V are binary).  For fp32 device tensors of
+at least four tokens the two ``Conv1d(k=1) -> BatchNorm1d -> LIF`` chains run fused as well (``layer/fused.py``:
 split-bf16 MFMA GEMMs, batch norm and the neuron in two passes over the convolution output); other inputs keep
 torch's convolution and batch norm around the hip neurons.
 """

@@ -130,7 +130,7 @@ def conv_bn_lif(x_seq: torch.Tensor, conv: Optional[nn.Module], bn: nn.Module, n
               if p is not None)
     need_grad = torch.is_grad_enabled() and (x_seq.requires_grad or any(p.requires_grad for p in params))
     x4 = x_seq.flatten(3)  # [T, B, C, L]
-    if not C.supported(x4, need_grad):
+    if not C.supported(x4, need_grad, channels):
         return None
     T, B, _, Lp = x4.shape
     if ssa is not None:

@@ -14,6 +14,10 @@
 //   leaves sum g and sum g y of its row.  bn_backward_finalize_kernel turns those into dgamma, dbeta and the three
 //   per-channel coefficients of  dy = p_c g + q_c y + r_c,  which bn_grad_input_kernel applies (in place over g).
 // Arithmetic of the neuron is neuron_step / surrogate_grad of the plain neuron kernels.
+// Rows of any length L >= 4 (with C * L a multiple of 4, so that every step starts on 16 bytes): a kernel that owns rows
+// gives the last work-item of a row that 4 does not divide the row's last four elements, the first of which its
+// neighbour has too (stored twice with the same bits, summed once); a kernel over the flat tensor keeps its aligned
+// groups of four and looks up both channels where a group runs over the end of a row.
 #include "neuron_bwd.h"
 #include "neuron_fwd.h"
 
@@ -55,7 +59,7 @@ __device__ __forceinline__ double wave_sum_all(double v) {
 // (consecutive work-items, consecutive rows): per wavefront one masked reduction per row it touches, the results left
 // in LDS, then one work-item per row adds the wavefronts' shares in their order and writes (sum0, sum1) of row
 // first_row + r to out[2 (first_row + r)].  Every work-item of the block must call it.
-constexpr int kBnRowsMax = 16;  // rows per block: rows of at least 16 quads
+constexpr int kBnRowsMax = 32;  // rows per block: rows of at least 8 quads
 __device__ __forceinline__ void block_row_sums(float (&part)[4][kBnRowsMax][2], int r_local, bool valid, int rows_per_block,
                                                float v0, float v1, float *out, int64_t first_row, int64_t rows) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -77,6 +81,27 @@ __device__ __forceinline__ void block_row_sums(float (&part)[4][kBnRowsMax][2], 
   }
 }
 
+// The group of four of a row of L >= 4 elements that begins at 4 q, moved back into the row: `first` is its first element,
+// and elements j < skip of it belong to the group before.
+struct RowQuad {
+  int first, skip;
+  __device__ __forceinline__ RowQuad(int q, int L) : first(min(4 * q, L - 4)), skip(4 * q - min(4 * q, L - 4)) {}
+};
+__device__ __forceinline__ f32x4 load_row_quad(const float *row, int q, int L) {
+  const RowQuad quad(q, L);
+  f32x4 v = *reinterpret_cast<const f32x4_any *>(row + quad.first);
+  if (quad.skip > 0) v.x = 0.0f;
+  if (quad.skip > 1) v.y = 0.0f;
+  if (quad.skip > 2) v.z = 0.0f;
+  return v;
+}
+// The channel of element j of an aligned group of four of the flat tensor, which starts at position l of channel c's row
+struct QuadChannels {
+  int c, next, left;
+  __device__ __forceinline__ QuadChannels(int c_, int l, int C, int L) : c(c_), next(c_ + 1 == C ? 0 : c_ + 1), left(L - l) {}
+  __device__ __forceinline__ int operator[](int j) const { return j < left ? c : next; }
+};
+
 // one wavefront per row of L contiguous elements: sum and sum of squares.  A wavefront takes kBnStatRows rows in a
 // row of at most 256 elements and has their loads all in flight before the first sum (37 -> 31 us on
 // [256, 1152, 196]); several whole rows per block with the row sums through LDS, as in bn_lif_backward_rows_kernel,
@@ -86,13 +111,13 @@ __global__ void __launch_bounds__(256) bn_stats_kernel(const float *y, int64_t r
   const int lane = threadIdx.x & 63;
   const int64_t row0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * kBnStatRows;
   if (row0 >= rows) return;
-  const int quads = L / 4;
+  const int quads = (L + 3) / 4;
   if (quads <= 64) {
     f32x4 v[kBnStatRows];
 #pragma unroll
     for (int r = 0; r < kBnStatRows; ++r) {
       const bool ok = row0 + r < rows && lane < quads;
-      v[r] = ok ? reinterpret_cast<const f32x4 *>(y + (row0 + r) * L)[lane] : (f32x4)(0.0f);
+      v[r] = ok ? load_row_quad(y + (row0 + r) * L, lane, L) : (f32x4)(0.0f);
     }
 #pragma unroll
     for (int r = 0; r < kBnStatRows; ++r) {
@@ -106,10 +131,10 @@ __global__ void __launch_bounds__(256) bn_stats_kernel(const float *y, int64_t r
     return;
   }
   for (int r = 0; r < kBnStatRows && row0 + r < rows; ++r) {
-    const f32x4 *p = reinterpret_cast<const f32x4 *>(y + (row0 + r) * L);
+    const float *p = y + (row0 + r) * L;
     float s = 0.0f, q = 0.0f;
     for (int i = lane; i < quads; i += 64) {
-      const f32x4 v = p[i];
+      const f32x4 v = load_row_quad(p, i, L);
       s += (v.x + v.y) + (v.z + v.w);
       q = fmaf(v.x, v.x, q); q = fmaf(v.y, v.y, q); q = fmaf(v.z, v.z, q); q = fmaf(v.w, v.w, q);
     }
@@ -159,7 +184,7 @@ __global__ void __launch_bounds__(256) bn_finalize_kernel(const float *partial, 
   invstd_out[c] = (float)invstd;
 }
 
-template <int CH, int RS, bool PACKED>
+template <int CH, int RS, bool PACKED, bool RAGGED>
 __device__ __forceinline__ void bn_lif_forward_body(const BnLifFwdArgs &a) {
   typedef Acc<float, true, false> A;
   const FwdArgs &f = a.f;
@@ -168,8 +193,15 @@ __device__ __forceinline__ void bn_lif_forward_body(const BnLifFwdArgs &a) {
   if (col >= N) return;
   // (32-bit quotients where the tensor allows it: a 64-bit integer division is some hundred instructions, as many as
   // the four steps of a short sequence)
-  const int c = N <= 0x7fffffffLL ? (int)(((uint32_t)col / (uint32_t)a.L) % (uint32_t)a.C) : (int)((col / a.L) % a.C);
-  const float sc = a.scale[c], sh = a.shift[c];
+  const int64_t row = N <= 0x7fffffffLL ? (int64_t)((uint32_t)col / (uint32_t)a.L) : col / a.L;
+  const int c = N <= 0x7fffffffLL ? (int)((uint32_t)row % (uint32_t)a.C) : (int)(row % a.C);
+  const QuadChannels ch(c, RAGGED ? (int)(col - row * a.L) : 0, a.C, a.L);
+  float sc[4], sh[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    sc[j] = (RAGGED || j == 0) ? a.scale[RAGGED ? ch[j] : c] : sc[0];
+    sh[j] = (RAGGED || j == 0) ? a.shift[RAGGED ? ch[j] : c] : sh[0];
+  }
   const float tau = f.k_device ? *f.k_device : f.tau;  // PLIF: k = sigmoid(w), read where torch left it
   const float *yp = (const float *)f.x + col;
   float *sp = (float *)f.spike + col;
@@ -187,7 +219,7 @@ __device__ __forceinline__ void bn_lif_forward_body(const BnLifFwdArgs &a) {
         float y[4], h[4], s[4];
         A::unpack(rows[i], y);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) neuron_step<float, CH, RS>(fmaf(y[j], sc, sh), v[j], h[j], s[j], tau, f);
+        for (int j = 0; j < 4; ++j) neuron_step<float, CH, RS>(fmaf(y[j], sc[j], sh[j]), v[j], h[j], s[j], tau, f);
         if (PACKED) store_spike_bits<4>((uint8_t *)f.spike + t * (N >> 3), col, N, s);
         else A::store(sp + t * N, s);
       }
@@ -196,18 +228,18 @@ __device__ __forceinline__ void bn_lif_forward_body(const BnLifFwdArgs &a) {
   if (f.v_last) A::store((float *)f.v_last + col, v);
 }
 
-template <int CH, bool PACKED> __device__ __forceinline__ void bn_lif_forward_reset(const BnLifFwdArgs &a) {
-  if (a.f.soft_reset) bn_lif_forward_body<CH, RESET_SOFT, PACKED>(a);
-  else bn_lif_forward_body<CH, RESET_HARD, PACKED>(a);
+template <int CH, bool PACKED, bool RAGGED> __device__ __forceinline__ void bn_lif_forward_reset(const BnLifFwdArgs &a) {
+  if (a.f.soft_reset) bn_lif_forward_body<CH, RESET_SOFT, PACKED, RAGGED>(a);
+  else bn_lif_forward_body<CH, RESET_HARD, PACKED, RAGGED>(a);
 }
 
-template <bool PACKED> __global__ void __launch_bounds__(256) bn_lif_forward_kernel(const BnLifFwdArgs a) {
+template <bool PACKED, bool RAGGED> __global__ void __launch_bounds__(256) bn_lif_forward_kernel(const BnLifFwdArgs a) {
   switch (a.f.charge) {
-    case CH_IF: bn_lif_forward_reset<CH_IF, PACKED>(a); break;
-    case CH_DECAY_INPUT_DIV: bn_lif_forward_reset<CH_DECAY_INPUT_DIV, PACKED>(a); break;
-    case CH_DECAY_INPUT_MUL: bn_lif_forward_reset<CH_DECAY_INPUT_MUL, PACKED>(a); break;
-    case CH_PLAIN_INPUT_DIV: bn_lif_forward_reset<CH_PLAIN_INPUT_DIV, PACKED>(a); break;
-    default: bn_lif_forward_reset<CH_PLAIN_INPUT_MUL, PACKED>(a); break;
+    case CH_IF: bn_lif_forward_reset<CH_IF, PACKED, RAGGED>(a); break;
+    case CH_DECAY_INPUT_DIV: bn_lif_forward_reset<CH_DECAY_INPUT_DIV, PACKED, RAGGED>(a); break;
+    case CH_DECAY_INPUT_MUL: bn_lif_forward_reset<CH_DECAY_INPUT_MUL, PACKED, RAGGED>(a); break;
+    case CH_PLAIN_INPUT_DIV: bn_lif_forward_reset<CH_PLAIN_INPUT_DIV, PACKED, RAGGED>(a); break;
+    default: bn_lif_forward_reset<CH_PLAIN_INPUT_MUL, PACKED, RAGGED>(a); break;
   }
 }
 
@@ -247,14 +279,14 @@ __device__ __forceinline__ void replay_h_charge(const FwdArgs &f, int len, const
   }
 }
 
-// BPTT over the replayed h (recurrence of neuron_bwd.h); writes g = dL/dz and adds this work-item's share of
-// sum g and sum g y.  PLIF: also of dL/dk = sum G_t dh_t/dk, dh_t/dk = (h_t - v_{t-1}) / k with input decay (the division
+// BPTT over the replayed h (recurrence of neuron_bwd.h); writes g = dL/dz and adds every neuron's share of
+// sum g and sum g y (four sums, because a neuron that a neighbour has too is counted once).  PLIF: also of dL/dk = sum G_t dh_t/dk, dh_t/dk = (h_t - v_{t-1}) / k with input decay (the division
 // is left to the final reduction) or v_reset - v_{t-1} without; v_{t-1} is re-derived from h_{t-1} with the forward's
 // reset arithmetic, v0 is the state in front of the first of these steps.
 template <int SG, int TMAX, bool PLIF>
 __device__ __forceinline__ void bptt_rows(const BwdArgs &b, float k, int64_t col, int64_t t0, int len, const f32x4 (&yv)[TMAX],
-                                          const float (&h)[TMAX][4], const float (&v0)[4], float (&carry)[4], float &acc_g,
-                                          float &acc_gy, float &acc_k) {
+                                          const float (&h)[TMAX][4], const float (&v0)[4], float (&carry)[4], float (&acc_g)[4],
+                                          float (&acc_gy)[4], float (&acc_k)[4]) {
 #pragma clang fp contract(fast)
   typedef Acc<float, true, true> A;
   const int64_t N = b.N;
@@ -277,15 +309,15 @@ __device__ __forceinline__ void bptt_rows(const BwdArgs &b, float k, int64_t col
         const float G = carry[j] * dvdh + gs[j] * sg;
         gz[j] = G * kx;
         carry[j] = G * km;
-        acc_g += gz[j];
-        acc_gy = fmaf(gz[j], y[j], acc_gy);
+        acc_g[j] += gz[j];
+        acc_gy[j] = fmaf(gz[j], y[j], acc_gy[j]);
         if constexpr (PLIF) {
           float v_prev = v0[j];
           if (t > 0) {
             const float h_prev = h[t > 0 ? t - 1 : 0][j];
             v_prev = reset_as_forward(h_prev, (h_prev - b.v_th >= 0.0f) ? 1.0f : 0.0f, b);
           }
-          acc_k = fmaf(G, b.decay_input ? (h[t][j] - v_prev) : (b.v_reset - v_prev), acc_k);
+          acc_k[j] = fmaf(G, b.decay_input ? (h[t][j] - v_prev) : (b.v_reset - v_prev), acc_k[j]);
         }
       }
       Acc<float, true, false>::store(gxp + (int64_t)t * N, gz);  // read again by the next kernel
@@ -296,7 +328,7 @@ __device__ __forceinline__ void bptt_rows(const BwdArgs &b, float k, int64_t col
 template <int TMAX, bool PLIF>
 __device__ __forceinline__ void bptt_rows_surrogate(const BwdArgs &b, float k, int64_t col, int64_t t0, int len,
                                                     const f32x4 (&yv)[TMAX], const float (&h)[TMAX][4], const float (&v0)[4],
-                                                    float (&carry)[4], float &acc_g, float &acc_gy, float &acc_k) {
+                                                    float (&carry)[4], float (&acc_g)[4], float (&acc_gy)[4], float (&acc_k)[4]) {
   switch (b.sg) {
     case SJHIP_SG_SIGMOID: bptt_rows<SJHIP_SG_SIGMOID, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
     case SJHIP_SG_ATAN: bptt_rows<SJHIP_SG_ATAN, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
@@ -306,6 +338,12 @@ __device__ __forceinline__ void bptt_rows_surrogate(const BwdArgs &b, float k, i
     case SJHIP_SG_SUPER_SPIKE: bptt_rows<SJHIP_SG_SUPER_SPIKE, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
     default: bptt_rows<SJHIP_SG_ERF, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
   }
+}
+
+// the shares of the neurons from `skip` on, added to the work-item's sums
+__device__ __forceinline__ void fold_shares(const float (&share)[4], int skip, float &sum) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sum += j >= skip ? share[j] : 0.0f;
 }
 
 // One work-item's four neurons (quad q of row `row`) for all T steps: replay, BPTT, g written, the sums extended.
@@ -319,7 +357,8 @@ __device__ __forceinline__ void bn_lif_backward_quad(const BnLifBwdArgs &a, int6
   const float sc = a.scale[c], sh = a.shift[c];
   const float k = (PLIF && b.k_device) ? *b.k_device : b.k;
   const int64_t N = f.N;
-  const int64_t col = row * a.L + 4 * q;
+  const RowQuad quad(q, a.L);
+  const int64_t col = row * a.L + quad.first;
   const float *yp = (const float *)f.x + col;
   f32x4 yv[TMAX];
 #pragma unroll
@@ -330,7 +369,11 @@ __device__ __forceinline__ void bn_lif_backward_quad(const BnLifBwdArgs &a, int6
   if (b.grad_v_last) A::unpack(A::load((const float *)b.grad_v_last + col), carry);
   else carry[0] = carry[1] = carry[2] = carry[3] = 0.0f;
   replay_h_charge<TMAX>(f, (int)f.T, yv, sc, sh, v, h);
-  bptt_rows_surrogate<TMAX, PLIF>(b, k, col, 0, (int)b.T, yv, h, v0, carry, acc_g, acc_gy, acc_k);
+  float g[4] = {}, gy[4] = {}, gk[4] = {};
+  bptt_rows_surrogate<TMAX, PLIF>(b, k, col, 0, (int)b.T, yv, h, v0, carry, g, gy, gk);
+  fold_shares(g, quad.skip, acc_g);
+  fold_shares(gy, quad.skip, acc_gy);
+  if (PLIF) fold_shares(gk, quad.skip, acc_k);
   if (b.grad_v_init) A::store((float *)b.grad_v_init + col, carry);
 }
 
@@ -349,7 +392,8 @@ __device__ __forceinline__ void bn_lif_backward_quad_long(const BnLifBwdArgs &a,
   const int c = (int)(row % a.C);
   const float sc = a.scale[c], sh = a.shift[c];
   const int64_t N = f.N;
-  const int64_t col = row * a.L + 4 * q;
+  const RowQuad quad(q, a.L);
+  const int64_t col = row * a.L + quad.first;
   const float *yp = (const float *)f.x + col;
   const int T = (int)f.T, pieces = (T + kBnPiece - 1) / kBnPiece;
   f32x4 yv[kBnPiece];
@@ -364,6 +408,7 @@ __device__ __forceinline__ void bn_lif_backward_quad_long(const BnLifBwdArgs &a,
   parked[(pieces - 1) * blockDim.x] = f32x4{v[0], v[1], v[2], v[3]};
   if (b.grad_v_last) A::unpack(A::load((const float *)b.grad_v_last + col), carry);
   else carry[0] = carry[1] = carry[2] = carry[3] = 0.0f;
+  float g[4] = {}, gy[4] = {}, gk[4] = {};
   for (int p = pieces - 1; p >= 0; --p) {
     const int t0 = p * kBnPiece, len = min(kBnPiece, T - t0);
 #pragma unroll
@@ -372,9 +417,11 @@ __device__ __forceinline__ void bn_lif_backward_quad_long(const BnLifBwdArgs &a,
     v[0] = s.x; v[1] = s.y; v[2] = s.z; v[3] = s.w;
     const float v0[4] = {s.x, s.y, s.z, s.w};
     replay_h_charge<kBnPiece>(f, len, yv, sc, sh, v, h);
-    bptt_rows_surrogate<kBnPiece, PLIF>(b, (PLIF && b.k_device) ? *b.k_device : b.k, col, t0, len, yv, h, v0, carry, acc_g,
-                                        acc_gy, acc_k);
+    bptt_rows_surrogate<kBnPiece, PLIF>(b, (PLIF && b.k_device) ? *b.k_device : b.k, col, t0, len, yv, h, v0, carry, g, gy, gk);
   }
+  fold_shares(g, quad.skip, acc_g);
+  fold_shares(gy, quad.skip, acc_gy);
+  if (PLIF) fold_shares(gk, quad.skip, acc_k);
   if (b.grad_v_init) A::store((float *)b.grad_v_init + col, carry);
 }
 
@@ -391,7 +438,7 @@ template <int TMAX, bool PLIF> __global__ void __launch_bounds__(256) bn_lif_bac
     return;
   }
   float acc_g = 0.0f, acc_gy = 0.0f, acc_k = 0.0f;
-  for (int q = lane; q < a.L / 4; q += 64) {
+  for (int q = lane; q < (a.L + 3) / 4; q += 64) {
     if constexpr (TMAX == 0) bn_lif_backward_quad_long<PLIF>(a, row, q, acc_g, acc_gy, acc_k, parked_states + threadIdx.x);
     else bn_lif_backward_quad<TMAX, PLIF>(a, row, q, acc_g, acc_gy, acc_k);
   }
@@ -474,31 +521,41 @@ __device__ __forceinline__ float finite_abs(float x) {
 // (they order like unsigned integers, and a maximum does not depend on the order it is taken in), with an atomic whose
 // result is not used, so that the block does not wait for it; and every wavefront the largest |dy| of its sample into
 // that sample's word, which follow the tensor's (one atomic when its lanes share a sample, else one per lane).
-template <bool AMAX>
+template <bool AMAX, bool RAGGED>
 __global__ void __launch_bounds__(256) bn_grad_input_kernel(const float *g, const float *y, const float *coef, int64_t S, int C,
                                                              int L, int64_t n, float *dy, unsigned *amax_bits) {
   const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   float amax = 0.0f;
   int sample = -1;
   if (i < n) {
-    int c;  // i = ((sample * C) + channel) * L + position
+    int c, l;  // i = ((sample * C) + channel) * L + position; a sample is a multiple of 4 elements
     if (n <= 0x7fffffffLL) {
       const uint32_t row = (uint32_t)i / (uint32_t)L, smp = row / (uint32_t)C;
       c = (int)(row - smp * (uint32_t)C);
       sample = (int)smp;
+      l = (int)((uint32_t)i - row * (uint32_t)L);
     } else {
       const int64_t row = i / L, smp = row / C;
       c = (int)(row - smp * C);
       sample = (int)smp;
+      l = (int)(i - row * L);
     }
-    const float p = coef[c], q = coef[C + c], r = coef[2 * C + c];
+    const QuadChannels ch(c, RAGGED ? l : 0, C, L);
+    float p[4], q[4], r[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int cj = RAGGED ? ch[j] : c;
+      p[j] = (RAGGED || j == 0) ? coef[cj] : p[0];
+      q[j] = (RAGGED || j == 0) ? coef[C + cj] : q[0];
+      r[j] = (RAGGED || j == 0) ? coef[2 * C + cj] : r[0];
+    }
     const f32x4 gv = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(g + i));
     const f32x4 yv = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(y + i));
     f32x4 o;
-    o.x = fmaf(p, gv.x, fmaf(q, yv.x, r));
-    o.y = fmaf(p, gv.y, fmaf(q, yv.y, r));
-    o.z = fmaf(p, gv.z, fmaf(q, yv.z, r));
-    o.w = fmaf(p, gv.w, fmaf(q, yv.w, r));
+    o.x = fmaf(p[0], gv.x, fmaf(q[0], yv.x, r[0]));
+    o.y = fmaf(p[1], gv.y, fmaf(q[1], yv.y, r[1]));
+    o.z = fmaf(p[2], gv.z, fmaf(q[2], yv.z, r[2]));
+    o.w = fmaf(p[3], gv.w, fmaf(q[3], yv.w, r[3]));
     *reinterpret_cast<f32x4 *>(dy + i) = o;
     if (AMAX) amax = fmaxf(fmaxf(finite_abs(o.x), finite_abs(o.y)), fmaxf(finite_abs(o.z), finite_abs(o.w)));
   }
@@ -542,7 +599,8 @@ __global__ void __launch_bounds__(256) bn_grad_input_kernel(const float *g, cons
 
 int check_layout(const char *what, int64_t T, int64_t B, int64_t C, int64_t L) {
   if (T < 1 || B < 1 || C < 1 || L < 1) return fail(SJHIP_ERR_INVALID, "%s: T=%lld B=%lld C=%lld L=%lld must be >= 1", what, (long long)T, (long long)B, (long long)C, (long long)L);
-  if (L % 4 != 0) return fail(SJHIP_ERR_UNSUPPORTED, "%s: L=%lld must be a multiple of 4", what, (long long)L);
+  if (L % 4 != 0 && (L < 4 || C > (1 << 24) || L > (1 << 24) || C * L % 4 != 0))
+    return fail(SJHIP_ERR_UNSUPPORTED, "%s: L=%lld must be a multiple of 4, or at least 4 with C*L a multiple of 4 (C=%lld)", what, (long long)L, (long long)C);
   if (C > (1 << 24) || L > (1 << 24) || B * C > (int64_t(1) << 40) || T > (int64_t(1) << 40) / (B * C * L))
     return fail(SJHIP_ERR_TOO_LARGE, "%s: T=%lld B=%lld C=%lld L=%lld", what, (long long)T, (long long)B, (long long)C, (long long)L);
   return SJHIP_OK;
@@ -596,8 +654,11 @@ int launch_bn_lif_forward(int neuron, const sjhip_neuron_params &p, int64_t T, i
   const int64_t blocks = (N / 4 + 255) / 256;
   if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "bn_lif_forward: N=%lld", (long long)N);
   ProfileScope prof(KC_BN_LIF_FORWARD, stream);
-  if (spike_bits) hipLaunchKernelGGL((bn_lif_forward_kernel<true>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
-  else hipLaunchKernelGGL((bn_lif_forward_kernel<false>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  auto launch = [&](auto packed, auto ragged) {
+    hipLaunchKernelGGL((bn_lif_forward_kernel<decltype(packed)::value, decltype(ragged)::value>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  };
+  if (L % 4 != 0) spike_bits ? launch(std::true_type(), std::true_type()) : launch(std::false_type(), std::true_type());
+  else spike_bits ? launch(std::true_type(), std::false_type()) : launch(std::false_type(), std::false_type());
   return check_launch("bn_lif_forward");
 }
 
@@ -638,7 +699,7 @@ int launch_bn_lif_backward(int neuron, const sjhip_neuron_params &p, int64_t T, 
   ProfileScope prof(KC_BN_LIF_BACKWARD, stream);
   // (the walk in pieces parks one state per piece and work-item in LDS: at most 64 KiB, no opt-in needed)
   const unsigned parked = T > kBnPiece ? (unsigned)((T + kBnPiece - 1) / kBnPiece) * 256u * 16u : 0u;
-  const int quads = (int)(L / 4);
+  const int quads = (int)((L + 3) / 4);
   const int per = quads > 0 ? 256 / quads : 0;
   // TMAX by sequence length (0: the walk in pieces), with or without the dL/dk term
   auto launch = [&](auto rows_kernel, auto plif_flag) {
@@ -660,7 +721,7 @@ int launch_bn_lif_backward(int neuron, const sjhip_neuron_params &p, int64_t T, 
     return nb;
   };
   // more than the four rows a block of the wavefront-per-row kernel takes: more lanes working
-  const bool by_rows = quads >= 16 && per > 4;
+  const bool by_rows = per > 4 && per <= kBnRowsMax;
   if (by_rows && (a.rows + per - 1) / per > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "bn_lif_backward: %lld rows", (long long)a.rows);
   int64_t nb;
   if (by_rows) nb = plif ? launch(std::true_type(), std::true_type()) : launch(std::true_type(), std::false_type());
@@ -688,12 +749,12 @@ int launch_bn_grad_input(const float *g, const float *y, const float *coef, int6
   const int64_t n = S * C * L, blocks = (n / 4 + 255) / 256;
   if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "bn_grad_input: %lld elements", (long long)n);
   ProfileScope prof(KC_BN_GRAD_INPUT, stream);
-  if (amax)
-    hipLaunchKernelGGL(bn_grad_input_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, stream, g, y, coef, S, (int)C, (int)L, n, dy,
-                       reinterpret_cast<unsigned *>(amax));
-  else
-    hipLaunchKernelGGL(bn_grad_input_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, stream, g, y, coef, S, (int)C, (int)L, n, dy,
-                       (unsigned *)nullptr);
+  auto launch = [&](auto with_amax, auto ragged) {
+    hipLaunchKernelGGL((bn_grad_input_kernel<decltype(with_amax)::value, decltype(ragged)::value>), dim3((unsigned)blocks), dim3(256), 0,
+                       stream, g, y, coef, S, (int)C, (int)L, n, dy, reinterpret_cast<unsigned *>(amax));
+  };
+  if (L % 4 != 0) amax ? launch(std::true_type(), std::true_type()) : launch(std::false_type(), std::true_type());
+  else amax ? launch(std::true_type(), std::false_type()) : launch(std::false_type(), std::false_type());
   return check_launch("bn_grad_input");
 }
 

@@ -342,8 +342,10 @@ struct PwGemmArgs {
   const float *b;            // [S][K][L]
   float *c;                  // [S][M][L]
   int64_t plane_stride;      // M_pad * K_pad
-  int64_t ncols;             // S * L
+  int64_t ncols;             // S * Lq
   int M, K, K_pad, L;
+  int Lq;                    // columns per sample of the column index: L rounded up to four (column_pitch), the rest hold zeros;
+                             // kBPlanes: L
   int m_blocks;
   float *stats;              // nullptr, or [2 x column blocks][M][2]: per row of c the sum and the sum of squares over
                              // each half (64 columns) of every column block
@@ -359,6 +361,16 @@ struct PwGemmArgs {
 #ifndef SJHIP_PW_WIDE_OUT
 #define SJHIP_PW_WIDE_OUT 1
 #endif
+typedef u32x4 u32x4_any __attribute__((aligned(4)));
+// the elements skip .. 3 of v at the places 0 .. 3 - skip, zeros behind them
+template <typename V> __device__ __forceinline__ V moved_down(V v, int skip) {
+  V r;
+  r.x = skip == 0 ? v.x : (skip == 1 ? v.y : (skip == 2 ? v.z : v.w));
+  r.y = skip == 0 ? v.y : (skip == 1 ? v.z : (skip == 2 ? v.w : 0));
+  r.z = skip == 0 ? v.z : (skip == 1 ? v.w : 0);
+  r.w = skip == 0 ? v.w : 0;
+  return r;
+}
 constexpr int kOutPitch = 68;                              // floats per row of the output staging buffer (64 columns + 4)
 constexpr unsigned kOutLds = 4 * 32 * kOutPitch * 4;       // 32 rows x 64 columns per wavefront
 constexpr int kStatPitch = 33;                             // floats per row of the transposing buffer: no bank conflicts
@@ -421,7 +433,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   const int64_t nb = logical / a.m_blocks;
   const int m0 = mb * kTile;
   const int64_t j0 = nb * kTile;
-  const int M = a.M, K = a.K, L = a.L;
+  const int M = a.M, K = a.K, L = a.L, Lq = a.Lq;
   const int K_pad = a.K_pad;
 
   // Addresses are a wavefront-uniform 64-bit base (scalar registers) plus a 32-bit per-lane byte offset, and every load
@@ -442,13 +454,11 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   const int bc = 2 * (tid & 63);
   const int bk = __builtin_amdgcn_readfirstlane(wave * 8);
   const int64_t jc = j0 + bc;
-  const bool col_ok = jc < a.ncols;  // L is even, so the two columns are in one sample and both valid or both not
+  const int64_t sc = jc / Lq;
+  const bool col_ok = jc < a.ncols && jc - sc * Lq < L;  // L is even, so the two columns are in one sample and both valid or both not
   uint32_t b_off = 0;  // byte offset of the column pair in row 0 of its sample; with BITS the bit index
-  if (col_ok) {
-    const int64_t s = jc / L;
-    b_off = (uint32_t)(((s * K) * (int64_t)L + (jc - s * L)) * (BITS ? 1 : 4));
-  }
-  const bool edge_cols = __builtin_amdgcn_readfirstlane(j0 + kTile > a.ncols ? 1 : 0) != 0;
+  if (col_ok) b_off = (uint32_t)(((sc * K) * (int64_t)L + (jc - sc * Lq)) * (BITS ? 1 : 4));
+  const bool edge_cols = __builtin_amdgcn_readfirstlane((j0 + kTile > a.ncols || L != Lq) ? 1 : 0) != 0;
   const char *a_base = reinterpret_cast<const char *>(a.a_planes);
   const char *b_base = reinterpret_cast<const char *>(a.b);
   // The scale of b: a sample's own power of two when b is split here (a work-item stages columns of one sample), the
@@ -458,8 +468,8 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   if (H && TB > 1 && !SAMPLE_SCALE && a.b_amax != nullptr) scale_for(tensor_amax(a.b_amax), b_scale, b_inverse);
   // A tile of 128 columns lies in at most two samples when a sample has that many positions: their two maxima are
   // fetched once per block from addresses that do not depend on the lane; shorter samples are looked up per column.
-  const bool two_samples = L >= kTile;
-  const int64_t tile_sample = j0 / L, next_sample_col = (tile_sample + 1) * L;
+  const bool two_samples = Lq >= kTile;
+  const int64_t tile_sample = j0 / Lq, next_sample_col = (tile_sample + 1) * Lq;
   float tile_amax[2] = {0.0f, 0.0f};
   if (SAMPLE_SCALE && a.b_amax_samples != nullptr && two_samples) {
     const int64_t s_a = a.amax_s0 + tile_sample, s_b = s_a + 1 < a.amax_S ? s_a + 1 : s_a;
@@ -467,7 +477,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
     tile_amax[1] = sample_amax(a.b_amax_samples, s_b);
   }
   auto column_amax = [&](int64_t j) {
-    return two_samples ? (j < next_sample_col ? tile_amax[0] : tile_amax[1]) : sample_amax(a.b_amax_samples, a.amax_s0 + j / L);
+    return two_samples ? (j < next_sample_col ? tile_amax[0] : tile_amax[1]) : sample_amax(a.b_amax_samples, a.amax_s0 + j / Lq);
   };
   if (SAMPLE_SCALE && a.b_amax_samples != nullptr && col_ok) scale_for(column_amax(jc), b_scale, b_inverse);
   // planes: 16-byte chunk pc (eight columns) of the k rows pr and pr + 16 of every plane
@@ -705,8 +715,9 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
     for (int nt = 0; nt < 2; ++nt) {
       const int64_t j = j0 + wn * 64 + nt * 32 + (lane & 31);
       if (j >= a.ncols) continue;
-      const int64_t s = j / L;
-      const int l = (int)(j - s * L);
+      const int64_t s = j / Lq;
+      const int l = (int)(j - s * Lq);
+      if (l >= L) continue;
       float *cp = a.c + (s * M) * (int64_t)L + l;
   #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
@@ -760,12 +771,15 @@ constexpr unsigned rows_inverse_offset(int tb) { return 2u * tb * kRowPlane > kO
 //   * a wavefront owns 32 rows of the tile and all 128 columns, and fetches its A fragments straight from the weight
 //     planes (the 16 bytes a lane needs are contiguous in the tile-ordered planes): A never passes through LDS and no two
 //     wavefronts fetch the same fragment;
-//   * B is fetched as 16-byte pieces of a k row (four positions of one sample; L is a multiple of 4), half the load
+//   * B is fetched as 16-byte pieces of a k row (four positions of one sample), half the load
 //     instructions, split, and stored as it lies in memory (k rows of 128 columns); the wavefronts fetch their
 //     fragments with the transposing LDS read, as pw_gemm_kernel does for term planes;
 //   * two B tiles alternate in LDS, so a K step has one barrier.
 // Per K step of a block: 16 KB written to and 64 KB read from LDS, 16 + 16 load instructions; 146 registers, three
 // wavefronts per SIMD.
+// Samples of any length L >= 4: the column index gives every sample Lq = L rounded up to four columns, so that a piece
+// lies in one sample; a piece that runs over the end of its row is fetched as the row's last four elements (at any
+// 4-byte address) and moved down by one to three places with zeros behind it.
 template <int TB>
 __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu(3, 3))) pw_gemm_rows_kernel(const PwGemmArgs a) {
   constexpr int TA = 2;
@@ -776,7 +790,8 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   const int mb = (int)(logical % a.m_blocks);
   const int64_t nb = logical / a.m_blocks;
   const int64_t j0 = nb * kTile;
-  const int M = a.M, K = a.K, L = a.L;
+  const int M = a.M, K = a.K, L = a.L, Lq = a.Lq;
+  const bool ragged = L != Lq;
   const int steps = a.K_pad / kTileK;
 
   // the inverse row scales of the tile wait in LDS (beyond the operand tiles) for the epilogue
@@ -791,9 +806,12 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   const int64_t jc = j0 + 4 * q4;
   const bool col_ok = jc < a.ncols;
   uint32_t b_off = 0;
+  int b_skip = 0;  // places that the piece is moved down
   if (col_ok) {
-    const int64_t s = jc / L;
-    b_off = (uint32_t)(((s * K) * (int64_t)L + (jc - s * L)) * 4);
+    const int64_t s = jc / Lq;
+    const int l = (int)(jc - s * Lq), first = min(l, L - 4);
+    b_off = (uint32_t)(((s * K) * (int64_t)L + first) * 4);
+    b_skip = l - first;
   }
   const uint32_t row_bytes = (uint32_t)L * 4u;
   const bool edge_cols = __builtin_amdgcn_readfirstlane(j0 + kTile > a.ncols ? 1 : 0) != 0;
@@ -801,8 +819,8 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   float b_scale = 1.0f, b_inverse = 1.0f;
   const bool per_sample = TB > 1 && a.b_amax_samples != nullptr;
   if (TB > 1 && !per_sample && a.b_amax != nullptr) scale_for(tensor_amax(a.b_amax), b_scale, b_inverse);
-  const bool two_samples = L >= kTile;
-  const int64_t tile_sample = j0 / L, next_sample_col = (tile_sample + 1) * L;
+  const bool two_samples = Lq >= kTile;
+  const int64_t tile_sample = j0 / Lq, next_sample_col = (tile_sample + 1) * Lq;
   float tile_amax[2] = {0.0f, 0.0f};
   if (per_sample && two_samples) {
     const int64_t s_a = a.amax_s0 + tile_sample, s_b = s_a + 1 < a.amax_S ? s_a + 1 : s_a;
@@ -810,7 +828,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
     tile_amax[1] = sample_amax(a.b_amax_samples, s_b);
   }
   auto column_amax = [&](int64_t j) {
-    return two_samples ? (j < next_sample_col ? tile_amax[0] : tile_amax[1]) : sample_amax(a.b_amax_samples, a.amax_s0 + j / L);
+    return two_samples ? (j < next_sample_col ? tile_amax[0] : tile_amax[1]) : sample_amax(a.b_amax_samples, a.amax_s0 + j / Lq);
   };
   if (per_sample && col_ok) scale_for(column_amax(jc), b_scale, b_inverse);
 
@@ -826,11 +844,15 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int k = tile * kTileK + kr + 8 * i;
-      rb[set][i] = *reinterpret_cast<const u32x4 *>(b_base + (b_off + (uint32_t)(k < K ? k : K - 1) * row_bytes));
+      rb[set][i] = *reinterpret_cast<const u32x4_any *>(b_base + (b_off + (uint32_t)(k < K ? k : K - 1) * row_bytes));
     }
   };
   auto stage = [&](int tile, int set) {
     uint8_t *Bs = lds + (tile & 1) * kBuf;
+    if (ragged) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) rb[set][i] = moved_down(rb[set][i], b_skip);
+    }
     if (edge_cols || (tile + 1) * kTileK > K) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
@@ -955,8 +977,10 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   for (int half = 0; half < 2; ++half) {
     const int64_t j4 = j0 + half * 64 + c4;
     const bool ok4 = j4 < a.ncols;
-    const int64_t s4 = ok4 ? j4 / L : 0;
-    float *cp4 = a.c + (s4 * M) * (int64_t)L + (ok4 ? (int)(j4 - s4 * L) : 0);
+    const int64_t s4 = ok4 ? j4 / Lq : 0;
+    const int l4 = ok4 ? (int)(j4 - s4 * Lq) : 0;
+    const int left = L - l4;  // positions of the sample from here on
+    float *cp4 = a.c + (s4 * M) * (int64_t)L + l4;
     __builtin_amdgcn_wave_barrier();  // the piece staged before has been read (LDS serves a wavefront's accesses in order)
 #pragma unroll
     for (int ntl = 0; ntl < 2; ++ntl)
@@ -969,7 +993,16 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
       const int row_local = 4 * q + rsub;
       const int row = wave_row0 + row_local;
       const f32x4 v = *reinterpret_cast<const f32x4 *>(buf + row_local * kOutPitch + c4);
-      if (ok4 && row < M) *reinterpret_cast<f32x4 *>(cp4 + (int64_t)row * L) = v;
+      if (ok4 && row < M) {
+        float *at = cp4 + (int64_t)row * L;
+        if (left >= 4) {
+          *reinterpret_cast<f32x4_any *>(at) = v;
+        } else {
+          at[0] = v.x;
+          if (left > 1) at[1] = v.y;
+          if (left > 2) at[2] = v.z;
+        }
+      }
     }
     if (a.stats && lane < 32) {
       const float *rowp = buf + lane * kOutPitch;
@@ -997,6 +1030,7 @@ struct PwDwArgs {
   float *partials;   // [chunks][M][N]
   int64_t S;
   int M, N, L;
+  int Lq;    // L rounded up to four: a row that four does not divide ends with a group that is partly zeros
   int s_per_chunk;
   int flat;  // the K steps run over the positions of all samples of a chunk in a row (see pw_dw_kernel)
   int m_blocks, n_blocks;
@@ -1019,16 +1053,17 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   const int tile = (int)(logical % tiles);
   const int mb = tile % a.m_blocks, nb = tile / a.m_blocks;
   const int m0 = mb * kTile, n0 = nb * kTile;
-  const int M = a.M, N = a.N, L = a.L;
+  const int M = a.M, N = a.N, L = a.L, Lq = a.Lq;
+  const bool ragged = L != Lq;
   const int64_t s_begin = (int64_t)chunk * a.s_per_chunk;
   const int64_t s_end = s_begin + a.s_per_chunk < a.S ? s_begin + a.s_per_chunk : a.S;
-  const int l_steps = (L + kTileK - 1) / kTileK;
+  const int l_steps = (Lq + kTileK - 1) / kTileK;
   // flat: the contraction index runs over the quads (four positions) of all samples of the chunk in a row, so a K step of
   // eight quads may take the last quads of one sample and the first of the next, and only the last step of a chunk is
   // partly empty (a row of 196 positions is 6.125 steps instead of 7).  Needs at least eight quads per sample (a step
   // then touches two samples at most) and samples of less than 2^31 bytes (a lane's offset reaches into the second).
   const bool flat = a.flat != 0;
-  const int Q = L >> 2;
+  const int Q = Lq >> 2;
   const int n_samples = (int)(s_end - s_begin);
   const int64_t total_quads = (int64_t)n_samples * Q;
   const int64_t iters = flat ? (total_quads + 7) / 8 : (int64_t)n_samples * l_steps;
@@ -1063,7 +1098,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
       if (second) q -= Q;
       const bool ok = f_s + (second ? 1 : 0) < n_samples;
       s = s_begin + f_s;
-      l_off = ok ? (uint32_t)q * 16u : 0u;
+      l_off = ok ? (uint32_t)min(4 * q, L - 4) * 4u : 0u;
       if (ok && second) {
         sa = a_sample;
         sb = b_sample;
@@ -1076,18 +1111,18 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
     } else {
       s = s_begin + it / l_steps;
       const int l = (int)(it % l_steps) * kTileK + 4 * q4;
-      l_off = (uint32_t)((l < L ? l : L - 4) * 4);
+      l_off = (uint32_t)(min(l, L - 4) * 4);
     }
     const char *pa = dy_base + (s * M) * (int64_t)L * 4;
     const char *pb = x_base + (BITS ? ((s * N) * (int64_t)L >> 3) : (s * N) * (int64_t)L * 4);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      ra[set][i] = *reinterpret_cast<const f32x4 *>(pa + (a_off[i] + sa + l_off));
+      ra[set][i] = *reinterpret_cast<const f32x4_any *>(pa + (a_off[i] + sa + l_off));
       if (BITS) {
         const uint32_t e = b_off[i] + sb + (l_off >> 2);
         rb[set][i].x = __builtin_bit_cast(float, (uint32_t)*reinterpret_cast<const uint8_t *>(pb + (e >> 3)));
       } else {
-        rb[set][i] = *reinterpret_cast<const f32x4 *>(pb + (b_off[i] + sb + l_off));
+        rb[set][i] = *reinterpret_cast<const f32x4_any *>(pb + (b_off[i] + sb + l_off));
       }
     }
   };
@@ -1111,6 +1146,14 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
       l_ok = l0 + 4 * q4 < L;
       lq = l_ok ? l0 + 4 * q4 : L - 4;
       tail = l0 + kTileK > L;
+    }
+    if (ragged && !BITS) {  // (as in pw_gemm_rows_kernel)
+      const int skip = lq - min(lq, L - 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ra[set][i] = moved_down(ra[set][i], skip);
+        rb[set][i] = moved_down(rb[set][i], skip);
+      }
     }
     if (edge_rows || tail) {
 #pragma unroll
@@ -1451,6 +1494,7 @@ __global__ void __launch_bounds__(256) dw_reduce_kernel(const float *partials, i
 }
 
 int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
+int64_t column_pitch(int64_t L) { return round_up(L, 4); }
 
 template <int TA, int TB, bool H = false, int BSRC = kBFloat>
 int launch_gemm_terms(const PwGemmArgs &a, int64_t blocks, hipStream_t stream) {
@@ -1534,15 +1578,17 @@ int64_t pwconv_gemm_stats_rows(int64_t K, int64_t S, int64_t L) {
   int64_t rows = 0;
   for (int64_t s0 = 0; s0 < S; s0 += s_step) {
     const int64_t s_count = S - s0 < s_step ? S - s0 : s_step;
-    rows += 2 * ((s_count * L + kTile - 1) / kTile);
+    rows += 2 * ((s_count * column_pitch(L) + kTile - 1) / kTile);
   }
   return rows;
 }
 
 int launch_pwconv_gemm(const uint16_t *a_planes, int a_terms, int64_t M, int64_t K, const float *b, int b_terms,
                        const float *b_amax, int64_t S, int64_t L, float *c, float *stats, hipStream_t stream, bool b_bits) {
-  if (L % 2 != 0 || !aligned16(a_planes) || (!b_bits && (reinterpret_cast<uintptr_t>(b) & 7u)))
-    return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_gemm: L=%lld must be even, the weight planes 16-byte and the activations 8-byte aligned", (long long)L);
+  // real fp32 activations on fp16 planes, at least four positions: the kernel that keeps A out of LDS
+  const bool rows_kernel = SJHIP_PW_ROWS != 0 && a_terms == (SJHIP_PW_F16 | 2) && !b_bits && L >= 4 && (b_terms == 1 || b_terms == 2);
+  if ((L % 2 != 0 && !rows_kernel) || !aligned16(a_planes) || (!b_bits && (reinterpret_cast<uintptr_t>(b) & 7u)))
+    return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_gemm: L=%lld must be even (or, on fp16 planes and fp32 activations, at least 4), the weight planes 16-byte and the activations 8-byte aligned", (long long)L);
   if (b_bits && ((K * L) % 8 != 0 || a_terms != (SJHIP_PW_F16 | 2) || b_terms != 1))
     return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_gemm: bit-packed activations need K*L=%lld to be a multiple of 8, fp16 weight planes and one activation term", (long long)(K * L));
   const int64_t limit = kPwOffsetLimit;
@@ -1555,9 +1601,9 @@ int launch_pwconv_gemm(const uint16_t *a_planes, int a_terms, int64_t M, int64_t
     PwGemmArgs a;
     a.a_planes = a_planes; a.c = c + s0 * M * L;
     a.b = b_bits ? reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(b) + s0 * K * L / 8) : b + s0 * K * L;
-    a.M = (int)M; a.K = (int)K; a.K_pad = (int)round_up(K, kTileK); a.L = (int)L;
+    a.M = (int)M; a.K = (int)K; a.K_pad = (int)round_up(K, kTileK); a.L = (int)L; a.Lq = (int)column_pitch(L);
     a.plane_stride = round_up(M, kTile) * a.K_pad;
-    a.ncols = s_count * L;
+    a.ncols = s_count * a.Lq;
     a.m_blocks = (int)(round_up(M, kTile) / kTile);
     a.stats = stats;
     a.a_inverse = reinterpret_cast<const float *>(a_planes + 2 * a.plane_stride);
@@ -1570,9 +1616,7 @@ int launch_pwconv_gemm(const uint16_t *a_planes, int a_terms, int64_t M, int64_t
     const int64_t blocks = a.m_blocks * ((a.ncols + kTile - 1) / kTile);
     if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "pwconv_gemm: %lld blocks", (long long)blocks);
     int rc;
-    // real fp32 activations, positions in fours, everything 16-byte aligned: the kernel that keeps A out of LDS
-    const bool rows_kernel = SJHIP_PW_ROWS != 0 && a_terms == (SJHIP_PW_F16 | 2) && !b_bits && L % 4 == 0 && aligned16(b) && aligned16(c);
-    if (rows_kernel && (b_terms == 1 || b_terms == 2)) {
+    if (rows_kernel) {
       rc = b_terms == 2 ? launch_gemm_rows<2>(a, blocks, stream) : launch_gemm_rows<1>(a, blocks, stream);
       if (rc != SJHIP_OK) return rc;
       continue;
@@ -1605,15 +1649,15 @@ int launch_pwconv_grad_weight(const float *dy, int dy_terms, const float *dy_ama
                               hipStream_t stream, bool x_bits) {
   if (x_bits && ((N * L) % 8 != 0 || dy_terms != (SJHIP_PW_F16 | 2) || x_terms != 1))
     return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_grad_weight: bit-packed activations need N*L=%lld to be a multiple of 8, two fp16 gradient terms and one activation term", (long long)(N * L));
-  if (L % 4 != 0 || !aligned16(dy) || (!x_bits && !aligned16(x)))
-    return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_grad_weight: L=%lld must be a multiple of 4 and the tensors 16-byte aligned", (long long)L);
+  if ((L % 4 != 0 && (x_bits || L < 4)) || !aligned16(dy) || (!x_bits && !aligned16(x)))
+    return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_grad_weight: L=%lld must be a multiple of 4 (or at least 4 with fp32 activations) and the tensors 16-byte aligned", (long long)L);
   if (M * L >= (int64_t(1) << 30) || N * L >= (int64_t(1) << 30) || M * N >= (int64_t(1) << 40))  // 32-bit per-lane byte offsets
     return fail(SJHIP_ERR_TOO_LARGE, "pwconv_grad_weight: M=%lld N=%lld L=%lld", (long long)M, (long long)N, (long long)L);
   PwDwArgs a;
   a.dy = dy; a.x = x; a.partials = workspace; a.S = S;
   a.dy_amax = dy_amax; a.x_amax = x_amax;
   a.flat = (L >= 32 && M * L < (int64_t(1) << 29) && N * L < (int64_t(1) << 29)) ? 1 : 0;
-  a.M = (int)M; a.N = (int)N; a.L = (int)L;
+  a.M = (int)M; a.N = (int)N; a.L = (int)L; a.Lq = (int)column_pitch(L);
   a.m_blocks = (int)(round_up(M, kTile) / kTile);
   a.n_blocks = (int)(round_up(N, kTile) / kTile);
   const int tiles = a.m_blocks * a.n_blocks;
@@ -1693,7 +1737,7 @@ int launch_pwconv_gemm_planes(const uint16_t *a_planes, int64_t M, int64_t K, co
     return fail(SJHIP_ERR_TOO_LARGE, "pwconv_gemm_planes: M=%lld K=%lld S=%lld L=%lld", (long long)M, (long long)K, (long long)S, (long long)L);
   PwGemmArgs a;
   a.a_planes = a_planes; a.b = nullptr; a.c = c;
-  a.M = (int)M; a.K = (int)K; a.K_pad = (int)round_up(K, kTileK); a.L = (int)L;
+  a.M = (int)M; a.K = (int)K; a.K_pad = (int)round_up(K, kTileK); a.L = a.Lq = (int)L;
   a.plane_stride = round_up(M, kTile) * a.K_pad;
   a.ncols = S * L;
   a.m_blocks = (int)(round_up(M, kTile) / kTile);

@@ -1,0 +1,146 @@
+"""Convolution, batch norm and neuron over samples whose number of positions four does not divide.
+
+Every kernel is compared with itself on the same rows padded with zeros to a multiple of four (the layout the other tests
+pin against the oracle): element-wise results and sums in the same order have the same bits, sums in another order the
+rounding of fp32 sums of their length."""
+
+import pytest
+import torch
+
+from helpers import seeded_randn
+from oracle import neuron_oracle as no
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [4, 5, 6, 7, 9, 31, 33, 49, 81, 127, 129, 198, 257, 259, 1025]
+
+
+@pytest.fixture(scope="module")
+def C():
+    from spikingjelly_amd.activation_based.hip_kernel import conv_bn_lif
+
+    return conv_bn_lif
+
+
+def _padded(x):
+    return torch.nn.functional.pad(x, (0, -x.shape[-1] % 4)).contiguous()
+
+
+def _spec(T):
+    from spikingjelly_amd.activation_based.hip_kernel import neuron_kernel as K
+
+    return (2.0, 1.0, 0.0, K._flags(False, False, True, 0), no.SG_IDS["atan"], no.SG_DEFAULT_ALPHA["atan"])
+
+
+@pytest.mark.parametrize("L", LENGTHS)
+@pytest.mark.parametrize("S, M, K", [(1, 5, 3), (5, 130, 70), (2, 256, 96)])
+@pytest.mark.parametrize("spikes", [False, True])
+def test_gemms(C, L, S, M, K, spikes):
+    F = C.F16 | 2
+    terms = C.F16 | 1 if spikes else F
+    x = (seeded_randn((S, K, L), 1) > 0.3).float().cuda() if spikes else seeded_randn((S, K, L), 1).cuda()
+    dy, w = seeded_randn((S, M, L), 2).cuda(), seeded_randn((M, K), 3).cuda()
+    xp, dyp = _padded(x), _padded(dy)
+    planes = C.split_weight(w, False, F)
+    got, sums = C.pw_gemm(planes, F, M, K, x, terms, True)
+    want, want_sums = C.pw_gemm(planes, F, M, K, xp, terms, True)
+    assert torch.equal(got, want[..., :L]) and torch.equal(sums, want_sums)
+    assert torch.equal(C.pw_grad_weight(dy, F, x, terms), C.pw_grad_weight(dyp, F, xp, terms))
+    # (and the padded form against 64 bits: what the split drops, 2^-22, and 2^-24 per fp32 addition of K terms)
+    exact = w.double() @ x.double()
+    bound = (2.0 ** -22 + K * 2.0 ** -24) * (w.double().abs() @ x.double().abs())
+    assert ((got.double() - exact).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("L", LENGTHS)
+@pytest.mark.parametrize("T", [1, 4, 9, 35])
+def test_normalise_and_neuron(C, L, T):
+    B, Ch = 3, 8
+    y = seeded_randn((T, B, Ch, L), 4, 0.4, 1.2).cuda()
+    gs = seeded_randn((T, B, Ch, L), 5).cuda()
+    gamma = seeded_randn((Ch,), 6, 1.0, 0.2).cuda()
+    stats = C._bn_map(y.flatten(0, 1), gamma, None, None, None, True, 0.1, 1e-5)
+    y64 = y.double().transpose(0, 2).reshape(Ch, -1)
+    torch.testing.assert_close(stats[2].double(), y64.mean(1), rtol=1e-5, atol=1e-6)
+    torch.testing.assert_close(stats[3].double(), (y64.var(1, unbiased=False) + 1e-5).rsqrt(), rtol=1e-5, atol=0)
+    v0 = seeded_randn((B, Ch, L), 7, 0.0, 0.3).cuda()
+    spec = _spec(T)
+    yp, gp, vp = _padded(y), _padded(gs), _padded(v0)
+    spikes, v = C._bn_lif_forward(y, stats, v0, spec, False)
+    want, want_v = C._bn_lif_forward(yp, stats, vp, spec, False)
+    assert torch.equal(spikes, want[..., :L]) and torch.equal(v, want_v[..., :L])
+    bits, _ = C._bn_lif_forward(y, stats, v0, spec, True) if B * Ch * L % 8 == 0 else (None, None)
+    if bits is not None:
+        unpacked = (bits[:, None] >> torch.arange(8, device="cuda", dtype=torch.uint8)) & 1
+        assert torch.equal(unpacked.flatten().float(), spikes.flatten())
+    for batch_stats in (False, True):
+        dy, dgamma, dbeta, gvi, dy_amax = C._bn_lif_backward(y, stats, gamma, v0, spec, batch_stats, gs, None, True, True)
+        pdy, pdgamma, pdbeta, pgvi, _ = C._bn_lif_backward(yp, stats, gamma, vp, spec, False, gp, None, True, True)
+        assert torch.equal(gvi, pgvi[..., :L])
+        torch.testing.assert_close(dgamma, pdgamma, rtol=1e-5, atol=1e-4)  # sums of up to T B L = 1e5 terms of order one, in another order
+        torch.testing.assert_close(dbeta, pdbeta, rtol=1e-5, atol=1e-4)
+        assert torch.equal(C.sample_amax(dy_amax), dy.abs().amax(dim=(2, 3)).flatten())
+        if not batch_stats:
+            assert torch.equal(dy, pdy[..., :L])
+        else:   # dy = a (g - mean(g) - yhat mean(g yhat)), a g being the gradient without batch statistics
+            yhat = (y - stats[2].view(-1, 1)) * stats[3].view(-1, 1)
+            n, a = T * B * L, (gamma * stats[3]).view(-1, 1)
+            ref = pdy[..., :L].double() - (a * (dbeta.view(-1, 1) + yhat * dgamma.view(-1, 1)) / n).double()
+            torch.testing.assert_close(dy.double(), ref, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("T", [3, 20])
+def test_parametric_time_constant(C, T):
+    B, Ch, L = 2, 20, 49
+    y, gs = seeded_randn((T, B, Ch, L), 8, 0.4, 1.2).cuda(), seeded_randn((T, B, Ch, L), 9).cuda()
+    stats = C._bn_map(y.flatten(0, 1), None, None, None, None, True, 0.1, 1e-5)
+    v0 = torch.zeros((B, Ch, L), device="cuda")
+    k = torch.tensor([0.4], device="cuda")
+    spec = (0.0, *_spec(T)[1:])
+    out = C._bn_lif_backward(y, stats, None, v0, spec, False, gs, None, False, False, k)
+    ref = C._bn_lif_backward(_padded(y), stats, None, _padded(v0), spec, False, _padded(gs), None, False, False, k)
+    # padded positions have no upstream gradient, hence no share in dL/dk
+    assert torch.equal(out[0], ref[0][..., :L])
+    torch.testing.assert_close(out[-1], ref[-1], rtol=1e-4, atol=1e-3)
+
+
+@pytest.mark.parametrize("train", [False, True])
+def test_modules_take_the_fused_chain(train):
+    """The attention block over 7 x 7 positions and a convolution block over 5 x 5: the fused chain runs, and equals the
+    chain run module by module up to spikes at their threshold (another order of the convolution's sums)."""
+    from spikingjelly_amd import configure
+    from spikingjelly_amd.activation_based import functional, layer
+    from spikingjelly_amd.activation_based.hip_kernel import conv_bn_lif
+    from spikingjelly_amd.activation_based.model.spikformer import SpikformerConv2dBNLIF
+
+    for make, shape in ((lambda: layer.SpikingSelfAttention(64, 2, backend="hip"), (4, 3, 64, 49)),
+                        (lambda: SpikformerConv2dBNLIF(24, 40, 1, backend="hip"), (3, 2, 24, 5, 5))):
+        torch.manual_seed(11)
+        block = make().cuda().train(train)
+        for m in block.modules():   # (scales and offsets that make the neurons fire)
+            if isinstance(m, (torch.nn.BatchNorm1d, torch.nn.BatchNorm2d)):
+                torch.nn.init.constant_(m.weight, 1.5), torch.nn.init.constant_(m.bias, 0.4), m.running_var.fill_(0.1)
+        x = seeded_randn(shape, 12).cuda()
+        results = []
+        for fuse in (True, False):
+            configure.hip_fuse_conv_bn_lif = fuse
+            calls = []
+            run = conv_bn_lif.pw_gemm
+            conv_bn_lif.pw_gemm = lambda *a, **k: (calls.append(1), run(*a, **k))[1]
+            try:
+                xd = x.clone().requires_grad_()
+                out = block(xd)
+                out.backward(seeded_randn(tuple(out.shape), 13).cuda())
+            finally:
+                conv_bn_lif.pw_gemm = run
+                configure.hip_fuse_conv_bn_lif = True
+            assert bool(calls) == fuse
+            states = [m.v.clone() for m in block.modules() if hasattr(m, "v") and isinstance(m.v, torch.Tensor)]
+            functional.reset_net(block)
+            results.append((out.detach(), xd.grad, states, [p.grad.clone() for p in block.parameters()]))
+            block.zero_grad()
+        (a, ga, sa, pa), (b, gb, sb, pb) = results
+        assert a.shape == b.shape and [s.shape for s in sa] == [s.shape for s in sb]
+        assert 0.0 < float(b.mean()) < 1.0 and float((a != b).float().mean()) < 1e-3
+        for p, q in zip([ga, *pa], [gb, *pb]):
+            assert float((p - q).norm()) < 2e-2 * float(q.norm())
