@@ -560,6 +560,34 @@ int sjhip_pwconv_grad_weight_f16_bits(const float *dy, const float *dy_amax, con
                                       int64_t N, int64_t L, float *dw, float *workspace, void *stream);
 
 /*
+ * Convolution (kernel size 1) -> batch norm -> neuron of a training or inference step, all launches from one call, with
+ * the fp16 split and one workspace (16-byte aligned, sjhip_conv_bn_lif_*_workspace_floats; free when the stream has passed
+ * the call).  The launches and their results are those of the single entry points, in this order:
+ *   forward    sjhip_pwconv_split_weight_f16, sjhip_pwconv_amax (x_amax != NULL), sjhip_pwconv_gemm_f16[_bits] with
+ *              statistics (batch_stats), sjhip_bn_finalize[_rows], sjhip_bn_lif_forward / sjhip_bn_plif_forward
+ *   backward   sjhip_bn_lif_backward / sjhip_bn_plif_backward, sjhip_bn_backward_finalize, and for dx or dw
+ *              sjhip_bn_grad_input_amax, then sjhip_pwconv_grad_weight_f16[_bits] (dw != NULL),
+ *              sjhip_pwconv_split_weight_f16 and sjhip_pwconv_gemm_f16 (dx != NULL)
+ * x [T*B][Cin][L] fp32 or x_bits (bit-packed spikes, L a multiple of 4); x_amax: sjhip_pwconv_amax_floats(T*B) words to
+ * fill (forward) or filled (backward) for real-valued x, NULL for x that fp16 holds exactly; weight [Cout][Cin]; bn_map
+ * [4][Cout]: scale, shift, mean, 1/std; k_device and grad_k with SJHIP_NEURON_PLIF and only with it; channel_grads
+ * [5][Cout]: dgamma, dbeta and the three coefficients of the input gradient.
+ */
+int64_t sjhip_conv_bn_lif_forward_workspace_floats(int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L);
+int sjhip_conv_bn_lif_forward(int neuron, const sjhip_neuron_params *p, int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L,
+                              const float *x, const uint8_t *x_bits, const float *weight, const float *gamma, const float *beta,
+                              float *running_mean, float *running_var, int batch_stats, float momentum, float eps,
+                              int64_t *batches_tracked, const float *v_init, const float *k_device, float *x_amax, float *y,
+                              float *bn_map, float *spike_seq, uint8_t *spike_bits, float *v_last, float *workspace, void *stream);
+int64_t sjhip_conv_bn_lif_backward_workspace_floats(int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L, int need_dx, int need_dw,
+                                                    int plif);
+int sjhip_conv_bn_lif_backward(int neuron, const sjhip_neuron_params *p, int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L,
+                               const float *x, const uint8_t *x_bits, const float *x_amax, const float *weight, const float *gamma,
+                               const float *v_init, const float *k_device, const float *y, const float *bn_map, int batch_stats,
+                               const float *grad_spike_seq, const float *grad_v_last, float *dx, float *dw, float *channel_grads,
+                               float *grad_v_init, float *grad_k, float *workspace, void *stream);
+
+/*
  * The same GEMMs with the activations / gradients arriving as fp16 term planes that their producer wrote already scaled
  * and split (sjhip_pwconv_split_planes), instead of
  * fp32 tensors that every block of a GEMM splits again while it stages them (same reference lines:

@@ -449,6 +449,96 @@ def _conv_backward(dy, x_seq, weight, x_exact, need_dx, need_dw, dy_amax=None, x
     return dx, dw
 
 
+# The chain with all its launches in one call (fp16 split): a launch through ctypes costs 15 to 20 us of host time (device
+# guard, stream, outputs, workspace), and at few samples a kernel runs 3 to 6 us.
+def _chain_forward(x_seq, bits, shape, weight, gamma, beta, v_init, bn, spec, x_exact: bool, packed: bool, k):
+    """Convolution, batch norm and neuron of ``x_seq [T, B, Cin, L]`` or of its spikes as ``bits`` (``shape``: that of the
+    sequence): ``(spikes or bits, v_last, y, bn_map, x_amax)``."""
+    running_mean, running_var, batch_stats, momentum, eps, tracked = _bn_config(bn)
+    T, B, Cin, Lp = shape
+    Cout = weight.shape[0]
+    terms = _terms()
+    if not terms & F16:
+        y, partial, x_amax = _conv_forward(x_seq, weight, x_exact, batch_stats)
+        bn_map = _bn_map(y.flatten(0, 1), gamma, beta, running_mean, running_var, batch_stats, momentum, eps, partial, tracked)
+        return (*_bn_lif_forward(y, bn_map, v_init, spec, packed, k), y, bn_map, x_amax)
+    source = x_seq if bits is None else bits
+    dev = source.device
+    w = L.aligned16(weight.detach().to(torch.float32))
+    v_keep, broadcast = K._state_arg(v_init, True)
+    params = _lif_params(spec, broadcast)
+    k_keep, k_ptr = K._k_pointer(k, source)
+    lib = L.load()
+    f32 = dict(dtype=torch.float32, device=dev)
+    x_amax = torch.empty((amax_floats(T * B) if bits is None and not x_exact else 0,), **f32)
+    y = torch.empty((T, B, Cout, Lp), **f32)
+    bn_map = torch.empty((4, Cout), **f32)
+    v_last = torch.empty((B, Cout, Lp), **f32)
+    spikes = torch.empty((T * B * Cout * Lp // 8,), dtype=torch.uint8, device=dev) if packed else torch.empty_like(y)
+    workspace = torch.empty((lib.sjhip_conv_bn_lif_forward_workspace_floats(T, B, Cin, Cout, Lp),), **f32)
+    with torch.cuda.device(dev):
+        rc = lib.sjhip_conv_bn_lif_forward(
+            L.NEURON_PLIF if k is not None else _neuron_id(spec, k), ctypes.byref(params), T, B, Cin, Cout, Lp,
+            source.data_ptr() if bits is None else None, None if bits is None else bits.data_ptr(), w.data_ptr(), L.ptr(gamma), L.ptr(beta),
+            L.ptr(running_mean), L.ptr(running_var), 1 if batch_stats else 0, momentum, eps, L.ptr(tracked), v_keep.data_ptr(), k_ptr,
+            x_amax.data_ptr() if x_amax.numel() else None, y.data_ptr(), bn_map.data_ptr(), None if packed else spikes.data_ptr(),
+            spikes.data_ptr() if packed else None, v_last.data_ptr(), workspace.data_ptr(), _stream(source))
+    L.check(rc, "conv_bn_lif_forward")
+    return spikes, v_last, y, bn_map, x_amax
+
+
+def _chain_backward(x_seq, bits, shape, weight, gamma, v_init, y, bn_map, x_amax, spec, batch_stats: bool, x_exact: bool, grad_spikes,
+                    grad_v_last, need_dx: bool, need_dw: bool, need_gvi: bool, k=None):
+    """Backward of ``_chain_forward``: ``(dx, dw, dgamma, dbeta, grad_v_init)``, ``None`` where not needed; with ``k``
+    (parametric LIF) a sixth element, ``dL/dk``."""
+    T, B, Cin, Lp = shape
+    Cout = weight.shape[0]
+    overlap = (need_dx and need_dw and bits is None and getattr(configure, "hip_conv_overlap_gradients", False)
+               and not torch.cuda.is_current_stream_capturing())  # (the two gradients on two streams)
+    if overlap or not _terms() & F16:
+        dy, dgamma, dbeta, gvi, dy_amax, *grad_k = _bn_lif_backward(y, bn_map, gamma, v_init, spec, batch_stats, grad_spikes,
+                                                                     grad_v_last, need_gvi, True, k)
+        if bits is None:
+            dx, dw = _conv_backward(dy, x_seq, weight, x_exact, need_dx, need_dw, dy_amax, x_amax)
+        else:
+            terms, dy3 = _terms(), dy.view(T * B, Cout, Lp)
+            if dy_amax is None:
+                dy_amax = amax(dy3)
+            dw = pw_grad_weight_bits(dy3, bits, Cin, dy_amax) if need_dw else None
+            dx = (pw_gemm(split_weight(weight, True, terms), terms, Cin, Cout, dy3, terms, False, dy_amax).view(T, B, Cin, Lp)
+                  if need_dx else None)
+        return (dx, dw, dgamma, dbeta, gvi, *grad_k)
+    dev = y.device
+    lib = L.load()
+    f32 = dict(dtype=torch.float32, device=dev)
+    grad_spikes = L.aligned16(grad_spikes.to(torch.float32)) if grad_spikes is not None else torch.zeros_like(y)
+    if grad_v_last is not None:
+        grad_v_last = L.aligned16(grad_v_last.to(torch.float32))
+    w = L.aligned16(weight.detach().to(torch.float32))
+    if bits is not None or x_exact:
+        x_amax = None
+    elif need_dw and x_amax.numel() == 0:  # (the forward ran on bf16 terms)
+        x_amax = amax(x_seq.reshape(T * B, Cin, Lp))
+    v_keep, broadcast = K._state_arg(v_init, True)
+    params = _lif_params(spec, broadcast)
+    k_keep, k_ptr = K._k_pointer(k, y)
+    dx = torch.empty((T, B, Cin, Lp), **f32) if need_dx else None
+    dw = torch.empty((Cout, Cin), **f32) if need_dw else None
+    grads = torch.empty((5, Cout), **f32)  # dgamma, dbeta, then the coefficients of the input gradient
+    gvi = torch.empty((B, Cout, Lp), **f32) if need_gvi else None
+    grad_k = torch.empty((1,), **f32) if k is not None else None
+    workspace = torch.empty((lib.sjhip_conv_bn_lif_backward_workspace_floats(T, B, Cin, Cout, Lp, need_dx, need_dw, k is not None),), **f32)
+    with torch.cuda.device(dev):
+        rc = lib.sjhip_conv_bn_lif_backward(
+            L.NEURON_PLIF if k is not None else _neuron_id(spec, k), ctypes.byref(params), T, B, Cin, Cout, Lp,
+            x_seq.data_ptr() if bits is None else None, L.ptr(bits), L.ptr(x_amax), w.data_ptr(), L.ptr(gamma), v_keep.data_ptr(), k_ptr,
+            y.data_ptr(), bn_map.data_ptr(), 1 if batch_stats else 0, grad_spikes.data_ptr(), L.ptr(grad_v_last), L.ptr(dx), L.ptr(dw),
+            grads.data_ptr(), L.ptr(gvi), L.ptr(grad_k), workspace.data_ptr(), _stream(y))
+    L.check(rc, "conv_bn_lif_backward")
+    out = (dx, dw, grads[0], grads[1], gvi)
+    return out if k is None else (*out, grad_k)
+
+
 _SIDE_STREAMS: dict = {}
 
 
@@ -475,10 +565,8 @@ def _conv_chain_backward(x_seq, weight, gamma, v_init, y, bn_map, bits, x_amax, 
         heads, cph, scale = ssa
         T, B, _, Lp = x_seq.shape
         grad_spikes = A._ssa_packed(bits, grad_out, torch.float32, T * B, heads, cph, Lp, scale).view(y.shape)
-    dy, dgamma, dbeta, gvi, dy_amax, *grad_k = _bn_lif_backward(y, bn_map, gamma, v_init, spec, batch_stats, grad_spikes,
-                                                                 grad_v_last, need_gvi, True, k)
-    dx, dw = _conv_backward(dy, x_seq, weight, x_exact, need_dx, need_dw, dy_amax, x_amax)
-    return (dx, dw, dgamma, dbeta, gvi, *grad_k)
+    return _chain_backward(x_seq, None, x_seq.shape, weight, gamma, v_init, y, bn_map, x_amax, spec, batch_stats, x_exact, grad_spikes,
+                           grad_v_last, need_dx, need_dw, need_gvi, k)
 
 
 def _lif_conv_chain_backward(pre_seq, pre_v_init, weight, gamma, v_init, y, bn_map, bits, pre_spec, spec, batch_stats: bool,
@@ -488,17 +576,11 @@ def _lif_conv_chain_backward(pre_seq, pre_v_init, weight, gamma, v_init, y, bn_m
     ``(grad of the first neuron's input, of its state, dw, dgamma, dbeta, grad_v_init)``; with ``k`` (the second neuron
     is a parametric LIF) a seventh element, ``dL/dk``."""
     T, B, Cin, Lp = pre_seq.shape
-    Cout = weight.shape[0]
-    terms = _terms()
-    dy, dgamma, dbeta, gvi, dy_amax, *grad_k = _bn_lif_backward(y, bn_map, gamma, v_init, spec, batch_stats, grad_spikes,
-                                                                 grad_v_last, need_gvi, True, k)
-    dy3 = dy.view(T * B, Cout, Lp)
-    if dy_amax is None:
-        dy_amax = amax(dy3)
-    dw = pw_grad_weight_bits(dy3, bits, Cin, dy_amax) if need_dw else None
+    grad_pre_spikes, dw, dgamma, dbeta, gvi, *grad_k = _chain_backward(None, bits, pre_seq.shape, weight, gamma, v_init, y, bn_map, None,
+                                                                       spec, batch_stats, True, grad_spikes, grad_v_last,
+                                                                       need_gx or need_gpv, need_dw, need_gvi, k)
     gx = gpv = None
     if need_gx or need_gpv:
-        grad_pre_spikes = pw_gemm(split_weight(weight, True, terms), terms, Cin, Cout, dy3, terms, False, dy_amax)
         tau, v_th, v_reset, flags, sg_id, sg_alpha = pre_spec
         glast = grad_pre_v_last.flatten() if grad_pre_v_last is not None else None
         gx, gpv, _ = K._run_backward(L.NEURON_LIF, grad_pre_spikes.view(T, -1), None, glast, None, pre_seq.view(T, -1),
@@ -538,12 +620,8 @@ class _BnLif(torch.autograd.Function):
 class _ConvBnLif(torch.autograd.Function):
     @staticmethod
     def forward(x_seq, weight, gamma, beta, v_init, bn, spec, x_exact, k=None):
-        running_mean, running_var, batch_stats, momentum, eps, tracked = _bn_config(bn)
         x_seq = L.aligned16(x_seq)
-        y, partial, x_amax = _conv_forward(x_seq, weight, x_exact, batch_stats)
-        bn_map = _bn_map(y.flatten(0, 1), gamma, beta, running_mean, running_var, batch_stats, momentum, eps, partial, tracked)
-        spikes, v_last = _bn_lif_forward(y, bn_map, v_init, spec, False, k)
-        return spikes, v_last, y, bn_map, x_amax
+        return _chain_forward(x_seq, None, x_seq.shape, weight, gamma, beta, v_init, bn, spec, x_exact, False, k)
 
     @staticmethod
     def setup_context(ctx, inputs, output):
@@ -572,13 +650,10 @@ class _ConvBnLifSsa(torch.autograd.Function):
     def forward(x_seq, weight, gamma, beta, v_init, bn, spec, x_exact, ssa, k=None):
         from . import attention_kernel as A
 
-        running_mean, running_var, batch_stats, momentum, eps, tracked = _bn_config(bn)
         heads, cph, scale = ssa
         x_seq = L.aligned16(x_seq)
         T, B, _, Lp = x_seq.shape
-        y, partial, x_amax = _conv_forward(x_seq, weight, x_exact, batch_stats)
-        bn_map = _bn_map(y.flatten(0, 1), gamma, beta, running_mean, running_var, batch_stats, momentum, eps, partial, tracked)
-        bits, v_last = _bn_lif_forward(y, bn_map, v_init, spec, True, k)
+        bits, v_last, y, bn_map, x_amax = _chain_forward(x_seq, None, x_seq.shape, weight, gamma, beta, v_init, bn, spec, x_exact, True, k)
         out = A._ssa_packed(bits, None, torch.float32, T * B, heads, cph, Lp, scale)
         return out, v_last, y, bn_map, bits, x_amax
 
@@ -612,13 +687,10 @@ class _ConvBnLifSsaLif(torch.autograd.Function):
     def forward(x_seq, weight, gamma, beta, v_init, attn_v_init, bn, spec, x_exact, ssa, attn_spec, save_h):
         from . import attention_kernel as A
 
-        running_mean, running_var, batch_stats, momentum, eps, tracked = _bn_config(bn)
         heads, cph, scale = ssa
         x_seq = L.aligned16(x_seq)
         T, B, _, Lp = x_seq.shape
-        y, partial, x_amax = _conv_forward(x_seq, weight, x_exact, batch_stats)
-        bn_map = _bn_map(y.flatten(0, 1), gamma, beta, running_mean, running_var, batch_stats, momentum, eps, partial, tracked)
-        bits, v_last = _bn_lif_forward(y, bn_map, v_init, spec, True)
+        bits, v_last, y, bn_map, x_amax = _chain_forward(x_seq, None, x_seq.shape, weight, gamma, beta, v_init, bn, spec, x_exact, True, None)
         v_keep, broadcast = K._state_arg(attn_v_init, True)
         spikes, h_seq, attn_v_last = A._ssa_lif_forward(bits, v_keep, _lif_params(attn_spec, broadcast), T, B, heads, cph,
                                                         Lp, scale, save_h)
@@ -649,9 +721,9 @@ class _ConvBnLifSsaLif(torch.autograd.Function):
             grad_qkv, _ = A._ssa_lif_backward(bits, h_seq, grad_attn_spikes, grad_attn_v_last, _lif_params(ctx.attn_spec), T, B,
                                               heads, cph, Lp, scale, False)
             grad_spikes = grad_qkv.view(y.shape)
-        dy, dgamma, dbeta, gvi, dy_amax = _bn_lif_backward(y, bn_map, gamma, v_init, ctx.spec, ctx.batch_stats, grad_spikes,
-                                                            grad_v_last, bool(need[4]), True)
-        dx, dw = _conv_backward(dy, x_seq, weight, ctx.x_exact, bool(need[0]), bool(need[1]), dy_amax, x_amax)
+        dx, dw, dgamma, dbeta, gvi = _chain_backward(x_seq, None, x_seq.shape, weight, gamma, v_init, y, bn_map, x_amax, ctx.spec,
+                                                     ctx.batch_stats, ctx.x_exact, grad_spikes, grad_v_last, bool(need[0]),
+                                                     bool(need[1]), bool(need[4]))
         return (dx, dw, dgamma if need[2] else None, dbeta if need[3] else None, gvi, None, None, None, None, None, None, None)
 
 
@@ -665,20 +737,12 @@ class _LifConvBnLif(torch.autograd.Function):
 
     @staticmethod
     def forward(pre_seq, pre_v_init, weight, gamma, beta, v_init, bn, pre_spec, spec, k=None):
-        running_mean, running_var, batch_stats, momentum, eps, tracked = _bn_config(bn)
         pre_seq = L.aligned16(pre_seq)
         T, B, Cin, Lp = pre_seq.shape
-        Cout = weight.shape[0]
         tau, v_th, v_reset, flags, _, _ = pre_spec
         bits, _, pre_v_last = K._run_forward_packed(L.NEURON_LIF, pre_seq.view(T, -1), pre_v_init.flatten(), None, tau, v_th,
                                                     v_reset, flags, False)
-        terms = _terms()
-        planes = split_weight(weight, False, terms)
-        out = pw_gemm_bits(planes, Cout, Cin, bits, T * B, Lp, batch_stats)
-        y, partial = (out[0], out[1]) if batch_stats else (out, None)
-        y = y.view(T, B, Cout, Lp)
-        bn_map = _bn_map(y.flatten(0, 1), gamma, beta, running_mean, running_var, batch_stats, momentum, eps, partial, tracked)
-        spikes, v_last = _bn_lif_forward(y, bn_map, v_init, spec, False, k)
+        spikes, v_last, y, bn_map, _ = _chain_forward(None, bits, pre_seq.shape, weight, gamma, beta, v_init, bn, spec, True, False, k)
         return spikes, v_last, pre_v_last.view(B, Cin, Lp), y, bn_map, bits
 
     @staticmethod

@@ -82,6 +82,10 @@ EXPORTED_SYMBOLS = (
     "sjhip_pwconv_gemm_f16",
     "sjhip_pwconv_grad_weight_f16",
     "sjhip_bn_grad_input_amax",
+    "sjhip_conv_bn_lif_forward_workspace_floats",
+    "sjhip_conv_bn_lif_forward",
+    "sjhip_conv_bn_lif_backward_workspace_floats",
+    "sjhip_conv_bn_lif_backward",
     "sjhip_pwconv_gemm_f16_bits",
     "sjhip_pwconv_grad_weight_f16_bits",
     "sjhip_pwconv_plane_elems",
@@ -286,6 +290,16 @@ def load() -> ctypes.CDLL:
         lib.sjhip_pwconv_grad_weight_f16.restype = c_int
         lib.sjhip_pwconv_grad_weight_f16.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int64, c_int64, c_int64,
                                                      c_int64, c_void_p, c_void_p, c_void_p]
+        lib.sjhip_conv_bn_lif_forward_workspace_floats.restype = c_int64
+        lib.sjhip_conv_bn_lif_forward_workspace_floats.argtypes = [c_int64] * 5
+        lib.sjhip_conv_bn_lif_forward.restype = c_int
+        lib.sjhip_conv_bn_lif_forward.argtypes = ([c_int, POINTER(NeuronParams)] + [c_int64] * 5 + [c_void_p] * 7 + [c_int, c_float, c_float]
+                                                  + [c_void_p] * 11)
+        lib.sjhip_conv_bn_lif_backward_workspace_floats.restype = c_int64
+        lib.sjhip_conv_bn_lif_backward_workspace_floats.argtypes = [c_int64] * 5 + [c_int] * 3
+        lib.sjhip_conv_bn_lif_backward.restype = c_int
+        lib.sjhip_conv_bn_lif_backward.argtypes = ([c_int, POINTER(NeuronParams)] + [c_int64] * 5 + [c_void_p] * 9 + [c_int]
+                                                   + [c_void_p] * 9)
         lib.sjhip_pwconv_gemm_f16_bits.restype = c_int
         lib.sjhip_pwconv_gemm_f16_bits.argtypes = [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p,
                                                    c_void_p]

@@ -755,6 +755,133 @@ int sjhip_pwconv_grad_weight_planes(const uint16_t *dy_planes, const float *dy_a
                                           static_cast<hipStream_t>(stream));
 }
 
+// ---- the whole chain in one call ---------------------------------------------------------------------------------------------
+namespace {
+// Hands out the parts of one workspace, each on 256 bytes; without a base it only counts.
+struct Carver {
+  float *base;
+  int64_t used = 0;
+  float *take(int64_t floats) {
+    float *p = base ? base + used : nullptr;
+    used += (floats + 63) / 64 * 64;
+    return p;
+  }
+};
+struct ChainForwardParts {
+  uint16_t *planes;
+  float *partial;
+  int64_t rows;
+  int64_t floats;
+  ChainForwardParts(float *workspace, int64_t S, int64_t Cin, int64_t Cout, int64_t L) {
+    Carver carve{workspace};
+    planes = reinterpret_cast<uint16_t *>(carve.take((pwconv_planes_elems(Cout, Cin) + 1) / 2));
+    rows = pwconv_gemm_stats_rows(Cin, S, L);
+    partial = carve.take(rows * Cout * 2);
+    floats = carve.used;
+  }
+};
+struct ChainBackwardParts {
+  float *dy, *partial, *amax, *k_shares, *dw_partials;
+  uint16_t *planes;
+  int64_t floats;
+  // (the weight gradient's partial tiles and the planes of the transposed weights are used one after the other)
+  ChainBackwardParts(float *workspace, int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L, bool dx, bool dw, bool plif) {
+    Carver carve{workspace};
+    dy = carve.take(T * B * Cout * L);
+    partial = carve.take(B * Cout * 2);
+    amax = carve.take(SJHIP_PW_AMAX_FLOATS + SJHIP_PW_AMAX_SAMPLE_WORDS * T * B);
+    k_shares = carve.take(plif ? bn_lif_backward_k_workspace_floats(B, Cout, L) : 0);
+    const int64_t dw_floats = dw ? pwconv_dw_workspace_floats(Cout, Cin, T * B) : 0;
+    const int64_t planes_floats = dx ? (pwconv_planes_elems(Cin, Cout) + 1) / 2 : 0;
+    dw_partials = carve.take(dw_floats > planes_floats ? dw_floats : planes_floats);
+    planes = reinterpret_cast<uint16_t *>(dw_partials);
+    floats = carve.used;
+  }
+};
+int check_chain(const char *what, int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L) {
+  const int64_t limit = int64_t(1) << 40;
+  if (T < 1 || B < 1 || Cin < 1 || Cout < 1 || L < 1)
+    return fail(SJHIP_ERR_INVALID, "%s: T=%lld B=%lld Cin=%lld Cout=%lld L=%lld must be >= 1", what, (long long)T, (long long)B, (long long)Cin, (long long)Cout, (long long)L);
+  if (T > (1 << 24) || B > (1 << 24) || Cin > (1 << 24) || Cout > (1 << 24) || L > (1 << 24) || T * B > limit / L ||
+      T * B * L > limit / Cin || T * B * L > limit / Cout)
+    return fail(SJHIP_ERR_TOO_LARGE, "%s: T=%lld B=%lld Cin=%lld Cout=%lld L=%lld", what, (long long)T, (long long)B, (long long)Cin, (long long)Cout, (long long)L);
+  return SJHIP_OK;
+}
+}  // namespace
+
+int64_t sjhip_conv_bn_lif_forward_workspace_floats(int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L) {
+  if (check_chain("conv_bn_lif", T, B, Cin, Cout, L) != SJHIP_OK) return 0;
+  return ChainForwardParts(nullptr, T * B, Cin, Cout, L).floats;
+}
+
+int sjhip_conv_bn_lif_forward(int neuron, const sjhip_neuron_params *p, int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L,
+                              const float *x, const uint8_t *x_bits, const float *weight, const float *gamma, const float *beta,
+                              float *running_mean, float *running_var, int batch_stats, float momentum, float eps,
+                              int64_t *batches_tracked, const float *v_init, const float *k_device, float *x_amax, float *y,
+                              float *bn_map, float *spike_seq, uint8_t *spike_bits, float *v_last, float *workspace, void *stream_) {
+  if (!p || !weight || !v_init || !y || !bn_map || !v_last || !workspace || (x == nullptr) == (x_bits == nullptr) ||
+      (spike_seq == nullptr) == (spike_bits == nullptr))
+    return fail(SJHIP_ERR_INVALID, "conv_bn_lif_forward: NULL buffer, or not exactly one of x / x_bits and of spike_seq / spike_bits");
+  if (x_bits && x_amax) return fail(SJHIP_ERR_INVALID, "conv_bn_lif_forward: x_amax goes with fp32 activations");
+  int rc = check_chain("conv_bn_lif_forward", T, B, Cin, Cout, L);
+  if (rc != SJHIP_OK) return rc;
+  if (!aligned16(workspace) || !aligned16(y) || (x_amax && !aligned16(x_amax)))
+    return fail(SJHIP_ERR_UNSUPPORTED, "conv_bn_lif_forward: workspace, y and x_amax must be 16-byte aligned");
+  const hipStream_t stream = static_cast<hipStream_t>(stream_);
+  const int64_t S = T * B;
+  const ChainForwardParts w(workspace, S, Cin, Cout, L);
+  rc = launch_pwconv_split_weight_f16(weight, Cout, Cin, 0, w.planes, x_amax, SJHIP_PW_AMAX_FLOATS + SJHIP_PW_AMAX_SAMPLE_WORDS * S, stream);
+  if (rc == SJHIP_OK && x_amax) rc = launch_pwconv_amax(x, S, Cin * L, x_amax, stream);
+  float *partial = batch_stats ? w.partial : nullptr;
+  if (rc == SJHIP_OK)
+    rc = launch_pwconv_gemm(w.planes, SJHIP_PW_F16 | 2, Cout, Cin, x_bits ? reinterpret_cast<const float *>(x_bits) : x, x_amax ? 2 : 1,
+                            x_amax, S, L, y, partial, stream, x_bits != nullptr);
+  if (rc == SJHIP_OK)
+    rc = launch_bn_finalize(partial, w.rows, S * L, Cout, gamma, beta, eps, momentum, running_mean, running_var, bn_map, bn_map + Cout,
+                            bn_map + 2 * Cout, bn_map + 3 * Cout, batches_tracked, stream);
+  if (rc == SJHIP_OK)
+    rc = launch_bn_lif_forward(neuron, *p, T, B, Cout, L, y, bn_map, bn_map + Cout, v_init, k_device, spike_seq, spike_bits, v_last, stream);
+  return rc;
+}
+
+int64_t sjhip_conv_bn_lif_backward_workspace_floats(int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L, int need_dx, int need_dw,
+                                                    int plif) {
+  if (check_chain("conv_bn_lif", T, B, Cin, Cout, L) != SJHIP_OK) return 0;
+  return ChainBackwardParts(nullptr, T, B, Cin, Cout, L, need_dx != 0, need_dw != 0, plif != 0).floats;
+}
+
+int sjhip_conv_bn_lif_backward(int neuron, const sjhip_neuron_params *p, int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L,
+                               const float *x, const uint8_t *x_bits, const float *x_amax, const float *weight, const float *gamma,
+                               const float *v_init, const float *k_device, const float *y, const float *bn_map, int batch_stats,
+                               const float *grad_spike_seq, const float *grad_v_last, float *dx, float *dw, float *channel_grads,
+                               float *grad_v_init, float *grad_k, float *workspace, void *stream_) {
+  if (!p || !weight || !v_init || !y || !bn_map || !grad_spike_seq || !channel_grads || !workspace || (dw && (x == nullptr) == (x_bits == nullptr)))
+    return fail(SJHIP_ERR_INVALID, "conv_bn_lif_backward: NULL buffer, or not exactly one of x / x_bits");
+  int rc = check_chain("conv_bn_lif_backward", T, B, Cin, Cout, L);
+  if (rc != SJHIP_OK) return rc;
+  if (!aligned16(workspace) || (x_amax && !aligned16(x_amax)))
+    return fail(SJHIP_ERR_UNSUPPORTED, "conv_bn_lif_backward: workspace and x_amax must be 16-byte aligned");
+  const hipStream_t stream = static_cast<hipStream_t>(stream_);
+  const int64_t S = T * B;
+  const ChainBackwardParts w(workspace, T, B, Cin, Cout, L, dx != nullptr, dw != nullptr, k_device != nullptr);
+  float *coef = channel_grads + 2 * Cout;
+  rc = launch_bn_lif_backward(neuron, *p, T, B, Cout, L, y, bn_map, bn_map + Cout, v_init, k_device, grad_spike_seq, grad_v_last, w.dy,
+                              grad_v_init, w.partial, grad_k, w.k_shares, stream);
+  if (rc == SJHIP_OK)
+    rc = launch_bn_backward_finalize(w.partial, T, B, Cout, L, batch_stats, gamma, bn_map + 2 * Cout, bn_map + 3 * Cout, channel_grads,
+                                     channel_grads + Cout, coef, w.amax, stream);
+  if (!dx && !dw) return rc;
+  if (rc == SJHIP_OK) rc = launch_bn_grad_input(w.dy, y, coef, S, Cout, L, w.dy, w.amax, stream);
+  if (rc == SJHIP_OK && dw)
+    rc = launch_pwconv_grad_weight(w.dy, SJHIP_PW_F16 | 2, w.amax, x_bits ? reinterpret_cast<const float *>(x_bits) : x, x_amax ? 2 : 1,
+                                   x_amax, S, Cout, Cin, L, dw, w.dw_partials, stream, x_bits != nullptr);
+  if (rc == SJHIP_OK && dx) {
+    rc = launch_pwconv_split_weight_f16(weight, Cout, Cin, 1, w.planes, nullptr, 0, stream);
+    if (rc == SJHIP_OK) rc = launch_pwconv_gemm(w.planes, SJHIP_PW_F16 | 2, Cin, Cout, w.dy, 2, w.amax, S, L, dx, nullptr, stream);
+  }
+  return rc;
+}
+
 int sjhip_bn_stats(const float *y, int64_t S, int64_t C, int64_t L, float *partial, void *stream) {
   if (!y || !partial) return fail(SJHIP_ERR_INVALID, "bn_stats: NULL buffer");
   return launch_bn_stats(y, S, C, L, partial, static_cast<hipStream_t>(stream));
