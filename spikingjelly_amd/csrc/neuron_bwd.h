@@ -351,12 +351,15 @@ __device__ __forceinline__ float backward_body(const BwdArgs &a, bool active, in
     float v0[V];
     load_state_from<S, VECTOR, SJHIP_BWD_NT != 0>(a.v_init, col, a.v_init_broadcast, v0);
     // neurons that the work-item shares with its neighbour (whole_group) are counted there
-    const int64_t shared = ((int64_t)column_block(a.spread) * blockDim.x + threadIdx.x) * V - col;
+    const int rest = (int)(a.N % V);
+    int shared = 0;
+    if (rest != 0) shared = col + V == a.N ? V - rest : 0;
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       const float dh_dk = a.decay_input ? (h_next[j] - v0[j]) : (a.v_reset - v0[j]);
       acc[j] += g_next[j] * dh_dk;
-      if (j >= shared) acc_total += acc[j];
+      if (rest == 0) acc_total += acc[j];
+      else if (j >= shared) acc_total += acc[j];
     }
   }
   return acc_total;

@@ -394,7 +394,7 @@ __device__ __forceinline__ unsigned column_block(int spread) {
 // fp16 with every op rounded [6, 3580137] 35 / 264 -> 20 / 34.
 #ifdef __HIPCC__
 template <int V> __device__ __forceinline__ int64_t whole_group(int64_t col, int64_t N) {
-  if (V == 1) return col;
+  if (V == 1 || N % V == 0) return col;  // (the same for every lane: whole rows pay one scalar test)
   return col + V <= N ? col : N - V;
 }
 #endif
