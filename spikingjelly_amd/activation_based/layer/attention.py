@@ -2,10 +2,10 @@
 
 ``Conv1d+BN -> LIF -> scale * (V K^T) Q -> LIF(v_threshold=0.5) -> Conv1d+BN -> LIF`` on ``[T, N, C, L]``
 input.  With ``backend='hip'`` the three LIF nodes run the HIP neuron kernels and the contraction runs on
-the matrix cores (int8 / bf16 MFMA, fp32 accumulation; exact because Q/K/V are binary).  For fp32 device tensors of
-at least four tokens the two ``Conv1d(k=1) -> BatchNorm1d -> LIF`` chains run fused as well (``layer/fused.py``:
-split-bf16 MFMA GEMMs, batch norm and the neuron in two passes over the convolution output); other inputs keep
-torch's convolution and batch norm around the hip neurons.
+the matrix cores (int8 / bf16 MFMA, fp32 accumulation; exact because Q/K/V are binary).  For fp32 device tensors whose
+token count is a multiple of 4 the two ``Conv1d(k=1) -> BatchNorm1d -> LIF`` chains run fused as well (``layer/fused.py``:
+split-operand MFMA GEMMs, batch norm and the neuron in two passes over the convolution output), for other counts of at
+least four the second of them; other inputs keep torch's convolution and batch norm around the hip neurons.
 """
 
 from __future__ import annotations
@@ -108,7 +108,10 @@ class SpikingSelfAttention(nn.Module, base.MultiStepModule):
         hip = self.backend == "hip"
         out = None
         attn_spikes = None
-        if hip and len(self.qkv_conv_bn) == 2:
+        if hip and len(self.qkv_conv_bn) == 2 and L % 4 == 0:
+            # (Other token counts keep torch's convolution in front of the contraction: with the sums of a convolution in
+            # another order a few spikes in a million fall on the other side of their threshold, and the contraction
+            # spreads each over a head.)
             # convolution, batch norm, LIF (bit-packed spikes), the contraction and the attention's LIF in one autograd
             # node; without the last of them when it cannot run inside the contraction
             if configure.hip_fuse_ssa_lif:
