@@ -571,7 +571,9 @@ int sjhip_pwconv_grad_weight_f16_bits(const float *dy, const float *dy_amax, con
  * x [T*B][Cin][L] fp32 or x_bits (bit-packed spikes, L a multiple of 4); x_amax: sjhip_pwconv_amax_floats(T*B) words to
  * fill (forward) or filled (backward) for real-valued x, NULL for x that fp16 holds exactly; weight [Cout][Cin]; bn_map
  * [4][Cout]: scale, shift, mean, 1/std; k_device and grad_k with SJHIP_NEURON_PLIF and only with it; channel_grads
- * [5][Cout]: dgamma, dbeta and the three coefficients of the input gradient.
+ * [5][Cout]: dgamma, dbeta and the three coefficients of the input gradient; dy [T*B][Cout][L]: the gradient of the
+ * convolution's output (that of the batch norm's output when neither dx nor dw is asked for), apart from the workspace
+ * because it is as large as y.
  */
 int64_t sjhip_conv_bn_lif_forward_workspace_floats(int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L);
 int sjhip_conv_bn_lif_forward(int neuron, const sjhip_neuron_params *p, int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L,
@@ -584,8 +586,8 @@ int64_t sjhip_conv_bn_lif_backward_workspace_floats(int64_t T, int64_t B, int64_
 int sjhip_conv_bn_lif_backward(int neuron, const sjhip_neuron_params *p, int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L,
                                const float *x, const uint8_t *x_bits, const float *x_amax, const float *weight, const float *gamma,
                                const float *v_init, const float *k_device, const float *y, const float *bn_map, int batch_stats,
-                               const float *grad_spike_seq, const float *grad_v_last, float *dx, float *dw, float *channel_grads,
-                               float *grad_v_init, float *grad_k, float *workspace, void *stream);
+                               const float *grad_spike_seq, const float *grad_v_last, float *dy, float *dx, float *dw,
+                               float *channel_grads, float *grad_v_init, float *grad_k, float *workspace, void *stream);
 
 /*
  * The same GEMMs with the activations / gradients arriving as fp16 term planes that their producer wrote already scaled

@@ -522,18 +522,19 @@ def _chain_backward(x_seq, bits, shape, weight, gamma, v_init, y, bn_map, x_amax
     v_keep, broadcast = K._state_arg(v_init, True)
     params = _lif_params(spec, broadcast)
     k_keep, k_ptr = K._k_pointer(k, y)
-    dx = torch.empty((T, B, Cin, Lp), **f32) if need_dx else None
-    dw = torch.empty((Cout, Cin), **f32) if need_dw else None
+    dy = torch.empty_like(y)
     grads = torch.empty((5, Cout), **f32)  # dgamma, dbeta, then the coefficients of the input gradient
     gvi = torch.empty((B, Cout, Lp), **f32) if need_gvi else None
     grad_k = torch.empty((1,), **f32) if k is not None else None
     workspace = torch.empty((lib.sjhip_conv_bn_lif_backward_workspace_floats(T, B, Cin, Cout, Lp, need_dx, need_dw, k is not None),), **f32)
+    dw = torch.empty((Cout, Cin), **f32) if need_dw else None
+    dx = torch.empty((T, B, Cin, Lp), **f32) if need_dx else None
     with torch.cuda.device(dev):
         rc = lib.sjhip_conv_bn_lif_backward(
             L.NEURON_PLIF if k is not None else _neuron_id(spec, k), ctypes.byref(params), T, B, Cin, Cout, Lp,
             x_seq.data_ptr() if bits is None else None, L.ptr(bits), L.ptr(x_amax), w.data_ptr(), L.ptr(gamma), v_keep.data_ptr(), k_ptr,
-            y.data_ptr(), bn_map.data_ptr(), 1 if batch_stats else 0, grad_spikes.data_ptr(), L.ptr(grad_v_last), L.ptr(dx), L.ptr(dw),
-            grads.data_ptr(), L.ptr(gvi), L.ptr(grad_k), workspace.data_ptr(), _stream(y))
+            y.data_ptr(), bn_map.data_ptr(), 1 if batch_stats else 0, grad_spikes.data_ptr(), L.ptr(grad_v_last), dy.data_ptr(), L.ptr(dx),
+            L.ptr(dw), grads.data_ptr(), L.ptr(gvi), L.ptr(grad_k), workspace.data_ptr(), _stream(y))
     L.check(rc, "conv_bn_lif_backward")
     out = (dx, dw, grads[0], grads[1], gvi)
     return out if k is None else (*out, grad_k)

@@ -299,7 +299,7 @@ def load() -> ctypes.CDLL:
         lib.sjhip_conv_bn_lif_backward_workspace_floats.argtypes = [c_int64] * 5 + [c_int] * 3
         lib.sjhip_conv_bn_lif_backward.restype = c_int
         lib.sjhip_conv_bn_lif_backward.argtypes = ([c_int, POINTER(NeuronParams)] + [c_int64] * 5 + [c_void_p] * 9 + [c_int]
-                                                   + [c_void_p] * 9)
+                                                   + [c_void_p] * 10)
         lib.sjhip_pwconv_gemm_f16_bits.restype = c_int
         lib.sjhip_pwconv_gemm_f16_bits.argtypes = [c_void_p, c_int64, c_int64, c_void_p, c_int64, c_int64, c_void_p, c_void_p,
                                                    c_void_p]

@@ -781,13 +781,12 @@ struct ChainForwardParts {
   }
 };
 struct ChainBackwardParts {
-  float *dy, *partial, *amax, *k_shares, *dw_partials;
+  float *partial, *amax, *k_shares, *dw_partials;
   uint16_t *planes;
   int64_t floats;
   // (the weight gradient's partial tiles and the planes of the transposed weights are used one after the other)
   ChainBackwardParts(float *workspace, int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L, bool dx, bool dw, bool plif) {
     Carver carve{workspace};
-    dy = carve.take(T * B * Cout * L);
     partial = carve.take(B * Cout * 2);
     amax = carve.take(SJHIP_PW_AMAX_FLOATS + SJHIP_PW_AMAX_SAMPLE_WORDS * T * B);
     k_shares = carve.take(plif ? bn_lif_backward_k_workspace_floats(B, Cout, L) : 0);
@@ -853,9 +852,9 @@ int64_t sjhip_conv_bn_lif_backward_workspace_floats(int64_t T, int64_t B, int64_
 int sjhip_conv_bn_lif_backward(int neuron, const sjhip_neuron_params *p, int64_t T, int64_t B, int64_t Cin, int64_t Cout, int64_t L,
                                const float *x, const uint8_t *x_bits, const float *x_amax, const float *weight, const float *gamma,
                                const float *v_init, const float *k_device, const float *y, const float *bn_map, int batch_stats,
-                               const float *grad_spike_seq, const float *grad_v_last, float *dx, float *dw, float *channel_grads,
-                               float *grad_v_init, float *grad_k, float *workspace, void *stream_) {
-  if (!p || !weight || !v_init || !y || !bn_map || !grad_spike_seq || !channel_grads || !workspace || (dw && (x == nullptr) == (x_bits == nullptr)))
+                               const float *grad_spike_seq, const float *grad_v_last, float *dy, float *dx, float *dw,
+                               float *channel_grads, float *grad_v_init, float *grad_k, float *workspace, void *stream_) {
+  if (!p || !weight || !v_init || !y || !bn_map || !grad_spike_seq || !dy || !channel_grads || !workspace || (dw && (x == nullptr) == (x_bits == nullptr)))
     return fail(SJHIP_ERR_INVALID, "conv_bn_lif_backward: NULL buffer, or not exactly one of x / x_bits");
   int rc = check_chain("conv_bn_lif_backward", T, B, Cin, Cout, L);
   if (rc != SJHIP_OK) return rc;
@@ -865,19 +864,19 @@ int sjhip_conv_bn_lif_backward(int neuron, const sjhip_neuron_params *p, int64_t
   const int64_t S = T * B;
   const ChainBackwardParts w(workspace, T, B, Cin, Cout, L, dx != nullptr, dw != nullptr, k_device != nullptr);
   float *coef = channel_grads + 2 * Cout;
-  rc = launch_bn_lif_backward(neuron, *p, T, B, Cout, L, y, bn_map, bn_map + Cout, v_init, k_device, grad_spike_seq, grad_v_last, w.dy,
+  rc = launch_bn_lif_backward(neuron, *p, T, B, Cout, L, y, bn_map, bn_map + Cout, v_init, k_device, grad_spike_seq, grad_v_last, dy,
                               grad_v_init, w.partial, grad_k, w.k_shares, stream);
   if (rc == SJHIP_OK)
     rc = launch_bn_backward_finalize(w.partial, T, B, Cout, L, batch_stats, gamma, bn_map + 2 * Cout, bn_map + 3 * Cout, channel_grads,
                                      channel_grads + Cout, coef, w.amax, stream);
   if (!dx && !dw) return rc;
-  if (rc == SJHIP_OK) rc = launch_bn_grad_input(w.dy, y, coef, S, Cout, L, w.dy, w.amax, stream);
+  if (rc == SJHIP_OK) rc = launch_bn_grad_input(dy, y, coef, S, Cout, L, dy, w.amax, stream);
   if (rc == SJHIP_OK && dw)
-    rc = launch_pwconv_grad_weight(w.dy, SJHIP_PW_F16 | 2, w.amax, x_bits ? reinterpret_cast<const float *>(x_bits) : x, x_amax ? 2 : 1,
+    rc = launch_pwconv_grad_weight(dy, SJHIP_PW_F16 | 2, w.amax, x_bits ? reinterpret_cast<const float *>(x_bits) : x, x_amax ? 2 : 1,
                                    x_amax, S, Cout, Cin, L, dw, w.dw_partials, stream, x_bits != nullptr);
   if (rc == SJHIP_OK && dx) {
     rc = launch_pwconv_split_weight_f16(weight, Cout, Cin, 1, w.planes, nullptr, 0, stream);
-    if (rc == SJHIP_OK) rc = launch_pwconv_gemm(w.planes, SJHIP_PW_F16 | 2, Cin, Cout, w.dy, 2, w.amax, S, L, dx, nullptr, stream);
+    if (rc == SJHIP_OK) rc = launch_pwconv_gemm(w.planes, SJHIP_PW_F16 | 2, Cin, Cout, dy, 2, w.amax, S, L, dx, nullptr, stream);
   }
   return rc;
 }
