@@ -246,6 +246,43 @@ __global__ void __launch_bounds__(256) split_weight_f16_kernel(const float *src,
   if (lane == 0) reinterpret_cast<float *>(planes + 2 * rows_pad * cols_pad)[r] = inverse;
 }
 
+// The same planes of the transposed matrix: A[r][c] = src[c * ld_c + r], rows contiguous.  A wavefront per row would fetch
+// one line per element; here a block takes 16 rows (64 contiguous bytes of every c) and four k steps: 64 x 16 work-items
+// walk all of c for the rows' largest magnitudes (again for every block of the same rows, from L2), then each splits one
+// pair of c.
+constexpr int kSplitSteps = 4;
+__global__ void __launch_bounds__(1024) split_weight_f16_transposed_kernel(const float *src, int64_t rows, int64_t cols, int64_t ld_c,
+                                                                            int64_t rows_pad, int64_t cols_pad, uint16_t *planes) {
+  __shared__ float part[16][17];
+  const int ri = threadIdx.x & 15, ci = threadIdx.x >> 4;
+  const int64_t r = (int64_t)blockIdx.x * 16 + ri;
+  const bool row_ok = r < rows;
+  const int64_t steps = cols_pad / kTileK, step = (int64_t)blockIdx.y * kSplitSteps + (ci >> 4), c = step * kTileK + 2 * (ci & 15);
+  const float raw0 = row_ok && c < cols ? src[c * ld_c + r] : 0.0f;
+  const float raw1 = row_ok && c + 1 < cols ? src[(c + 1) * ld_c + r] : 0.0f;
+  float amax = 0.0f;
+  if (row_ok) {
+#pragma unroll 16
+    for (int64_t i = ci; i < cols; i += 64) amax = fmaxf(amax, finite_abs(src[i * ld_c + r]));
+  }
+  amax = fmaxf(amax, __shfl_xor(amax, 16));  // the four c of a wavefront
+  amax = fmaxf(amax, __shfl_xor(amax, 32));
+  if ((threadIdx.x & 48) == 0) part[threadIdx.x >> 6][ri] = amax;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) amax = fmaxf(amax, part[i][ri]);
+  float scale, inverse;
+  scale_for(amax, scale, inverse);
+  if (step < steps) {
+    uint32_t w[2];
+    split_pair<2, true>(raw0 * scale, raw1 * scale, w);
+    const int64_t at = (((r / kTile) * steps + step) * kTile + r % kTile) * kTileK + 2 * (ci & 15);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) reinterpret_cast<uint32_t *>(planes + (int64_t)t * rows_pad * cols_pad)[at / 2] = w[t];
+  }
+  if (blockIdx.y == 0 && ci == 0) reinterpret_cast<float *>(planes + 2 * rows_pad * cols_pad)[r] = inverse;
+}
+
 // The largest magnitude of a tensor is kept as SJHIP_PW_AMAX_FLOATS non-negative floats whose maximum it is: blocks fold
 // their share into word (block % SJHIP_PW_AMAX_FLOATS) with an integer atomic maximum (the bit patterns of non-negative
 // floats order like unsigned integers, and a maximum does not depend on the order it is taken in).  Several words,
@@ -777,10 +814,13 @@ constexpr unsigned rows_inverse_offset(int tb) { return 2u * tb * kRowPlane > kO
 //   * two B tiles alternate in LDS, so a K step has one barrier.
 // Per K step of a block: 16 KB written to and 64 KB read from LDS, 16 + 16 load instructions; 146 registers, three
 // wavefronts per SIMD.
+// BITS: b is a spike tensor that arrives bit-packed (as in pw_gemm_kernel, L a multiple of 4): a byte per piece, one term.
 // Samples of any length L >= 4: the column index gives every sample Lq = L rounded up to four columns, so that a piece
 // lies in one sample; a piece that runs over the end of its row is fetched as the row's last four elements (at any
 // 4-byte address) and moved down by one to three places with zeros behind it.
-template <int TB>
+// (RAGGED is a template parameter: asked at run time the moves cost the aligned case 4 %, 106 -> 110 us at M = 1536, K = 384,
+// 25 088 columns.)
+template <int TB, bool BITS, bool RAGGED>
 __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu(3, 3))) pw_gemm_rows_kernel(const PwGemmArgs a) {
   constexpr int TA = 2;
   constexpr int kBuf = TB * kRowPlane;  // one B tile: [TB][32 k][kPlanePitch]
@@ -790,8 +830,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   const int mb = (int)(logical % a.m_blocks);
   const int64_t nb = logical / a.m_blocks;
   const int64_t j0 = nb * kTile;
-  const int M = a.M, K = a.K, L = a.L, Lq = a.Lq;
-  const bool ragged = L != Lq;
+  const int M = a.M, K = a.K, L = a.L, Lq = RAGGED ? a.Lq : a.L;
   const int steps = a.K_pad / kTileK;
 
   // the inverse row scales of the tile wait in LDS (beyond the operand tiles) for the epilogue
@@ -809,11 +848,11 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   int b_skip = 0;  // places that the piece is moved down
   if (col_ok) {
     const int64_t s = jc / Lq;
-    const int l = (int)(jc - s * Lq), first = min(l, L - 4);
-    b_off = (uint32_t)(((s * K) * (int64_t)L + first) * 4);
+    const int l = (int)(jc - s * Lq), first = RAGGED ? min(l, L - 4) : l;
+    b_off = (uint32_t)(((s * K) * (int64_t)L + first) * (BITS ? 1 : 4));  // with BITS the bit index
     b_skip = l - first;
   }
-  const uint32_t row_bytes = (uint32_t)L * 4u;
+  const uint32_t row_bytes = (uint32_t)L * (BITS ? 1u : 4u);
   const bool edge_cols = __builtin_amdgcn_readfirstlane(j0 + kTile > a.ncols ? 1 : 0) != 0;
   const char *b_base = reinterpret_cast<const char *>(a.b);
   float b_scale = 1.0f, b_inverse = 1.0f;
@@ -844,12 +883,14 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int k = tile * kTileK + kr + 8 * i;
-      rb[set][i] = *reinterpret_cast<const u32x4_any *>(b_base + (b_off + (uint32_t)(k < K ? k : K - 1) * row_bytes));
+      const uint32_t at = b_off + (uint32_t)(k < K ? k : K - 1) * row_bytes;
+      if constexpr (BITS) rb[set][i].x = *reinterpret_cast<const uint8_t *>(b_base + (at >> 3)) >> (at & 7u);
+      else rb[set][i] = *reinterpret_cast<const u32x4_any *>(b_base + at);
     }
   };
   auto stage = [&](int tile, int set) {
     uint8_t *Bs = lds + (tile & 1) * kBuf;
-    if (ragged) {
+    if constexpr (RAGGED) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) rb[set][i] = moved_down(rb[set][i], b_skip);
     }
@@ -860,6 +901,14 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+      if constexpr (BITS) {  // four positions: 0 or 1 in fp16
+        const uint32_t four = rb[set][i].x;
+        u32x2 v;
+        v.x = (four & 1u) * 0x3c00u | (four & 2u) * 0x1e000000u;
+        v.y = (four & 4u) * 0x0f00u | (four & 8u) * 0x07800000u;
+        *reinterpret_cast<u32x2 *>(Bs + (kr + 8 * i) * kPlanePitch + q4 * 8) = v;
+        continue;
+      }
       // (the components go through scalars first: a bit cast applied to a vector component directly reads component 0)
       const uint32_t u0 = rb[set][i].x, u1 = rb[set][i].y, u2 = rb[set][i].z, u3 = rb[set][i].w;
       float x0 = __builtin_bit_cast(float, u0), x1 = __builtin_bit_cast(float, u1);
@@ -995,7 +1044,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
       const f32x4 v = *reinterpret_cast<const f32x4 *>(buf + row_local * kOutPitch + c4);
       if (ok4 && row < M) {
         float *at = cp4 + (int64_t)row * L;
-        if (left >= 4) {
+        if (!RAGGED || left >= 4) {
           *reinterpret_cast<f32x4_any *>(at) = v;
         } else {
           at[0] = v.x;
@@ -1037,11 +1086,17 @@ struct PwDwArgs {
   const float *dy_amax, *x_amax;  // fp16 terms: nullptr (no scale), or the words whose maximum is the tensor's max |.|
 };
 
+// four elements at a 16-byte or, with ANY, at a 4-byte address
+template <bool ANY> __device__ __forceinline__ f32x4 load4(const char *p) {
+  if (ANY) return *reinterpret_cast<const f32x4_any *>(p);
+  return *reinterpret_cast<const f32x4 *>(p);
+}
+
 // BITS: x is a spike tensor that arrives bit-packed (as in pw_gemm_kernel); a work-item fetches the byte whose low or
 // high half holds its four consecutive positions of a row (L and N * L are multiples of 4 and 8).
-template <int TA, int TB, bool H, bool BITS = false>
+template <int TA, int TB, bool H, bool BITS = false, bool RAGGED = false>
 __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) pw_dw_kernel(const PwDwArgs a) {
-  static_assert(!BITS || TB == 1, "a bit-packed operand has one term");
+  static_assert(!BITS || (TB == 1 && !RAGGED), "a bit-packed operand has one term and rows of a multiple of four");
   extern __shared__ __align__(16) uint8_t lds[];
   uint8_t *As = lds;                   // [TA][128][kRowBytes]
   uint8_t *Bs = lds + TA * kRowPlane;  // [TB][128][kRowBytes]
@@ -1053,8 +1108,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   const int tile = (int)(logical % tiles);
   const int mb = tile % a.m_blocks, nb = tile / a.m_blocks;
   const int m0 = mb * kTile, n0 = nb * kTile;
-  const int M = a.M, N = a.N, L = a.L, Lq = a.Lq;
-  const bool ragged = L != Lq;
+  const int M = a.M, N = a.N, L = a.L, Lq = RAGGED ? a.Lq : a.L;
   const int64_t s_begin = (int64_t)chunk * a.s_per_chunk;
   const int64_t s_end = s_begin + a.s_per_chunk < a.S ? s_begin + a.s_per_chunk : a.S;
   const int l_steps = (Lq + kTileK - 1) / kTileK;
@@ -1098,7 +1152,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
       if (second) q -= Q;
       const bool ok = f_s + (second ? 1 : 0) < n_samples;
       s = s_begin + f_s;
-      l_off = ok ? (uint32_t)min(4 * q, L - 4) * 4u : 0u;
+      l_off = ok ? (uint32_t)(RAGGED ? min(4 * q, L - 4) : 4 * q) * 4u : 0u;
       if (ok && second) {
         sa = a_sample;
         sb = b_sample;
@@ -1117,12 +1171,12 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
     const char *pb = x_base + (BITS ? ((s * N) * (int64_t)L >> 3) : (s * N) * (int64_t)L * 4);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      ra[set][i] = *reinterpret_cast<const f32x4_any *>(pa + (a_off[i] + sa + l_off));
+      ra[set][i] = load4<RAGGED>(pa + (a_off[i] + sa + l_off));
       if (BITS) {
         const uint32_t e = b_off[i] + sb + (l_off >> 2);
         rb[set][i].x = __builtin_bit_cast(float, (uint32_t)*reinterpret_cast<const uint8_t *>(pb + (e >> 3)));
       } else {
-        rb[set][i] = *reinterpret_cast<const f32x4_any *>(pb + (b_off[i] + sb + l_off));
+        rb[set][i] = load4<RAGGED>(pb + (b_off[i] + sb + l_off));
       }
     }
   };
@@ -1147,7 +1201,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
       lq = l_ok ? l0 + 4 * q4 : L - 4;
       tail = l0 + kTileK > L;
     }
-    if (ragged && !BITS) {  // (as in pw_gemm_rows_kernel)
+    if constexpr (RAGGED) {  // (as in pw_gemm_rows_kernel)
       const int skip = lq - min(lq, L - 4);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1505,16 +1559,19 @@ int launch_gemm_terms(const PwGemmArgs &a, int64_t blocks, hipStream_t stream) {
   return check_launch("pwconv_gemm");
 }
 
-template <int TB>
+template <int TB, bool BITS = false>
 int launch_gemm_rows(const PwGemmArgs &a, int64_t blocks, hipStream_t stream) {
-  hipLaunchKernelGGL((pw_gemm_rows_kernel<TB>), dim3((unsigned)blocks), dim3(kPwThreads), rows_inverse_offset(TB) + kTile * 4, stream, a);
+  const unsigned lds = rows_inverse_offset(TB) + kTile * 4;
+  if (BITS || a.L == a.Lq) hipLaunchKernelGGL((pw_gemm_rows_kernel<TB, BITS, false>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
+  else hipLaunchKernelGGL((pw_gemm_rows_kernel<TB, false, true>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
   return check_launch("pwconv_gemm");
 }
 
 template <int TA, int TB, bool H = false, bool BITS = false>
 int launch_dw_terms(const PwDwArgs &a, int64_t blocks, hipStream_t stream) {
   const unsigned lds = (TA + TB) * kRowPlane;
-  hipLaunchKernelGGL((pw_dw_kernel<TA, TB, H, BITS>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
+  if (BITS || a.L == a.Lq) hipLaunchKernelGGL((pw_dw_kernel<TA, TB, H, BITS>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
+  else hipLaunchKernelGGL((pw_dw_kernel<TA, TB, H, false, true>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
   return check_launch("pwconv_grad_weight");
 }
 
@@ -1554,6 +1611,14 @@ int launch_pwconv_split_weight_f16(const float *w, int64_t rows, int64_t cols, i
   const int64_t rows_pad = round_up(ar, kTile), cols_pad = round_up(ac, kTileK);
   const int64_t blocks = rows_pad / 4;
   if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "pwconv_split_weight_f16: %lld x %lld", (long long)rows, (long long)cols);
+  if (transpose && !amax_reset) {
+    const int64_t step_blocks = (cols_pad / kTileK + kSplitSteps - 1) / kSplitSteps;
+    if (step_blocks <= 65535) {
+      hipLaunchKernelGGL(split_weight_f16_transposed_kernel, dim3((unsigned)(rows_pad / 16), (unsigned)step_blocks), dim3(1024), 0, stream,
+                         w, ar, ac, cols, rows_pad, cols_pad, planes);
+      return check_launch("pwconv_split_weight_f16");
+    }
+  }
   hipLaunchKernelGGL(split_weight_f16_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, w, ar, ac,
                      transpose ? (int64_t)1 : cols, transpose ? cols : (int64_t)1, rows_pad, cols_pad, planes, amax_reset, amax_floats);
   return check_launch("pwconv_split_weight_f16");
@@ -1585,8 +1650,8 @@ int64_t pwconv_gemm_stats_rows(int64_t K, int64_t S, int64_t L) {
 
 int launch_pwconv_gemm(const uint16_t *a_planes, int a_terms, int64_t M, int64_t K, const float *b, int b_terms,
                        const float *b_amax, int64_t S, int64_t L, float *c, float *stats, hipStream_t stream, bool b_bits) {
-  // real fp32 activations on fp16 planes, at least four positions: the kernel that keeps A out of LDS
-  const bool rows_kernel = SJHIP_PW_ROWS != 0 && a_terms == (SJHIP_PW_F16 | 2) && !b_bits && L >= 4 && (b_terms == 1 || b_terms == 2);
+  // fp16 planes and at least four positions (bits: a multiple of four): the kernel that keeps A out of LDS
+  const bool rows_kernel = SJHIP_PW_ROWS != 0 && a_terms == (SJHIP_PW_F16 | 2) && (b_bits ? L % 4 == 0 && b_terms == 1 : L >= 4 && (b_terms == 1 || b_terms == 2));
   if ((L % 2 != 0 && !rows_kernel) || !aligned16(a_planes) || (!b_bits && (reinterpret_cast<uintptr_t>(b) & 7u)))
     return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_gemm: L=%lld must be even (or, on fp16 planes and fp32 activations, at least 4), the weight planes 16-byte and the activations 8-byte aligned", (long long)L);
   if (b_bits && ((K * L) % 8 != 0 || a_terms != (SJHIP_PW_F16 | 2) || b_terms != 1))
@@ -1617,7 +1682,8 @@ int launch_pwconv_gemm(const uint16_t *a_planes, int a_terms, int64_t M, int64_t
     if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "pwconv_gemm: %lld blocks", (long long)blocks);
     int rc;
     if (rows_kernel) {
-      rc = b_terms == 2 ? launch_gemm_rows<2>(a, blocks, stream) : launch_gemm_rows<1>(a, blocks, stream);
+      rc = b_bits ? launch_gemm_rows<1, true>(a, blocks, stream)
+                  : (b_terms == 2 ? launch_gemm_rows<2>(a, blocks, stream) : launch_gemm_rows<1>(a, blocks, stream));
       if (rc != SJHIP_OK) return rc;
       continue;
     }
