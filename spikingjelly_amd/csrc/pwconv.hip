@@ -64,6 +64,8 @@
 // round-robin over the eight XCDs).
 #include "sjhip_common.h"
 
+#include <mutex>
+
 namespace sjhip {
 
 namespace {
@@ -1086,6 +1088,9 @@ struct PwDwArgs {
   const float *dy_amax, *x_amax;  // fp16 terms: nullptr (no scale), or the words whose maximum is the tensor's max |.|
 };
 
+// Two LDS buffers (fp16 terms: 2 x 40 KiB, two blocks per compute unit still fit): the next tile is split and stored while
+// the current one is multiplied, with one barrier per K step instead of two.
+constexpr bool dw_two_buffers(bool h) { return h; }
 // four elements at a 16-byte or, with ANY, at a 4-byte address
 template <bool ANY> __device__ __forceinline__ f32x4 load4(const char *p) {
   if (ANY) return *reinterpret_cast<const f32x4_any *>(p);
@@ -1098,8 +1103,10 @@ template <int TA, int TB, bool H, bool BITS = false, bool RAGGED = false>
 __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) pw_dw_kernel(const PwDwArgs a) {
   static_assert(!BITS || (TB == 1 && !RAGGED), "a bit-packed operand has one term and rows of a multiple of four");
   extern __shared__ __align__(16) uint8_t lds[];
-  uint8_t *As = lds;                   // [TA][128][kRowBytes]
-  uint8_t *Bs = lds + TA * kRowPlane;  // [TB][128][kRowBytes]
+  // [TA][128][kRowBytes] of dy, then [TB][128][kRowBytes] of x; DOUBLE: twice
+  uint8_t *As = lds, *Bs = lds + TA * kRowPlane;
+  constexpr bool DOUBLE = dw_two_buffers(H);
+  constexpr int kBuf = DOUBLE ? (TA + TB) * kRowPlane : 0;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const int64_t logical = xcd_order(blockIdx.x, gridDim.x);
@@ -1229,7 +1236,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
           u32x2 w;
           w.x = w01[t];
           w.y = w23[t];
-          *reinterpret_cast<u32x2 *>(As + t * kRowPlane + off) = w;
+          *reinterpret_cast<u32x2 *>(As + set * kBuf + t * kRowPlane + off) = w;
         }
       }
       {
@@ -1250,7 +1257,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
           u32x2 w;
           w.x = w01[t];
           w.y = w23[t];
-          *reinterpret_cast<u32x2 *>(Bs + t * kRowPlane + off) = w;
+          *reinterpret_cast<u32x2 *>(Bs + set * kBuf + t * kRowPlane + off) = w;
         }
       }
     }
@@ -1264,7 +1271,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.0f;
 
-  auto multiply = [&](int64_t it) {
+  auto multiply = [&](int64_t it, int set) {
     // the second half of the last stage of a row (flat: of the chunk) may hold nothing
     const int ksteps = flat ? ((it + 1 == iters && total_quads - 8 * it <= 4) ? 1 : 2)
                             : (((int)(it % l_steps) * kTileK + 16 < L) ? 2 : 1);
@@ -1273,32 +1280,55 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-        for (int t = 0; t < TA; ++t) af[mt][t] = row_fragment(As + t * kRowPlane, wm * 64 + mt * 32 + (lane & 31), ks, lane);
+        for (int t = 0; t < TA; ++t) af[mt][t] = row_fragment(As + set * kBuf + t * kRowPlane, wm * 64 + mt * 32 + (lane & 31), ks, lane);
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-        for (int t = 0; t < TB; ++t) bf[nt][t] = row_fragment(Bs + t * kRowPlane, wn * 64 + nt * 32 + (lane & 31), ks, lane);
+        for (int t = 0; t < TB; ++t) bf[nt][t] = row_fragment(Bs + set * kBuf + t * kRowPlane, wn * 64 + nt * 32 + (lane & 31), ks, lane);
       mfma_step<TA, TB, H>(af, bf, acc);
     }
-  };
-  // as in pw_gemm_kernel: unconditional requests in the steady state, conditions only in the last steps
-  auto step = [&](int64_t it, int set, bool more) {
-    __syncthreads();
-    stage(it, set);
-    __syncthreads();
-    if (more) fetch(it + 2, set);
-    multiply(it);
   };
   if (iters > 0) fetch(0, 0);
   if (iters > 1) fetch(1, 1);
   int64_t it = 0;
-  for (; it + 3 < iters; it += 2) {
-    step(it, 0, true);
-    step(it + 1, 1, true);
+  if constexpr (DOUBLE) {
+    // step it: tile it + 1 (requested two steps ago) goes into the other LDS buffer, tile it + 3 is requested into the
+    // registers that frees, tile it is multiplied; one barrier.  Requests are unconditional in the steady state only.
+    auto step = [&](int64_t it, int set, bool stage_next, bool more) {
+      if (stage_next) stage(it + 1, set ^ 1);
+      if (more) fetch(it + 3, set ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(it, set);
+      __syncthreads();
+    };
+    if (iters > 0) stage(0, 0);
+    if (iters > 2) fetch(2, 0);
+    __syncthreads();
+    for (; it + 4 < iters; it += 2) {
+      step(it, 0, true, true);
+      step(it + 1, 1, true, true);
+    }
+    if (it < iters) step(it, 0, it + 1 < iters, it + 3 < iters);
+    if (it + 1 < iters) step(it + 1, 1, it + 2 < iters, false);
+    if (it + 2 < iters) step(it + 2, 0, it + 3 < iters, false);
+    if (it + 3 < iters) step(it + 3, 1, false, false);
+  } else {
+    // as in pw_gemm_kernel: unconditional requests in the steady state, conditions only in the last steps
+    auto step = [&](int64_t it, int set, bool more) {
+      __syncthreads();
+      stage(it, set);
+      __syncthreads();
+      if (more) fetch(it + 2, set);
+      multiply(it, set);
+    };
+    for (; it + 3 < iters; it += 2) {
+      step(it, 0, true);
+      step(it + 1, 1, true);
+    }
+    if (it < iters) step(it, 0, it + 2 < iters);
+    if (it + 1 < iters) step(it + 1, 1, false);
+    if (it + 2 < iters) step(it + 2, 0, false);
   }
-  if (it < iters) step(it, 0, it + 2 < iters);
-  if (it + 1 < iters) step(it + 1, 1, false);
-  if (it + 2 < iters) step(it + 2, 0, false);
 
   float *out = a.partials + (int64_t)chunk * M * N;
   if (H) {
@@ -1567,12 +1597,26 @@ int launch_gemm_rows(const PwGemmArgs &a, int64_t blocks, hipStream_t stream) {
   return check_launch("pwconv_gemm");
 }
 
+template <int TA, int TB, bool H, bool BITS, bool RAGGED>
+int launch_dw(const PwDwArgs &a, int64_t blocks, hipStream_t stream) {
+  constexpr unsigned lds = (dw_two_buffers(H) ? 2 : 1) * (TA + TB) * kRowPlane;
+  if constexpr (lds > 64u * 1024u) {
+    static std::once_flag once;
+    static hipError_t attr_rc = hipSuccess;
+    std::call_once(once, [&]() {
+      attr_rc = hipFuncSetAttribute(reinterpret_cast<const void *>(&pw_dw_kernel<TA, TB, H, BITS, RAGGED>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      (void)hipGetLastError();
+    });
+    if (attr_rc != hipSuccess) return fail(SJHIP_ERR_LAUNCH, "pwconv_grad_weight: cannot raise the dynamic LDS limit: %s", hipGetErrorString(attr_rc));
+  }
+  hipLaunchKernelGGL((pw_dw_kernel<TA, TB, H, BITS, RAGGED>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
+  return check_launch("pwconv_grad_weight");
+}
 template <int TA, int TB, bool H = false, bool BITS = false>
 int launch_dw_terms(const PwDwArgs &a, int64_t blocks, hipStream_t stream) {
-  const unsigned lds = (TA + TB) * kRowPlane;
-  if (BITS || a.L == a.Lq) hipLaunchKernelGGL((pw_dw_kernel<TA, TB, H, BITS>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
-  else hipLaunchKernelGGL((pw_dw_kernel<TA, TB, H, false, true>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
-  return check_launch("pwconv_grad_weight");
+  if (BITS || a.L == a.Lq) return launch_dw<TA, TB, H, BITS, false>(a, blocks, stream);
+  return launch_dw<TA, TB, H, false, true>(a, blocks, stream);
 }
 
 // Samples per partial tile of dW.  Two blocks are resident per compute unit (512 on the chip); the chunk count is the
