@@ -564,7 +564,8 @@ int sjhip_pwconv_grad_weight_f16_bits(const float *dy, const float *dy_amax, con
  * the fp16 split and one workspace (16-byte aligned, sjhip_conv_bn_lif_*_workspace_floats; free when the stream has passed
  * the call).  The launches and their results are those of the single entry points, in this order:
  *   forward    sjhip_pwconv_split_weight_f16, sjhip_pwconv_amax (x_amax != NULL), sjhip_pwconv_gemm_f16[_bits] with
- *              statistics (batch_stats), sjhip_bn_finalize[_rows], sjhip_bn_lif_forward / sjhip_bn_plif_forward
+ *              statistics (batch_stats), sjhip_bn_finalize[_rows] (without batch_stats its map is made by the first
+ *              launch), sjhip_bn_lif_forward / sjhip_bn_plif_forward
  *   backward   sjhip_bn_lif_backward / sjhip_bn_plif_backward, sjhip_bn_backward_finalize, and for dx or dw
  *              sjhip_bn_grad_input_amax, then sjhip_pwconv_grad_weight_f16[_bits] (dw != NULL),
  *              sjhip_pwconv_split_weight_f16 and sjhip_pwconv_gemm_f16 (dx != NULL)

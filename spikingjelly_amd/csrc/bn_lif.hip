@@ -18,6 +18,7 @@
 // gives the last work-item of a row that 4 does not divide the row's last four elements, the first of which its
 // neighbour has too (stored twice with the same bits, summed once); a kernel over the flat tensor keeps its aligned
 // groups of four and looks up both channels where a group runs over the end of a row.
+#include "bn_map.h"
 #include "neuron_bwd.h"
 #include "neuron_fwd.h"
 
@@ -175,13 +176,7 @@ __global__ void __launch_bounds__(256) bn_finalize_kernel(const float *partial, 
     mean = (double)running_mean[c];
     var = (double)running_var[c];
   }
-  const double invstd = 1.0 / sqrt(var + (double)eps);
-  const double g = gamma ? (double)gamma[c] : 1.0, b = beta ? (double)beta[c] : 0.0;
-  const double a = g * invstd;
-  scale[c] = (float)a;
-  shift[c] = (float)(b - mean * a);
-  mean_out[c] = (float)mean;
-  invstd_out[c] = (float)invstd;
+  store_bn_map(c, mean, var, gamma, beta, eps, scale, shift, mean_out, invstd_out);
 }
 
 template <int CH, int RS, bool PACKED, bool RAGGED>

@@ -62,6 +62,7 @@
 //       of samples and writes its partial tile, dw_reduce_kernel adds the chunks in a fixed order.
 // Blocks that share operand tiles are numbered so that they run on the same XCD (one L2 each, blocks are dealt
 // round-robin over the eight XCDs).
+#include "bn_map.h"
 #include "sjhip_common.h"
 
 #include <mutex>
@@ -213,10 +214,12 @@ __global__ void __launch_bounds__(256) split_weight_kernel(const float *src, int
 
 // fp16 planes[t][tile order] = term t of scale_r * src[r][c], with a power-of-two scale per row r (a row of A is a row
 // of the product, so the GEMM's epilogue takes the scale out again); the inverse scales follow the two planes as
-// rows_pad floats.  One wavefront per row.
+// rows_pad floats.  One wavefront per row.  In evaluation mode (bn.map) it also makes the map of its row's batch norm
+// channel, which depends on parameters only: a launch less between the convolution and the neuron.
 __global__ void __launch_bounds__(256) split_weight_f16_kernel(const float *src, int64_t rows, int64_t cols, int64_t ld_r,
                                                                 int64_t ld_c, int64_t rows_pad, int64_t cols_pad,
-                                                                uint16_t *planes, float *amax_reset, int64_t amax_floats) {
+                                                                uint16_t *planes, float *amax_reset, int64_t amax_floats,
+                                                                const BnEvalMap bn) {
   if (amax_reset && blockIdx.x == 0)
     for (int64_t i = threadIdx.x; i < amax_floats; i += 256) amax_reset[i] = 0.0f;
   const int lane = threadIdx.x & 63;
@@ -245,7 +248,10 @@ __global__ void __launch_bounds__(256) split_weight_f16_kernel(const float *src,
     for (int t = 0; t < 2; ++t)
       reinterpret_cast<uint32_t *>(planes + (int64_t)t * rows_pad * cols_pad)[at / 2] = w[t];
   }
-  if (lane == 0) reinterpret_cast<float *>(planes + 2 * rows_pad * cols_pad)[r] = inverse;
+  if (lane == 0) {
+    reinterpret_cast<float *>(planes + 2 * rows_pad * cols_pad)[r] = inverse;
+    if (bn.map && r < rows) store_bn_map(bn, (int)r);
+  }
 }
 
 // The same planes of the transposed matrix: A[r][c] = src[c * ld_c + r], rows contiguous.  A wavefront per row would fetch
@@ -1664,7 +1670,17 @@ int launch_pwconv_split_weight_f16(const float *w, int64_t rows, int64_t cols, i
     }
   }
   hipLaunchKernelGGL(split_weight_f16_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, w, ar, ac,
-                     transpose ? (int64_t)1 : cols, transpose ? cols : (int64_t)1, rows_pad, cols_pad, planes, amax_reset, amax_floats);
+                     transpose ? (int64_t)1 : cols, transpose ? cols : (int64_t)1, rows_pad, cols_pad, planes, amax_reset, amax_floats, BnEvalMap{});
+  return check_launch("pwconv_split_weight_f16");
+}
+
+int launch_pwconv_split_weight_f16_bn(const float *w, int64_t rows, int64_t cols, uint16_t *planes, float *amax_reset,
+                                      int64_t amax_floats, const BnEvalMap &bn, hipStream_t stream) {
+  if (rows != bn.C || rows > (1 << 24) || !bn.running_mean || !bn.running_var)
+    return fail(SJHIP_ERR_INVALID, "pwconv_split_weight_f16: %lld rows, batch norm of %d channels; evaluation mode needs the running statistics", (long long)rows, bn.C);
+  const int64_t rows_pad = round_up(rows, kTile), cols_pad = round_up(cols, kTileK);
+  hipLaunchKernelGGL(split_weight_f16_kernel, dim3((unsigned)(rows_pad / 4)), dim3(256), 0, stream, w, rows, cols, cols, (int64_t)1, rows_pad,
+                     cols_pad, planes, amax_reset, amax_floats, bn);
   return check_launch("pwconv_split_weight_f16");
 }
 

@@ -1,6 +1,7 @@
 // C ABI of libsjhip.so (declared in include/sjhip.h): argument validation, thread-local error
 // text, launch tuning and the optional event profiler.  No entry point allocates device memory or
 // synchronises the host (sjhip_profile_read excepted, which waits for the events it reports on).
+#include "bn_map.h"
 #include "sjhip_common.h"
 
 #include <atomic>
@@ -829,13 +830,19 @@ int sjhip_conv_bn_lif_forward(int neuron, const sjhip_neuron_params *p, int64_t 
   const hipStream_t stream = static_cast<hipStream_t>(stream_);
   const int64_t S = T * B;
   const ChainForwardParts w(workspace, S, Cin, Cout, L);
-  rc = launch_pwconv_split_weight_f16(weight, Cout, Cin, 0, w.planes, x_amax, SJHIP_PW_AMAX_FLOATS + SJHIP_PW_AMAX_SAMPLE_WORDS * S, stream);
+  const int64_t amax_floats = SJHIP_PW_AMAX_FLOATS + SJHIP_PW_AMAX_SAMPLE_WORDS * S;
+  const bool map_with_weights = !batch_stats && !batches_tracked;  // the map does not wait for the convolution
+  if (map_with_weights)
+    rc = launch_pwconv_split_weight_f16_bn(weight, Cout, Cin, w.planes, x_amax, amax_floats,
+                                           BnEvalMap{gamma, beta, running_mean, running_var, eps, bn_map, (int)Cout}, stream);
+  else
+    rc = launch_pwconv_split_weight_f16(weight, Cout, Cin, 0, w.planes, x_amax, amax_floats, stream);
   if (rc == SJHIP_OK && x_amax) rc = launch_pwconv_amax(x, S, Cin * L, x_amax, stream);
   float *partial = batch_stats ? w.partial : nullptr;
   if (rc == SJHIP_OK)
     rc = launch_pwconv_gemm(w.planes, SJHIP_PW_F16 | 2, Cout, Cin, x_bits ? reinterpret_cast<const float *>(x_bits) : x, x_amax ? 2 : 1,
                             x_amax, S, L, y, partial, stream, x_bits != nullptr);
-  if (rc == SJHIP_OK)
+  if (rc == SJHIP_OK && !map_with_weights)
     rc = launch_bn_finalize(partial, w.rows, S * L, Cout, gamma, beta, eps, momentum, running_mean, running_var, bn_map, bn_map + Cout,
                             bn_map + 2 * Cout, bn_map + 3 * Cout, batches_tracked, stream);
   if (rc == SJHIP_OK)

@@ -144,3 +144,16 @@ def test_modules_take_the_fused_chain(train):
         assert 0.0 < float(b.mean()) < 1.0 and float((a != b).float().mean()) < 1e-3
         for p, q in zip([ga, *pa], [gb, *pb]):
             assert float((p - q).norm()) < 2e-2 * float(q.norm())
+
+
+def test_evaluation_map_made_with_the_weights(C):
+    """Without batch statistics the chain's first launch makes the batch norm's map: the bits of the finalizing launch."""
+    T, B, Cin, Cout, L = 2, 3, 20, 133, 8
+    x, w = seeded_randn((T, B, Cin, L), 20).cuda(), seeded_randn((Cout, Cin), 21).cuda()
+    gamma, beta = seeded_randn((Cout,), 22, 1.0, 0.2).cuda(), seeded_randn((Cout,), 23, 0.2, 0.2).cuda()
+    mean, var = seeded_randn((Cout,), 24).cuda(), seeded_randn((Cout,), 25).square().cuda()
+    v0 = torch.zeros((B, Cout, L), device="cuda")
+    for g, b in ((gamma, beta), (None, None)):
+        for before in (mean.clone(),):
+            _, _, y, bn_map, _ = C._chain_forward(x, None, x.shape, w, g, b, v0, (mean, var, False, 0.1, 1e-5), _spec(T), False, False, None)
+            assert torch.equal(bn_map, C._bn_map(y.flatten(0, 1), g, b, mean, var, False, 0.1, 1e-5)) and torch.equal(mean, before)
