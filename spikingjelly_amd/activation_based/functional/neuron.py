@@ -243,8 +243,16 @@ def _hip_replays(x2: torch.Tensor) -> bool:
     divide (``whole_group`` of ``csrc/sjhip_common.h``): only rows shorter than one vector keep the saved ``h_seq``."""
     if not configure.hip_backward_recompute:
         return False
-    width, steps = _replay_limits(x2.dtype, _hip_mode_flags(x2))
-    return width > 0 and x2.shape[1] >= width and x2.shape[0] <= steps
+    flags = _hip_mode_flags(x2)
+    width, steps = _replay_limits(x2.dtype, flags)
+    return width > 0 and _replays_row(x2.shape[1], width, flags) and x2.shape[0] <= steps
+
+
+def _replays_row(N: int, width: int, flags: int) -> bool:
+    """Rows of whole vectors and, where the saved ``h_seq`` holds what the replay recomputes, all that are not shorter than
+    one.  With fp32 state it does not: 16-bit storage rounds it, the gradients of the two routes differ (bf16 hard reset:
+    1.4e-2 in the 2-norm, spikes of rounded potentials at their threshold), and ragged rows keep the route they had."""
+    return N % width == 0 if flags & _REPLAY_POLICY_FLAGS else N >= width
 
 
 _native = None  # (extension module, resolver of surrogate ids), imported at the first call of a hip functional
@@ -281,7 +289,9 @@ def _native_sequence(neuron: int, x_seq: torch.Tensor, v: torch.Tensor, k: Optio
     if torch.is_grad_enabled() and (x_seq.requires_grad or v.requires_grad or (k is not None and k.requires_grad)):
         sg_id, sg_alpha = (_MULTI_LEVEL, 0.0) if surrogate_function is None else resolve(surrogate_function)
         if configure.hip_backward_recompute and dtype in _FLOAT_DTYPES:
-            steps = _replay_limits(dtype, mode)[1]
+            width, steps = _replay_limits(dtype, mode)
+            if mode & _REPLAY_POLICY_FLAGS and not (width and _replays_row(v.numel(), width, mode)):
+                steps = 0
     return module.neuron_sequence(x_seq, v, k, single, neuron, tau, v_threshold, float(v_reset), flags, sg_id, sg_alpha, store_v_seq,
                                   steps, extra)
 

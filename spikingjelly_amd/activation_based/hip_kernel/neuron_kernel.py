@@ -886,8 +886,10 @@ def replay_chunk(dtype: torch.dtype, T: int, N: int, flags: int) -> int:
     chunk = int(configure.hip_replay_chunk)
     if not configure.hip_backward_recompute or chunk <= 0 or T <= chunk:
         return 0
-    # (a row that the vector width does not divide is replayed like the whole vectors it begins with)
-    return chunk if L.recompute_preferred(dtype, chunk, N & ~7 if N > 8 else N, flags) else 0
+    # (a row that the vector width does not divide is replayed like the whole vectors it begins with, except where a saved
+    # h_seq would be rounded to the storage dtype: such rows keep that route)
+    whole = N if N <= 8 or flags & L.FLAG_FP32_STATE else N & ~7
+    return chunk if L.recompute_preferred(dtype, chunk, whole, flags) else 0
 
 
 def eager_multistep(neuron: int, x_seq: torch.Tensor, v_init: torch.Tensor, k: Optional[torch.Tensor], tau: float,

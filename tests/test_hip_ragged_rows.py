@@ -53,7 +53,10 @@ def test_ragged_rows_equal_padded_rows(kind, dtype, mode, N, T, monkeypatch):
     x, gs, gv = (t.to(dtype).cuda() for t in (x, gs, gv))
     cut = lambda t: t[..., :N].contiguous()
     gv = gv if N % 2 else None
-    want = _run(kind, x, gs, gv)
+    # 16-bit storage with fp32 state: a saved h_seq is rounded, a replayed one is not; ragged rows keep the saved route
+    with monkeypatch.context() as m:
+        m.setattr(configure, "hip_backward_recompute", mode != "fp32_state" or N % 8 == 0)
+        want = _run(kind, x, gs, gv)
     got = _run(kind, cut(x), cut(gs), None if gv is None else cut(gv))
     for name, a, b in zip(("spikes", "v", "v_seq", "grad_x"), got[:4], want[:4]):
         if b is not None:
