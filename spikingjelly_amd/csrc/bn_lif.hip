@@ -86,6 +86,7 @@ __device__ __forceinline__ void block_row_sums(float (&part)[4][kBnRowsMax][2], 
 // and elements j < skip of it belong to the group before.
 struct RowQuad {
   int first, skip;
+  __device__ __forceinline__ explicit RowQuad(int q) : first(4 * q), skip(0) {}  // (rows of a multiple of four)
   __device__ __forceinline__ RowQuad(int q, int L) : first(min(4 * q, L - 4)), skip(4 * q - min(4 * q, L - 4)) {}
 };
 __device__ __forceinline__ f32x4 load_row_quad(const float *row, int q, int L) {
@@ -275,13 +276,15 @@ __device__ __forceinline__ void replay_h_charge(const FwdArgs &f, int len, const
 }
 
 // BPTT over the replayed h (recurrence of neuron_bwd.h); writes g = dL/dz and adds every neuron's share of
-// sum g and sum g y (four sums, because a neuron that a neighbour has too is counted once).  PLIF: also of dL/dk = sum G_t dh_t/dk, dh_t/dk = (h_t - v_{t-1}) / k with input decay (the division
+// sum g and sum g y.  SUMS: one sum of the four neurons, or (ragged rows) one of each, because a neuron that a neighbour has
+// too is counted once; whole rows keep the order, and with it the bits, of a single sum (four: 184 instead of 182 us for the two
+// backwards of an attention block [4, 64, 384, 196]).  PLIF: also of dL/dk = sum G_t dh_t/dk, dh_t/dk = (h_t - v_{t-1}) / k with input decay (the division
 // is left to the final reduction) or v_reset - v_{t-1} without; v_{t-1} is re-derived from h_{t-1} with the forward's
 // reset arithmetic, v0 is the state in front of the first of these steps.
-template <int SG, int TMAX, bool PLIF>
+template <int SG, int TMAX, bool PLIF, int SUMS>
 __device__ __forceinline__ void bptt_rows(const BwdArgs &b, float k, int64_t col, int64_t t0, int len, const f32x4 (&yv)[TMAX],
-                                          const float (&h)[TMAX][4], const float (&v0)[4], float (&carry)[4], float (&acc_g)[4],
-                                          float (&acc_gy)[4], float (&acc_k)[4]) {
+                                          const float (&h)[TMAX][4], const float (&v0)[4], float (&carry)[4], float (&acc_g)[SUMS],
+                                          float (&acc_gy)[SUMS], float (&acc_k)[SUMS]) {
 #pragma clang fp contract(fast)
   typedef Acc<float, true, true> A;
   const int64_t N = b.N;
@@ -304,15 +307,16 @@ __device__ __forceinline__ void bptt_rows(const BwdArgs &b, float k, int64_t col
         const float G = carry[j] * dvdh + gs[j] * sg;
         gz[j] = G * kx;
         carry[j] = G * km;
-        acc_g[j] += gz[j];
-        acc_gy[j] = fmaf(gz[j], y[j], acc_gy[j]);
+        const int n = SUMS == 1 ? 0 : j;
+        acc_g[n] += gz[j];
+        acc_gy[n] = fmaf(gz[j], y[j], acc_gy[n]);
         if constexpr (PLIF) {
           float v_prev = v0[j];
           if (t > 0) {
             const float h_prev = h[t > 0 ? t - 1 : 0][j];
             v_prev = reset_as_forward(h_prev, (h_prev - b.v_th >= 0.0f) ? 1.0f : 0.0f, b);
           }
-          acc_k[j] = fmaf(G, b.decay_input ? (h[t][j] - v_prev) : (b.v_reset - v_prev), acc_k[j]);
+          acc_k[n] = fmaf(G, b.decay_input ? (h[t][j] - v_prev) : (b.v_reset - v_prev), acc_k[n]);
         }
       }
       Acc<float, true, false>::store(gxp + (int64_t)t * N, gz);  // read again by the next kernel
@@ -320,18 +324,18 @@ __device__ __forceinline__ void bptt_rows(const BwdArgs &b, float k, int64_t col
   }
 }
 
-template <int TMAX, bool PLIF>
+template <int TMAX, bool PLIF, int SUMS>
 __device__ __forceinline__ void bptt_rows_surrogate(const BwdArgs &b, float k, int64_t col, int64_t t0, int len,
                                                     const f32x4 (&yv)[TMAX], const float (&h)[TMAX][4], const float (&v0)[4],
-                                                    float (&carry)[4], float (&acc_g)[4], float (&acc_gy)[4], float (&acc_k)[4]) {
+                                                    float (&carry)[4], float (&acc_g)[SUMS], float (&acc_gy)[SUMS], float (&acc_k)[SUMS]) {
   switch (b.sg) {
-    case SJHIP_SG_SIGMOID: bptt_rows<SJHIP_SG_SIGMOID, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
-    case SJHIP_SG_ATAN: bptt_rows<SJHIP_SG_ATAN, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
-    case SJHIP_SG_PIECEWISE_QUADRATIC: bptt_rows<SJHIP_SG_PIECEWISE_QUADRATIC, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
-    case SJHIP_SG_PIECEWISE_EXP: bptt_rows<SJHIP_SG_PIECEWISE_EXP, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
-    case SJHIP_SG_SOFT_SIGN: bptt_rows<SJHIP_SG_SOFT_SIGN, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
-    case SJHIP_SG_SUPER_SPIKE: bptt_rows<SJHIP_SG_SUPER_SPIKE, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
-    default: bptt_rows<SJHIP_SG_ERF, TMAX, PLIF>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
+    case SJHIP_SG_SIGMOID: bptt_rows<SJHIP_SG_SIGMOID, TMAX, PLIF, SUMS>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
+    case SJHIP_SG_ATAN: bptt_rows<SJHIP_SG_ATAN, TMAX, PLIF, SUMS>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
+    case SJHIP_SG_PIECEWISE_QUADRATIC: bptt_rows<SJHIP_SG_PIECEWISE_QUADRATIC, TMAX, PLIF, SUMS>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
+    case SJHIP_SG_PIECEWISE_EXP: bptt_rows<SJHIP_SG_PIECEWISE_EXP, TMAX, PLIF, SUMS>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
+    case SJHIP_SG_SOFT_SIGN: bptt_rows<SJHIP_SG_SOFT_SIGN, TMAX, PLIF, SUMS>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
+    case SJHIP_SG_SUPER_SPIKE: bptt_rows<SJHIP_SG_SUPER_SPIKE, TMAX, PLIF, SUMS>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
+    default: bptt_rows<SJHIP_SG_ERF, TMAX, PLIF, SUMS>(b, k, col, t0, len, yv, h, v0, carry, acc_g, acc_gy, acc_k); break;
   }
 }
 
@@ -340,9 +344,10 @@ __device__ __forceinline__ void fold_shares(const float (&share)[4], int skip, f
 #pragma unroll
   for (int j = 0; j < 4; ++j) sum += j >= skip ? share[j] : 0.0f;
 }
+__device__ __forceinline__ void fold_shares(const float (&share)[1], int, float &sum) { sum += share[0]; }
 
 // One work-item's four neurons (quad q of row `row`) for all T steps: replay, BPTT, g written, the sums extended.
-template <int TMAX, bool PLIF>
+template <int TMAX, bool PLIF, int SUMS>
 __device__ __forceinline__ void bn_lif_backward_quad(const BnLifBwdArgs &a, int64_t row, int q, float &acc_g, float &acc_gy,
                                                      float &acc_k) {
   typedef Acc<float, true, false> A;
@@ -352,7 +357,7 @@ __device__ __forceinline__ void bn_lif_backward_quad(const BnLifBwdArgs &a, int6
   const float sc = a.scale[c], sh = a.shift[c];
   const float k = (PLIF && b.k_device) ? *b.k_device : b.k;
   const int64_t N = f.N;
-  const RowQuad quad(q, a.L);
+  const RowQuad quad = SUMS == 1 ? RowQuad(q) : RowQuad(q, a.L);
   const int64_t col = row * a.L + quad.first;
   const float *yp = (const float *)f.x + col;
   f32x4 yv[TMAX];
@@ -364,8 +369,8 @@ __device__ __forceinline__ void bn_lif_backward_quad(const BnLifBwdArgs &a, int6
   if (b.grad_v_last) A::unpack(A::load((const float *)b.grad_v_last + col), carry);
   else carry[0] = carry[1] = carry[2] = carry[3] = 0.0f;
   replay_h_charge<TMAX>(f, (int)f.T, yv, sc, sh, v, h);
-  float g[4] = {}, gy[4] = {}, gk[4] = {};
-  bptt_rows_surrogate<TMAX, PLIF>(b, k, col, 0, (int)b.T, yv, h, v0, carry, g, gy, gk);
+  float g[SUMS] = {}, gy[SUMS] = {}, gk[SUMS] = {};
+  bptt_rows_surrogate<TMAX, PLIF, SUMS>(b, k, col, 0, (int)b.T, yv, h, v0, carry, g, gy, gk);
   fold_shares(g, quad.skip, acc_g);
   fold_shares(gy, quad.skip, acc_gy);
   if (PLIF) fold_shares(gk, quad.skip, acc_k);
@@ -378,7 +383,7 @@ __device__ __forceinline__ void bn_lif_backward_quad(const BnLifBwdArgs &a, int6
 // replayed from its parked state into registers and walked backwards; y is read twice.
 constexpr int kBnPiece = 16;
 constexpr int kBnMaxPieces = 16;  // 256 work-items x 16 bytes x 16 pieces = 64 KiB of LDS
-template <bool PLIF>
+template <bool PLIF, int SUMS>
 __device__ __forceinline__ void bn_lif_backward_quad_long(const BnLifBwdArgs &a, int64_t row, int q, float &acc_g, float &acc_gy,
                                                           float &acc_k, f32x4 *parked) {
   typedef Acc<float, true, false> A;
@@ -387,7 +392,7 @@ __device__ __forceinline__ void bn_lif_backward_quad_long(const BnLifBwdArgs &a,
   const int c = (int)(row % a.C);
   const float sc = a.scale[c], sh = a.shift[c];
   const int64_t N = f.N;
-  const RowQuad quad(q, a.L);
+  const RowQuad quad = SUMS == 1 ? RowQuad(q) : RowQuad(q, a.L);
   const int64_t col = row * a.L + quad.first;
   const float *yp = (const float *)f.x + col;
   const int T = (int)f.T, pieces = (T + kBnPiece - 1) / kBnPiece;
@@ -403,7 +408,7 @@ __device__ __forceinline__ void bn_lif_backward_quad_long(const BnLifBwdArgs &a,
   parked[(pieces - 1) * blockDim.x] = f32x4{v[0], v[1], v[2], v[3]};
   if (b.grad_v_last) A::unpack(A::load((const float *)b.grad_v_last + col), carry);
   else carry[0] = carry[1] = carry[2] = carry[3] = 0.0f;
-  float g[4] = {}, gy[4] = {}, gk[4] = {};
+  float g[SUMS] = {}, gy[SUMS] = {}, gk[SUMS] = {};
   for (int p = pieces - 1; p >= 0; --p) {
     const int t0 = p * kBnPiece, len = min(kBnPiece, T - t0);
 #pragma unroll
@@ -412,7 +417,7 @@ __device__ __forceinline__ void bn_lif_backward_quad_long(const BnLifBwdArgs &a,
     v[0] = s.x; v[1] = s.y; v[2] = s.z; v[3] = s.w;
     const float v0[4] = {s.x, s.y, s.z, s.w};
     replay_h_charge<kBnPiece>(f, len, yv, sc, sh, v, h);
-    bptt_rows_surrogate<kBnPiece, PLIF>(b, (PLIF && b.k_device) ? *b.k_device : b.k, col, t0, len, yv, h, v0, carry, g, gy, gk);
+    bptt_rows_surrogate<kBnPiece, PLIF, SUMS>(b, (PLIF && b.k_device) ? *b.k_device : b.k, col, t0, len, yv, h, v0, carry, g, gy, gk);
   }
   fold_shares(g, quad.skip, acc_g);
   fold_shares(gy, quad.skip, acc_gy);
@@ -424,7 +429,7 @@ __device__ __forceinline__ void bn_lif_backward_quad_long(const BnLifBwdArgs &a,
 // (TMAX = 0: the walk in pieces, with pieces x 256 x 16 bytes of dynamic LDS)
 // PLIF: every wavefront also leaves its share of dL/dk in k_partial[4 * block + wavefront] (summed afterwards in a fixed
 // order by plif_reduce_kernel, which also divides by k where the charge calls for it).
-template <int TMAX, bool PLIF> __global__ void __launch_bounds__(256) bn_lif_backward_kernel(const BnLifBwdArgs a) {
+template <int TMAX, bool PLIF, int SUMS> __global__ void __launch_bounds__(256) bn_lif_backward_kernel(const BnLifBwdArgs a) {
   extern __shared__ f32x4 parked_states[];
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -434,8 +439,8 @@ template <int TMAX, bool PLIF> __global__ void __launch_bounds__(256) bn_lif_bac
   }
   float acc_g = 0.0f, acc_gy = 0.0f, acc_k = 0.0f;
   for (int q = lane; q < (a.L + 3) / 4; q += 64) {
-    if constexpr (TMAX == 0) bn_lif_backward_quad_long<PLIF>(a, row, q, acc_g, acc_gy, acc_k, parked_states + threadIdx.x);
-    else bn_lif_backward_quad<TMAX, PLIF>(a, row, q, acc_g, acc_gy, acc_k);
+    if constexpr (TMAX == 0) bn_lif_backward_quad_long<PLIF, SUMS>(a, row, q, acc_g, acc_gy, acc_k, parked_states + threadIdx.x);
+    else bn_lif_backward_quad<TMAX, PLIF, SUMS>(a, row, q, acc_g, acc_gy, acc_k);
   }
   acc_g = wave_sum(acc_g);
   acc_gy = wave_sum(acc_gy);
@@ -452,7 +457,7 @@ template <int TMAX, bool PLIF> __global__ void __launch_bounds__(256) bn_lif_bac
 // quads: 245 working); a row's sums are formed per wavefront (a wavefront holds parts of a few rows: one masked
 // reduction per row it touches), left in LDS, and added over the wavefronts in their order by one work-item per row,
 // so the result does not depend on timing.
-template <int TMAX, bool PLIF>
+template <int TMAX, bool PLIF, int SUMS>
 __global__ void __launch_bounds__(256) bn_lif_backward_rows_kernel(const BnLifBwdArgs a, int quads, int rows_per_block,
                                                                    float inv_quads) {
   __shared__ float part[4][kBnRowsMax][2];
@@ -465,8 +470,8 @@ __global__ void __launch_bounds__(256) bn_lif_backward_rows_kernel(const BnLifBw
   if (r_local >= rows_per_block) r_local = rows_per_block - 1;
   float acc_g = 0.0f, acc_gy = 0.0f, acc_k = 0.0f;
   if (valid) {
-    if constexpr (TMAX == 0) bn_lif_backward_quad_long<PLIF>(a, row, q, acc_g, acc_gy, acc_k, parked_states + tid);
-    else bn_lif_backward_quad<TMAX, PLIF>(a, row, q, acc_g, acc_gy, acc_k);
+    if constexpr (TMAX == 0) bn_lif_backward_quad_long<PLIF, SUMS>(a, row, q, acc_g, acc_gy, acc_k, parked_states + tid);
+    else bn_lif_backward_quad<TMAX, PLIF, SUMS>(a, row, q, acc_g, acc_gy, acc_k);
   }
   if (PLIF) {
     acc_k = wave_sum(acc_k);
@@ -697,30 +702,33 @@ int launch_bn_lif_backward(int neuron, const sjhip_neuron_params &p, int64_t T, 
   const int quads = (int)((L + 3) / 4);
   const int per = quads > 0 ? 256 / quads : 0;
   // TMAX by sequence length (0: the walk in pieces), with or without the dL/dk term
-  auto launch = [&](auto rows_kernel, auto plif_flag) {
+  auto launch = [&](auto rows_kernel, auto plif_flag, auto ragged) {
     constexpr bool ROWS = decltype(rows_kernel)::value, P = decltype(plif_flag)::value;
+    constexpr int S = decltype(ragged)::value ? 4 : 1;
     const int64_t nb = ROWS ? (a.rows + per - 1) / per : blocks;
     const float inv = quads > 0 ? 1.0f / (float)quads : 0.0f;
     const dim3 grid((unsigned)nb), threads(256);
     if constexpr (ROWS) {
-      if (T <= 4) hipLaunchKernelGGL((bn_lif_backward_rows_kernel<4, P>), grid, threads, 0, stream, a, quads, per, inv);
-      else if (T <= 8) hipLaunchKernelGGL((bn_lif_backward_rows_kernel<8, P>), grid, threads, 0, stream, a, quads, per, inv);
-      else if (T <= 16) hipLaunchKernelGGL((bn_lif_backward_rows_kernel<16, P>), grid, threads, 0, stream, a, quads, per, inv);
-      else hipLaunchKernelGGL((bn_lif_backward_rows_kernel<0, P>), grid, threads, parked, stream, a, quads, per, inv);
+      if (T <= 4) hipLaunchKernelGGL((bn_lif_backward_rows_kernel<4, P, S>), grid, threads, 0, stream, a, quads, per, inv);
+      else if (T <= 8) hipLaunchKernelGGL((bn_lif_backward_rows_kernel<8, P, S>), grid, threads, 0, stream, a, quads, per, inv);
+      else if (T <= 16) hipLaunchKernelGGL((bn_lif_backward_rows_kernel<16, P, S>), grid, threads, 0, stream, a, quads, per, inv);
+      else hipLaunchKernelGGL((bn_lif_backward_rows_kernel<0, P, S>), grid, threads, parked, stream, a, quads, per, inv);
     } else {
-      if (T <= 4) hipLaunchKernelGGL((bn_lif_backward_kernel<4, P>), grid, threads, 0, stream, a);
-      else if (T <= 8) hipLaunchKernelGGL((bn_lif_backward_kernel<8, P>), grid, threads, 0, stream, a);
-      else if (T <= 16) hipLaunchKernelGGL((bn_lif_backward_kernel<16, P>), grid, threads, 0, stream, a);
-      else hipLaunchKernelGGL((bn_lif_backward_kernel<0, P>), grid, threads, parked, stream, a);
+      if (T <= 4) hipLaunchKernelGGL((bn_lif_backward_kernel<4, P, S>), grid, threads, 0, stream, a);
+      else if (T <= 8) hipLaunchKernelGGL((bn_lif_backward_kernel<8, P, S>), grid, threads, 0, stream, a);
+      else if (T <= 16) hipLaunchKernelGGL((bn_lif_backward_kernel<16, P, S>), grid, threads, 0, stream, a);
+      else hipLaunchKernelGGL((bn_lif_backward_kernel<0, P, S>), grid, threads, parked, stream, a);
     }
     return nb;
   };
   // more than the four rows a block of the wavefront-per-row kernel takes: more lanes working
   const bool by_rows = per > 4 && per <= kBnRowsMax;
   if (by_rows && (a.rows + per - 1) / per > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "bn_lif_backward: %lld rows", (long long)a.rows);
-  int64_t nb;
-  if (by_rows) nb = plif ? launch(std::true_type(), std::true_type()) : launch(std::true_type(), std::false_type());
-  else nb = plif ? launch(std::false_type(), std::true_type()) : launch(std::false_type(), std::false_type());
+  auto by_shape = [&](auto plif_flag, auto ragged) {
+    return by_rows ? launch(std::true_type(), plif_flag, ragged) : launch(std::false_type(), plif_flag, ragged);
+  };
+  auto by_row = [&](auto plif_flag) { return L % 4 != 0 ? by_shape(plif_flag, std::true_type()) : by_shape(plif_flag, std::false_type()); };
+  const int64_t nb = plif ? by_row(std::true_type()) : by_row(std::false_type());
   rc = check_launch("bn_lif_backward");
   if (rc != SJHIP_OK || !plif) return rc;
   return launch_plif_reduce(a.b, 4 * nb, grad_k, stream);
