@@ -149,7 +149,9 @@ py::object neuron_sequence(const Tensor &x_seq, const Tensor &v_init, const c10:
   const Tensor k = k_opt.has_value() ? *k_opt : Tensor();
   const bool grad = at::GradMode::is_enabled() && (x_seq.requires_grad() || v_init.requires_grad() || (k.defined() && k.requires_grad()));
   const bool broadcast = is_broadcast(v_init);
-  if (torch::autograd::isFwGradDefined(v_init) || (!broadcast && !v_init.is_contiguous())) return py::none();
+  if (torch::autograd::isFwGradDefined(v_init) || (k.defined() && torch::autograd::isFwGradDefined(k)) ||
+      (!broadcast && !v_init.is_contiguous()))
+    return py::none();
   if (k.defined() && (k.scalar_type() != at::kFloat || k.device() != x_seq.device() || k.numel() != 1)) return py::none();
   if (grad && (T > replay_steps || N < (dtype == SJHIP_F32 ? 4 : 8))) return py::none();
 

@@ -118,6 +118,18 @@ def test_what_the_native_path_leaves_alone(monkeypatch):
     assert seen == [True]
 
 
+@pytest.mark.parametrize("dual", ["x", "v", "w"])
+def test_forward_mode_derivatives_are_refused_not_dropped(dual):
+    """The kernels carry no tangents: a call that would have to produce one raises, whichever argument brings it."""
+    import torch.autograd.forward_ad as fwAD
+
+    t = {"x": torch.randn(4, 64, device="cuda"), "v": torch.zeros(64, device="cuda"), "w": torch.tensor(0.2, device="cuda")}
+    with fwAD.dual_level():
+        t[dual] = fwAD.make_dual(t[dual].requires_grad_(), torch.ones_like(t[dual]))
+        with pytest.raises(NotImplementedError, match="jvp"):
+            functional.plif_multi_step_hip(t["x"], t["v"], t["w"], True, 1.0, 0.0, surrogate.ATan())
+
+
 def test_saved_tensors_go_through_hooks_and_are_freed():
     packed = []
     x = torch.randn(4, 64, device="cuda").requires_grad_()
