@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/torch.h>
 
@@ -56,8 +57,8 @@ bool plain(const Tensor &t) {
   return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has(c10::DispatchKey::Python) && !t.is_neg() &&
          !torch::autograd::isFwGradDefined(t);
 }
-bool transforms_active() {
-  return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+bool transforms_active() {  // (torch.jit.trace among them: a node made here would enter the trace as a constant)
+  return torch::jit::tracer::isTracing() || c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
          c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Python);
 }
 

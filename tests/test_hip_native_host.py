@@ -130,6 +130,16 @@ def test_forward_mode_derivatives_are_refused_not_dropped(dual):
             functional.plif_multi_step_hip(t["x"], t["v"], t["w"], True, 1.0, 0.0, surrogate.ATan())
 
 
+def test_traced_call_follows_its_input():
+    """``torch.jit.trace`` records the autograd function; an untraced call would leave its result in the trace as a constant."""
+    x, v = torch.randn(4, 64, device="cuda").requires_grad_(), torch.zeros(64, device="cuda")
+    fn = lambda t: functional.lif_multi_step_hip(t, v, 2.0, True, 1.0, 0.0, surrogate.ATan())[0]
+    traced = torch.jit.trace(fn, (x,), check_trace=False)
+    for shift in (0.0, 1.0, 3.0):
+        y = (x.detach() + shift).requires_grad_()
+        assert torch.equal(traced(y), fn(y))
+
+
 def test_saved_tensors_go_through_hooks_and_are_freed():
     packed = []
     x = torch.randn(4, 64, device="cuda").requires_grad_()
