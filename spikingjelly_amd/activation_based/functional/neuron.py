@@ -266,8 +266,10 @@ def _native_sequence(neuron: int, x_seq: torch.Tensor, v: torch.Tensor, k: Optio
                      store_v_seq: bool, single: bool = False, extra: tuple = _NO_EXTRA):
     """One eager call through the native host path (``csrc/torch_binding.cpp``): ``(spike_seq, v_next, v_seq or None)`` in the
     shapes of ``x_seq``, or ``None`` when it does not serve the call (the general path below then does: layouts that need a
-    copy, a saved ``h_seq``, a sequence replayed in pieces, function transforms).  ``single``: ``x_seq`` is one step.
+    copy, a saved ``h_seq``, a sequence replayed in pieces, function transforms, tensor subclasses).  ``single``: ``x_seq`` is one step.
     ``surrogate_function`` ``None``: the windowed gradient of the integer-valued neuron, whose limits are in ``extra``."""
+    if type(x_seq) not in _PLAIN_TYPES:
+        return None
     global _native
     if _native is None:
         from ..hip_kernel import native
@@ -297,6 +299,8 @@ def _native_sequence(neuron: int, x_seq: torch.Tensor, v: torch.Tensor, k: Optio
 
 
 _FLOAT_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
+# (results of a subclass of torch.Tensor are of that subclass: the general path makes them with its __torch_function__)
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
 def _native_packed(neuron: int, x_seq: torch.Tensor, v: torch.Tensor, k: Optional[torch.Tensor], tau: float, v_threshold: float,
@@ -304,6 +308,8 @@ def _native_packed(neuron: int, x_seq: torch.Tensor, v: torch.Tensor, k: Optiona
     """The same for inference with bit-packed spikes: ``(spike_bits, v_next, v_seq or None)`` or ``None``."""
     from ..hip_kernel import native
 
+    if type(x_seq) not in _PLAIN_TYPES:
+        return None
     flags = _hip_mode_flags(x_seq) | (0x02 if v_reset is None else 0) | (0x01 if decay_input else 0)
     return native.load().neuron_sequence_packed(x_seq, v, k, neuron, tau, v_threshold, 0.0 if v_reset is None else float(v_reset),
                                                 flags, store_v_seq)

@@ -140,6 +140,22 @@ def test_traced_call_follows_its_input():
         assert torch.equal(traced(y), fn(y))
 
 
+class _Tagged(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_results_keep_the_type_of_a_tensor_subclass(grad):
+    x, v = torch.randn(4, 64, device="cuda").as_subclass(_Tagged).requires_grad_(grad), torch.zeros(64, device="cuda")
+    out = functional.lif_multi_step_hip(x, v, 2.0, True, 1.0, 0.0, surrogate.ATan(), store_v_seq=True)
+    assert [type(t) for t in out] == [_Tagged] * 3
+    step = functional.lif_step_hip(x[0], v, 2.0, True, 1.0, 0.0, surrogate.ATan())
+    assert [type(t) for t in step] == [_Tagged] * 2
+    if not grad:
+        _, v_last, v_seq = functional.lif_multi_step_hip_packed(x, v, 2.0, True, 1.0, 0.0, True)
+        assert type(v_last) is _Tagged and type(v_seq) is _Tagged
+
+
 def test_saved_tensors_go_through_hooks_and_are_freed():
     packed = []
     x = torch.randn(4, 64, device="cuda").requires_grad_()
