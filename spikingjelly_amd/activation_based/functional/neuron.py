@@ -267,7 +267,7 @@ def _native_sequence(neuron: int, x_seq: torch.Tensor, v: torch.Tensor, k: Optio
     """One eager call through the native host path (``csrc/torch_binding.cpp``): ``(spike_seq, v_next, v_seq or None)`` in the
     shapes of ``x_seq``, or ``None`` when it does not serve the call (the general path below then does: layouts that need a
     copy, a saved ``h_seq``, a sequence replayed in pieces, function transforms, tensor subclasses).  ``single``: ``x_seq`` is one step.
-    ``surrogate_function`` ``None``: the windowed gradient of the integer-valued neuron, whose limits are in ``extra``."""
+    The integer-valued neuron has no ``surrogate_function`` but a windowed gradient, whose limits are in ``extra``."""
     if type(x_seq) not in _PLAIN_TYPES:
         return None
     global _native
@@ -289,7 +289,7 @@ def _native_sequence(neuron: int, x_seq: torch.Tensor, v: torch.Tensor, k: Optio
         flags |= 0x01  # FLAG_DECAY_INPUT
     sg_id, sg_alpha, steps = 0, 0.0, 0
     if torch.is_grad_enabled() and (x_seq.requires_grad or v.requires_grad or (k is not None and k.requires_grad)):
-        sg_id, sg_alpha = (_MULTI_LEVEL, 0.0) if surrogate_function is None else resolve(surrogate_function)
+        sg_id, sg_alpha = (_MULTI_LEVEL, 0.0) if neuron == _ILIF else resolve(surrogate_function)
         if configure.hip_backward_recompute and dtype in _FLOAT_DTYPES:
             width, steps = _replay_limits(dtype, mode)
             if mode & _REPLAY_POLICY_FLAGS and not (width and _replays_row(v.numel(), width, mode)):

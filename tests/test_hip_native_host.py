@@ -140,6 +140,18 @@ def test_traced_call_follows_its_input():
         assert torch.equal(traced(y), fn(y))
 
 
+def test_training_call_without_a_surrogate_function_is_refused():
+    x, v, w = torch.randn(4, 64, device="cuda").requires_grad_(), torch.zeros(64, device="cuda"), torch.zeros((), device="cuda")
+    for call in (lambda: functional.if_multi_step_hip(x, v, 1.0, 0.0, None),
+                 lambda: functional.lif_multi_step_hip(x, v, 2.0, True, 1.0, 0.0, None),
+                 lambda: functional.plif_multi_step_hip(x, v, w, True, 1.0, 0.0, None),
+                 lambda: functional.lif_step_hip(x[0], v, 2.0, True, 1.0, 0.0, None)):
+        with pytest.raises(NotImplementedError, match="surrogate"):
+            call()
+        with torch.no_grad():
+            call()
+
+
 class _Tagged(torch.Tensor):
     pass
 
