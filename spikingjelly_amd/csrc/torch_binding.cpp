@@ -142,7 +142,7 @@ py::object neuron_sequence(const Tensor &x_seq, const Tensor &v_init, const c10:
                            double tau, double v_th, double v_reset, int64_t flags, int64_t sg_id, double sg_alpha, bool store_v_seq,
                            int64_t replay_steps, const std::array<double, 6> &extra) {
   const int dtype = dtype_id(x_seq.scalar_type());
-  if (dtype < 0 || x_seq.dim() < (single ? 0 : 1) || !plain(x_seq) || !x_seq.is_contiguous() || x_seq.numel() == 0 || transforms_active())
+  if (dtype < 0 || x_seq.dim() < (single ? 1 : 2) || !plain(x_seq) || !x_seq.is_contiguous() || x_seq.numel() == 0 || transforms_active())
     return py::none();
   const int64_t T = single ? 1 : x_seq.size(0), N = x_seq.numel() / T;
   const auto step = single ? x_seq.sizes() : x_seq.sizes().slice(1);
@@ -193,7 +193,7 @@ py::object neuron_sequence(const Tensor &x_seq, const Tensor &v_init, const c10:
 py::object neuron_sequence_packed(const Tensor &x_seq, const Tensor &v_init, const c10::optional<Tensor> &k_opt, int neuron, double tau,
                                   double v_th, double v_reset, int64_t flags, bool store_v_seq) {
   const int dtype = dtype_id(x_seq.scalar_type());
-  if (dtype < 0 || x_seq.dim() < 1 || !plain(x_seq) || !x_seq.is_contiguous() || x_seq.numel() == 0 || transforms_active()) return py::none();
+  if (dtype < 0 || x_seq.dim() < 2 || !plain(x_seq) || !x_seq.is_contiguous() || x_seq.numel() == 0 || transforms_active()) return py::none();
   const int64_t T = x_seq.size(0), N = x_seq.numel() / T;
   const auto step = x_seq.sizes().slice(1);
   const bool broadcast = is_broadcast(v_init);

@@ -152,6 +152,15 @@ def test_training_call_without_a_surrogate_function_is_refused():
             call()
 
 
+def test_sequences_without_a_neuron_dimension_are_refused():
+    x = torch.randn(4, device="cuda")
+    for call in (lambda: functional.lif_multi_step_hip(x, x[0], 2.0, True, 1.0, 0.0, surrogate.ATan()),
+                 lambda: functional.lif_step_hip(x[0], x[1], 2.0, True, 1.0, 0.0, surrogate.ATan()),
+                 lambda: functional.lif_multi_step_hip_packed(torch.randn(8, device="cuda"), x[0], 2.0, True, 1.0, 0.0)):
+        with pytest.raises(IndexError):
+            call()
+
+
 class _Tagged(torch.Tensor):
     pass
 
