@@ -73,11 +73,24 @@ bool is_broadcast(const Tensor &v) {
 
 Tensor empty(at::IntArrayRef sizes, const Tensor &like) { return at::empty(sizes, like.options()); }
 
+// dense and on 16 bytes
+Tensor dense16(const Tensor &t) {
+  const Tensor d = t.contiguous();
+  return aligned16(d) ? d : d.clone();
+}
+
 // A gradient as the kernels take it: dense, in the storage dtype, on 16 bytes.
 Tensor dense_grad(const Tensor &g, at::ScalarType dtype) {
   if (!g.defined()) return g;
-  Tensor d = g.to(dtype).contiguous();
-  return aligned16(d) ? d : d.clone();
+  return dense16(g.to(dtype));
+}
+
+// A saved tensor as the kernels take it.  A saved-tensor hook may hand the values back in another layout or type; what is
+// not on the device, or has another size, is refused before a kernel reads it.
+Tensor saved_values(const Tensor &t, const char *name, at::ScalarType dtype, int64_t numel) {
+  TORCH_CHECK(t.is_cuda(), "backend='hip' runs on a ROCm device only, but the saved ", name, " is on ", t.device());
+  TORCH_CHECK(t.layout() == at::kStrided && t.numel() == numel, "the saved ", name, " has ", t.numel(), " elements instead of ", numel);
+  return t.scalar_type() == dtype ? t : t.to(dtype);
 }
 
 const void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
@@ -85,7 +98,8 @@ const void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; 
 struct NeuronBackward : public torch::autograd::Node {
   SavedVariable x_, v_, k_;
   bool with_k = false;
-  sjhip_neuron_params params{};
+  sjhip_neuron_params params{};  // without SJHIP_FLAG_V_INIT_BROADCAST, which follows the state as it is unpacked
+  at::ScalarType storage = at::kFloat;
   int neuron = 0, dtype = 0;
   int64_t T = 0, N = 0;
 
@@ -101,13 +115,16 @@ struct NeuronBackward : public torch::autograd::Node {
     std::lock_guard<std::mutex> lock(mutex_);
     variable_list out(3);
     if (!grads[0].defined() && !grads[1].defined() && !grads[2].defined()) return out;
-    Tensor x = x_.unpack(), v = v_.unpack();
-    const Tensor k = with_k ? k_.unpack() : Tensor();
+    const Tensor saved_x = x_.unpack(), saved_v = v_.unpack(), saved_k = with_k ? k_.unpack() : Tensor();
     at::AutoDispatchBelowADInplaceOrView below;
-    c10::DeviceGuard guard(x.device());
+    c10::DeviceGuard guard(saved_x.device());
     // (the library asks for tensors that begin on 16 bytes; a step taken out of a sequence may not)
-    if (!aligned16(x)) x = x.clone();
-    if (!(params.flags & SJHIP_FLAG_V_INIT_BROADCAST) && !aligned16(v)) v = v.clone();
+    const Tensor x = dense16(saved_values(saved_x, "x_seq", storage, T * N));
+    Tensor v = saved_values(saved_v, "v_init", storage, N);
+    const Tensor k = with_k ? saved_values(saved_k, "k", at::kFloat, 1) : Tensor();
+    sjhip_neuron_params p = params;
+    if (is_broadcast(v)) p.flags |= SJHIP_FLAG_V_INIT_BROADCAST;
+    else v = dense16(v);
     const Tensor gs = dense_grad(grads[0], x.scalar_type()), glast = dense_grad(grads[1], x.scalar_type()),
                  gv = dense_grad(grads[2], x.scalar_type());
     const Tensor gx = at::empty_like(x);
@@ -115,14 +132,14 @@ struct NeuronBackward : public torch::autograd::Node {
     if (task_should_compute_output(1)) gv0 = empty(v.sizes(), x);
     if (with_k) {
       const auto f32 = x.options().dtype(at::kFloat);
-      if (params.flags & SJHIP_FLAG_ATOMIC_REDUCE) {
+      if (p.flags & SJHIP_FLAG_ATOMIC_REDUCE) {
         gk = at::zeros(k.sizes(), f32);
       } else {
         gk = at::empty(k.sizes(), f32);
         workspace = at::empty({sjhip_plif_workspace_floats(dtype, N)}, f32);
       }
     }
-    check(sjhip_neuron_backward_recompute(neuron, dtype, &params, T, N, ptr(x), ptr(v), static_cast<const float *>(ptr(k)), ptr(gs),
+    check(sjhip_neuron_backward_recompute(neuron, dtype, &p, T, N, ptr(x), ptr(v), static_cast<const float *>(ptr(k)), ptr(gs),
                                           ptr(gv), ptr(glast), gx.data_ptr(), gv0.defined() ? gv0.data_ptr() : nullptr,
                                           gk.defined() ? gk.data_ptr<float>() : nullptr,
                                           workspace.defined() ? workspace.data_ptr<float>() : nullptr, stream_of(x)),
@@ -179,6 +196,8 @@ py::object neuron_sequence(const Tensor &x_seq, const Tensor &v_init, const c10:
     node->with_k = k.defined();
     if (k.defined()) node->k_ = SavedVariable(k, false);
     node->params = p;
+    node->params.flags &= ~(uint32_t)SJHIP_FLAG_V_INIT_BROADCAST;
+    node->storage = x_seq.scalar_type();
     node->neuron = neuron; node->dtype = dtype; node->T = T; node->N = N;
     torch::autograd::set_history(spikes, node);
     torch::autograd::set_history(v_last, node);

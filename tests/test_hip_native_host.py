@@ -194,6 +194,42 @@ def test_saved_tensors_go_through_hooks_and_are_freed():
         s.sum().backward()
 
 
+def _reversed_strides(t):
+    out = torch.empty(t.shape[::-1], dtype=t.dtype, device=t.device).permute(*range(t.dim() - 1, -1, -1))
+    return out.copy_(t)
+
+
+@pytest.mark.parametrize("unpack", [_reversed_strides, lambda t: t.clone(memory_format=torch.contiguous_format), lambda t: t.double(),
+                                    lambda t: t[..., :1].clone().expand(t.shape) if t.dim() == 2 and bool((t == t.flatten()[0]).all()) else t,
+                                    lambda t: torch.cat([t.flatten()[:1], t.flatten()])[1:].view(t.shape)],
+                         ids=["strided", "dense", "double", "expanded", "off 16 bytes"])
+@pytest.mark.parametrize("state", ["one element", "constant", "dense"])
+def test_saved_tensors_come_back_in_any_layout(unpack, state):
+    g = torch.Generator().manual_seed(7)
+    x0, gs = (torch.randn(3, 8, 5, generator=g) + 0.4).cuda(), torch.randn(3, 8, 5, generator=g).cuda()
+    v0 = {"one element": torch.full((1, 1), 0.25).cuda().expand(8, 5), "constant": torch.full((8, 5), 0.25).cuda(),
+          "dense": (torch.randn(8, 5, generator=g) * 0.2).cuda()}[state]
+    results = []
+    for hook in (lambda t: t, lambda t: unpack(t) if t.dim() else t):  # (sigmoid(w), which sigmoid saves as well, stays as it is)
+        x, w = x0.clone().requires_grad_(), torch.tensor(0.2, device="cuda").requires_grad_()
+        v = v0 if state == "one element" else v0.clone().requires_grad_()
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, hook):
+            s = functional.plif_multi_step_hip(x, v, w, True, 1.0, 0.0, surrogate.ATan())[0]
+        s.backward(gs)
+        results.append([x.grad, v.grad, w.grad])
+    _equal(*results)
+
+
+@pytest.mark.parametrize("what", ["device", "size"])
+def test_saved_tensors_that_are_not_the_saved_ones_are_refused(what):
+    x = torch.randn(4, 64, device="cuda").requires_grad_()
+    unpack = (lambda t: t.cpu()) if what == "device" else (lambda t: t[..., :32].contiguous())
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        s = functional.lif_multi_step_hip(x, torch.zeros(64, device="cuda"), 2.0, True, 1.0, 0.0, surrogate.ATan())[0]
+    with pytest.raises(RuntimeError, match="saved x_seq"):
+        s.sum().backward()
+
+
 def test_packed_inference_equals_the_operator():
     x = (torch.rand(6, 5, 16, device="cuda") * 0.6).half()
     v = torch.zeros(5, 16, dtype=torch.float16, device="cuda")
