@@ -877,6 +877,37 @@ class _EagerNeuron(torch.autograd.Function):
         return gx, (gvi if need else None), gk, None
 
 
+def backward_as_operator(neuron: int, grad_spike_seq: Optional[torch.Tensor], grad_v_seq: Optional[torch.Tensor],
+                         grad_v_last: Optional[torch.Tensor], x_seq: torch.Tensor, v_init: torch.Tensor, k: Optional[torch.Tensor],
+                         single: bool, params: tuple, need_grad_v_init: bool
+                         ) -> tuple[torch.Tensor, Optional[torch.Tensor], Optional[torch.Tensor]]:
+    """The backward of a node of the native host path as a call of the traceable operators, for a compiler that records the
+    backward graph (compiled autograd): ``(grad_x_seq, grad_v_init, grad_k)`` in the shapes of the inputs.  ``single``: they
+    have no time dimension.  ``params``: the fields of ``sjhip_neuron_params`` in their order."""
+    tau, v_th, v_reset, sg_alpha, sg_id, flags, *extra = params
+    T = 1 if single else x_seq.shape[0]
+    rows = lambda t: None if t is None else t.reshape(T, -1)
+    tensors = (rows(grad_spike_seq), rows(grad_v_seq), None if grad_v_last is None else grad_v_last.reshape(-1), None, rows(x_seq),
+               v_init.reshape(-1))
+    mode = flags & (L.FLAG_FP32_STATE | L.FLAG_RECIPROCAL_TAU | L.FLAG_ATOMIC_REDUCE)
+    soft, detach, decay = (bool(flags & f) for f in (L.FLAG_SOFT_RESET, L.FLAG_DETACH_RESET, L.FLAG_DECAY_INPUT))
+    last, gk = (sg_id, sg_alpha, mode, need_grad_v_init), None
+    if neuron == L.NEURON_IF:
+        gx, gvi = hip_multistep_if_backward(*tensors, v_th, v_reset, soft, detach, *last)
+    elif neuron == L.NEURON_LIF:
+        gx, gvi = hip_multistep_lif_backward(*tensors, v_th, v_reset, soft, detach, tau, decay, *last)
+    elif neuron == L.NEURON_PLIF:
+        gx, gvi, gk = hip_multistep_plif_backward(*tensors, k, v_th, v_reset, soft, detach, decay, *last)
+        gk = gk.reshape(k.shape)
+    elif neuron == L.NEURON_QIF:
+        gx, gvi = hip_multistep_qif_backward(*tensors, v_th, v_reset, soft, detach, tau, *extra[:3], *last)
+    elif neuron == L.NEURON_EIF:
+        gx, gvi = hip_multistep_eif_backward(*tensors, v_th, v_reset, soft, detach, tau, *extra[:3], *last)
+    else:
+        gx, gvi = hip_multistep_ilif_backward(*tensors, tau, v_th, int(extra[3]), extra[4], extra[5], detach, mode, need_grad_v_init)
+    return gx.reshape(x_seq.shape), gvi.reshape(v_init.shape) if need_grad_v_init else None, gk
+
+
 def replay_chunk(dtype: torch.dtype, T: int, N: int, flags: int) -> int:
     """Steps per piece when a sequence of ``T`` steps should be replayed piece by piece in the backward, else 0: the
     replay is switched on, one piece of the configured length is a shape the replay kernel prefers, and the sequence

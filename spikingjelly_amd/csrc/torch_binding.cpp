@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/dynamo/compiled_autograd.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 #include <torch/torch.h>
@@ -97,7 +98,7 @@ const void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; 
 
 struct NeuronBackward : public torch::autograd::Node {
   SavedVariable x_, v_, k_;
-  bool with_k = false;
+  bool with_k = false, single = false;  // single: one step without a time dimension
   sjhip_neuron_params params{};  // without SJHIP_FLAG_V_INIT_BROADCAST, which follows the state as it is unpacked
   at::ScalarType storage = at::kFloat;
   int neuron = 0, dtype = 0;
@@ -149,6 +150,47 @@ struct NeuronBackward : public torch::autograd::Node {
     if (with_k && task_should_compute_output(2)) out[2] = gk;
     return out;
   }
+
+  // Compiled autograd records the backward graph instead of running it: what the node holds (scalars are constants of the
+  // graph), and the same backward as a call of the traceable operators.
+  void compiled_args(torch::dynamo::autograd::CompiledNodeArgs &args) const override {
+    args.collect(x_, false);
+    args.collect(v_, false);
+    args.collect(with_k);
+    if (with_k) args.collect(k_, false);
+    args.collect(single);
+    args.collect((int64_t)neuron);
+    args.collect((int64_t)params.sg_id);
+    args.collect((int64_t)params.flags);
+    for (float f : {params.tau, params.v_threshold, params.v_reset, params.sg_alpha, params.v_rest, params.v_c, params.a0, params.level_max,
+                    params.grad_min, params.grad_max})
+      args.collect((double)f);
+  }
+  variable_list apply_with_saved(const variable_list &grads, torch::dynamo::autograd::SwapSavedVariables &saved) override {
+    saved.before(x_);
+    saved.before(v_);
+    if (with_k) saved.before(k_);
+    variable_list out(3);
+    if (grads[0].defined() || grads[1].defined() || grads[2].defined()) {
+      py::gil_scoped_acquire gil;
+      auto arg = [](const Tensor &t) { return t.defined() ? py::cast(t) : py::object(py::none()); };
+      const auto result = py::cast<std::tuple<Tensor, c10::optional<Tensor>, c10::optional<Tensor>>>(
+          py::module_::import("spikingjelly_amd.activation_based.hip_kernel.neuron_kernel")
+              .attr("backward_as_operator")(neuron, arg(grads[0]), arg(grads[2]), arg(grads[1]), x_.unpack(), v_.unpack(),
+                                            arg(with_k ? k_.unpack() : Tensor()), single,
+                                            py::make_tuple(params.tau, params.v_threshold, params.v_reset, params.sg_alpha, params.sg_id,
+                                                           params.flags, params.v_rest, params.v_c, params.a0, params.level_max,
+                                                           params.grad_min, params.grad_max),
+                                            should_compute_output(1)));
+      if (should_compute_output(0)) out[0] = std::get<0>(result);
+      if (should_compute_output(1)) out[1] = *std::get<1>(result);
+      if (with_k && should_compute_output(2)) out[2] = *std::get<2>(result);
+    }
+    saved.after(x_);
+    saved.after(v_);
+    if (with_k) saved.after(k_);
+    return out;
+  }
 };
 
 // (spikes, v after the last step, v after every step or None), or None when the general path has to serve.
@@ -194,6 +236,7 @@ py::object neuron_sequence(const Tensor &x_seq, const Tensor &v_init, const c10:
     node->x_ = SavedVariable(x_seq, false);
     node->v_ = SavedVariable(v_init, false);
     node->with_k = k.defined();
+    node->single = single;
     if (k.defined()) node->k_ = SavedVariable(k, false);
     node->params = p;
     node->params.flags &= ~(uint32_t)SJHIP_FLAG_V_INIT_BROADCAST;

@@ -194,6 +194,45 @@ def test_saved_tensors_go_through_hooks_and_are_freed():
         s.sum().backward()
 
 
+def _calls(x, v, w):
+    sg = surrogate.ATan()
+    levels = surrogate.MultiLevelSpikeCount(4)
+    return {
+        "if": lambda: functional.if_multi_step_hip(x, v, 1.0, None, sg, True),
+        "lif": lambda: functional.lif_multi_step_hip(x, v, 2.0, True, 1.0, 0.0, sg, store_v_seq=True),
+        "plif": lambda: functional.plif_multi_step_hip(x, v, w, False, 1.0, 0.0, sg),
+        "qif": lambda: functional.qif_multi_step_hip(x, v, 2.0, 1.0, 0.0, 0.0, 0.8, 1.0, False, sg),
+        "eif": lambda: functional.eif_multi_step_hip(x, v, 2.0, 1.0, 0.0, 0.0, 0.8, 1.0, False, sg),
+        "ilif": lambda: functional.ilif_multi_step_hip(x, v, 2.0, 1.0, levels),
+        "step": lambda: functional.lif_step_hip(x[0], v, 2.0, True, 1.0, 0.0, sg),
+    }
+
+
+@pytest.mark.parametrize("compiler", ["graph module", "eager", "aot_eager"])
+@pytest.mark.parametrize("kind", ["if", "lif", "plif", "qif", "eif", "ilif", "step"])
+def test_compiled_autograd_records_the_operators(kind, compiler):
+    """Compiled autograd asks a C++ node for its arguments and for its backward on recorded tensors."""
+    from torch._dynamo import compiled_autograd
+
+    torch._dynamo.reset()
+    enable = (lambda gm: gm) if compiler == "graph module" else torch.compile(backend=compiler)
+    g = torch.Generator().manual_seed(8)
+    for T, v_th in ((4, 1.0), (3, 1.0)):
+        x0, v0 = (torch.randn(T, 8, 5, generator=g) + 0.4).cuda(), (torch.randn(8, 5, generator=g) * 0.2).cuda()
+        results = []
+        for compiled in (False, True):
+            x, v, w = x0.clone().requires_grad_(), v0.clone().requires_grad_(), torch.tensor(0.2, device="cuda").requires_grad_()
+            s, v_last, *rest = _calls(x * 1.5, v, w)[kind]()
+            loss = (s * torch.arange(5.0, device="cuda")).sum() + v_last.sum() + sum(r.square().sum() for r in rest if r is not None)
+            if compiled:
+                with compiled_autograd._enable(enable):
+                    loss.backward()
+            else:
+                loss.backward()
+            results.append([x.grad, v.grad, w.grad])
+        _equal(*results)
+
+
 def _reversed_strides(t):
     out = torch.empty(t.shape[::-1], dtype=t.dtype, device=t.device).permute(*range(t.dim() - 1, -1, -1))
     return out.copy_(t)
