@@ -515,6 +515,8 @@ def _chain_backward(x_seq, bits, shape, weight, gamma, v_init, y, bn_map, x_amax
     if grad_v_last is not None:
         grad_v_last = L.aligned16(grad_v_last.to(torch.float32))
     w = L.aligned16(weight.detach().to(torch.float32))
+    if bits is None and need_dw:
+        x_seq = L.aligned16(x_seq)  # (a saved-tensor hook may have handed it back in another layout)
     if bits is not None or x_exact:
         x_amax = None
     elif need_dw and x_amax.numel() == 0:  # (the forward ran on bf16 terms)

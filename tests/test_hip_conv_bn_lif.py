@@ -818,6 +818,35 @@ def test_convolution_gradients_on_two_streams_equal_those_on_one(monkeypatch):
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("block", ["attention", "convolution"])
+def test_saved_input_comes_back_in_another_layout(block):
+    """A saved-tensor hook that hands the input of a chain back with other strides: the same values, so the same gradients."""
+    from spikingjelly_amd.activation_based.model.spikformer import SpikformerConv2dBNLIF
+
+    shape = (4, 3, 64, 36) if block == "attention" else (4, 3, 64, 6, 6)
+
+    def strided(t):
+        if t.numel() != x.numel() or not torch.equal(t.flatten(), x.flatten()):
+            return t
+        return torch.empty(t.shape[::-1], device="cuda").permute(*range(t.dim() - 1, -1, -1)).copy_(t)
+
+    x, g = seeded_randn(shape, 64, 0.0, 2.0).cuda(), None
+    results = []
+    for hook in (lambda t: t, strided):
+        net = (_make_block(64, 2, 61) if block == "attention" else SpikformerConv2dBNLIF(64, 40, 1, backend="hip")).cuda().train()
+        if block == "convolution":
+            with torch.no_grad():
+                net.conv_bn.block[0].weight.copy_(seeded_randn((40, 64, 1, 1), 65))
+        xi = x.clone().requires_grad_()
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, hook):
+            out = net(xi)
+        g = seeded_randn(tuple(out.shape), 66).cuda() if g is None else g
+        out.backward(g)
+        results.append([xi.grad] + [p_.grad for p_ in net.parameters()])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("training", [True, False])
 def test_bit_packed_spikes_between_attention_neuron_and_projection_change_nothing(training, monkeypatch):
     """``configure.hip_conv_bit_spikes``: the attention neuron writes bits and the projection's GEMMs read bits, or the
