@@ -150,7 +150,8 @@ const char *sjhip_last_error(void);
  *             address of one fp32 holding k = sigmoid(w), read by the kernel in place of p->tau so that no host
  *             synchronisation is needed to fetch it
  * T >= 1, N >= 1, T*N < 2^62.  128-bit accesses are used when N is at least 16/sizeof(dtype), at any alignment of
- * the rows; shorter rows run an element-wise kernel.  No output may overlap an input.
+ * the rows; shorter rows run an element-wise kernel, and so does a call with an N that is no multiple of that and with
+ * an output in the place of an input (spike_seq == x_seq, v_last == v_init).
  */
 int sjhip_neuron_forward(int neuron, int dtype, const sjhip_neuron_params *p,
                          int64_t T, int64_t N,
@@ -229,9 +230,9 @@ int sjhip_neuron_backward_static(int neuron, int dtype, const sjhip_neuron_param
  * in LDS) and then runs the same BPTT.  A forward whose backward will use this entry point can be
  * called with h_seq = NULL, which saves its largest write.  Same argument meaning as
  * sjhip_neuron_backward with (x_seq, v_init) in place of h_seq; `p` carries the forward flags too
- * (SJHIP_FLAG_FP32_STATE, SJHIP_FLAG_RECIPROCAL_TAU).  Requires N of at least one 128-bit vector, the T of
- * sjhip_recompute_supported() and tensors that begin on 16 bytes; returns SJHIP_ERR_UNSUPPORTED / SJHIP_ERR_INVALID
- * otherwise.
+ * (SJHIP_FLAG_FP32_STATE, SJHIP_FLAG_RECIPROCAL_TAU).  Requires N of at least one 128-bit vector (where it is no
+ * multiple of one, no output may overlap an input), the T of sjhip_recompute_supported() and tensors that begin on 16
+ * bytes; returns SJHIP_ERR_UNSUPPORTED / SJHIP_ERR_INVALID otherwise.
  * Stands in for the same reference backward ops as sjhip_neuron_backward; the reference has no
  * recomputing variant (its kernels always read the saved h_seq, multi_step/base.py:137-409).
  */
@@ -254,7 +255,7 @@ int sjhip_neuron_backward_recompute(int neuron, int dtype, const sjhip_neuron_pa
  * states and checkpoints are bit-identical to sjhip_neuron_forward's; gradients are those of the walk over the whole
  * sequence (in fp32 storage also those of sjhip_neuron_backward_recompute applied piece by piece with grad_v_init
  * handed on as grad_v_last).  N must be at least one 128-bit
- * vector and every tensor 16-byte aligned.  With 16-bit storage and SJHIP_FLAG_FP32_STATE the checkpoints are
+ * vector (where it is no multiple of one, no output may overlap an input) and every tensor 16-byte aligned.  With 16-bit storage and SJHIP_FLAG_FP32_STATE the checkpoints are
  * fp32 rows ([pieces - 1][N] floats: a checkpoint in the storage dtype would round the state).  The saved state per
  * neuron is 1 / chunk of an h_seq; chunk = 16 keeps
  * five or more blocks resident per compute unit, which is where the single-piece kernel runs fastest.  No counterpart

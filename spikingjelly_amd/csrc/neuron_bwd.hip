@@ -86,7 +86,12 @@ int launch_backward(int neuron, int dtype, const sjhip_neuron_params &p, int64_t
   if (rc != SJHIP_OK) return rc;
   const int mode = neuron == SJHIP_NEURON_PLIF ? BWD_PLIF : ((neuron == SJHIP_NEURON_QIF || neuron == SJHIP_NEURON_EIF) ? BWD_QIF : BWD_PLAIN);
 
-  const bool vector = N >= (dtype == SJHIP_F32 ? 4 : 8);  // any N and any alignment: see whole_group()
+  // any N and any alignment, but rows that V does not divide only apart from the inputs: see whole_group()
+  const int V = dtype == SJHIP_F32 ? 4 : 8;
+  const uint64_t row = (uint64_t)N * (16 / V), all = (uint64_t)T * row;
+  const bool vector = N % V == 0 || (N >= V && !any_overlap({{grad_x_seq, all}, {grad_v_init, row}},
+                                                            {{grad_spike_seq, all}, {grad_v_seq, all}, {h_seq, all}, {grad_v_last, row},
+                                                             {v_init, a.v_init_broadcast ? 4 : row}}));
 
   switch (dtype) {
     case SJHIP_F32: return launch_typed<float>(a, vector, mode, grad_rtau, stream);

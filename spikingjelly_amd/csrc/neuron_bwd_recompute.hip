@@ -74,6 +74,14 @@ int launch_replay(int neuron, int dtype, const sjhip_neuron_params &p, int64_t T
                       grad_x_seq, grad_v_init, grad_rtau, workspace);
   if (rc != SJHIP_OK) return rc;
 
+  const int whole = dtype == SJHIP_F32 ? 4 : 8;
+  const uint64_t row = (uint64_t)N * (16 / whole), all = (uint64_t)T * row;
+  const uint64_t kept = (uint64_t)(chunk > 0 && T > chunk ? (T + chunk - 1) / chunk - 1 : 0) * N * (checkpoints_are_f32(dtype, p.flags) ? 4 : 16 / whole);
+  if (N % whole != 0 && any_overlap({{grad_x_seq, all}, {grad_v_init, row}},
+                                    {{x_seq, all}, {v_init, broadcast ? 4 : row}, {checkpoints, kept}, {grad_spike_seq, all},
+                                     {grad_v_seq, all}, {grad_v_last, row}}))
+    return fail(SJHIP_ERR_UNSUPPORTED, "backward(recompute): N=%lld is not a multiple of %d: no output may overlap an input", (long long)N, whole);
+
   const bool narrow = dtype != SJHIP_F32 && !round_each;  // 16-bit storage, fp32 state: four neurons per work-item
   const int V = (dtype == SJHIP_F32 || narrow) ? 4 : 8;
   // The walk over several pieces measured faster with each XCD on a contiguous eighth of the columns at every row

@@ -83,6 +83,11 @@ int launch_forward_pieces(int neuron, int dtype, const sjhip_neuron_params &p, i
   if (N < V || !aligned16(x_seq) || !(a.v_init_broadcast || aligned16(v_init)) || !aligned16(spike_seq) || !aligned16(v_seq) ||
       !aligned16(v_last) || !aligned16(checkpoints))
     return fail(SJHIP_ERR_UNSUPPORTED, "forward(pieces): N=%lld must be at least %d and every tensor 16-byte aligned", (long long)N, V);
+  const uint64_t row = (uint64_t)N * (16 / V), all = (uint64_t)T * row;
+  const uint64_t kept = (uint64_t)(T > chunk ? (T + chunk - 1) / chunk - 1 : 0) * N * (checkpoints_are_f32(dtype, p.flags) ? 4 : 16 / V);
+  if (N % V != 0 && any_overlap({{spike_seq, all}, {v_seq, all}, {v_last, row}, {checkpoints, kept}},
+                                {{x_seq, all}, {v_init, a.v_init_broadcast ? 4 : row}}))
+    return fail(SJHIP_ERR_UNSUPPORTED, "forward(pieces): N=%lld is not a multiple of %d: no output may overlap an input", (long long)N, V);
   a.checkpoints = checkpoints; a.chunk = chunk;
   switch (dtype) {
     case SJHIP_F32: return launch_pieces_typed<float, false>(a, stream);
@@ -118,7 +123,11 @@ int launch_forward(int neuron, int dtype, const sjhip_neuron_params &p, int64_t 
   int rc = build_fwd_args(a, round_each, neuron, dtype, p, T, N, x_seq, v_init, k_device, spike_seq, v_seq, v_last, h_seq);
   if (rc != SJHIP_OK) return rc;
 
-  const bool vector = N >= (dtype == SJHIP_F32 ? 4 : 8);  // any N and any alignment: see whole_group()
+  // any N and any alignment, but rows that V does not divide only apart from the inputs: see whole_group()
+  const int V = dtype == SJHIP_F32 ? 4 : 8;
+  const uint64_t row = (uint64_t)N * (16 / V), all = (uint64_t)T * row;
+  const bool vector = N % V == 0 || (N >= V && !any_overlap({{spike_seq, all}, {v_seq, all}, {h_seq, all}, {v_last, row}},
+                                                            {{x_seq, all}, {v_init, a.v_init_broadcast ? 4 : row}}));
 
   switch (dtype) {
     case SJHIP_F32: return launch_typed<float, false>(a, vector, stream);

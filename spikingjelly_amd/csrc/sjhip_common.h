@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include <cmath>
+#include <initializer_list>
 
 #include <type_traits>
 
@@ -387,7 +388,8 @@ __device__ __forceinline__ unsigned column_block(int spread) {
 
 // First of the V neurons of the work-item whose share of a row begins at `col`: the last work-item of a row that V does
 // not divide takes the row's last V neurons, the first of which its neighbour has too (both compute and store the same
-// bits; nothing they read is written by the kernel).  So a row of any N >= V runs on V-wide accesses; shorter ones on the
+// bits; nothing they read is written by the kernel: a call whose outputs share memory with its inputs keeps the
+// element-wise kernels, where a work-item reads its neuron before it writes it, or is refused).  So a row of any N >= V runs on V-wide accesses; shorter ones on the
 // element-wise kernels, which such rows had to take before: one 2- or 4-byte access per lane and row keeps too few bytes in
 // flight, and without the replay h_seq is written and read as well.  Measured (forward / backward, us; element-wise and
 // saved h -> this and the replay): fp32 [8, 2979423] 78 / 157 -> 35 / 53 (5.4 TB/s; a row of whole vectors takes the same),
@@ -398,6 +400,20 @@ template <int V> __device__ __forceinline__ int64_t whole_group(int64_t col, int
   return col + V <= N ? col : N - V;
 }
 #endif
+
+// One buffer of a call, for the question whether an output shares memory with an input (a null buffer shares nothing).
+struct Span {
+  const void *p;
+  uint64_t bytes;
+};
+static inline bool any_overlap(std::initializer_list<Span> outputs, std::initializer_list<Span> inputs) {
+  for (const Span &o : outputs)
+    for (const Span &i : inputs) {
+      const uintptr_t a = reinterpret_cast<uintptr_t>(o.p), b = reinterpret_cast<uintptr_t>(i.p);
+      if (a && b && a < b + i.bytes && b < a + o.bytes) return true;
+    }
+  return false;
+}
 
 static inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
