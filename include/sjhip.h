@@ -644,7 +644,8 @@ int sjhip_pwconv_grad_weight_planes(const uint16_t *dy_planes, const float *dy_a
  *                       one of the two is given; v_last [B][C][L] or NULL
  *   sjhip_bn_lif_backward  replays the neuron from y (T <= 256; beyond 16 steps in pieces of 16), runs the BPTT recurrence of sjhip_neuron_backward with
  *                       grad_spike_seq and (optionally) grad_v_last, writes grad_z = dL/dz [T][B][C][L], grad_v_init
- *                       (or NULL) and partial[b][c] = (sum g, sum g y) over the row and all steps
+ *                       (or NULL) and partial[b][c] = (sum g, sum g y) over the row and all steps (where L is no multiple
+ *                       of 4, no output may overlap an input)
  *   sjhip_bn_backward_finalize   dgamma, dbeta (either may be NULL) and coef [3][C] = (p, q, r) of dy = p g + q y + r;
  *                       training != 0: batch statistics took part in the forward, else q = r = 0; amax_reset: NULL, or
  *                       the amax buffer (sjhip_pwconv_amax_floats(T * B) floats) of a following sjhip_bn_grad_input_amax,

@@ -686,6 +686,11 @@ int launch_bn_lif_backward(int neuron, const sjhip_neuron_params &p, int64_t T, 
   if (!aligned16(y) || (!broadcast && !aligned16(v_init)) || !aligned16(grad_spike_seq) || !aligned16(grad_z) ||
       (grad_v_last && !aligned16(grad_v_last)) || (grad_v_init && !aligned16(grad_v_init)))
     return fail(SJHIP_ERR_UNSUPPORTED, "bn_lif_backward: tensors must be 16-byte aligned");
+  // (groups of four overlap at the end of a row that four does not divide: nothing they read may be written)
+  const uint64_t step = (uint64_t)N * 4, all = (uint64_t)T * step;
+  if (L % 4 != 0 && any_overlap({{grad_z, all}, {grad_v_init, step}},
+                                {{y, all}, {v_init, broadcast ? 4 : step}, {grad_spike_seq, all}, {grad_v_last, step}}))
+    return fail(SJHIP_ERR_UNSUPPORTED, "bn_lif_backward: L=%lld is not a multiple of 4: no output may overlap an input", (long long)L);
   BnLifBwdArgs a;
   bool round_each = false;
   rc = build_fwd_args(a.f, round_each, neuron, SJHIP_F32, p, T, N, y, v_init, k_device, nullptr, nullptr, nullptr, nullptr);

@@ -36,6 +36,29 @@ def test_forward_in_pieces_refuses_shared_memory_in_ragged_rows(N):
         assert rc == -2 and b"overlap" in lib.sjhip_last_error(), (s, v_seq, v_last)
 
 
+@pytest.mark.parametrize("T", [4, 20])
+def test_batch_norm_backward_refuses_shared_memory_in_ragged_rows(T):
+    lib, p = L.load(), _params(1)
+    for g, gv0, gl in ((GS, None, None), (X, None, None), (GX, V, None), (GX, GV, GV)):
+        rc = lib.sjhip_bn_lif_backward(L.NEURON_LIF, ctypes.byref(p), T, 2, 4, 9, X, CK, CK, V, GS, gl, g, gv0, CK, None)
+        assert rc == -2 and b"overlap" in lib.sjhip_last_error(), (g, gv0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [4, 20])
+def test_batch_norm_backward_of_whole_rows_in_place(T):
+    lib, p, B, C, Lp = L.load(), ctypes.byref(_params(1)), 2, 4, 12
+    g = torch.Generator().manual_seed(T)
+    y, gs = (torch.randn(T, B, C, Lp, generator=g).cuda() for _ in range(2))
+    one, zero, v0 = torch.ones(C).cuda(), torch.zeros(C).cuda(), torch.zeros(B, C, Lp).cuda()
+    sums, sums2, dz = torch.empty(B * C, 2).cuda(), torch.empty(B * C, 2).cuda(), torch.empty_like(y)
+    st, ptr = L.current_stream_ptr(y.device), lambda t: t.data_ptr()
+    call = lambda grad, out, part: lib.sjhip_bn_lif_backward(L.NEURON_LIF, p, T, B, C, Lp, ptr(y), ptr(one), ptr(zero), ptr(v0), ptr(grad), None,
+                                                             ptr(out), None, ptr(part), st)
+    assert call(gs, dz, sums) == 0 and call(gs, gs, sums2) == 0
+    assert torch.equal(dz, gs) and torch.equal(sums, sums2)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("N", [3, 8, 9, 1027, 262147])
