@@ -2,8 +2,6 @@
 // translation units so the three sets of kernels compile in parallel.
 #pragma once
 
-#include <mutex>
-
 #include "neuron_bwd_recompute.h"
 
 namespace sjhip {
@@ -14,14 +12,9 @@ constexpr unsigned kRecomputeMaxLds = 159u * 1024u;
 template <typename S, bool ROUND_EACH, int MODE>
 int launch_kernel(const FwdArgs &f, const BwdArgs &b, int block, unsigned lds, int64_t blocks, hipStream_t stream) {
   auto kernel = backward_recompute_kernel<S, ROUND_EACH, MODE>;
-  // a block may use more than the default 64 KiB of dynamic LDS only after this opt-in (once per kernel)
-  static std::once_flag once;
-  static hipError_t attr_rc = hipSuccess;
-  std::call_once(once, [&]() {
-    attr_rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)kRecomputeMaxLds);
-    (void)hipGetLastError();  // a refusal is reported below, only if the launch really needs the larger limit
-  });
+  // a block may use more than the default 64 KiB of dynamic LDS only after this opt-in (once per kernel and device)
+  static OncePerDevice once;
+  const hipError_t attr_rc = allow_dynamic_lds(once, reinterpret_cast<const void *>(kernel), (int)kRecomputeMaxLds);
   if (lds > 64u * 1024u && attr_rc != hipSuccess)
     return fail(SJHIP_ERR_LAUNCH, "backward(recompute): cannot raise the dynamic LDS limit: %s", hipGetErrorString(attr_rc));
   hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(block), lds, stream, f, b);
@@ -34,13 +27,8 @@ int launch_pieces_kernel(const FwdArgs &f, const BwdArgs &b, const PieceArgs &p,
   auto kernel = backward_recompute_pieces_kernel<S, ROUND_EACH, MODE>;
   // pieces of 16 steps stay below the default 64 KiB of dynamic LDS; longer pieces (17 steps and more at 256 lanes,
   // 33 and more at 128) do not and need the same opt-in as launch_kernel
-  static std::once_flag once;
-  static hipError_t attr_rc = hipSuccess;
-  std::call_once(once, [&]() {
-    attr_rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)kRecomputeMaxLds);
-    (void)hipGetLastError();
-  });
+  static OncePerDevice once;
+  const hipError_t attr_rc = allow_dynamic_lds(once, reinterpret_cast<const void *>(kernel), (int)kRecomputeMaxLds);
   if (lds > kRecomputeMaxLds)
     return fail(SJHIP_ERR_UNSUPPORTED, "backward(recompute, pieces): %u bytes of LDS per block exceed %u", lds, kRecomputeMaxLds);
   if (lds > 64u * 1024u && attr_rc != hipSuccess)

@@ -65,8 +65,6 @@
 #include "bn_map.h"
 #include "sjhip_common.h"
 
-#include <mutex>
-
 namespace sjhip {
 
 namespace {
@@ -1610,13 +1608,8 @@ template <int TA, int TB, bool H, bool BITS, bool RAGGED>
 int launch_dw(const PwDwArgs &a, int64_t blocks, hipStream_t stream) {
   constexpr unsigned lds = (dw_two_buffers(H) ? 2 : 1) * (TA + TB) * kRowPlane;
   if constexpr (lds > 64u * 1024u) {
-    static std::once_flag once;
-    static hipError_t attr_rc = hipSuccess;
-    std::call_once(once, [&]() {
-      attr_rc = hipFuncSetAttribute(reinterpret_cast<const void *>(&pw_dw_kernel<TA, TB, H, BITS, RAGGED>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      (void)hipGetLastError();
-    });
+    static OncePerDevice once;
+    const hipError_t attr_rc = allow_dynamic_lds(once, reinterpret_cast<const void *>(&pw_dw_kernel<TA, TB, H, BITS, RAGGED>), (int)lds);
     if (attr_rc != hipSuccess) return fail(SJHIP_ERR_LAUNCH, "pwconv_grad_weight: cannot raise the dynamic LDS limit: %s", hipGetErrorString(attr_rc));
   }
   hipLaunchKernelGGL((pw_dw_kernel<TA, TB, H, BITS, RAGGED>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);

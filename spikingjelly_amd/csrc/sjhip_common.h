@@ -10,6 +10,7 @@
 
 #include <type_traits>
 
+#include "once_per_device.h"
 #include "sjhip.h"
 
 namespace sjhip {
@@ -400,6 +401,16 @@ template <int V> __device__ __forceinline__ int64_t whole_group(int64_t col, int
   return col + V <= N ? col : N - V;
 }
 #endif
+
+// Raises a kernel's limit of dynamic LDS to `bytes` on the current device, the first time it is asked there.
+static inline hipError_t allow_dynamic_lds(OncePerDevice &once, const void *kernel, int bytes) {
+  int device = 0;
+  hipError_t rc = hipGetDevice(&device);
+  if (rc == hipSuccess)
+    rc = (hipError_t)once(device, [&]() { return (int)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); });
+  if (rc != hipSuccess) (void)hipGetLastError();  // (for the caller to report, if its launch needs the larger limit)
+  return rc;
+}
 
 // One buffer of a call, for the question whether an output shares memory with an input (a null buffer shares nothing).
 struct Span {

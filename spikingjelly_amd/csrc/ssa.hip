@@ -35,7 +35,6 @@
 #include "sjhip_common.h"
 
 #include <algorithm>
-#include <mutex>
 
 // Resident blocks per compute unit the backward kernel's register allocation is sized for (heads of up to 32
 // channels).  Sized for 2 the kernel takes 124 registers and keeps the split dS operands across the column tiles
@@ -949,13 +948,8 @@ unsigned backward_lds(int cph, int L) {
 }
 
 template <typename K>
-int launch_with_lds(K kernel, const SsaArgs &a, int threads, unsigned lds, hipStream_t stream, std::once_flag &once,
-                    hipError_t &attr_rc, const char *what) {
-  std::call_once(once, [&]() {
-    attr_rc = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)kSsaMaxLds);
-    (void)hipGetLastError();
-  });
+int launch_with_lds(K kernel, const SsaArgs &a, int threads, unsigned lds, hipStream_t stream, OncePerDevice &once, const char *what) {
+  const hipError_t attr_rc = allow_dynamic_lds(once, reinterpret_cast<const void *>(kernel), (int)kSsaMaxLds);
   if (lds > 64u * 1024u && attr_rc != hipSuccess)
     return fail(SJHIP_ERR_LAUNCH, "%s: cannot raise the dynamic LDS limit: %s", what, hipGetErrorString(attr_rc));
   hipLaunchKernelGGL(kernel, dim3((unsigned)a.problems), dim3(threads), lds, stream, a);
@@ -964,15 +958,13 @@ int launch_with_lds(K kernel, const SsaArgs &a, int threads, unsigned lds, hipSt
 
 template <typename S, int MC>
 int launch_fwd(const SsaArgs &a, hipStream_t stream) {
-  static std::once_flag once;
-  static hipError_t attr_rc = hipSuccess;
-  return launch_with_lds(ssa_forward_kernel<S, MC>, a, ssa_threads(MC), forward_lds(a.cph, a.L), stream, once, attr_rc, "ssa_forward");
+  static OncePerDevice once;
+  return launch_with_lds(ssa_forward_kernel<S, MC>, a, ssa_threads(MC), forward_lds(a.cph, a.L), stream, once, "ssa_forward");
 }
 template <typename S, int MC>
 int launch_bwd(const SsaArgs &a, hipStream_t stream) {
-  static std::once_flag once;
-  static hipError_t attr_rc = hipSuccess;
-  return launch_with_lds(ssa_backward_kernel<S, MC>, a, ssa_threads(MC), backward_lds(a.cph, a.L), stream, once, attr_rc, "ssa_backward");
+  static OncePerDevice once;
+  return launch_with_lds(ssa_backward_kernel<S, MC>, a, ssa_threads(MC), backward_lds(a.cph, a.L), stream, once, "ssa_backward");
 }
 
 template <typename S>
@@ -1056,15 +1048,10 @@ int launch_ssa_lif(bool backward, int neuron, const sjhip_neuron_params &p, int6
                                 : forward_lds(cph, (int)L) + (unsigned)(padded_rows(cph) * lds_row_f32((int)L) * 4);
   const void *kernel = backward ? (mc == 1 ? (const void *)ssa_lif_backward_kernel<1> : (const void *)ssa_lif_backward_kernel<2>)
                                 : (mc == 1 ? (const void *)ssa_lif_forward_kernel<1> : (const void *)ssa_lif_forward_kernel<2>);
-  static std::once_flag once[4];
-  static hipError_t attr_rc[4] = {hipSuccess, hipSuccess, hipSuccess, hipSuccess};
-  const int slot = (backward ? 2 : 0) + (mc - 1);
-  std::call_once(once[slot], [&]() {
-    attr_rc[slot] = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSsaMaxLds);
-    (void)hipGetLastError();
-  });
-  if (lds > 64u * 1024u && attr_rc[slot] != hipSuccess)
-    return fail(SJHIP_ERR_LAUNCH, "%s: cannot raise the dynamic LDS limit: %s", what, hipGetErrorString(attr_rc[slot]));
+  static OncePerDevice once[4];
+  const hipError_t attr_rc = allow_dynamic_lds(once[(backward ? 2 : 0) + (mc - 1)], kernel, (int)kSsaMaxLds);
+  if (lds > 64u * 1024u && attr_rc != hipSuccess)
+    return fail(SJHIP_ERR_LAUNCH, "%s: cannot raise the dynamic LDS limit: %s", what, hipGetErrorString(attr_rc));
   ProfileScope prof(backward ? KC_SSA_BACKWARD : KC_SSA_FORWARD, stream);
   const dim3 grid((unsigned)(B * heads)), threads(ssa_threads(mc));
   if (backward) {
