@@ -1109,6 +1109,7 @@ template <bool ANY> __device__ __forceinline__ f32x4 load4(const char *p) {
 template <int TA, int TB, bool H, bool BITS = false, bool RAGGED = false>
 __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) pw_dw_kernel(const PwDwArgs a) {
   static_assert(!BITS || (TB == 1 && !RAGGED), "a bit-packed operand has one term and rows of a multiple of four");
+  static_assert(H || !RAGGED, "rows of other lengths run on fp16 terms");
   extern __shared__ __align__(16) uint8_t lds[];
   // [TA][128][kRowBytes] of dy, then [TB][128][kRowBytes] of x; DOUBLE: twice
   uint8_t *As = lds, *Bs = lds + TA * kRowPlane;
@@ -1617,8 +1618,10 @@ int launch_dw(const PwDwArgs &a, int64_t blocks, hipStream_t stream) {
 }
 template <int TA, int TB, bool H = false, bool BITS = false>
 int launch_dw_terms(const PwDwArgs &a, int64_t blocks, hipStream_t stream) {
-  if (BITS || a.L == a.Lq) return launch_dw<TA, TB, H, BITS, false>(a, blocks, stream);
-  return launch_dw<TA, TB, H, false, true>(a, blocks, stream);
+  if constexpr (H && !BITS) {
+    if (a.L != a.Lq) return launch_dw<TA, TB, H, false, true>(a, blocks, stream);
+  }
+  return launch_dw<TA, TB, H, BITS, false>(a, blocks, stream);
 }
 
 // Samples per partial tile of dW.  Two blocks are resident per compute unit (512 on the chip); the chunk count is the
@@ -1771,8 +1774,9 @@ int launch_pwconv_grad_weight(const float *dy, int dy_terms, const float *dy_ama
                               hipStream_t stream, bool x_bits) {
   if (x_bits && ((N * L) % 8 != 0 || dy_terms != (SJHIP_PW_F16 | 2) || x_terms != 1))
     return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_grad_weight: bit-packed activations need N*L=%lld to be a multiple of 8, two fp16 gradient terms and one activation term", (long long)(N * L));
-  if ((L % 4 != 0 && (x_bits || L < 4)) || !aligned16(dy) || (!x_bits && !aligned16(x)))
-    return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_grad_weight: L=%lld must be a multiple of 4 (or at least 4 with fp32 activations) and the tensors 16-byte aligned", (long long)L);
+  // (other lengths: fp16 terms only, the GEMM beside it has no bf16 form for them)
+  if ((L % 4 != 0 && (x_bits || L < 4 || !(dy_terms & SJHIP_PW_F16))) || !aligned16(dy) || (!x_bits && !aligned16(x)))
+    return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_grad_weight: L=%lld must be a multiple of 4 (or, with fp16 terms and fp32 activations, at least 4) and the tensors 16-byte aligned", (long long)L);
   if (M * L >= (int64_t(1) << 30) || N * L >= (int64_t(1) << 30) || M * N >= (int64_t(1) << 40))  // 32-bit per-lane byte offsets
     return fail(SJHIP_ERR_TOO_LARGE, "pwconv_grad_weight: M=%lld N=%lld L=%lld", (long long)M, (long long)N, (long long)L);
   PwDwArgs a;

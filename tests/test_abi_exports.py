@@ -249,3 +249,11 @@ def test_fp16_split_convolution_arguments_without_a_device():
     assert lib.sjhip_pwconv_amax_floats(10) == 256 + 16 * 10
     rc = lib.sjhip_pwconv_split_weight_f16(16, 8, 8, 0, 8, None, 0, None)
     assert rc == -2 and b"aligned" in lib.sjhip_last_error()
+
+
+@pytest.mark.parametrize("terms", [(3, 3), (3, 1), (2, 2), (2, 1), (1, 1)])
+@pytest.mark.parametrize("Lp", [1, 2, 3, 5, 6, 49])
+def test_bf16_weight_gradient_takes_rows_of_a_multiple_of_four_only(terms, Lp):
+    lib = L.load()
+    rc = lib.sjhip_pwconv_grad_weight(0x10000, terms[0], 0x20000, terms[1], 4, 8, 8, Lp, 0x30000, 0x40000, None)
+    assert rc == -2 and b"multiple of 4" in lib.sjhip_last_error()
