@@ -632,9 +632,11 @@ int launch_bn_finalize(const float *partial, int64_t rows, int64_t count, int64_
   return check_launch("bn_finalize");
 }
 
-int launch_bn_lif_forward(int neuron, const sjhip_neuron_params &p, int64_t T, int64_t B, int64_t C, int64_t L, const float *y,
-                          const float *scale, const float *shift, const float *v_init, const float *k_device, float *spike_seq,
-                          uint8_t *spike_bits, float *v_last, hipStream_t stream) {
+// The checks of the forward stage, without a launch: a chain asks before its first launch, because batch norm's running
+// statistics have been updated by the time this stage is reached.
+static int prepare_bn_lif_forward(BnLifFwdArgs &a, int neuron, const sjhip_neuron_params &p, int64_t T, int64_t B, int64_t C, int64_t L,
+                                  const float *y, const float *v_init, const float *k_device, float *spike_seq, uint8_t *spike_bits,
+                                  float *v_last) {
   int rc = check_layout("bn_lif_forward", T, B, C, L);
   if (rc != SJHIP_OK) return rc;
   if (!lif_like(neuron)) return fail(SJHIP_ERR_UNSUPPORTED, "bn_lif_forward: neuron %d (IF, LIF and PLIF only)", neuron);
@@ -645,14 +647,29 @@ int launch_bn_lif_forward(int neuron, const sjhip_neuron_params &p, int64_t T, i
   if (!aligned16(y) || (!broadcast && !aligned16(v_init)) || (spike_seq && !aligned16(spike_seq)) || (v_last && !aligned16(v_last)))
     return fail(SJHIP_ERR_UNSUPPORTED, "bn_lif_forward: tensors must be 16-byte aligned");
   if (spike_bits && N % 8 != 0) return fail(SJHIP_ERR_UNSUPPORTED, "bn_lif_forward: B*C*L=%lld must be a multiple of 8 for bit-packed spikes", (long long)N);
-  BnLifFwdArgs a;
   bool round_each = false;
   rc = build_fwd_args(a.f, round_each, neuron, SJHIP_F32, p, T, N, y, v_init, k_device,
                       spike_bits ? (void *)spike_bits : (void *)spike_seq, nullptr, v_last, nullptr);
   if (rc != SJHIP_OK) return rc;
-  a.scale = scale; a.shift = shift; a.C = (int)C; a.L = (int)L;
-  const int64_t blocks = (N / 4 + 255) / 256;
-  if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "bn_lif_forward: N=%lld", (long long)N);
+  a.C = (int)C; a.L = (int)L;
+  if ((N / 4 + 255) / 256 > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "bn_lif_forward: N=%lld", (long long)N);
+  return SJHIP_OK;
+}
+
+int check_bn_lif_forward(int neuron, const sjhip_neuron_params &p, int64_t T, int64_t B, int64_t C, int64_t L, const float *y,
+                         const float *v_init, const float *k_device, float *spike_seq, uint8_t *spike_bits, float *v_last) {
+  BnLifFwdArgs a;
+  return prepare_bn_lif_forward(a, neuron, p, T, B, C, L, y, v_init, k_device, spike_seq, spike_bits, v_last);
+}
+
+int launch_bn_lif_forward(int neuron, const sjhip_neuron_params &p, int64_t T, int64_t B, int64_t C, int64_t L, const float *y,
+                          const float *scale, const float *shift, const float *v_init, const float *k_device, float *spike_seq,
+                          uint8_t *spike_bits, float *v_last, hipStream_t stream) {
+  BnLifFwdArgs a;
+  const int rc = prepare_bn_lif_forward(a, neuron, p, T, B, C, L, y, v_init, k_device, spike_seq, spike_bits, v_last);
+  if (rc != SJHIP_OK) return rc;
+  a.scale = scale; a.shift = shift;
+  const int64_t blocks = (a.f.N / 4 + 255) / 256;
   ProfileScope prof(KC_BN_LIF_FORWARD, stream);
   auto launch = [&](auto packed, auto ragged) {
     hipLaunchKernelGGL((bn_lif_forward_kernel<decltype(packed)::value, decltype(ragged)::value>), dim3((unsigned)blocks), dim3(256), 0, stream, a);

@@ -827,6 +827,8 @@ int sjhip_conv_bn_lif_forward(int neuron, const sjhip_neuron_params *p, int64_t 
   if (rc != SJHIP_OK) return rc;
   if (!aligned16(workspace) || !aligned16(y) || (x_amax && !aligned16(x_amax)))
     return fail(SJHIP_ERR_UNSUPPORTED, "conv_bn_lif_forward: workspace, y and x_amax must be 16-byte aligned");
+  rc = check_bn_lif_forward(neuron, *p, T, B, Cout, L, y, v_init, k_device, spike_seq, spike_bits, v_last);
+  if (rc != SJHIP_OK) return rc;
   const hipStream_t stream = static_cast<hipStream_t>(stream_);
   const int64_t S = T * B;
   const ChainForwardParts w(workspace, S, Cin, Cout, L);
@@ -865,8 +867,8 @@ int sjhip_conv_bn_lif_backward(int neuron, const sjhip_neuron_params *p, int64_t
     return fail(SJHIP_ERR_INVALID, "conv_bn_lif_backward: NULL buffer, or not exactly one of x / x_bits");
   int rc = check_chain("conv_bn_lif_backward", T, B, Cin, Cout, L);
   if (rc != SJHIP_OK) return rc;
-  if (!aligned16(workspace) || (x_amax && !aligned16(x_amax)))
-    return fail(SJHIP_ERR_UNSUPPORTED, "conv_bn_lif_backward: workspace and x_amax must be 16-byte aligned");
+  if (!aligned16(workspace) || (x_amax && !aligned16(x_amax)) || (dw && x && !aligned16(x)))
+    return fail(SJHIP_ERR_UNSUPPORTED, "conv_bn_lif_backward: workspace, x and x_amax must be 16-byte aligned");
   const hipStream_t stream = static_cast<hipStream_t>(stream_);
   const int64_t S = T * B;
   const ChainBackwardParts w(workspace, T, B, Cin, Cout, L, dx != nullptr, dw != nullptr, k_device != nullptr);

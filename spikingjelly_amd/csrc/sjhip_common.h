@@ -544,6 +544,8 @@ int launch_bn_finalize(const float *partial, int64_t rows, int64_t count, int64_
                        float momentum, float *running_mean, float *running_var, float *scale, float *shift, float *mean,
                        float *invstd, int64_t *batches_tracked, hipStream_t stream);
 // (k_device: PLIF's k = sigmoid(w) in device memory, else nullptr; grad_k + k_workspace: where dL/dk goes, PLIF only)
+int check_bn_lif_forward(int neuron, const sjhip_neuron_params &p, int64_t T, int64_t B, int64_t C, int64_t L, const float *y,
+                         const float *v_init, const float *k_device, float *spike_seq, uint8_t *spike_bits, float *v_last);
 int launch_bn_lif_forward(int neuron, const sjhip_neuron_params &p, int64_t T, int64_t B, int64_t C, int64_t L, const float *y,
                           const float *scale, const float *shift, const float *v_init, const float *k_device, float *spike_seq,
                           uint8_t *spike_bits, float *v_last, hipStream_t stream);

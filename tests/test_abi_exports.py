@@ -257,3 +257,22 @@ def test_bf16_weight_gradient_takes_rows_of_a_multiple_of_four_only(terms, Lp):
     lib = L.load()
     rc = lib.sjhip_pwconv_grad_weight(0x10000, terms[0], 0x20000, terms[1], 4, 8, 8, Lp, 0x30000, 0x40000, None)
     assert rc == -2 and b"multiple of 4" in lib.sjhip_last_error()
+
+
+@pytest.mark.parametrize("change,code,text", [
+    (dict(v_init=0x50004), -2, b"16-byte"), (dict(spikes=0x70008), -2, b"16-byte"), (dict(v_last=0x80004), -2, b"16-byte"),
+    (dict(neuron=4), -2, b"neuron 4"), (dict(neuron=2), -1, b"PLIF"), (dict(k=0x90000), -1, b"PLIF"), (dict(tau=0.0), -1, b"tau"),
+    (dict(L=9, Cout=7), -2, b"multiple of 4"), (dict(bits=0x70000, spikes=None, B=1, Cout=3), -2, b"multiple of 8"),
+    (dict(batch_stats=0, mean=None), -1, b"running statistics")])
+def test_convolution_chain_refuses_before_its_first_launch(change, code, text):
+    """Without a device a launch fails with an error of its own (-3): what is refused here has launched nothing, in
+    particular not the kernel that updates batch norm's running statistics."""
+    a = dict(neuron=L.NEURON_LIF, tau=2.0, B=2, Cout=8, L=4, v_init=0x50000, k=None, spikes=0x70000, bits=None, v_last=0x80000, mean=0xa0000,
+             batch_stats=1)
+    a.update(change)
+    p = L.NeuronParams(a["tau"], 1.0, 0.0, 2.0, 1, 1)
+    lib = L.load()
+    rc = lib.sjhip_conv_bn_lif_forward(a["neuron"], ctypes.byref(p), 4, a["B"], 8, a["Cout"], a["L"], 0x10000, None, 0x20000, None, None, a["mean"],
+                                       0xb0000, a["batch_stats"], 0.1, 1e-5, None, a["v_init"], a["k"], None, 0x30000, 0x40000, a["spikes"],
+                                       a["bits"], a["v_last"], 0x60000, None)
+    assert rc == code and text in lib.sjhip_last_error(), (rc, lib.sjhip_last_error())
