@@ -818,7 +818,7 @@ constexpr unsigned rows_inverse_offset(int tb) { return 2u * tb * kRowPlane > kO
 //     instructions, split, and stored as it lies in memory (k rows of 128 columns); the wavefronts fetch their
 //     fragments with the transposing LDS read, as pw_gemm_kernel does for term planes;
 //   * two B tiles alternate in LDS, so a K step has one barrier.
-// Per K step of a block: 16 KB written to and 64 KB read from LDS, 16 + 16 load instructions; 146 registers, three
+// Per K step of a block: 16 KB written to and 64 KB read from LDS, 16 + 16 load instructions; 148 to 154 registers, three
 // wavefronts per SIMD.
 // BITS: b is a spike tensor that arrives bit-packed (as in pw_gemm_kernel, L a multiple of 4): a byte per piece, one term;
 // M = K = 384, 50 176 columns: 41 us, pw_gemm_kernel 47.
@@ -827,8 +827,15 @@ constexpr unsigned rows_inverse_offset(int tb) { return 2u * tb * kRowPlane > kO
 // 4-byte address) and moved down by one to three places with zeros behind it.
 // (RAGGED is a template parameter: asked at run time the moves cost the aligned case 4 %, 106 -> 110 us at M = 1536, K = 384,
 // 25 088 columns.)
+// The products of a K step of such rows are summed by themselves, the small terms of both halves first, and reach the
+// accumulators with one rounding: with one chain over all of K (as the rows of a multiple of four have it) the error
+// against float64 was above that of the library's fp32 GEMM, which serves these lengths otherwise (relative 2-norm, spikes,
+// [48, 512, 49] -> 128 channels: library 1.11e-7, chain 1.54e-7, now 9.9e-8; real values, [4, 1536, 49] -> 512: 3.5e-7, 4.4e-7,
+// 1.6e-7; over 70 shapes of 96 to 576 channels, 7 x 7 and 9 x 9: 0.87 of the library's forward and 0.33 of its input gradient on
+// average, at most 1.09).  It takes 256 registers, two wavefronts per SIMD: [128, 384, 49] -> 1536 38.9 -> 46.0 us, its input
+// gradient 53.5 -> 59.1, [96, 512, 81] -> 512 25.8 -> 28.6.
 template <int TB, bool BITS, bool RAGGED>
-__global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu(3, 3))) pw_gemm_rows_kernel(const PwGemmArgs a) {
+__global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu(RAGGED ? 2 : 3, RAGGED ? 2 : 3))) pw_gemm_rows_kernel(const PwGemmArgs a) {
   constexpr int TA = 2;
   constexpr int kBuf = TB * kRowPlane;  // one B tile: [TB][32 k][kPlanePitch]
   extern __shared__ __align__(16) uint8_t lds[];
@@ -878,13 +885,15 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   };
   if (per_sample && col_ok) scale_for(column_amax(jc), b_scale, b_inverse);
 
-  u32x4 af[2][TA];  // [ks][term]: the fragments of the step being multiplied, refilled as they are used up
+  // [ks][term]: the fragments of the step being multiplied, refilled as they are used up; RAGGED: those of the next step
+  // arrive in the other set
+  u32x4 af[RAGGED ? 4 : 2][TA];
   u32x4 rb[2][4];   // [set][i]: k row kr + 8 i of a tile, fp32 bit patterns of four columns
-  auto fetch_a = [&](int tile, int ks) {  // every request is unconditional: k steps beyond the last repeat it
+  auto fetch_a = [&](int tile, int ks, int set = 0) {  // every request is unconditional: k steps beyond the last repeat it
     const int t_ = tile < steps ? tile : steps - 1;
     const char *src = a_base + (int64_t)t_ * (kTile * kTileK * 2) + ks * 32;
 #pragma unroll
-    for (int ta = 0; ta < TA; ++ta) af[ks][ta] = *reinterpret_cast<const u32x4 *>(src + (int64_t)ta * a.plane_stride * 2 + a_lane);
+    for (int ta = 0; ta < TA; ++ta) af[2 * set + ks][ta] = *reinterpret_cast<const u32x4 *>(src + (int64_t)ta * a.plane_stride * 2 + a_lane);
   };
   auto fetch_b = [&](int tile, int set) {
 #pragma unroll
@@ -942,20 +951,60 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   const int tr_g = lane >> 4, tr_i = lane & 15;
   const uint32_t tr_off = (uint32_t)((8 * (tr_g >> 1) + (tr_i >> 2)) * kPlanePitch + (16 * (tr_g & 1) + 4 * (tr_i & 3)) * 2);
   typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  auto multiply = [&](int tile, int next_a) {
+  auto fragment_b = [&](const uint8_t *Bs, int tb, int ks, int nt) {
+    const uint8_t *src = Bs + tb * kRowPlane + ks * 16 * kPlanePitch + nt * 64;
+    const u32x2 k03 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(src)));
+    const u32x2 k47 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(src + 4 * kPlanePitch)));
+    u32x4 v;
+    v.x = k03.x; v.y = k03.y; v.z = k47.x; v.w = k47.y;
+    return v;
+  };
+  auto multiply = [&](auto parity, int tile, int next_a) {  // parity: of the tile
     const uint8_t *Bs = lds + (tile & 1) * kBuf + tr_off;
+    if constexpr (RAGGED) {
+      constexpr int set = decltype(parity)::value;
+      fetch_a(next_a, 0, set ^ 1);
+      fetch_a(next_a, 1, set ^ 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int pair = 0; pair < 4; pair += 2) {
+        u32x4 bf[2][2][TB];
+        f32x16 part[2];  // the products of this step, smallest terms first
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) bf[n][ks][tb] = fragment_b(Bs, tb, ks, pair + n);
+#pragma unroll
+          for (int q = 0; q < 16; ++q) part[n][q] = 0.0f;
+        }
+#pragma unroll
+        for (int order = Pairs<TA, TB>::kMax; order >= 0; --order) {
+#pragma unroll
+          for (int ta = 0; ta < TA; ++ta) {
+            const int tb = order - ta;
+            if (tb < 0 || tb >= TB) continue;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+              for (int n = 0; n < 2; ++n)
+                part[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, af[2 * set + ks][ta]),
+                                                                  __builtin_bit_cast(f16x8, bf[n][ks][tb]), part[n], 0, 0, 0);
+          }
+        }
+        acc[pair] += part[0];
+        acc[pair + 1] += part[1];
+      }
+      return;
+    }
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
       u32x4 bf[4][TB];
 #pragma unroll
       for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-        for (int tb = 0; tb < TB; ++tb) {
-          const uint8_t *src = Bs + tb * kRowPlane + ks * 16 * kPlanePitch + nt * 64;
-          const u32x2 k03 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(src)));
-          const u32x2 k47 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(src + 4 * kPlanePitch)));
-          bf[nt][tb].x = k03.x; bf[nt][tb].y = k03.y; bf[nt][tb].z = k47.x; bf[nt][tb].w = k47.y;
-        }
+        for (int tb = 0; tb < TB; ++tb) bf[nt][tb] = fragment_b(Bs, tb, ks, nt);
       // smallest terms first, as mfma_step
 #pragma unroll
       for (int order = Pairs<TA, TB>::kMax; order >= 0; --order) {
@@ -989,16 +1038,16 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
     stage(i + 1, 1);
     fetch_b(i + 3, 1);
     __builtin_amdgcn_sched_barrier(0);
-    multiply(i, i + 1);
+    multiply(std::integral_constant<int, 0>(), i, i + 1);
     __syncthreads();
     if (i + 2 < steps) stage(i + 2, 0);
     fetch_b(i + 4, 0);
     __builtin_amdgcn_sched_barrier(0);
-    multiply(i + 1, i + 2);
+    multiply(std::integral_constant<int, 1>(), i + 1, i + 2);
     __syncthreads();
   }
   if (i < steps) {
-    multiply(i, i);
+    multiply(std::integral_constant<int, 0>(), i, i);
     __syncthreads();
   }
 
@@ -1562,27 +1611,29 @@ __global__ void __launch_bounds__(256) split_planes_kernel(const float *x, int64
 __global__ void __launch_bounds__(256) dw_reduce_scalar_kernel(const float *partials, int chunks, int64_t count, float *out) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= count) return;
-  float sum = 0.0f;
-  for (int c = 0; c < chunks; ++c) sum += partials[(int64_t)c * count + i];
-  out[i] = sum;
+  double sum = 0.0;
+  for (int c = 0; c < chunks; ++c) sum += (double)partials[(int64_t)c * count + i];
+  out[i] = (float)sum;
 }
 
 // count a multiple of 4 and 16-byte aligned buffers: four elements per work-item, the chunks in their order, four
-// loads in flight
+// loads in flight; in 64 bits, which the loads hide (error of the weight gradient against float64, relative 2-norm, [64, 512, 49]
+// spikes, 96 output channels: 1.67e-7 with fp32 sums over the 64 chunks, 8.3e-8 now; the library's fp32 1.49e-7)
 __global__ void __launch_bounds__(256) dw_reduce_kernel(const float *partials, int chunks, int64_t count, float *out) {
   const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= count) return;
-  f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+  typedef double f64x4 __attribute__((ext_vector_type(4)));
+  f64x4 sum = {0.0, 0.0, 0.0, 0.0};
   int c = 0;
   for (; c + 4 <= chunks; c += 4) {
     f32x4 v[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(partials + (int64_t)(c + u) * count + i));
 #pragma unroll
-    for (int u = 0; u < 4; ++u) sum += v[u];
+    for (int u = 0; u < 4; ++u) sum += __builtin_convertvector(v[u], f64x4);
   }
-  for (; c < chunks; ++c) sum += __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(partials + (int64_t)c * count + i));
-  *reinterpret_cast<f32x4 *>(out + i) = sum;
+  for (; c < chunks; ++c) sum += __builtin_convertvector(__builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(partials + (int64_t)c * count + i)), f64x4);
+  *reinterpret_cast<f32x4 *>(out + i) = __builtin_convertvector(sum, f32x4);
 }
 
 int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
