@@ -472,7 +472,7 @@ int sjhip_ssa_lif_backward_packed(int neuron, const sjhip_neuron_params *p, int6
  * the accuracy of an fp32 GEMM; an operand that bf16 holds exactly (spikes) needs 1 term.  Supported (a_terms, b_terms):
  * (3,3) (3,1) (2,2) (2,1) (1,1).  sjhip_pwconv_gemm needs an even L, 16-byte aligned weight planes and 8-byte
  * aligned activations; sjhip_pwconv_grad_weight needs L a multiple of 4 and 16-byte aligned tensors
- * (SJHIP_ERR_UNSUPPORTED otherwise).
+ * (SJHIP_ERR_UNSUPPORTED otherwise).  The fp16 forms below take more lengths.
  *
  *   sjhip_pwconv_split_weight   planes = bf16 terms [3][rows_pad * cols_pad] (zero padded to multiples of 128 and 32, and
  *                               stored as tiles of 128 rows x 32 columns in the order sjhip_pwconv_gemm reads them: an
@@ -538,6 +538,8 @@ int sjhip_pwconv_grad_weight(const float *dy, int dy_terms, const float *x, int 
  *                                  b_terms 2 with the b_amax buffer of b (sjhip_pwconv_amax_floats(S) floats; larger
  *                                  maxima are safe, smaller ones are not), or 1 with NULL
  *   sjhip_pwconv_grad_weight_f16   sjhip_pwconv_grad_weight with two terms of dy (dy_amax) and x_terms of x
+ * Lengths: sjhip_pwconv_gemm_f16 takes L = 2 and any L >= 4, sjhip_pwconv_grad_weight_f16 any L >= 4 (alignment as above).
+ * Where 4 does not divide L, the products of 32 consecutive k are summed before they are added to the rest.
  */
 #define SJHIP_PW_F16 16          /* internal term code of an fp16 operand: SJHIP_PW_F16 | terms */
 #define SJHIP_PW_AMAX_FLOATS 256
@@ -570,7 +572,9 @@ int sjhip_pwconv_grad_weight_f16_bits(const float *dy, const float *dy_amax, con
  *   backward   sjhip_bn_lif_backward / sjhip_bn_plif_backward, sjhip_bn_backward_finalize, and for dx or dw
  *              sjhip_bn_grad_input_amax, then sjhip_pwconv_grad_weight_f16[_bits] (dw != NULL),
  *              sjhip_pwconv_split_weight_f16 and sjhip_pwconv_gemm_f16 (dx != NULL)
- * x [T*B][Cin][L] fp32 or x_bits (bit-packed spikes, L a multiple of 4); x_amax: sjhip_pwconv_amax_floats(T*B) words to
+ * The neuron stage's arguments are checked before the first launch: a refused call has not touched the running statistics.
+ * L: a multiple of 4 or, with fp32 x, at least 4 with Cout * L a multiple of 4 (SJHIP_ERR_UNSUPPORTED otherwise).
+ * x [T*B][Cin][L] fp32 or x_bits (bit-packed spikes, Cin * L a multiple of 8); x_amax: sjhip_pwconv_amax_floats(T*B) words to
  * fill (forward) or filled (backward) for real-valued x, NULL for x that fp16 holds exactly; weight [Cout][Cin]; bn_map
  * [4][Cout]: scale, shift, mean, 1/std; k_device and grad_k with SJHIP_NEURON_PLIF and only with it; channel_grads
  * [5][Cout]: dgamma, dbeta and the three coefficients of the input gradient; dy [T*B][Cout][L]: the gradient of the
@@ -627,7 +631,7 @@ int sjhip_pwconv_grad_weight_planes(const uint16_t *dy_planes, const float *dy_a
 
 /*
  * Batch normalisation fused with the multi-step IF / LIF neuron behind it, for fp32 activations [T][B][C][L]
- * (L contiguous, a multiple of 4).  Stands in for nn.BatchNorm1d / nn.BatchNorm2d followed by LIFNode in the reference's
+ * (L contiguous, a multiple of 4, or at least 4 with C * L a multiple of 4).  Stands in for nn.BatchNorm1d / nn.BatchNorm2d followed by LIFNode in the reference's
  * SpikingSelfAttention (layer/attention.py:314-329, 370-384) and SpikformerConv2dBNLIF (model/spikformer.py:196-212),
  * which torch runs as separate passes; here the normalised tensor is never written.
  *

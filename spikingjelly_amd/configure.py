@@ -27,9 +27,11 @@ for its CuPy/Triton backends).
     ``True``: training forwards write no ``h_seq``; the backward kernel replays the forward from
     ``x_seq`` and ``v_init`` (bit-identical ``h``, held in LDS), so autograd keeps ``x_seq`` alive
     instead of a same-sized ``h_seq`` and the forward's largest write disappears.  Used whenever the
-    library prefers it for the shape (``sjhip_recompute_preferred``: ``N`` at least one 128-bit
+    library prefers it for the shape (``sjhip_recompute_preferred``: ``N`` a multiple of the 128-bit
     vector and the sequence short enough for the replayed ``h`` to stay in LDS with enough
-    resident wavefronts); other shapes and ``False`` fall back to saving ``h_seq``.
+    resident wavefronts) and, by IF, LIF, parametric LIF, QIF, EIF and ILIF, for other ``N`` of at least
+    one vector as well, except with 16-bit storage and fp32 state: there a saved ``h_seq`` is rounded to
+    the storage type and a replayed one is not.  Other shapes and ``False`` fall back to saving ``h_seq``.
 """
 
 hip_half_precision_mode = "torch"

@@ -277,7 +277,7 @@ __device__ __forceinline__ void replay_h_charge(const FwdArgs &f, int len, const
 
 // BPTT over the replayed h (recurrence of neuron_bwd.h); writes g = dL/dz and adds every neuron's share of
 // sum g and sum g y.  SUMS: one sum of the four neurons, or (ragged rows) one of each, because a neuron that a neighbour has
-// too is counted once; whole rows keep the order, and with it the bits, of a single sum (four: 184 instead of 182 us for the two
+// too is counted once; whole rows keep a single sum per work-item (four: 184 instead of 182 us for the two
 // backwards of an attention block [4, 64, 384, 196]).  PLIF: also of dL/dk = sum G_t dh_t/dk, dh_t/dk = (h_t - v_{t-1}) / k with input decay (the division
 // is left to the final reduction) or v_reset - v_{t-1} without; v_{t-1} is re-derived from h_{t-1} with the forward's
 // reset arithmetic, v0 is the state in front of the first of these steps.
@@ -743,7 +743,11 @@ int launch_bn_lif_backward(int neuron, const sjhip_neuron_params &p, int64_t T, 
     }
     return nb;
   };
-  // more than the four rows a block of the wavefront-per-row kernel takes: more lanes working
+  // More than the four rows a block of the wavefront-per-row kernel takes, hence more lanes working: rows of 8 to 51 groups
+  // (L = 29 to 204; the partial sums of a block hold 32 rows, shorter ones stay with the other kernel).  Wavefront per row / this,
+  // us: [4, 64, 384, L] at L = 32 31.9 / 11.1, 48 33.7 / 12.7, 60 34.8 / 17.0; [8, 32, 512, L] at 32 52.0 / 13.4, 60 55.3 / 20.7;
+  // [20, 16, 256, L] at 32 41.5 / 22.0, 60 44.3 / 24.9; [4, 16, 256, L], few blocks, at 32 6.5 / 6.5, 60 7.4 / 6.2.  The two
+  // add a row in different orders.
   const bool by_rows = per > 4 && per <= kBnRowsMax;
   if (by_rows && (a.rows + per - 1) / per > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "bn_lif_backward: %lld rows", (long long)a.rows);
   auto by_shape = [&](auto plif_flag, auto ragged) {

@@ -805,8 +805,8 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
 // LDS of pw_gemm_rows_kernel: two B tiles (or the output staging of the epilogue, whichever is larger), then 128 floats
 constexpr unsigned rows_inverse_offset(int tb) { return 2u * tb * kRowPlane > kOutLds ? 2u * tb * kRowPlane : kOutLds; }
 
-// pw_gemm_rows_kernel: the same product, term order and batch-norm sums as pw_gemm_kernel<2, TB, true, kBFloat> (bit for
-// bit), laid out for what a compute unit can move.  Measured per compute unit: LDS reads of 16 bytes per lane run at
+// pw_gemm_rows_kernel: the same product, term order and batch-norm sums as pw_gemm_kernel<2, TB, true, kBFloat> (on rows of a
+// multiple of four bit for bit), laid out for what a compute unit can move.  Measured per compute unit: LDS reads of 16 bytes per lane run at
 // 256 bytes per cycle but writes at 64-78, and the vector memory path issues one wavefront load of 8 or 16 bytes per lane
 // every 16 cycles (58 bytes per cycle from L1), so in pw_gemm_kernel a K step of a block costs about as many cycles of LDS
 // (16 KB of A and 16 KB of B written, 64 KB read) and of the load path (32 eight-byte loads of B, 16 of A) as of the matrix
@@ -1760,7 +1760,8 @@ int64_t pwconv_gemm_stats_rows(int64_t K, int64_t S, int64_t L) {
 
 int launch_pwconv_gemm(const uint16_t *a_planes, int a_terms, int64_t M, int64_t K, const float *b, int b_terms,
                        const float *b_amax, int64_t S, int64_t L, float *c, float *stats, hipStream_t stream, bool b_bits) {
-  // fp16 planes and at least four positions (bits: a multiple of four): the kernel that keeps A out of LDS
+  // fp16 planes and at least four positions (bits: a multiple of four): the kernel that keeps A out of LDS, whose pieces are
+  // four positions of one sample.  What is left of the fp16 forms for pw_gemm_kernel are two positions, and bits with L % 4 == 2.
   const bool rows_kernel = SJHIP_PW_ROWS != 0 && a_terms == (SJHIP_PW_F16 | 2) && (b_bits ? L % 4 == 0 && b_terms == 1 : L >= 4 && (b_terms == 1 || b_terms == 2));
   if ((L % 2 != 0 && !rows_kernel) || !aligned16(a_planes) || (!b_bits && (reinterpret_cast<uintptr_t>(b) & 7u)))
     return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_gemm: L=%lld must be even (or, on fp16 planes and fp32 activations, at least 4), the weight planes 16-byte and the activations 8-byte aligned", (long long)L);
