@@ -283,6 +283,29 @@ def test_fp16_gemms_read_bit_packed_spikes(C, S, M, Kd, Lp):
     assert torch.equal(C.pw_grad_weight_bits(dy, bits, Kd), C.pw_grad_weight(dy, F, x, C.F16 | 1))
 
 
+@pytest.mark.parametrize("S,M,Kd", [(3, 100, 52), (1, 7, 4), (67, 130, 260)])
+@pytest.mark.parametrize("Lp,source", [(2, "real"), (2, "spikes"), (2, "bits"), (6, "bits"), (10, "bits")])
+def test_fp16_gemm_of_the_lengths_its_row_kernel_leaves(C, S, M, Kd, Lp, source):
+    """Two positions, and bit-packed spikes over a length with remainder 2: the general kernel on fp16 planes, with its batch-norm
+    sums, against 64 bits (2^-22 of the split and 2^-24 per fp32 addition; sums and sums of squares on top of that)."""
+    from spikingjelly_amd.activation_based.hip_kernel.compress import bit_spike_compress
+
+    F = C.F16 | 2
+    w = seeded_randn((M, Kd), 84).cuda()
+    x = seeded_randn((S, Kd, Lp), 85).cuda() if source == "real" else (seeded_randn((S, Kd, Lp), 85) > 0.4).float().cuda()
+    planes = C.split_weight(w, False, F)
+    if source == "bits":
+        got, sums = C.pw_gemm_bits(planes, M, Kd, bit_spike_compress(x), S, Lp, stats=True)
+    else:
+        got, sums = C.pw_gemm(planes, F, M, Kd, x, F if source == "real" else C.F16 | 1, stats=True)
+    exact, terms = w.double() @ x.double(), w.double().abs() @ x.double().abs()
+    rel = 2.0 ** -22 + Kd * 2.0 ** -24
+    assert ((got.double() - exact).abs() <= rel * terms).all()
+    for i, power in ((0, 1), (1, 2)):
+        bound = power * (rel + 64 * 2.0 ** -24) * terms.pow(power).sum((0, 2))
+        assert ((sums[..., i].double().sum(0) - exact.pow(power).sum((0, 2))).abs() <= bound).all()
+
+
 def test_amax(C):
     """``amax(x)``: the maximum of the first 256 words is the largest magnitude among the numbers of ``x``, for any length
     and alignment, ``sample_amax`` of the words that of every sample, and both fold into what the words already hold."""

@@ -269,6 +269,31 @@ def test_saved_tensors_that_are_not_the_saved_ones_are_refused(what):
         s.sum().backward()
 
 
+def test_calls_on_a_side_stream():
+    """Forward on a stream of its own, backward asked for from the main stream: kernels and memory stay with the forward's
+    stream, also while the main stream allocates and works."""
+    g = torch.Generator().manual_seed(9)
+    x0, gs = (torch.randn(6, 1 << 16, generator=g) + 0.4).cuda(), torch.randn(6, 1 << 16, generator=g).cuda()
+    v = torch.zeros(1 << 16, device="cuda")
+
+    def run(stream):
+        x = x0.clone().requires_grad_()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            out = functional.lif_multi_step_hip(x * 1.25, v, 2.0, True, 1.0, 0.0, surrogate.ATan(), store_v_seq=True)
+        noise = [torch.randn(6, 1 << 16, device="cuda") for _ in range(4)]
+        torch.cuda.current_stream().wait_stream(stream)
+        (out[0] * gs + out[2]).sum().backward()
+        return [t.detach() for t in out] + [x.grad, sum(noise)]
+
+    want = run(torch.cuda.current_stream())[:4]
+    side = torch.cuda.Stream()
+    for _ in range(5):
+        got = run(side)[:4]
+        torch.cuda.synchronize()
+        _equal(got, want)
+
+
 def test_packed_inference_equals_the_operator():
     x = (torch.rand(6, 5, 16, device="cuda") * 0.6).half()
     v = torch.zeros(5, 16, dtype=torch.float16, device="cuda")

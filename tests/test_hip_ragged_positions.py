@@ -127,9 +127,13 @@ def test_normalise_and_neuron(C, L, T):
 
 
 @pytest.mark.parametrize("T", [3, 20])
-def test_parametric_time_constant(C, T):
-    B, Ch, L = 2, 20, 49
+@pytest.mark.parametrize("L", [5, 49, 257])  # (a wavefront per row, rows packed into blocks, several rounds of a wavefront per row)
+@pytest.mark.parametrize("last", [False, True])
+def test_parametric_time_constant(C, T, L, last):
+    B, Ch = 2, 20
     y, gs = seeded_randn((T, B, Ch, L), 8, 0.4, 1.2).cuda(), seeded_randn((T, B, Ch, L), 9).cuda()
+    if last:  # only the row's last four positions, most of which two groups hold, have an upstream gradient
+        gs[..., :-4] = 0.0
     stats = C._bn_map(y.flatten(0, 1), None, None, None, None, True, 0.1, 1e-5)
     v0 = torch.zeros((B, Ch, L), device="cuda")
     k = torch.tensor([0.4], device="cuda")

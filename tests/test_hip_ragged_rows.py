@@ -67,6 +67,27 @@ def test_ragged_rows_equal_padded_rows(kind, dtype, mode, N, T, monkeypatch):
         assert abs(float(got[4]) - float(want[4])) <= (T + 60) * 2.0 ** -24 * 2.0 * T * N, (float(got[4]), float(want[4]))
 
 
+@pytest.mark.parametrize("T", [8, 45])
+@pytest.mark.parametrize("N", [9, 15, 1025, 1027, 4099])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("saved_h", [False, True])
+def test_a_neuron_held_twice_counts_once_in_the_time_constant(dtype, N, T, saved_h, monkeypatch):
+    """Only the last vector of a row has an upstream gradient: dL/dk is then a sum of few terms, most of them of the neurons that
+    two work-items hold."""
+    monkeypatch.setattr(configure, "hip_backward_recompute", not saved_h)
+    g = torch.Generator().manual_seed(N * 100 + T)
+    pad, V = (N + 7) // 8 * 8, 16 // dtype.itemsize
+    x, gs = torch.zeros(T, pad), torch.zeros(T, pad)
+    x[:, :N] = torch.randn(T, N, generator=g) * 0.8 + 0.4
+    gs[:, N - V:N] = torch.rand(T, V, generator=g) + 0.5
+    x, gs = x.to(dtype).cuda(), gs.to(dtype).cuda()
+    got = float(_run("plif", x[:, :N].contiguous(), gs[:, :N].contiguous(), None)[4])
+    want = float(_run("plif", x, gs, None)[4])
+    # (fp32 sums of T V terms below 8: the carried gradient reaches 1.5 / (1 - 1/2) and more through the reset, times |h - v| < 2)
+    assert abs(got - want) <= (T + 60) * 2.0 ** -24 * 8.0 * T * V, (got, want)
+    assert abs(want) > 0.05  # a shared neuron counted twice would show
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("offset", [1, 3])
 def test_rows_that_begin_off_the_vector_alignment(dtype, offset):
