@@ -1142,11 +1142,13 @@ struct PwDwArgs {
   const float *dy_amax, *x_amax;  // fp16 terms: nullptr (no scale), or the words whose maximum is the tensor's max |.|
 };
 
-// Two LDS buffers (fp16 terms: 2 x 40 KiB, two blocks per compute unit still fit): the next tile is split and stored while
-// the current one is multiplied, with one barrier per K step instead of two.
-// (M = 1536, N = 384, 25 088 columns: 148 -> 145 us; M = 1152, 50 176 columns: 216 -> 213.  The bf16 split's three planes per
-// operand would leave one block per compute unit.)
-constexpr bool dw_two_buffers(bool h) { return h; }
+// Two LDS buffers where x has one fp16 term (spikes, 2 x 30 KiB): the next tile is split and stored while the current one is
+// multiplied, with one barrier per K step instead of two.  One buffer / two, us with the reduction, three processes of each in
+// turn on one box: x as bits, dy [256, 1152, 196] and x [256, 384, 196] 146.6 / 142.0, [128, 1536, 196] and [128, 384, 196]
+// 108.6 / 105.1, [256, 384, 196] both 58.3 / 55.5; x as fp32 spikes 197.6 / 189.4, 110.1 / 110.1, 59.9 / 59.9.  With two terms of x
+// (2 x 40 KiB) two buffers measured 210.4 -> 214.0, 138.8 -> 138.4, 74.7 -> 74.5: those keep one, and every launch stays within
+// the default limit of dynamic LDS.  (The bf16 split's three planes per operand would leave one block per compute unit.)
+constexpr bool dw_two_buffers(bool h, int tb) { return h && tb == 1; }
 // four elements at a 16-byte or, with ANY, at a 4-byte address
 template <bool ANY> __device__ __forceinline__ f32x4 load4(const char *p) {
   if (ANY) return *reinterpret_cast<const f32x4_any *>(p);
@@ -1162,7 +1164,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   extern __shared__ __align__(16) uint8_t lds[];
   // [TA][128][kRowBytes] of dy, then [TB][128][kRowBytes] of x; DOUBLE: twice
   uint8_t *As = lds, *Bs = lds + TA * kRowPlane;
-  constexpr bool DOUBLE = dw_two_buffers(H);
+  constexpr bool DOUBLE = dw_two_buffers(H, TB);
   constexpr int kBuf = DOUBLE ? (TA + TB) * kRowPlane : 0;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
@@ -1616,7 +1618,7 @@ __global__ void __launch_bounds__(256) dw_reduce_scalar_kernel(const float *part
   out[i] = (float)sum;
 }
 
-// count a multiple of 4 and 16-byte aligned buffers: four elements per work-item, the chunks in their order, four
+// count a multiple of 4 and 16-byte aligned buffers: four elements per work-item, the chunks in their order, eight
 // loads in flight; in 64 bits, which the loads hide (error of the weight gradient against float64, relative 2-norm, [64, 512, 49]
 // spikes, 96 output channels: 1.67e-7 with fp32 sums over the 64 chunks, 8.3e-8 now; the library's fp32 1.49e-7)
 __global__ void __launch_bounds__(256) dw_reduce_kernel(const float *partials, int chunks, int64_t count, float *out) {
@@ -1625,14 +1627,19 @@ __global__ void __launch_bounds__(256) dw_reduce_kernel(const float *partials, i
   typedef double f64x4 __attribute__((ext_vector_type(4)));
   f64x4 sum = {0.0, 0.0, 0.0, 0.0};
   int c = 0;
-  for (; c + 4 <= chunks; c += 4) {
-    f32x4 v[4];
+  auto add = [&](auto loads) {  // (all of them in flight before the first is used)
+    constexpr int kLoads = decltype(loads)::value;
+    for (; c + kLoads <= chunks; c += kLoads) {
+      f32x4 v[kLoads];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(partials + (int64_t)(c + u) * count + i));
+      for (int u = 0; u < kLoads; ++u) v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(partials + (int64_t)(c + u) * count + i));
 #pragma unroll
-    for (int u = 0; u < 4; ++u) sum += __builtin_convertvector(v[u], f64x4);
-  }
-  for (; c < chunks; ++c) sum += __builtin_convertvector(__builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(partials + (int64_t)c * count + i)), f64x4);
+      for (int u = 0; u < kLoads; ++u) sum += __builtin_convertvector(v[u], f64x4);
+    }
+  };
+  add(std::integral_constant<int, 8>());
+  add(std::integral_constant<int, 2>());
+  add(std::integral_constant<int, 1>());
   *reinterpret_cast<f32x4 *>(out + i) = __builtin_convertvector(sum, f32x4);
 }
 
@@ -1658,12 +1665,8 @@ int launch_gemm_rows(const PwGemmArgs &a, int64_t blocks, hipStream_t stream) {
 
 template <int TA, int TB, bool H, bool BITS, bool RAGGED>
 int launch_dw(const PwDwArgs &a, int64_t blocks, hipStream_t stream) {
-  constexpr unsigned lds = (dw_two_buffers(H) ? 2 : 1) * (TA + TB) * kRowPlane;
-  if constexpr (lds > 64u * 1024u) {
-    static OncePerDevice once;
-    const hipError_t attr_rc = allow_dynamic_lds(once, reinterpret_cast<const void *>(&pw_dw_kernel<TA, TB, H, BITS, RAGGED>), (int)lds);
-    if (attr_rc != hipSuccess) return fail(SJHIP_ERR_LAUNCH, "pwconv_grad_weight: cannot raise the dynamic LDS limit: %s", hipGetErrorString(attr_rc));
-  }
+  constexpr unsigned lds = (dw_two_buffers(H, TB) ? 2 : 1) * (TA + TB) * kRowPlane;
+  static_assert(lds <= 64u * 1024u, "within the default limit of dynamic LDS");
   hipLaunchKernelGGL((pw_dw_kernel<TA, TB, H, BITS, RAGGED>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
   return check_launch("pwconv_grad_weight");
 }
