@@ -405,14 +405,20 @@ struct PwGemmArgs {
 #define SJHIP_PW_WIDE_OUT 1
 #endif
 typedef u32x4 u32x4_any __attribute__((aligned(4)));
-// the elements skip .. 3 of v at the places 0 .. 3 - skip, zeros behind them
+// the elements skip .. 3 of v at the places 0 .. 3 - skip, zeros behind them: down by one where bit 0 of skip is set, then by two
+// where bit 1 is (eight selects; chosen among four by the value of skip, the compiler branches for every vector)
 template <typename V> __device__ __forceinline__ V moved_down(V v, int skip) {
+  const bool one = (skip & 1) != 0, two = (skip & 2) != 0;
   V r;
-  r.x = skip == 0 ? v.x : (skip == 1 ? v.y : (skip == 2 ? v.z : v.w));
-  r.y = skip == 0 ? v.y : (skip == 1 ? v.z : (skip == 2 ? v.w : 0));
-  r.z = skip == 0 ? v.z : (skip == 1 ? v.w : 0);
-  r.w = skip == 0 ? v.w : 0;
-  return r;
+  r.x = one ? v.y : v.x;
+  r.y = one ? v.z : v.y;
+  r.z = one ? v.w : v.z;
+  r.w = one ? 0 : v.w;
+  v.x = two ? r.z : r.x;
+  v.y = two ? r.w : r.y;
+  v.z = two ? 0 : r.z;
+  v.w = two ? 0 : r.w;
+  return v;
 }
 constexpr int kOutPitch = 68;                              // floats per row of the output staging buffer (64 columns + 4)
 constexpr unsigned kOutLds = 4 * 32 * kOutPitch * 4;       // 32 rows x 64 columns per wavefront
@@ -832,8 +838,8 @@ constexpr unsigned rows_inverse_offset(int tb) { return 2u * tb * kRowPlane > kO
 // against float64 was above that of the library's fp32 GEMM, which serves these lengths otherwise (relative 2-norm, spikes,
 // [48, 512, 49] -> 128 channels: library 1.11e-7, chain 1.54e-7, now 9.9e-8; real values, [4, 1536, 49] -> 512: 3.5e-7, 4.4e-7,
 // 1.6e-7; over 70 shapes of 96 to 576 channels, 7 x 7 and 9 x 9: 0.87 of the library's forward and 0.33 of its input gradient on
-// average, at most 1.09).  It takes 256 registers, two wavefronts per SIMD: [128, 384, 49] -> 1536 38.9 -> 46.0 us, its input
-// gradient 53.5 -> 59.1, [96, 512, 81] -> 512 25.8 -> 28.6.
+// average, at most 1.09).  It takes 256 registers, two wavefronts per SIMD: [128, 384, 49] -> 1536 (624 blocks, more
+// than are resident then) 37.9 -> 44.1 us, its input gradient 53.1 -> 51.8, [96, 512, 81] -> 512 25.8 -> 26.2.
 template <int TB, bool BITS, bool RAGGED>
 __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu(RAGGED ? 2 : 3, RAGGED ? 2 : 3))) pw_gemm_rows_kernel(const PwGemmArgs a) {
   constexpr int TA = 2;
