@@ -66,27 +66,34 @@ def test_gemms(C, L, S, M, K, spikes):
         assert ((a - b).abs() <= power * 2 * (2.0 ** -22 + K * 2.0 ** -24 + 64 * 2.0 ** -24) * scale).all()
 
 
-@pytest.mark.parametrize("T, B, Cin, Cout, side", [(6, 8, 512, 128, 7), (4, 1, 512, 1536, 7), (4, 16, 256, 256, 7), (2, 32, 512, 96, 7)])
+# Relative 2-norm errors against 64 bits, in 1e-7, of torch's fp32 convolution (y, dx, dw) on the inputs of the test below: the smallest of
+# four processes, which differ in the last digits of dw only.
+LIBRARY_ERRORS = {
+    (6, 8, 512, 128): {False: (2.065, 2.033, 2.321), True: (1.149, 2.033, 2.264)},
+    (4, 1, 512, 1536): {False: (2.880, 3.540, 1.333), True: (1.478, 3.540, 0.8018)},
+    (4, 16, 256, 256): {False: (1.498, 2.049, 2.065), True: (0.8767, 2.049, 1.901)},
+    (2, 32, 512, 96): {False: (2.068, 1.760, 1.939), True: (1.144, 1.760, 1.477)},
+}
+
+
+@pytest.mark.parametrize("T, B, Cin, Cout", LIBRARY_ERRORS)
 @pytest.mark.parametrize("spikes", [False, True])
-def test_no_further_from_64_bits_than_the_library(C, T, B, Cin, Cout, side, spikes):
-    """What ran on the library's fp32 convolution before it ran on the fp16 split: the split's sums (the K steps of a column, and
-    the sample groups of a weight gradient in 64 bits) are no further from 64 bits.  2-norm over the whole result, which
-    varies by 1 % between seeds; measured 0.3 to 0.9 of the library's error (1.4 without the order of the sums)."""
-    F, S = C.F16 | 2, T * B
-    x = (seeded_randn((S, Cin, side * side), 30) > 0.7).float().cuda() if spikes else seeded_randn((S, Cin, side * side), 30).cuda()
-    w, dy = (seeded_randn((Cout, Cin), 31) * Cin ** -0.5).cuda(), seeded_randn((S, Cout, side * side), 32).cuda()
-    xr, wr = x.view(S, Cin, side, side).clone().requires_grad_(), w.view(Cout, Cin, 1, 1).clone().requires_grad_()
-    y = torch.nn.functional.conv2d(xr, wr)
-    y.backward(dy.view(S, Cout, side, side))
-    library = (y.detach().view_as(dy), xr.grad.view_as(x), wr.grad.view_as(w))
+def test_no_further_from_64_bits_than_the_library(C, T, B, Cin, Cout, spikes):
+    """Position counts that four does not divide ran on the library's fp32 convolution before they ran on the fp16 split: the
+    split's sums (the K steps of a column, and the sample groups of a weight gradient in 64 bits) are no further from 64 bits.
+    The kernels add in a fixed order, so the errors are the same on every run: 0.35 to 0.98 of the library's (with one chain over
+    all of K and fp32 sums over the groups up to 1.34)."""
+    F, S, L = C.F16 | 2, T * B, 49
+    x = (seeded_randn((S, Cin, L), 30) > 0.7).float().cuda() if spikes else seeded_randn((S, Cin, L), 30).cuda()
+    w, dy = (seeded_randn((Cout, Cin), 31) * Cin ** -0.5).cuda(), seeded_randn((S, Cout, L), 32).cuda()
     terms = C.F16 | 1 if spikes else F
     split = (C.pw_gemm(C.split_weight(w, False, F), F, Cout, Cin, x, terms), C.pw_gemm(C.split_weight(w, True, F), F, Cin, Cout, dy, F),
              C.pw_grad_weight(dy, F, x, terms))
     x64, w64, dy64 = x.double(), w.double(), dy.double()
     exact = (w64 @ x64, w64.t().contiguous() @ dy64,
              dy64.transpose(0, 1).reshape(Cout, -1) @ x64.transpose(0, 1).reshape(Cin, -1).t().contiguous())
-    for name, a, b, r in zip(("y", "dx", "dw"), split, library, exact):
-        assert float((a - r).norm()) <= 1.02 * float((b - r).norm()), name
+    for name, a, r, library in zip(("y", "dx", "dw"), split, exact, LIBRARY_ERRORS[T, B, Cin, Cout][spikes]):
+        assert float((a.double() - r).norm() / r.norm()) <= library * 1e-7, name
 
 
 @pytest.mark.parametrize("L", LENGTHS)
