@@ -87,9 +87,9 @@ Tensor dense_grad(const Tensor &g, at::ScalarType dtype) {
 }
 
 // A saved tensor as the kernels take it.  A saved-tensor hook may hand the values back in another layout or type; what is
-// not on the device, or has another size, is refused before a kernel reads it.
-Tensor saved_values(const Tensor &t, const char *name, at::ScalarType dtype, int64_t numel) {
-  TORCH_CHECK(t.is_cuda(), "backend='hip' runs on a ROCm device only, but the saved ", name, " is on ", t.device());
+// not on the device of the forward, or has another size, is refused before a kernel reads it.
+Tensor saved_values(const Tensor &t, const char *name, c10::Device device, at::ScalarType dtype, int64_t numel) {
+  TORCH_CHECK(t.device() == device, "backend='hip': the saved ", name, " is on ", t.device(), " and not on ", device);
   TORCH_CHECK(t.layout() == at::kStrided && t.numel() == numel, "the saved ", name, " has ", t.numel(), " elements instead of ", numel);
   return t.scalar_type() == dtype ? t : t.to(dtype);
 }
@@ -101,6 +101,7 @@ struct NeuronBackward : public torch::autograd::Node {
   bool with_k = false, single = false;  // single: one step without a time dimension
   sjhip_neuron_params params{};  // without SJHIP_FLAG_V_INIT_BROADCAST, which follows the state as it is unpacked
   at::ScalarType storage = at::kFloat;
+  c10::Device device = at::kCUDA;
   int neuron = 0, dtype = 0;
   int64_t T = 0, N = 0;
 
@@ -118,11 +119,11 @@ struct NeuronBackward : public torch::autograd::Node {
     if (!grads[0].defined() && !grads[1].defined() && !grads[2].defined()) return out;
     const Tensor saved_x = x_.unpack(), saved_v = v_.unpack(), saved_k = with_k ? k_.unpack() : Tensor();
     at::AutoDispatchBelowADInplaceOrView below;
-    c10::DeviceGuard guard(saved_x.device());
+    c10::DeviceGuard guard(device);
     // (the library asks for tensors that begin on 16 bytes; a step taken out of a sequence may not)
-    const Tensor x = dense16(saved_values(saved_x, "x_seq", storage, T * N));
-    Tensor v = saved_values(saved_v, "v_init", storage, N);
-    const Tensor k = with_k ? saved_values(saved_k, "k", at::kFloat, 1) : Tensor();
+    const Tensor x = dense16(saved_values(saved_x, "x_seq", device, storage, T * N));
+    Tensor v = saved_values(saved_v, "v_init", device, storage, N);
+    const Tensor k = with_k ? saved_values(saved_k, "k", device, at::kFloat, 1) : Tensor();
     sjhip_neuron_params p = params;
     if (is_broadcast(v)) p.flags |= SJHIP_FLAG_V_INIT_BROADCAST;
     else v = dense16(v);
@@ -241,6 +242,7 @@ py::object neuron_sequence(const Tensor &x_seq, const Tensor &v_init, const c10:
     node->params = p;
     node->params.flags &= ~(uint32_t)SJHIP_FLAG_V_INIT_BROADCAST;
     node->storage = x_seq.scalar_type();
+    node->device = x_seq.device();
     node->neuron = neuron; node->dtype = dtype; node->T = T; node->N = N;
     torch::autograd::set_history(spikes, node);
     torch::autograd::set_history(v_last, node);

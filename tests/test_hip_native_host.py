@@ -260,12 +260,15 @@ def test_saved_tensors_come_back_in_any_layout(unpack, state):
 
 
 @pytest.mark.parametrize("what", ["device", "size"])
-def test_saved_tensors_that_are_not_the_saved_ones_are_refused(what):
-    x = torch.randn(4, 64, device="cuda").requires_grad_()
-    unpack = (lambda t: t.cpu()) if what == "device" else (lambda t: t[..., :32].contiguous())
-    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
-        s = functional.lif_multi_step_hip(x, torch.zeros(64, device="cuda"), 2.0, True, 1.0, 0.0, surrogate.ATan())[0]
-    with pytest.raises(RuntimeError, match="saved x_seq"):
+@pytest.mark.parametrize("which", ["x_seq", "v_init", "k"])
+def test_saved_tensors_that_are_not_the_saved_ones_are_refused(what, which):
+    x, v = torch.randn(4, 64, device="cuda").requires_grad_(), torch.zeros(64, device="cuda")
+    k = torch.tensor(0.4, device="cuda").requires_grad_()
+    other = (lambda t: t.cpu()) if what == "device" else (lambda t: t[..., :32].contiguous() if t.dim() else t.expand(2).contiguous())
+    dim = {"x_seq": 2, "v_init": 1, "k": 0}[which]
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: other(t) if t.dim() == dim else t):
+        s = native.load().neuron_sequence(x, v, k, False, 2, 0.0, 1.0, 0.0, 1, 1, 2.0, False, 39, EXTRA)[0]
+    with pytest.raises(RuntimeError, match=f"saved {which}"):
         s.sum().backward()
 
 
