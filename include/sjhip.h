@@ -539,7 +539,8 @@ int sjhip_pwconv_grad_weight(const float *dy, int dy_terms, const float *x, int 
  *                                  maxima are safe, smaller ones are not), or 1 with NULL
  *   sjhip_pwconv_grad_weight_f16   sjhip_pwconv_grad_weight with two terms of dy (dy_amax) and x_terms of x
  * Lengths: sjhip_pwconv_gemm_f16 takes L = 2 and any L >= 4, sjhip_pwconv_grad_weight_f16 any L >= 4 (alignment as above).
- * Where 4 does not divide L, the products of 32 consecutive k are summed before they are added to the rest.
+ * Where 4 does not divide L, the GEMM sums the products of 32 consecutive k before it adds them to the rest (and with one
+ * term, or K <= 192, carries what that addition rounds off).
  */
 #define SJHIP_PW_F16 16          /* internal term code of an fp16 operand: SJHIP_PW_F16 | terms */
 #define SJHIP_PW_AMAX_FLOATS 256

@@ -834,15 +834,22 @@ constexpr unsigned rows_inverse_offset(int tb) { return 2u * tb * kRowPlane > kO
 // (RAGGED is a template parameter: asked at run time the moves cost the aligned case 4 %, 106 -> 110 us at M = 1536, K = 384,
 // 25 088 columns.)
 // The products of a K step of such rows are summed by themselves, the small terms of both halves first, and reach the
-// accumulators with one rounding: with one chain over all of K (as the rows of a multiple of four have it) the error
-// against float64 was above that of the library's fp32 GEMM, which serves these lengths otherwise (relative 2-norm, spikes,
-// [48, 512, 49] -> 128 channels: library 1.11e-7, chain 1.54e-7, now 9.9e-8; real values, [4, 1536, 49] -> 512: 3.5e-7, 4.4e-7,
-// 1.6e-7; over 70 shapes of 96 to 576 channels, 7 x 7 and 9 x 9: 0.87 of the library's forward and 0.33 of its input gradient on
-// average, at most 1.09).  It takes 256 registers, two wavefronts per SIMD: [128, 384, 49] -> 1536 (624 blocks, more
-// than are resident then) 37.9 -> 44.1 us, its input gradient 53.1 -> 51.8, [96, 512, 81] -> 512 25.8 -> 26.2.
-template <int TB, bool BITS, bool RAGGED>
-__global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu(RAGGED ? 2 : 3, RAGGED ? 2 : 3))) pw_gemm_rows_kernel(const PwGemmArgs a) {
+// accumulators with one rounding (kStepSums); with one activation term, or few steps, what that rounding takes off is carried
+// into the next step's sum (kStepSumsCompensated).  With one chain over all of K, as the rows of a multiple of four have it, the
+// error against float64 was above that of the library's fp32 GEMM, which serves these lengths otherwise.  Relative 2-norm,
+// library / chain / now: spikes, [48, 512, 49] -> 128 channels 1.11e-7 / 1.54e-7 / 9.9e-8 (6.8e-8 as one term); real values,
+// [4, 1536, 49] -> 512 3.5e-7 / 4.4e-7 / 1.6e-7.  Over 70 shapes of 96 to 576 channels, 7 x 7 and 9 x 9, in units of the library's
+// error: forward 0.78 on average and 0.96 at most (chain 1.25 and 1.53; step sums alone 0.87 and 1.09), input gradient 0.33 and 1.02,
+// where the library settles on its most exact algorithm.  Where the line lies: the step sums alone exceed the library's
+// error with one term (96 to 576 channels, by 3 to 9 %) and with two terms up to 128 channels (1 %); carried everywhere,
+// [96, 512, 81] -> 512 takes 30.7 us instead of 26.2.
+// 256 registers, two wavefronts per SIMD: [128, 384, 49] -> 1536 (624 blocks, more than are resident then) 37.9 us with one chain,
+// 44.1 now, its input gradient 53.1 and 51.8, [96, 512, 81] -> 512 25.8 and 26.2.
+enum RowSums { kOneChain = 0, kStepSums = 1, kStepSumsCompensated = 2 };
+template <int TB, bool BITS, int SUMS>
+__global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu(SUMS == kOneChain ? 3 : 2, SUMS == kOneChain ? 3 : 2))) pw_gemm_rows_kernel(const PwGemmArgs a) {
   constexpr int TA = 2;
+  constexpr bool RAGGED = SUMS != kOneChain, COMPENSATED = SUMS == kStepSumsCompensated;
   constexpr int kBuf = TB * kRowPlane;  // one B tile: [TB][32 k][kPlanePitch]
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -891,9 +898,9 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   };
   if (per_sample && col_ok) scale_for(column_amax(jc), b_scale, b_inverse);
 
-  // [ks][term]: the fragments of the step being multiplied, refilled as they are used up; RAGGED: those of the next step
+  // [ks][term]: the fragments of the step being multiplied, refilled as they are used up; kStepSums: those of the next step
   // arrive in the other set
-  u32x4 af[RAGGED ? 4 : 2][TA];
+  u32x4 af[SUMS == kStepSums ? 4 : 2][TA];
   u32x4 rb[2][4];   // [set][i]: k row kr + 8 i of a tile, fp32 bit patterns of four columns
   auto fetch_a = [&](int tile, int ks, int set = 0) {  // every request is unconditional: k steps beyond the last repeat it
     const int t_ = tile < steps ? tile : steps - 1;
@@ -947,11 +954,18 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
     }
   };
 
-  f32x16 acc[4];
+  auto clear = [](f32x16 &v) {
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt)
+    for (int q = 0; q < 16; ++q) v[q] = 0.0f;
+  };
+  // part: the sum of a K step; COMPENSATED: between the steps, what the last addition to acc rounded off, on which the next
+  // step's products are summed
+  f32x16 acc[4], part[COMPENSATED ? 4 : 2];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) acc[nt][q] = 0.0f;
+  for (int nt = 0; nt < 4; ++nt) {
+    clear(acc[nt]);
+    if constexpr (COMPENSATED) clear(part[nt]);
+  }
   // the transposing read: group g = lane / 16 fetches columns 16 (g % 2) + 0..15 of the 32, k rows 8 (g / 2) + 0..3 (and
   // + 4 in the second read) of the 16; lane i of the group points at columns 4 (i % 4) + 0..3 of row i / 4
   const int tr_g = lane >> 4, tr_i = lane & 15;
@@ -968,23 +982,25 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   auto multiply = [&](auto parity, int tile, int next_a) {  // parity: of the tile
     const uint8_t *Bs = lds + (tile & 1) * kBuf + tr_off;
     if constexpr (RAGGED) {
-      constexpr int set = decltype(parity)::value;
-      fetch_a(next_a, 0, set ^ 1);
-      fetch_a(next_a, 1, set ^ 1);
-      __builtin_amdgcn_sched_barrier(0);
+      constexpr int set = COMPENSATED ? 0 : decltype(parity)::value;
+      if constexpr (!COMPENSATED) {
+        fetch_a(next_a, 0, set ^ 1);
+        fetch_a(next_a, 1, set ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int pair = 0; pair < 4; pair += 2) {
         u32x4 bf[2][2][TB];
-        f32x16 part[2];  // the products of this step, smallest terms first
+        constexpr int stay = COMPENSATED ? 1 : 0;
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
 #pragma unroll
           for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
             for (int tb = 0; tb < TB; ++tb) bf[n][ks][tb] = fragment_b(Bs, tb, ks, pair + n);
-#pragma unroll
-          for (int q = 0; q < 16; ++q) part[n][q] = 0.0f;
+          if constexpr (!COMPENSATED) clear(part[n]);
         }
+        // smallest terms first, of both halves of the step
 #pragma unroll
         for (int order = Pairs<TA, TB>::kMax; order >= 0; --order) {
 #pragma unroll
@@ -995,12 +1011,23 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
             for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
               for (int n = 0; n < 2; ++n)
-                part[n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, af[2 * set + ks][ta]),
-                                                                  __builtin_bit_cast(f16x8, bf[n][ks][tb]), part[n], 0, 0, 0);
+                part[stay * pair + n] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, af[2 * set + ks][ta]),
+                                                                                __builtin_bit_cast(f16x8, bf[n][ks][tb]), part[stay * pair + n], 0, 0, 0);
           }
         }
-        acc[pair] += part[0];
-        acc[pair + 1] += part[1];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          const f32x16 sum = acc[pair + n] + part[stay * pair + n];
+          if constexpr (COMPENSATED) part[pair + n] -= sum - acc[pair + n];
+          acc[pair + n] = sum;
+        }
+        if constexpr (COMPENSATED) {
+          if (pair == 2) {
+            fetch_a(next_a, 0);
+            fetch_a(next_a, 1);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
       return;
     }
@@ -1661,11 +1688,17 @@ int launch_gemm_terms(const PwGemmArgs &a, int64_t blocks, hipStream_t stream) {
   return check_launch("pwconv_gemm");
 }
 
+// Rows of other lengths: compensated sums for one activation term, and for two up to so many K (see pw_gemm_rows_kernel).
+constexpr int kCompensateK = 192;
 template <int TB, bool BITS = false>
 int launch_gemm_rows(const PwGemmArgs &a, int64_t blocks, hipStream_t stream) {
   const unsigned lds = rows_inverse_offset(TB) + kTile * 4;
-  if (BITS || a.L == a.Lq) hipLaunchKernelGGL((pw_gemm_rows_kernel<TB, BITS, false>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
-  else hipLaunchKernelGGL((pw_gemm_rows_kernel<TB, false, true>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
+  auto launch = [&](auto bits, auto sums) {
+    hipLaunchKernelGGL((pw_gemm_rows_kernel<TB, decltype(bits)::value, decltype(sums)::value>), dim3((unsigned)blocks), dim3(kPwThreads), lds, stream, a);
+  };
+  if (BITS || a.L == a.Lq) launch(std::bool_constant<BITS>(), std::integral_constant<int, kOneChain>());
+  else if (TB == 1 || a.K <= kCompensateK) launch(std::false_type(), std::integral_constant<int, kStepSumsCompensated>());
+  else if constexpr (TB == 2) launch(std::false_type(), std::integral_constant<int, kStepSums>());
   return check_launch("pwconv_gemm");
 }
 

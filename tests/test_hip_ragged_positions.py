@@ -81,7 +81,7 @@ LIBRARY_ERRORS = {
 def test_no_further_from_64_bits_than_the_library(C, T, B, Cin, Cout, spikes):
     """Position counts that four does not divide ran on the library's fp32 convolution before they ran on the fp16 split: the
     split's sums (the K steps of a column, and the sample groups of a weight gradient in 64 bits) are no further from 64 bits.
-    The kernels add in a fixed order, so the errors are the same on every run: 0.35 to 0.98 of the library's (with one chain over
+    The kernels add in a fixed order, so the errors are the same on every run: 0.35 to 0.92 of the library's (with one chain over
     all of K and fp32 sums over the groups up to 1.34)."""
     F, S, L = C.F16 | 2, T * B, 49
     x = (seeded_randn((S, Cin, L), 30) > 0.7).float().cuda() if spikes else seeded_randn((S, Cin, L), 30).cuda()
