@@ -54,8 +54,8 @@
 //       Raising the wavefront priority for the multiplication (s_setprio 2 around it): 0.348 and 0.331 ms
 //       (Y = W X and dX) against 0.338 and 0.300; not kept.
 //       By number of products (M = 1152, K = 384, random data): 1 product 0.15-0.16 ms, 2: 0.17-0.18, 3: 0.22,
-//       6: 0.33-0.35.  The weight planes are stored tile by tile ([row tile][k step][row][k], 8 KiB per staged tile in
-//       a row) so that every 128-byte line a block fetches is used whole: 0.345 -> 0.338 ms, one-term activations
+//       6: 0.33-0.35.  The weight planes are stored tile by tile ([row tile][k step][row][k], for fp16 in
+//       fragments of 32 rows x 16 k, 8 KiB per staged tile in a row) so that every 128-byte line a block fetches is used whole: 0.345 -> 0.338 ms, one-term activations
 //       0.229 -> 0.215 ms.
 //   pw_dw_kernel       dW[m][n] = sum_{s,l} dY[s][m][l] X[s][n][l]
 //       both operands are contiguous along the contraction index l; a block owns a 128 x 128 tile of dW for a chunk
@@ -188,6 +188,12 @@ __device__ __forceinline__ int64_t xcd_order(int64_t b, int64_t n) {
   return x * q + (x < r ? x : r) + i;
 }
 
+// the same in 32 bits (a 64-bit integer division is some hundred instructions, also where every lane has the same operands)
+__device__ __forceinline__ uint32_t xcd_order32(uint32_t b, uint32_t n) {
+  const uint32_t q = n / kXcds, r = n % kXcds, x = b % kXcds, i = b / kXcds;
+  return x * q + (x < r ? x : r) + i;
+}
+
 // planes[t][r][c] = term t of src[r * ld_r + c * ld_c] for r < rows, c < cols, zero in the padding
 __global__ void __launch_bounds__(256) split_weight_kernel(const float *src, int64_t rows, int64_t cols, int64_t ld_r,
                                                             int64_t ld_c, int64_t rows_pad, int64_t cols_pad,
@@ -210,6 +216,11 @@ __global__ void __launch_bounds__(256) split_weight_kernel(const float *src, int
     reinterpret_cast<uint32_t *>(planes + (int64_t)t * rows_pad * cols_pad)[at / 2] = w[t];
 }
 
+// Where element (row r of 128, k c of 32) of a tile of fp16 planes lies: the 16 bytes (eight k) that a lane of
+// v_mfma_f32_32x32x16_f16 takes, in lane order, so that a wavefront fetches the fragment of 32 rows and 16 k as 1 KiB in a row.
+__device__ __forceinline__ int fragment_place(int r, int c) {
+  return (r >> 5) * 1024 + (c >> 4) * 512 + (((c >> 3) & 1) * 32 + (r & 31)) * 8 + (c & 7);
+}
 // fp16 planes[t][tile order] = term t of scale_r * src[r][c], with a power-of-two scale per row r (a row of A is a row
 // of the product, so the GEMM's epilogue takes the scale out again); the inverse scales follow the two planes as
 // rows_pad floats.  One wavefront per row.  In evaluation mode (bn.map) it also makes the map of its row's batch norm
@@ -241,7 +252,7 @@ __global__ void __launch_bounds__(256) split_weight_f16_kernel(const float *src,
     }
     uint32_t w[2];
     split_pair<2, true>(x0, x1, w);
-    const int64_t at = (((r / kTile) * (cols_pad / kTileK) + c / kTileK) * kTile + r % kTile) * kTileK + c % kTileK;
+    const int64_t at = ((r / kTile) * (cols_pad / kTileK) + c / kTileK) * (kTile * kTileK) + fragment_place((int)(r % kTile), (int)(c % kTileK));
 #pragma unroll
     for (int t = 0; t < 2; ++t)
       reinterpret_cast<uint32_t *>(planes + (int64_t)t * rows_pad * cols_pad)[at / 2] = w[t];
@@ -282,7 +293,7 @@ __global__ void __launch_bounds__(1024) split_weight_f16_transposed_kernel(const
   if (step < steps) {
     uint32_t w[2];
     split_pair<2, true>(raw0 * scale, raw1 * scale, w);
-    const int64_t at = (((r / kTile) * steps + step) * kTile + r % kTile) * kTileK + 2 * (ci & 15);
+    const int64_t at = ((r / kTile) * steps + step) * (kTile * kTileK) + fragment_place((int)(r % kTile), 2 * (ci & 15));
 #pragma unroll
     for (int t = 0; t < 2; ++t) reinterpret_cast<uint32_t *>(planes + (int64_t)t * rows_pad * cols_pad)[at / 2] = w[t];
   }
@@ -389,6 +400,7 @@ struct PwGemmArgs {
   int M, K, K_pad, L;
   int Lq;                    // columns per sample of the column index: L rounded up to four (column_pitch), the rest hold zeros;
                              // kBPlanes: L
+  float inv_Lq;              // 1 / Lq
   int m_blocks;
   float *stats;              // nullptr, or [2 x column blocks][M][2]: per row of c the sum and the sum of squares over
                              // each half (64 columns) of every column block
@@ -493,7 +505,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   int a_dst[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int q = tid + kPwThreads * i, row = q >> 2, kc = q & 3;
+    const int q = tid + kPwThreads * i, row = H ? 32 * (q >> 7) + (q & 31) : q >> 2, kc = H ? (q >> 5) & 3 : q & 3;
     a_off[i] = (uint32_t)((mb * (K_pad / kTileK) * (kTile * kTileK) + 8 * q) * 2);
     a_dst[i] = row * kRowBytes + kc * 16;
   }
@@ -826,6 +838,11 @@ constexpr unsigned rows_inverse_offset(int tb) { return 2u * tb * kRowPlane > kO
 //   * two B tiles alternate in LDS, so a K step has one barrier.
 // Per K step of a block: 16 KB written to and 64 KB read from LDS, 16 + 16 load instructions; 148 to 154 registers, three
 // wavefronts per SIMD.
+// The planes hold the 16 bytes of every lane of a fragment in lane order (fragment_place): eight lines per request instead of sixteen
+// half used ones.  Where a column lies is worked out in 32 bits from one division per tile: as 64-bit divisions, eight of them in a
+// wavefront's prologue and epilogue, it was half of the kernel's vector instructions at K = 384.  Both together, before / now, us:
+// M = 1152, K = 384, 50 176 columns 194 / 187, M = 384, K = 1152 156 / 148; [64, 256, 100] -> 768 20.1 / 19.4, [16, 384, 196] -> 384
+// 16.4 / 15.7, [4, 384, 196] -> 1152 16.1 / 15.4.
 // BITS: b is a spike tensor that arrives bit-packed (as in pw_gemm_kernel, L a multiple of 4): a byte per piece, one term;
 // M = K = 384, 50 176 columns: 41 us, pw_gemm_kernel 47.
 // Samples of any length L >= 4: the column index gives every sample Lq = L rounded up to four columns, so that a piece
@@ -853,11 +870,18 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   constexpr int kBuf = TB * kRowPlane;  // one B tile: [TB][32 k][kPlanePitch]
   extern __shared__ __align__(16) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t logical = xcd_order(blockIdx.x, gridDim.x);
-  const int mb = (int)(logical % a.m_blocks);
-  const int64_t nb = logical / a.m_blocks;
-  const int64_t j0 = nb * kTile;
+  const uint32_t logical = xcd_order32(blockIdx.x, gridDim.x);
+  const uint32_t nb = logical / (uint32_t)a.m_blocks;
+  const int mb = (int)(logical - nb * (uint32_t)a.m_blocks);
+  // Columns are counted in 32 bits (a launch has fewer than 2^31), and a column's sample from that of the tile's first column, the
+  // one quotient that is formed by a division: `at` = position in that sample + column in the tile, less than Lq + 128.
+  const uint32_t j0 = nb * kTile, ncols = (uint32_t)a.ncols;
   const int M = a.M, K = a.K, L = a.L, Lq = RAGGED ? a.Lq : a.L;
+  const uint32_t tile_sample = j0 / (uint32_t)Lq;
+  const int l0 = (int)(j0 - tile_sample * (uint32_t)Lq);
+  const bool two_samples = Lq >= kTile;
+  // (exact: at + 1/2 is at least 1 / (2 Lq) of a sample away from a whole number, with Lq + 128 below 2^24 far more than the product's error)
+  auto samples_on = [&](int at) { return two_samples ? (at >= Lq ? 1 : 0) : (int)(((float)at + 0.5f) * a.inv_Lq); };
   const int steps = a.K_pad / kTileK;
 
   // the inverse row scales of the tile wait in LDS (beyond the operand tiles) for the epilogue
@@ -866,37 +890,38 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
 
   // A: lane (r, g) wants k chunk 2 ks + g (eight k, 16 bytes) of row r of the wavefront's 32 rows
   const char *a_base = reinterpret_cast<const char *>(a.a_planes) + (int64_t)mb * steps * (kTile * kTileK * 2);
-  const uint32_t a_lane = (uint32_t)(((wave * 32 + (lane & 31)) * kTileK + (lane >> 5) * 8) * 2);
+  const uint32_t a_lane = (uint32_t)((wave * 1024 + lane * 8) * 2);
   // B: the 16 bytes of columns 4 (tid % 32) .. + 3 in the k rows tid / 32 + 8 i
   const int q4 = tid & 31, kr = tid >> 5;
-  const int64_t jc = j0 + 4 * q4;
-  const bool col_ok = jc < a.ncols;
+  const bool col_ok = j0 + 4 * q4 < ncols;
+  const int b_ds = col_ok ? samples_on(l0 + 4 * q4) : 0;
   uint32_t b_off = 0;
   int b_skip = 0;  // places that the piece is moved down
   if (col_ok) {
-    const int64_t s = jc / Lq;
-    const int l = (int)(jc - s * Lq), first = RAGGED ? min(l, L - 4) : l;
-    b_off = (uint32_t)(((s * K) * (int64_t)L + first) * (BITS ? 1 : 4));  // with BITS the bit index
+    const int l = l0 + 4 * q4 - b_ds * Lq, first = RAGGED ? min(l, L - 4) : l;
+    b_off = ((tile_sample + (uint32_t)b_ds) * (uint32_t)K * (uint32_t)L + (uint32_t)first) * (BITS ? 1u : 4u);  // with BITS the bit index
     b_skip = l - first;
   }
   const uint32_t row_bytes = (uint32_t)L * (BITS ? 1u : 4u);
-  const bool edge_cols = __builtin_amdgcn_readfirstlane(j0 + kTile > a.ncols ? 1 : 0) != 0;
+  // places of the rows kr + 8 i of a K step from its first row; rows beyond K repeat the last one (a minimum of offsets: one instruction)
+  uint32_t b_row[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) b_row[i] = b_off + (uint32_t)(kr + 8 * i) * row_bytes;
+  const bool edge_cols = __builtin_amdgcn_readfirstlane(j0 + kTile > ncols ? 1 : 0) != 0;
   const char *b_base = reinterpret_cast<const char *>(a.b);
   float b_scale = 1.0f, b_inverse = 1.0f;
   const bool per_sample = TB > 1 && a.b_amax_samples != nullptr;
   if (TB > 1 && !per_sample && a.b_amax != nullptr) scale_for(tensor_amax(a.b_amax), b_scale, b_inverse);
-  const bool two_samples = Lq >= kTile;
-  const int64_t tile_sample = j0 / Lq, next_sample_col = (tile_sample + 1) * Lq;
   float tile_amax[2] = {0.0f, 0.0f};
   if (per_sample && two_samples) {
     const int64_t s_a = a.amax_s0 + tile_sample, s_b = s_a + 1 < a.amax_S ? s_a + 1 : s_a;
     tile_amax[0] = sample_amax(a.b_amax_samples, s_a);
     tile_amax[1] = sample_amax(a.b_amax_samples, s_b);
   }
-  auto column_amax = [&](int64_t j) {
-    return two_samples ? (j < next_sample_col ? tile_amax[0] : tile_amax[1]) : sample_amax(a.b_amax_samples, a.amax_s0 + j / Lq);
+  auto column_amax = [&](int ds) {
+    return two_samples ? tile_amax[ds] : sample_amax(a.b_amax_samples, a.amax_s0 + tile_sample + ds);
   };
-  if (per_sample && col_ok) scale_for(column_amax(jc), b_scale, b_inverse);
+  if (per_sample && col_ok) scale_for(column_amax(b_ds), b_scale, b_inverse);
 
   // [ks][term]: the fragments of the step being multiplied, refilled as they are used up; kStepSums: those of the next step
   // arrive in the other set
@@ -904,17 +929,19 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   u32x4 rb[2][4];   // [set][i]: k row kr + 8 i of a tile, fp32 bit patterns of four columns
   auto fetch_a = [&](int tile, int ks, int set = 0) {  // every request is unconditional: k steps beyond the last repeat it
     const int t_ = tile < steps ? tile : steps - 1;
-    const char *src = a_base + (int64_t)t_ * (kTile * kTileK * 2) + ks * 32;
+    const char *src = a_base + (int64_t)t_ * (kTile * kTileK * 2) + ks * 1024;
 #pragma unroll
     for (int ta = 0; ta < TA; ++ta) af[2 * set + ks][ta] = *reinterpret_cast<const u32x4 *>(src + (int64_t)ta * a.plane_stride * 2 + a_lane);
   };
   auto fetch_b = [&](int tile, int set) {
+    const int t_ = tile < steps ? tile : steps - 1;
+    const uint32_t first = (uint32_t)(t_ * kTileK) * row_bytes;            // the same for every lane
+    const uint32_t last = b_off + (uint32_t)(K - 1 - t_ * kTileK) * row_bytes;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int k = tile * kTileK + kr + 8 * i;
-      const uint32_t at = b_off + (uint32_t)(k < K ? k : K - 1) * row_bytes;
-      if constexpr (BITS) rb[set][i].x = *reinterpret_cast<const uint8_t *>(b_base + (at >> 3)) >> (at & 7u);
-      else rb[set][i] = *reinterpret_cast<const u32x4_any *>(b_base + at);
+      const uint32_t at = min(b_row[i], last);
+      if constexpr (BITS) rb[set][i].x = *reinterpret_cast<const uint8_t *>(b_base + ((at + first) >> 3)) >> ((at + first) & 7u);
+      else rb[set][i] = *reinterpret_cast<const u32x4_any *>(b_base + first + at);
     }
   };
   auto stage = [&](int tile, int set) {
@@ -1089,10 +1116,10 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   if (per_sample) {
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
-      const int64_t j = j0 + nt * 32 + (lane & 31);
+      const int col = nt * 32 + (lane & 31);
       float unused;
       b_inv_col[nt] = 1.0f;
-      if (j < a.ncols) scale_for(column_amax(j), unused, b_inv_col[nt]);
+      if (j0 + col < ncols) scale_for(column_amax(samples_on(l0 + col)), unused, b_inv_col[nt]);
     }
   }
 #pragma unroll
@@ -1113,12 +1140,12 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   const int wave_row0 = mb * kTile + wave * 32;
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
-    const int64_t j4 = j0 + half * 64 + c4;
-    const bool ok4 = j4 < a.ncols;
-    const int64_t s4 = ok4 ? j4 / Lq : 0;
-    const int l4 = ok4 ? (int)(j4 - s4 * Lq) : 0;
+    const int col4 = half * 64 + c4;
+    const bool ok4 = j0 + col4 < ncols;
+    const int ds4 = ok4 ? samples_on(l0 + col4) : 0, l4 = ok4 ? l0 + col4 - ds4 * Lq : 0;
     const int left = L - l4;  // positions of the sample from here on
-    float *cp4 = a.c + (s4 * M) * (int64_t)L + l4;
+    float *at4 = a.c + ((int64_t)(tile_sample + ds4) * M + (wave_row0 + rsub)) * (int64_t)L + l4;
+    const int64_t step4 = 4 * (int64_t)L;
     __builtin_amdgcn_wave_barrier();  // the piece staged before has been read (LDS serves a wavefront's accesses in order)
 #pragma unroll
     for (int ntl = 0; ntl < 2; ++ntl)
@@ -1131,8 +1158,9 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
       const int row_local = 4 * q + rsub;
       const int row = wave_row0 + row_local;
       const f32x4 v = *reinterpret_cast<const f32x4 *>(buf + row_local * kOutPitch + c4);
+      float *at = at4;
+      at4 += step4;
       if (ok4 && row < M) {
-        float *at = cp4 + (int64_t)row * L;
         if (!RAGGED || left >= 4) {
           *reinterpret_cast<f32x4_any *>(at) = v;
         } else {
@@ -1154,7 +1182,7 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
       }
       const int row = wave_row0 + lane;
       if (row < M) {
-        float *out = a.stats + ((2 * nb + half) * (int64_t)M + row) * 2;
+        float *out = a.stats + ((2 * (int64_t)nb + half) * M + row) * 2;
         out[0] = sum;
         out[1] = squares;
       }
@@ -1819,7 +1847,7 @@ int launch_pwconv_gemm(const uint16_t *a_planes, int a_terms, int64_t M, int64_t
     PwGemmArgs a;
     a.a_planes = a_planes; a.c = c + s0 * M * L;
     a.b = b_bits ? reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(b) + s0 * K * L / 8) : b + s0 * K * L;
-    a.M = (int)M; a.K = (int)K; a.K_pad = (int)round_up(K, kTileK); a.L = (int)L; a.Lq = (int)column_pitch(L);
+    a.M = (int)M; a.K = (int)K; a.K_pad = (int)round_up(K, kTileK); a.L = (int)L; a.Lq = (int)column_pitch(L); a.inv_Lq = 1.0f / (float)a.Lq;
     a.plane_stride = round_up(M, kTile) * a.K_pad;
     a.ncols = s_count * a.Lq;
     a.m_blocks = (int)(round_up(M, kTile) / kTile);
@@ -1957,7 +1985,7 @@ int launch_pwconv_gemm_planes(const uint16_t *a_planes, int64_t M, int64_t K, co
     return fail(SJHIP_ERR_TOO_LARGE, "pwconv_gemm_planes: M=%lld K=%lld S=%lld L=%lld", (long long)M, (long long)K, (long long)S, (long long)L);
   PwGemmArgs a;
   a.a_planes = a_planes; a.b = nullptr; a.c = c;
-  a.M = (int)M; a.K = (int)K; a.K_pad = (int)round_up(K, kTileK); a.L = a.Lq = (int)L;
+  a.M = (int)M; a.K = (int)K; a.K_pad = (int)round_up(K, kTileK); a.L = a.Lq = (int)L; a.inv_Lq = 1.0f / (float)L;
   a.plane_stride = round_up(M, kTile) * a.K_pad;
   a.ncols = S * L;
   a.m_blocks = (int)(round_up(M, kTile) / kTile);
