@@ -62,6 +62,8 @@
 //       of samples and writes its partial tile, dw_reduce_kernel adds the chunks in a fixed order.
 // Blocks that share operand tiles are numbered so that they run on the same XCD (one L2 each, blocks are dealt
 // round-robin over the eight XCDs).
+#include <cmath>
+
 #include "bn_map.h"
 #include "sjhip_common.h"
 
@@ -1205,7 +1207,7 @@ struct PwDwArgs {
 
 // Two LDS buffers where x has one fp16 term (spikes, 2 x 30 KiB): the next tile is split and stored while the current one is
 // multiplied, with one barrier per K step instead of two.  One buffer / two, us with the reduction, three processes of each in
-// turn on one box: x as bits, dy [256, 1152, 196] and x [256, 384, 196] 146.6 / 142.0, [128, 1536, 196] and [128, 384, 196]
+// turn on one box: (on shapes that pw_dw_flat_kernel has taken over) x as bits, dy [256, 1152, 196] and x [256, 384, 196] 146.6 / 142.0, [128, 1536, 196] and [128, 384, 196]
 // 108.6 / 105.1, [256, 384, 196] both 58.3 / 55.5; x as fp32 spikes 197.6 / 189.4, 110.1 / 110.1, 59.9 / 59.9.  With two terms of x
 // (2 x 40 KiB) two buffers measured 210.4 -> 214.0, 138.8 -> 138.4, 74.7 -> 74.5: those keep one, and every launch stays within
 // the default limit of dynamic LDS.  (The bf16 split's three planes per operand would leave one block per compute unit.)
@@ -1475,6 +1477,274 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
   }
 }
 
+// pw_dw_flat_kernel: the weight gradient on fp16 terms where the contraction runs over the positions of all samples in a row (rows of at
+// least eight quads), the same products as pw_dw_kernel.  That kernel's K step (qkv shape: dy [256, 1152, 196], x [256, 384, 196], cycles of
+// a wavefront) was 1245 of split and LDS writes, 839 until the eight loads of the next tile had been accepted, 400 at barriers and 1301 of
+// multiplication, one after the other, for 768 of the matrix cores.  Here
+//   * the step is one straight line: behind every few multiplications stands a piece of the next tile's split and the request that
+//     refills its registers, so that nothing is issued in a burst; two LDS buffers, one barrier; rows of 64 bytes with exchanged
+//     chunks instead of padded ones, no bank conflicts.  With the requests taken out a step then takes 1606 cycles for two
+//     wavefronts per SIMD, 1536 being the matrix cores' own;
+//   * with them 2700: the loads bound it (128 x 128 tiles move 32 KB per step and tile through a compute unit's memory path).  A block is
+//     eight wavefronts, 128 rows of dy by 128 WN of x: with WN = 3 64 KB for three tiles.  acc 96 + two tiles in flight 64 + fragments
+//     of a half step and the next one's: 246 registers, two wavefronts per SIMD, one block per compute unit.
+// Kernel and reduction, before / now, us: this shape 207 / 163, x as bits 141 / 119; dy [128, 1536, 196], x [128, 384, 196] 139 / 117;
+// both [256, 384, 196] 75 / 64; dy [64, 768, 100], x [64, 256, 100] 28.0 / 20.6; both [128, 512, 49] 43.7 / 32.9; both [16, 384, 196]
+// 21.5 / 16.5; dy [4, 1152, 196], x [4, 384, 196] 20.0 / 15.4.
+// No sum is less exact than before (error against float64, relative 2-norm): the sums of 32 bits are no longer than pw_dw_kernel's chunks
+// were (dw_flat_plan), where needed a chunk leaves several partial tiles.  With WN = 1 registers are left for sums of their own for
+// the products of small terms: those of the large ones are rounded a third (one term of x: half) as often, which allows chains 2.5 times as
+// long.  qkv shape 4.6e-7 / 3.8e-7, spikes 2.2e-7 / 1.9e-7; [128, 512, 49] 1.48e-7 / 1.27e-7, spikes 8.9e-8 / 5.7e-8; twelve shapes, all lower.
+struct PwDwFlatArgs {
+  const float *dy, *x;
+  float *partials;
+  int S, M, N, L, Lq;
+  int m_blocks, n_blocks;
+  int total_quads;      // S * Lq / 4
+  int steps_per_chunk;  // K steps (eight quads) per partial tile
+  int steps_per_sum;    // K steps, an even number, after which the accumulators go out and start again
+  int sums;             // partial tiles per chunk
+  const float *dy_amax, *x_amax;
+};
+constexpr int kDwThreads = 512;
+constexpr int kDwRow = 64;  // bytes of a row of a plane: 32 fp16
+constexpr unsigned dw_flat_buffer(int tb, int wn) { return (2u + (unsigned)(tb * wn)) * kTile * kDwRow; }
+template <int TB, bool BITS, bool RAGGED, int WN>
+__global__ void __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) pw_dw_flat_kernel(const PwDwFlatArgs a) {
+  static_assert(!BITS || (TB == 1 && !RAGGED), "a bit-packed operand has one term and rows of a multiple of four");
+  constexpr int TA = 2, NT = kTile * WN, kPlaneA = kTile * kDwRow, kPlaneB = NT * kDwRow, kBuf = (int)dw_flat_buffer(TB, WN);
+  constexpr int UA = 2, UB = 2 * WN, U = UA + UB;  // 16-byte pieces of a K step per work-item: rows of dy, rows of x
+  extern __shared__ __align__(16) uint8_t lds[];   // two buffers of [TA][128][kDwRow] of dy, then [TB][NT][kDwRow] of x
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 2, wn = wave & 3;
+  const uint32_t logical = xcd_order32(blockIdx.x, gridDim.x);
+  const uint32_t tiles = (uint32_t)(a.m_blocks * a.n_blocks);
+  const uint32_t chunk = logical / tiles, tile = logical - chunk * tiles;
+  const uint32_t nb = tile / (uint32_t)a.m_blocks, mb = tile - nb * (uint32_t)a.m_blocks;
+  const int m0 = (int)mb * kTile, n0 = (int)nb * NT;
+  const int M = a.M, N = a.N, L = a.L, Lq = RAGGED ? a.Lq : a.L;
+  const int Q = Lq >> 2;  // quads (four positions) per sample, at least eight: the eight quads of a K step lie in two samples at most
+  const int first_quad = (int)chunk * a.steps_per_chunk * 8;
+  const int quads = min(a.steps_per_chunk * 8, a.total_quads - first_quad);  // of this chunk
+  const int iters = (quads + 7) / 8;
+  const uint32_t a_sample = (uint32_t)(M * L * 4), b_sample = (uint32_t)(N * L * (BITS ? 1 : 4));  // bytes; with BITS bits
+
+  // a work-item fetches quad q4 of the rows rr + 64 i of both tiles.  Rows beyond the matrices repeat the last one: what they hold
+  // reaches only rows and columns of the tile that are not written.
+  const int q4 = tid & 7, rr = tid >> 3;
+  uint32_t a_off[UA], b_off[UB];
+#pragma unroll
+  for (int i = 0; i < UA; ++i) a_off[i] = (uint32_t)(min(m0 + rr + 64 * i, M - 1) * L * 4);
+#pragma unroll
+  for (int i = 0; i < UB; ++i) b_off[i] = (uint32_t)(min(n0 + rr + 64 * i, N - 1) * L * (BITS ? 1 : 4));
+  float a_scale = 1.0f, a_inverse = 1.0f, b_scale = 1.0f, b_inverse = 1.0f;
+
+  // where a K step begins: sample, quad in it, quads of the chunk before it
+  struct Place {
+    int s, q, done = 0;
+    __device__ __forceinline__ void next(int Q) {
+      q += 8;
+      done += 8;
+      if (q >= Q) {
+        q -= Q;
+        ++s;
+      }
+    }
+  };
+  const int s_first = (int)((uint32_t)first_quad / (uint32_t)Q);
+  Place fetched{s_first, first_quad - s_first * Q}, staged = fetched;
+  f32x4 ra[2][UA], rb[2][UB];  // two tiles in flight; BITS: a byte in rb[..].x
+  const char *pa, *pb;         // of the tile being fetched
+  uint32_t la, lb;
+  auto aim = [&]() {  // at the next tile to be fetched (quads beyond the chunk: some place in the tensors)
+    int q = fetched.q + q4;
+    const bool second = q >= Q;
+    if (second) q -= Q;
+    const bool ok = fetched.done + q4 < quads;
+    const int l = ok ? (RAGGED ? min(4 * q, L - 4) : 4 * q) : 0;
+    la = (uint32_t)l * 4u + (ok && second ? a_sample : 0u);
+    lb = (BITS ? (uint32_t)l : (uint32_t)l * 4u) + (ok && second ? b_sample : 0u);
+    const int64_t s = min(fetched.s, a.S - 1);
+    pa = reinterpret_cast<const char *>(a.dy) + (s * M) * (int64_t)L * 4;
+    pb = reinterpret_cast<const char *>(a.x) + (BITS ? ((s * N) * (int64_t)L >> 3) : (s * N) * (int64_t)L * 4);
+    fetched.next(Q);
+  };
+  auto fetch_unit = [&](int u, int set) {
+    if (u < UA) ra[set][u] = load4<RAGGED>(pa + (a_off[u] + la));
+    else if constexpr (BITS) rb[set][u - UA].x = __builtin_bit_cast(float, (uint32_t)*reinterpret_cast<const uint8_t *>(pb + ((b_off[u - UA] + lb) >> 3)));
+    else rb[set][u - UA] = load4<RAGGED>(pb + (b_off[u - UA] + lb));
+  };
+  // A row's four 16-byte chunks (eight positions each) are exchanged by bits 2 and 3 of the row: the 16 rows a 16-byte fragment read
+  // of 16 lanes touches, and the four rows an 8-byte write of 32 lanes touches, fall on distinct banks
+  const uint32_t w_at = (uint32_t)(rr * kDwRow + (((q4 >> 1) ^ ((rr >> 2) & 3)) << 4) + (q4 & 1) * 8);
+  int place_q = 0, skip = 0;  // of the tile being staged
+  bool place_ok = true;
+  auto aim_stage = [&]() {
+    int q = staged.q + q4;
+    if (q >= Q) q -= Q;
+    place_ok = staged.done + q4 < quads;
+    place_q = place_ok ? 4 * q : 0;
+    if (RAGGED) skip = place_q - min(place_q, L - 4);
+    staged.next(Q);
+  };
+  auto stage_unit = [&](int u, int set, int buf, bool masked) {
+    uint8_t *dst = lds + buf * kBuf + w_at + (u < UA ? u * (64 * kDwRow) : TA * kPlaneA + (u - UA) * (64 * kDwRow));
+    f32x4 v = u < UA ? ra[set][u < UA ? u : 0] : rb[set][u < UA ? 0 : u - UA];
+    if (u >= UA && BITS) {  // (a whole sample is a multiple of 8 bits: the shift does not depend on the sample)
+      const uint32_t four = __builtin_bit_cast(uint32_t, v.x) >> ((b_off[u < UA ? 0 : u - UA] + (uint32_t)place_q) & 7u);
+      u32x2 w = {(four & 1u) * 0x3c00u | (four & 2u) * 0x1e000000u, (four & 4u) * 0x0f00u | (four & 8u) * 0x07800000u};
+      if (masked && !place_ok) w = (u32x2)(0u);
+      *reinterpret_cast<u32x2 *>(dst) = w;
+      return;
+    }
+    if constexpr (RAGGED) v = moved_down(v, skip);
+    if (masked && !place_ok) v = (f32x4)(0.0f);
+    if (u < UA) {
+      uint32_t w01[TA], w23[TA];
+      split_scaled_pair<TA, true>(v.x, v.y, a_scale, w01);
+      split_scaled_pair<TA, true>(v.z, v.w, a_scale, w23);
+#pragma unroll
+      for (int t = 0; t < TA; ++t) *reinterpret_cast<u32x2 *>(dst + t * kPlaneA) = u32x2{w01[t], w23[t]};
+    } else {
+      uint32_t w01[TB], w23[TB];
+      split_scaled_pair<TB, true>(v.x, v.y, b_scale, w01);
+      split_scaled_pair<TB, true>(v.z, v.w, b_scale, w23);
+#pragma unroll
+      for (int t = 0; t < TB; ++t) *reinterpret_cast<u32x2 *>(dst + t * kPlaneB) = u32x2{w01[t], w23[t]};
+    }
+  };
+
+  // SEP: the products of small terms have sums of their own, so that those of the large ones are rounded once where they would be three
+  // times (one term of x: once for twice)
+  constexpr bool SEP = WN == 1;
+  f32x16 acc[2][WN], small[SEP ? 2 : 1][SEP ? WN : 1];
+  auto clear = [&]() {
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < WN; ++nt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          acc[mt][nt][r] = 0.0f;
+          if (SEP) small[SEP ? mt : 0][SEP ? nt : 0][r] = 0.0f;
+        }
+  };
+  clear();
+  const uint32_t r_at = (uint32_t)((lane & 31) * kDwRow + (((lane >> 5) ^ ((lane >> 2) & 3)) << 4));  // (the second half: bit 5 flipped)
+  u32x4 af[2][2][TA], bf[2][WN][TB];  // [half][tile][term]
+  auto read_term = [&](int buf, int ks, int ta, int tb) {  // the fragments of term ta of dy, tb of x (-1: none)
+    const uint8_t *src = lds + buf * kBuf + (r_at ^ (ks * 32u));
+    if (ta >= 0) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) af[ks][t][ta] = *reinterpret_cast<const u32x4 *>(src + ta * kPlaneA + (wm * 64 + t * 32) * kDwRow);
+    }
+    if (tb >= 0) {
+#pragma unroll
+      for (int t = 0; t < WN; ++t) bf[ks][t][tb] = *reinterpret_cast<const u32x4 *>(src + TA * kPlaneA + tb * kPlaneB + (wn * (32 * WN) + t * 32) * kDwRow);
+    }
+  };
+  // Tile `it` (in LDS buffer P) is multiplied while tile it + 1 is split into the other buffer and tile it + 3 requested into the
+  // registers that frees, a piece of either between every few multiplications.
+  auto step = [&](auto parity, auto steady, bool stage_next, bool masked, bool more) {
+    constexpr int P = decltype(parity)::value;
+    constexpr bool STEADY = decltype(steady)::value;
+    constexpr int kProducts = TB == 2 ? 3 : 2, kMfmas = 2 * kProducts * 2 * WN;
+    if (STEADY || stage_next) aim_stage();
+    if (STEADY || more) aim();
+    read_term(P, 0, 0, TB - 1);
+    read_term(P, 0, 1, TB == 2 ? 0 : -1);
+    int n = 0, u = 0;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int g = 0; g < kProducts; ++g) {
+        // smallest terms first: (hi, lo), (lo, hi), (hi, hi); one term of x: (lo, x), (hi, x)
+        const int ta = g == kProducts - 2 ? 1 : 0, tb = TB == 2 && g == 0 ? 1 : 0;
+        if (ks == 0 && g == kProducts - 1) read_term(P, 1, 1, TB - 1);  // (into the registers of the small terms)
+        if (ks == 1 && g == 0) read_term(P, 1, 0, TB == 2 ? 0 : -1);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+          for (int nt = 0; nt < WN; ++nt) {
+            f32x16 &sum = SEP && g < kProducts - 1 ? small[SEP ? mt : 0][SEP ? nt : 0] : acc[mt][nt];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, af[ks][mt][ta]), __builtin_bit_cast(f16x8, bf[ks][nt][tb]), sum, 0, 0, 0);
+            ++n;
+            if (n * U >= (u + 1) * kMfmas) {
+              if (STEADY) {
+                stage_unit(u, P ^ 1, P ^ 1, false);
+                fetch_unit(u, P ^ 1);
+                __builtin_amdgcn_sched_barrier(0);
+              } else {
+                if (stage_next) stage_unit(u, P ^ 1, P ^ 1, masked);
+                if (more) fetch_unit(u, P ^ 1);
+              }
+              ++u;
+            }
+          }
+      }
+    __syncthreads();
+  };
+
+  // The accumulators into the next of the chunk's partial tiles.  (The address and the bounds pass through
+  // an empty asm: out of the loop, where the compiler would keep them, the addresses and masks of 32 WN stores spill.)
+  int64_t slot = (int64_t)chunk * a.sums;
+  auto flush = [&]() {
+    float *at = a.partials + (slot * M + (m0 + wm * 64 + 4 * (lane >> 5))) * N + (n0 + wn * (32 * WN) + (lane & 31));
+    int rows_left = M - (m0 + wm * 64 + 4 * (lane >> 5)), cols_left = N - (n0 + wn * (32 * WN) + (lane & 31));
+    asm volatile("" : "+v"(at), "+v"(rows_left), "+v"(cols_left));
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        if (mt * 32 + 8 * (r >> 2) + (r & 3) < rows_left) {
+#pragma unroll
+          for (int nt = 0; nt < WN; ++nt) {
+            const float sum = SEP ? acc[mt][nt][r] + small[SEP ? mt : 0][SEP ? nt : 0][r] : acc[mt][nt][r];
+            if (nt * 32 < cols_left) at[nt * 32] = sum * a_inverse * b_inverse;
+          }
+        }
+        at += (r & 3) < 3 ? N : 5 * N;
+      }
+    clear();
+    ++slot;
+  };
+
+  const std::integral_constant<int, 0> even;
+  const std::integral_constant<int, 1> odd;
+  // (every block has a K step; tiles beyond the last are requested at some place of the tensors and not staged)
+  aim();
+#pragma unroll
+  for (int u = 0; u < U; ++u) fetch_unit(u, 0);
+  aim();
+#pragma unroll
+  for (int u = 0; u < U; ++u) fetch_unit(u, 1);
+  if (a.dy_amax != nullptr) scale_for(tensor_amax(a.dy_amax), a_scale, a_inverse);
+  if (TB > 1 && a.x_amax != nullptr) scale_for(tensor_amax(a.x_amax), b_scale, b_inverse);
+  aim_stage();
+#pragma unroll
+  for (int u = 0; u < U; ++u) stage_unit(u, 0, 0, iters == 1);
+  aim();
+#pragma unroll
+  for (int u = 0; u < U; ++u) fetch_unit(u, 0);
+  __syncthreads();
+  int it = 0, sum_end = a.steps_per_sum;
+  for (; it + 4 < iters; it += 2) {  // (tile it + 2, staged by the second step, is not the last one)
+    if (it >= sum_end) {
+      flush();
+      sum_end += a.steps_per_sum;
+    }
+    step(even, std::true_type(), true, false, true);
+    step(odd, std::true_type(), true, false, true);
+  }
+  // at most four tiles are left; the last one may be partly empty
+  step(even, std::false_type(), it + 1 < iters, it + 2 >= iters, it + 3 < iters);
+  if (it + 1 < iters) step(odd, std::false_type(), it + 2 < iters, it + 3 >= iters, false);
+  if (it + 2 < iters) step(even, std::false_type(), it + 3 < iters, true, false);
+  if (it + 3 < iters) step(odd, std::false_type(), false, false, false);
+  const int64_t slots_end = ((int64_t)chunk + 1) * a.sums;
+  flush();
+  for (; slot < slots_end;) flush();  // (a last chunk shorter than the others: the accumulators are zeros now)
+}
 
 struct PwDwPlanesArgs {
   const uint16_t *dy_planes;  // [2][M][ld] fp16 terms of dy, column s * L + l of row m holds dy[s][m][l]
@@ -1745,6 +2015,10 @@ int launch_dw_terms(const PwDwArgs &a, int64_t blocks, hipStream_t stream) {
   return launch_dw<TA, TB, H, BITS, false>(a, blocks, stream);
 }
 
+bool dw_flat(int64_t S, int64_t M, int64_t N, int64_t L) {
+  return L >= 29 && M * L < (int64_t(1) << 29) && N * L < (int64_t(1) << 29) && S < (int64_t(1) << 31) && S * column_pitch(L) < (int64_t(1) << 31);
+}
+
 // Samples per partial tile of dW.  Two blocks are resident per compute unit (512 on the chip); the chunk count is the
 // largest that keeps tiles x chunks within one (few tiles) or two full generations of resident blocks, so that no
 // generation runs nearly empty.  Measured, kernel + reduction: 27 tiles: 38 chunks (1026 blocks) 312 + 11 us, 37 chunks
@@ -1756,6 +2030,59 @@ int dw_samples_per_chunk(int64_t S, int tiles) {
   if (chunks < 1) chunks = 1;
   if (chunks > S) chunks = S;
   return (int)((S + chunks - 1) / chunks);
+}
+
+// How pw_dw_flat_kernel cuts a weight gradient: tiles of 128 x 128 wn, the contraction's K steps into `chunks` of `spc`, a chunk's sums
+// into `sums` of `sps` steps.  Wide tiles load least per multiplication, narrow ones fill the chip where there are few K steps; every
+// partial tile is written and read once.  The fastest by this estimate of the widths and some numbers of chunks that fill the chip at
+// most once: 6 us for a block's first loads and its end, per K step 0.2 us + 0.3 us for each 128 columns of multiplication and up to 0.35 us
+// more for their loads with the whole chip at work (one term of x: less), partial tiles at 5.5 TB/s.
+struct DwFlatPlan {
+  int wn, m_blocks, n_blocks, chunks, spc, sums, sps;
+};
+// partial tiles that a workspace holds: those of pw_dw_kernel and as many more as fill the chip with the widest tiles
+int64_t dw_partial_tiles(int64_t M, int64_t N, int64_t S) {
+  const int tiles = (int)(round_up(M, kTile) / kTile * (round_up(N, kTile) / kTile));
+  const int spc = dw_samples_per_chunk(S, tiles);
+  return (S + spc - 1) / spc + 768 / tiles + 1;
+}
+DwFlatPlan dw_flat_plan(int64_t S, int64_t M, int64_t N, int64_t L, int x_terms) {
+  const int64_t steps = (S * (column_pitch(L) / 4) + 7) / 8;
+  const int tiles128 = (int)(round_up(M, kTile) / kTile * (round_up(N, kTile) / kTile));
+  const int64_t longest = dw_samples_per_chunk(S, tiles128) * column_pitch(L) / kTileK;  // of pw_dw_kernel's sums
+  const int64_t room = dw_partial_tiles(M, N, S);
+  const float tile_us = (float)M * (float)N * 1.45e-6f;  // a partial tile written and read
+  DwFlatPlan best = {};
+  float best_us = 0.0f;
+  for (int wn = 1; wn <= 3; ++wn) {
+    DwFlatPlan p;
+    p.wn = wn;
+    p.m_blocks = (int)((M + kTile - 1) / kTile);
+    p.n_blocks = (int)((N + kTile * wn - 1) / (kTile * wn));
+    const int64_t tiles = (int64_t)p.m_blocks * p.n_blocks;
+    const int64_t allowed = wn == 1 ? 5 * longest / 2 : longest;
+    const float width = (float)wn * (x_terms == 1 ? (wn == 1 ? 0.95f : 0.7f) : 1.0f);
+    int64_t want = tiles >= 256 ? 1 : 256 / tiles;
+    if (want > steps) want = steps;
+    for (int k = 0; k < 6 && want >= 1; ++k, want = want * 5 / 8) {
+      const int64_t spc = (steps + want - 1) / want, chunks = (steps + spc - 1) / spc;
+      const int64_t pairs = allowed > 3 ? allowed / 2 : 1;  // (the steps run in pairs)
+      int64_t sums = spc <= allowed ? 1 : (spc + 2 * pairs - 1) / (2 * pairs);
+      if (chunks * sums > room) {
+        if (wn != 1 || want != 1) continue;
+        sums = room / chunks;
+      }
+      const float rounds = (float)((tiles * chunks + 255) / 256), fill = fminf(1.0f, (float)(tiles * chunks) / 256.0f);
+      const float us = rounds * (6.0f + (float)spc * (0.2f + (0.3f + 0.35f * fill) * width)) + (float)(chunks * sums) * tile_us;
+      if (best.spc == 0 || us < best_us) {
+        best_us = us;
+        p.chunks = (int)chunks; p.spc = (int)spc; p.sums = (int)sums;
+        p.sps = (int)(((spc + sums - 1) / sums + 1) / 2 * 2);
+        best = p;
+      }
+    }
+  }
+  return best;
 }
 
 }  // namespace
@@ -1886,9 +2213,18 @@ int launch_pwconv_gemm(const uint16_t *a_planes, int a_terms, int64_t M, int64_t
 }
 
 int64_t pwconv_dw_workspace_floats(int64_t M, int64_t N, int64_t S) {
-  const int tiles = (int)(round_up(M, kTile) / kTile * (round_up(N, kTile) / kTile));
-  const int spc = dw_samples_per_chunk(S, tiles);
-  return (S + spc - 1) / spc * M * N;
+  return dw_partial_tiles(M, N, S) * M * N;
+}
+
+template <int TB, bool BITS, bool RAGGED, int WN> static int launch_dw_flat(const PwDwFlatArgs &a, int64_t blocks, hipStream_t stream) {
+  constexpr unsigned lds = 2 * dw_flat_buffer(TB, WN);
+  if constexpr (lds > 64u * 1024u) {
+    static OncePerDevice once;
+    if (allow_dynamic_lds(once, reinterpret_cast<const void *>(&pw_dw_flat_kernel<TB, BITS, RAGGED, WN>), (int)lds) != hipSuccess)
+      return fail(SJHIP_ERR_LAUNCH, "pwconv_grad_weight: %u bytes of LDS", lds);
+  }
+  hipLaunchKernelGGL((pw_dw_flat_kernel<TB, BITS, RAGGED, WN>), dim3((unsigned)blocks), dim3(kDwThreads), lds, stream, a);
+  return check_launch("pwconv_grad_weight");
 }
 
 int launch_pwconv_grad_weight(const float *dy, int dy_terms, const float *dy_amax, const float *x, int x_terms,
@@ -1901,6 +2237,41 @@ int launch_pwconv_grad_weight(const float *dy, int dy_terms, const float *dy_ama
     return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_grad_weight: L=%lld must be a multiple of 4 (or, with fp16 terms and fp32 activations, at least 4) and the tensors 16-byte aligned", (long long)L);
   if (M * L >= (int64_t(1) << 30) || N * L >= (int64_t(1) << 30) || M * N >= (int64_t(1) << 40))  // 32-bit per-lane byte offsets
     return fail(SJHIP_ERR_TOO_LARGE, "pwconv_grad_weight: M=%lld N=%lld L=%lld", (long long)M, (long long)N, (long long)L);
+  auto reduce = [&](int chunks) {
+    const int64_t count = M * N;
+    if (count % 4 == 0 && aligned16(workspace) && aligned16(dw))
+      hipLaunchKernelGGL(dw_reduce_kernel, dim3((unsigned)((count / 4 + 255) / 256)), dim3(256), 0, stream, workspace, chunks, count, dw);
+    else
+      hipLaunchKernelGGL(dw_reduce_scalar_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, workspace, chunks, count, dw);
+    return check_launch("pwconv_grad_weight(reduce)");
+  };
+  if (dy_terms == (SJHIP_PW_F16 | 2) && (x_terms == 2 || x_terms == 1 || x_terms == (SJHIP_PW_F16 | 1) || x_terms == (SJHIP_PW_F16 | 2)) && dw_flat(S, M, N, L)) {
+    const DwFlatPlan plan = dw_flat_plan(S, M, N, L, x_terms & ~SJHIP_PW_F16);
+    PwDwFlatArgs f;
+    f.dy = dy; f.x = x; f.partials = workspace; f.dy_amax = dy_amax; f.x_amax = x_amax;
+    f.S = (int)S; f.M = (int)M; f.N = (int)N; f.L = (int)L; f.Lq = (int)column_pitch(L);
+    f.m_blocks = plan.m_blocks; f.n_blocks = plan.n_blocks;
+    f.total_quads = (int)(S * f.Lq / 4);
+    f.steps_per_chunk = plan.spc; f.steps_per_sum = plan.sps; f.sums = plan.sums;
+    const int64_t blocks = (int64_t)plan.m_blocks * plan.n_blocks * plan.chunks;
+    if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "pwconv_grad_weight: %lld blocks", (long long)blocks);
+    ProfileScope prof(KC_PW_GRAD_WEIGHT, stream);
+    const int tb = x_terms & ~SJHIP_PW_F16;
+    auto by_width = [&](auto terms, auto bits, auto ragged) {
+      constexpr int TB = decltype(terms)::value;
+      constexpr bool BITS = decltype(bits)::value, RAGGED = decltype(ragged)::value;
+      if (plan.wn == 3) return launch_dw_flat<TB, BITS, RAGGED, 3>(f, blocks, stream);
+      if (plan.wn == 2) return launch_dw_flat<TB, BITS, RAGGED, 2>(f, blocks, stream);
+      return launch_dw_flat<TB, BITS, RAGGED, 1>(f, blocks, stream);
+    };
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, 2> two;
+    int rc;
+    if (x_bits) rc = by_width(one, std::true_type(), std::false_type());
+    else if (tb == 1) rc = L % 4 != 0 ? by_width(one, std::false_type(), std::true_type()) : by_width(one, std::false_type(), std::false_type());
+    else rc = L % 4 != 0 ? by_width(two, std::false_type(), std::true_type()) : by_width(two, std::false_type(), std::false_type());
+    return rc == SJHIP_OK ? reduce(plan.chunks * plan.sums) : rc;
+  }
   PwDwArgs a;
   a.dy = dy; a.x = x; a.partials = workspace; a.S = S;
   a.dy_amax = dy_amax; a.x_amax = x_amax;
@@ -1929,12 +2300,7 @@ int launch_pwconv_grad_weight(const float *dy, int dy_terms, const float *dy_ama
       default: return fail(SJHIP_ERR_UNSUPPORTED, "pwconv_grad_weight: %d gradient terms with %d activation terms (bf16: 3/3, 3/1, 2/2, 2/1, 1/1; fp16: 2/2, 2/1)", dy_terms, x_terms);
     }
     if (rc != SJHIP_OK) return rc;
-    const int64_t count = M * N;
-    if (count % 4 == 0 && aligned16(workspace) && aligned16(dw))
-      hipLaunchKernelGGL(dw_reduce_kernel, dim3((unsigned)((count / 4 + 255) / 256)), dim3(256), 0, stream, workspace, chunks, count, dw);
-    else
-      hipLaunchKernelGGL(dw_reduce_scalar_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, workspace, chunks, count, dw);
-    rc = check_launch("pwconv_grad_weight(reduce)");
+    rc = reduce(chunks);
   }
   return rc;
 }
