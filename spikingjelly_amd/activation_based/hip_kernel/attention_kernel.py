@@ -13,6 +13,7 @@ import ctypes
 
 import torch
 
+from . import eager
 from . import library as L
 
 __all__ = ["hip_ssa_forward", "hip_ssa_backward", "ssa_supported"]
@@ -211,5 +212,5 @@ def lif_ssa_fused(x_seq: torch.Tensor, v_init: torch.Tensor, tau: float, v_th: f
         from . import fused_ops as O
 
         return O.lif_ssa(x_seq, v_init, spec)
-    out, v_last, _ = _LifSsa.apply(x_seq, v_init, spec)
+    out, v_last, _ = eager.apply(_LifSsa, x_seq, v_init, spec)
     return out, v_last

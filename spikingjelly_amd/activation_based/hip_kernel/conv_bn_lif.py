@@ -33,6 +33,7 @@ from typing import Optional
 import torch
 
 from ... import configure
+from . import eager
 from . import library as L
 from . import neuron_kernel as K
 
@@ -776,7 +777,7 @@ def lif_conv_bn_lif(pre_seq: torch.Tensor, pre_v_init: torch.Tensor, weight: tor
         from . import fused_ops as O
 
         return O.lif_conv_bn_lif(pre_seq, pre_v_init, weight, gamma, beta, v_init, bn, pre_spec, spec, k)
-    out = _LifConvBnLif.apply(pre_seq, pre_v_init, weight, gamma, beta, v_init, bn, pre_spec, spec, k)
+    out = eager.apply(_LifConvBnLif, pre_seq, pre_v_init, weight, gamma, beta, v_init, bn, pre_spec, spec, k)
     return out[0], out[1], out[2]
 
 
@@ -796,7 +797,7 @@ def bn_lif(y_seq: torch.Tensor, gamma, beta, v_init: torch.Tensor, bn, spec, k: 
         from . import fused_ops as O
 
         return O.bn_lif(y_seq, gamma, beta, v_init, bn, spec, k)
-    spikes, v_last, _ = _BnLif.apply(y_seq, gamma, beta, v_init, bn, spec, k)
+    spikes, v_last, _ = eager.apply(_BnLif, y_seq, gamma, beta, v_init, bn, spec, k)
     return spikes, v_last
 
 
@@ -808,7 +809,7 @@ def conv_bn_lif(x_seq: torch.Tensor, weight: torch.Tensor, gamma, beta, v_init: 
         from . import fused_ops as O
 
         return O.conv_bn_lif(x_seq, weight, gamma, beta, v_init, bn, spec, x_exact, None, k)
-    spikes, v_last, _, _, _ = _ConvBnLif.apply(x_seq, weight, gamma, beta, v_init, bn, spec, x_exact, k)
+    spikes, v_last, _, _, _ = eager.apply(_ConvBnLif, x_seq, weight, gamma, beta, v_init, bn, spec, x_exact, k)
     return spikes, v_last
 
 
@@ -820,7 +821,7 @@ def conv_bn_lif_ssa(x_seq: torch.Tensor, weight: torch.Tensor, gamma, beta, v_in
         from . import fused_ops as O
 
         return O.conv_bn_lif(x_seq, weight, gamma, beta, v_init, bn, spec, x_exact, (heads, channels_per_head, scale), k)
-    out, v_last, _, _, _, _ = _ConvBnLifSsa.apply(x_seq, weight, gamma, beta, v_init, bn, spec, x_exact,
+    out, v_last, _, _, _, _ = eager.apply(_ConvBnLifSsa, x_seq, weight, gamma, beta, v_init, bn, spec, x_exact,
                                                (heads, channels_per_head, scale), k)
     return out, v_last
 
@@ -829,6 +830,6 @@ def conv_bn_lif_ssa_lif(x_seq: torch.Tensor, weight: torch.Tensor, gamma, beta, 
                         bn, spec, x_exact: bool, heads: int, channels_per_head: int, scale: float, attn_spec, save_h: bool):
     """``conv_bn_lif_ssa`` followed by the LIF of ``attn_spec`` on the contraction's output; returns
     ``(spikes [T, B, heads, channels_per_head, L], v_last of the first neuron, v_last of the attention neuron)``."""
-    out = _ConvBnLifSsaLif.apply(x_seq, weight, gamma, beta, v_init, attn_v_init, bn, spec, x_exact,
+    out = eager.apply(_ConvBnLifSsaLif, x_seq, weight, gamma, beta, v_init, attn_v_init, bn, spec, x_exact,
                                  (heads, channels_per_head, scale), attn_spec, save_h)
     return out[0], out[1], out[2]

@@ -31,6 +31,7 @@ from typing import Optional
 
 import torch
 
+from . import eager
 from . import library as L
 
 __all__ = [
@@ -939,6 +940,6 @@ def eager_multistep(neuron: int, x_seq: torch.Tensor, v_init: torch.Tensor, k: O
             chunk = replay_chunk(x_seq.dtype, x_seq.shape[0], x_seq.shape[1], flags)
             recompute = chunk > 0
         spec = (neuron, tau, v_th, v_reset, flags, sg_id, sg_alpha, store_v_seq, recompute, qif, levels, chunk)
-        return _EagerNeuron.apply(x_seq, v_init, k, spec)[:3]
+        return eager.apply(_EagerNeuron, x_seq, v_init, k, spec)[:3]
     return _run_forward(neuron, x_seq.detach(), v_init.detach(), None if k is None else k.detach(), tau, v_th, v_reset,
                         flags, store_v_seq, False, qif, levels)[:3]
