@@ -238,13 +238,12 @@ __device__ __forceinline__ void store_spike_bits(uint8_t *row, int64_t col, int6
   }
 }
 
-// OUT: what leaves the kernel besides the state, and with it the cache policy of the x loads.  Measured on MI355X with
+// OUT: what leaves the kernel besides the state, and with it the cache policy of its accesses.  Measured on MI355X with
 // both variants on one machine: bit-packed spikes (nothing but x moves) -> streaming everything (98.7 -> 94 us, fp16
 // T = 32, N = 6.4 M); 16-bit storage with fp32 state writing spikes plus v_seq / h_seq -> streaming x loads (bf16 T = 8,
-// N = 8.4 M: 88 -> 74 us); everything else -> default policy (fp32 with two outputs gained 4 % in a forward-only loop
-// but lost 1.2 % inside the training step, forward and backward alternating, which is the case that counts; 16-bit
-// with every op rounded lost 2 %).
-enum FwdOut { FWD_OUT_DENSE = 0, FWD_OUT_PACKED = 1, FWD_OUT_DENSE_STREAM_X = 2 };
+// N = 8.4 M: 88 -> 74 us); tensors that the cache in front of the memory cannot hold -> streaming x loads (16 bit) or
+// streaming stores (fp32), by the rule and the figures at beyond_cache(); everything else -> default policy.
+enum FwdOut { FWD_OUT_DENSE = 0, FWD_OUT_PACKED = 1, FWD_OUT_DENSE_STREAM_X = 2, FWD_OUT_DENSE_STREAM_OUT = 3 };
 // Added to a FwdOut for a sequence of one step (what step_mode='s' runs): two rows in flight instead of eight; the
 // registers the deep prefetch would hold go to resident wavefronts instead (T = 1, N = 134 M fp32: 3.7 -> 6.1 TB/s;
 // at T = 2 and 4 the effect is mixed and the deep prefetch stays).
@@ -258,7 +257,8 @@ __device__ __forceinline__ void forward_body(const FwdArgs &a) {
   // with bit-packed spikes the kernel is read-dominated (x in, one bit out): streaming policy like the backward
   constexpr bool NT = (SJHIP_FWD_NT != 0) || (PACKED && SJHIP_FWD_PACKED_NT != 0);
   typedef Acc<S, VECTOR, NT> A;
-  typedef Acc<S, VECTOR, NT || (OUT & 3) == FWD_OUT_DENSE_STREAM_X> AL;  // policy of the x loads alone
+  typedef Acc<S, VECTOR, NT || (OUT & 3) == FWD_OUT_DENSE_STREAM_X> AL;    // policy of the x loads alone
+  typedef Acc<S, VECTOR, NT || (OUT & 3) == FWD_OUT_DENSE_STREAM_OUT> AO;  // and of what is stored in every step
   typedef typename A::elem_t E;
   typedef typename std::conditional<ROUND_EACH, S, float>::type R;
   constexpr int V = A::V;
@@ -308,10 +308,10 @@ __device__ __forceinline__ void forward_body(const FwdArgs &a) {
 #pragma unroll
         for (int j = 0; j < V; ++j) neuron_step<R, CH, RS>(x[j], v[j], h[j], s[j], tau, a);
         if (PACKED) store_spike_bits<V>((uint8_t *)a.spike + t * (N >> 3), col, N, s);
-        else if (RS == RESET_COUNT) A::store(sp + t * N, s);
-        else A::store_spikes(sp + t * N, s);
-        if (hp) A::store(hp + t * N, h);
-        if (vp) A::store(vp + t * N, v);
+        else if (RS == RESET_COUNT) AO::store(sp + t * N, s);
+        else AO::store_spikes(sp + t * N, s);
+        if (hp) AO::store(hp + t * N, h);
+        if (vp) AO::store(vp + t * N, v);
         if (CKPT && t + 1 == next_checkpoint && t + 1 < T) {
           if constexpr (sizeof(S) == 2 && !ROUND_EACH) {
             // the state is kept in fp32 beside 16-bit storage: so is its checkpoint
@@ -370,18 +370,18 @@ __global__ void __launch_bounds__(SJHIP_MAX_BLOCK) forward_kernel(const FwdArgs 
 
 // The forward of a long sequence that the backward will replay in pieces: the ordinary walk over all T steps, which
 // also leaves the state after every a.chunk steps in a.checkpoints.
-template <typename S, bool ROUND_EACH>
+template <typename S, bool ROUND_EACH, int OUT = FWD_OUT_DENSE>
 __global__ void __launch_bounds__(SJHIP_MAX_BLOCK) forward_pieces_kernel(const FwdArgs a) {
   switch (a.charge) {
-    case CH_IF: forward_reset_dispatch<S, true, ROUND_EACH, CH_IF, FWD_OUT_DENSE, true>(a); break;
-    case CH_DECAY_INPUT_DIV: forward_reset_dispatch<S, true, ROUND_EACH, CH_DECAY_INPUT_DIV, FWD_OUT_DENSE, true>(a); break;
-    case CH_DECAY_INPUT_MUL: forward_reset_dispatch<S, true, ROUND_EACH, CH_DECAY_INPUT_MUL, FWD_OUT_DENSE, true>(a); break;
-    case CH_PLAIN_INPUT_DIV: forward_reset_dispatch<S, true, ROUND_EACH, CH_PLAIN_INPUT_DIV, FWD_OUT_DENSE, true>(a); break;
-    case CH_QIF_DIV: forward_reset_dispatch<S, true, ROUND_EACH, CH_QIF_DIV, FWD_OUT_DENSE, true>(a); break;
-    case CH_QIF_MUL: forward_reset_dispatch<S, true, ROUND_EACH, CH_QIF_MUL, FWD_OUT_DENSE, true>(a); break;
-    case CH_EIF_DIV: forward_reset_dispatch<S, true, ROUND_EACH, CH_EIF_DIV, FWD_OUT_DENSE, true>(a); break;
-    case CH_EIF_MUL: forward_reset_dispatch<S, true, ROUND_EACH, CH_EIF_MUL, FWD_OUT_DENSE, true>(a); break;
-    default: forward_reset_dispatch<S, true, ROUND_EACH, CH_PLAIN_INPUT_MUL, FWD_OUT_DENSE, true>(a); break;
+    case CH_IF: forward_reset_dispatch<S, true, ROUND_EACH, CH_IF, OUT, true>(a); break;
+    case CH_DECAY_INPUT_DIV: forward_reset_dispatch<S, true, ROUND_EACH, CH_DECAY_INPUT_DIV, OUT, true>(a); break;
+    case CH_DECAY_INPUT_MUL: forward_reset_dispatch<S, true, ROUND_EACH, CH_DECAY_INPUT_MUL, OUT, true>(a); break;
+    case CH_PLAIN_INPUT_DIV: forward_reset_dispatch<S, true, ROUND_EACH, CH_PLAIN_INPUT_DIV, OUT, true>(a); break;
+    case CH_QIF_DIV: forward_reset_dispatch<S, true, ROUND_EACH, CH_QIF_DIV, OUT, true>(a); break;
+    case CH_QIF_MUL: forward_reset_dispatch<S, true, ROUND_EACH, CH_QIF_MUL, OUT, true>(a); break;
+    case CH_EIF_DIV: forward_reset_dispatch<S, true, ROUND_EACH, CH_EIF_DIV, OUT, true>(a); break;
+    case CH_EIF_MUL: forward_reset_dispatch<S, true, ROUND_EACH, CH_EIF_MUL, OUT, true>(a); break;
+    default: forward_reset_dispatch<S, true, ROUND_EACH, CH_PLAIN_INPUT_MUL, OUT, true>(a); break;
   }
 }
 

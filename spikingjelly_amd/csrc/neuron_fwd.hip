@@ -7,11 +7,23 @@ namespace sjhip {
 
 namespace {
 
-#ifndef SJHIP_FWD_STREAM_X_FP32
-#define SJHIP_FWD_STREAM_X_FP32 0
-#endif
-template <typename S, bool ROUND_EACH>
-constexpr bool kStreamX = (sizeof(S) == 2 && !ROUND_EACH) || (sizeof(S) == 4 && SJHIP_FWD_STREAM_X_FP32 != 0);
+// Whether the [T, N] tensors of a call are together a third larger than the 256 MiB cache in front of the memory: what
+// the kernel moves then passes through that cache anyway, and marking one side of it as streaming leaves the cache to
+// the other side.  Which side was measured with both policies on one machine, forward plus replaying backward, us
+// (x tensor in MB; default -> streaming):
+//   * fp32, stores streaming (x stays for the backward, which gains as well).  Spikes only, T = 8: 160 MB 133 -> 136,
+//     192 MB 166 -> 162, 256 MB 226 -> 211, 320 MB 283 -> 261, 536 MB 471 -> 448; T = 128: 175 MB 190 -> 201, 320 MB
+//     389 -> 363, 536 MB 580 -> 534.  With v_seq, T = 8: 110 MB 143 -> 146, 128 MB 160 -> 149, 320 MB 398 -> 365,
+//     T = 16, 2.1 GB: 2617 -> 2563 (streaming the x loads instead: 2611 -> 2647).
+//   * 16 bit with spikes only, x loads streaming (streaming the stores: 150 -> 167 in the forward of T = 32, N = 6.4 M).
+//     fp16, T = 6: 140 MB 132 -> 131, 155 MB 144 -> 144, 170 MB 165 -> 160, 192 MB 187 -> 171, 400 MB 412 -> 410; T = 32,
+//     300 MB: 470 -> 450.  (With v_seq and every op rounded it loses from 400 MB on: 576 -> 608.)
+// Below the bound either policy costs up to 10 %: the next reader of the spikes, or the backward, finds them in the cache.
+bool beyond_cache(const FwdArgs &a, int element_bytes) {
+  constexpr int64_t kBytes = (int64_t)256 * 1024 * 1024 / 3 * 4;
+  const int64_t tensors = 2 + (a.v_seq != nullptr) + (a.h != nullptr);
+  return a.T > 1 && a.N > kBytes / (element_bytes * tensors) / a.T;
+}
 
 template <typename S, bool ROUND_EACH, bool PACKED = false>
 int launch_typed(const FwdArgs &a, bool vector, hipStream_t stream) {
@@ -35,14 +47,21 @@ int launch_typed(const FwdArgs &a, bool vector, hipStream_t stream) {
   const unsigned lds = (sizeof(S) == 4 && several_outputs) ? occupancy_cap_lds(cap) : 0u;
   ProfileScope prof(KC_FORWARD, stream);
   const dim3 grid((unsigned)blocks), threads(block);
+  // which accesses stream: see FwdOut and beyond_cache()
+  const bool stream_x = sizeof(S) == 2 && a.T > 1 && (several_outputs ? !ROUND_EACH : beyond_cache(a, 2));
+  const bool stream_out = sizeof(S) == 4 && beyond_cache(a, 4);
   if constexpr (PACKED) {
     if (vector) hipLaunchKernelGGL((forward_kernel<S, true, ROUND_EACH, FWD_OUT_PACKED>), grid, threads, lds, stream, a);
     else hipLaunchKernelGGL((forward_kernel<S, false, ROUND_EACH, FWD_OUT_PACKED>), grid, threads, lds, stream, a);
-  } else if (kStreamX<S, ROUND_EACH> && several_outputs && a.T > 1) {
-    // 16-bit storage with fp32 state writing spikes plus v_seq / h_seq: see FwdOut
-    if constexpr (kStreamX<S, ROUND_EACH>) {
+  } else if (stream_x) {
+    if constexpr (sizeof(S) == 2) {
       if (vector) hipLaunchKernelGGL((forward_kernel<S, true, ROUND_EACH, FWD_OUT_DENSE_STREAM_X>), grid, threads, lds, stream, a);
       else hipLaunchKernelGGL((forward_kernel<S, false, ROUND_EACH, FWD_OUT_DENSE_STREAM_X>), grid, threads, lds, stream, a);
+    }
+  } else if (stream_out) {
+    if constexpr (sizeof(S) == 4) {
+      if (vector) hipLaunchKernelGGL((forward_kernel<S, true, ROUND_EACH, FWD_OUT_DENSE_STREAM_OUT>), grid, threads, lds, stream, a);
+      else hipLaunchKernelGGL((forward_kernel<S, false, ROUND_EACH, FWD_OUT_DENSE_STREAM_OUT>), grid, threads, lds, stream, a);
     }
   } else if (a.T == 1) {
     if (vector) hipLaunchKernelGGL((forward_kernel<S, true, ROUND_EACH, FWD_OUT_DENSE | FWD_OUT_SHORT>), grid, threads, lds, stream, a);
@@ -66,7 +85,12 @@ template <typename S, bool ROUND_EACH> int launch_pieces_typed(const FwdArgs &a,
   if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "forward(pieces): N=%lld", (long long)a.N);
   const unsigned lds = (sizeof(S) == 4 && a.v_seq != nullptr) ? occupancy_cap_lds(tuning().fwd_blocks_per_cu) : 0u;
   ProfileScope prof(KC_FORWARD, stream);
-  hipLaunchKernelGGL((forward_pieces_kernel<S, ROUND_EACH>), dim3((unsigned)blocks), dim3(block), lds, stream, a);
+  if (sizeof(S) == 4 && beyond_cache(a, 4)) {
+    if constexpr (sizeof(S) == 4)
+      hipLaunchKernelGGL((forward_pieces_kernel<S, ROUND_EACH, FWD_OUT_DENSE_STREAM_OUT>), dim3((unsigned)blocks), dim3(block), lds, stream, a);
+  } else {
+    hipLaunchKernelGGL((forward_pieces_kernel<S, ROUND_EACH>), dim3((unsigned)blocks), dim3(block), lds, stream, a);
+  }
   return check_launch("forward(pieces)");
 }
 
