@@ -483,7 +483,7 @@ int sjhip_ssa_lif_backward_packed(int neuron, const sjhip_neuron_params *p, int6
  *                               (M = Cout, K = Cin), its input gradient with A = weight^T (M = Cin, K = Cout, b = dY)
  *   sjhip_pwconv_grad_weight    dw[m][n] = sum_{s,l} dy[s][m][l] x[s][n][l]; workspace of
  *                               sjhip_pwconv_grad_weight_workspace_floats(M, N, S) floats (partial sums over groups of
- *                               samples, added in a fixed order)
+ *                               samples or of columns, added in a fixed order)
  */
 int64_t sjhip_pwconv_planes_elems(int64_t rows, int64_t cols);
 int sjhip_pwconv_split_weight(const float *w, int64_t rows, int64_t cols, int transpose, uint16_t *planes, void *stream);
