@@ -1503,7 +1503,7 @@ struct PwDwFlatArgs {
   int total_quads;      // S * Lq / 4
   int steps_per_chunk;  // K steps (eight quads) per partial tile
   int steps_per_sum;    // K steps, an even number, after which the accumulators go out and start again
-  int sums;             // partial tiles per chunk
+  int sums;             // partial tiles per chunk: steps_per_chunk / steps_per_sum, rounded up
   const float *dy_amax, *x_amax;
 };
 constexpr int kDwThreads = 512;
@@ -1686,9 +1686,10 @@ __global__ void __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu
   };
 
   // The accumulators into the next of the chunk's partial tiles.  (The address and the bounds pass through
-  // an empty asm: out of the loop, where the compiler would keep them, the addresses and masks of 32 WN stores spill.)
+  // an empty asm: out of the loop, where the compiler would keep them, the addresses and masks of 32 WN stores spill.  Not inlined
+  // everywhere, the accumulators would live in scratch memory.)
   int64_t slot = (int64_t)chunk * a.sums;
-  auto flush = [&]() {
+  auto flush = [&]() __attribute__((always_inline)) {
     float *at = a.partials + (slot * M + (m0 + wm * 64 + 4 * (lane >> 5))) * N + (n0 + wn * (32 * WN) + (lane & 31));
     int rows_left = M - (m0 + wm * 64 + 4 * (lane >> 5)), cols_left = N - (n0 + wn * (32 * WN) + (lane & 31));
     asm volatile("" : "+v"(at), "+v"(rows_left), "+v"(cols_left));
@@ -1728,22 +1729,25 @@ __global__ void __launch_bounds__(kDwThreads) __attribute__((amdgpu_waves_per_eu
   for (int u = 0; u < U; ++u) fetch_unit(u, 0);
   __syncthreads();
   int it = 0, sum_end = a.steps_per_sum;
-  for (; it + 4 < iters; it += 2) {  // (tile it + 2, staged by the second step, is not the last one)
+  auto cut = [&]() {  // before a pair of steps: a full sum goes out
     if (it >= sum_end) {
       flush();
       sum_end += a.steps_per_sum;
     }
+  };
+  for (; it + 4 < iters; it += 2) {  // (tile it + 2, staged by the second step, is not the last one)
+    cut();
     step(even, std::true_type(), true, false, true);
     step(odd, std::true_type(), true, false, true);
   }
-  // at most four tiles are left; the last one may be partly empty
-  step(even, std::false_type(), it + 1 < iters, it + 2 >= iters, it + 3 < iters);
-  if (it + 1 < iters) step(odd, std::false_type(), it + 2 < iters, it + 3 >= iters, false);
-  if (it + 2 < iters) step(even, std::false_type(), it + 3 < iters, true, false);
-  if (it + 3 < iters) step(odd, std::false_type(), false, false, false);
+  for (; it < iters; it += 2) {  // at most four tiles are left; the last one may be partly empty
+    cut();
+    step(even, std::false_type(), it + 1 < iters, it + 2 >= iters, it + 3 < iters);
+    if (it + 1 < iters) step(odd, std::false_type(), it + 2 < iters, it + 3 >= iters, false);
+  }
   const int64_t slots_end = ((int64_t)chunk + 1) * a.sums;
-  flush();
-  for (; slot < slots_end;) flush();  // (a last chunk shorter than the others: the accumulators are zeros now)
+  do flush();  // (again: a last chunk shorter than the others, the accumulators are zeros then)
+  while (slot < slots_end);
 }
 
 struct PwDwPlanesArgs {
@@ -2072,12 +2076,13 @@ DwFlatPlan dw_flat_plan(int64_t S, int64_t M, int64_t N, int64_t L, int x_terms)
         if (wn != 1 || want != 1) continue;
         sums = room / chunks;
       }
+      const int64_t sps = ((spc + sums - 1) / sums + 1) / 2 * 2;
+      sums = (spc + sps - 1) / sps;  // (an even length may need fewer)
       const float rounds = (float)((tiles * chunks + 255) / 256), fill = fminf(1.0f, (float)(tiles * chunks) / 256.0f);
       const float us = rounds * (6.0f + (float)spc * (0.2f + (0.3f + 0.35f * fill) * width)) + (float)(chunks * sums) * tile_us;
       if (best.spc == 0 || us < best_us) {
         best_us = us;
-        p.chunks = (int)chunks; p.spc = (int)spc; p.sums = (int)sums;
-        p.sps = (int)(((spc + sums - 1) / sums + 1) / 2 * 2);
+        p.chunks = (int)chunks; p.spc = (int)spc; p.sums = (int)sums; p.sps = (int)sps;
         best = p;
       }
     }

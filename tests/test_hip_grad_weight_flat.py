@@ -57,3 +57,33 @@ def test_positions_beyond_the_last_chunk_do_not_count():
         got = C.pw_grad_weight(dy, C.F16 | 2, x, C.F16 | 2, *amax)
         want = torch.einsum("sml,snl->mn", dy.double().cpu(), x.double().cpu())
         torch.testing.assert_close(got.double().cpu(), want, rtol=1e-5, atol=1e-5)
+
+
+def _longest_sum(S, M, N, L):
+    """K steps (32 positions) that a sum of 32 bits may hold: the chunk of whole samples that one block took when every product went
+    into one sum (n), and 5 / 2 of it, at most 3 n - 2, on tiles where the products of small terms have sums of their own."""
+    tiles = -(-M // 128) * -(-N // 128)
+    samples = -(-S // min(S, max(1, (1024 if tiles >= 16 else 512) // tiles)))
+    n = -(-samples * (-(-L // 4) * 4) // 32)
+    return max(n, min(5 * n // 2, 3 * n - 2))
+
+
+@pytest.mark.parametrize("S, M, N, L", [
+    (32, 1152, 384, 64), (20, 1376, 480, 49), (20, 1408, 448, 49),  # chunks whose last pieces are the tail of the loop
+    (36, 1248, 160, 49), (128, 512, 512, 49), (100, 1152, 384, 36),
+])
+def test_no_sum_is_longer_than_its_limit(S, M, N, L):
+    """A term of 1/2 that is a whole limit of K steps away from 2^25 and from -2^25 is in neither's sum: the products are exact, the
+    partial tiles are added in 64 bits, so the result is 1/2 exactly; added to 2^25 in 32 bits it would be lost."""
+    from spikingjelly_amd.activation_based.hip_kernel import conv_bn_lif as C
+
+    limit, quads = _longest_sum(S, M, N, L), -(-L // 4)
+    last = S * quads // 8 - 1
+    assert last >= 2 * limit
+    first = torch.arange(M, device="cuda") % (last - 2 * limit + 1)
+    dy = torch.zeros((S, M, L), device="cuda")
+    for distance, value in ((0, 2.0 ** 25), (limit, 0.5), (2 * limit, -2.0 ** 25)):
+        quad = (first + distance) * 8
+        dy[quad // quads, torch.arange(M, device="cuda"), quad % quads * 4] = value
+    got = C.pw_grad_weight(dy, C.F16 | 2, torch.ones((S, N, L), device="cuda"), C.F16 | 2)
+    assert torch.equal(got, torch.full((M, N), 0.5, device="cuda"))
