@@ -1491,10 +1491,11 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
 // Kernel and reduction, before / now, us: this shape 207 / 163, x as bits 141 / 119; dy [128, 1536, 196], x [128, 384, 196] 139 / 117;
 // both [256, 384, 196] 75 / 64; dy [64, 768, 100], x [64, 256, 100] 28.0 / 20.6; both [128, 512, 49] 43.7 / 32.9; both [16, 384, 196]
 // 21.5 / 16.5; dy [4, 1152, 196], x [4, 384, 196] 20.0 / 15.4.
-// No sum is less exact than before (error against float64, relative 2-norm): the sums of 32 bits are no longer than pw_dw_kernel's chunks
-// were (dw_flat_plan), where needed a chunk leaves several partial tiles.  With WN = 1 registers are left for sums of their own for
-// the products of small terms: those of the large ones are rounded a third (one term of x: half) as often, which allows chains 2.5 times as
-// long.  qkv shape 4.6e-7 / 3.8e-7, spikes 2.2e-7 / 1.9e-7; [128, 512, 49] 1.48e-7 / 1.27e-7, spikes 8.9e-8 / 5.7e-8; twelve shapes, all lower.
+// No result is further from float64 than pw_dw_kernel's: sums of 32 bits are no longer than that kernel's chunks were (dw_longest_sum),
+// where needed a chunk leaves several partial tiles.  With WN = 1 registers are left for sums of their own for the products of small
+// terms: those of the large ones are rounded a third (one term of x: half) as often and may be longer.  Relative 2-norm of the error, before /
+// now: qkv shape 4.6e-7 / 3.8e-7, spikes 2.5e-7 / 2.1e-7; [128, 512, 49] 1.48e-7 / 1.29e-7, spikes 9.8e-8 / 5.7e-8; dy [32, 1152, 64], x
+// [32, 384, 64] 1.22e-7 / 1.14e-7; dy [20, 1376, 49], x [20, 480, 49] 1.19e-7 / 1.11e-7.
 struct PwDwFlatArgs {
   const float *dy, *x;
   float *partials;
@@ -2037,12 +2038,12 @@ int dw_samples_per_chunk(int64_t S, int tiles) {
 }
 
 // How pw_dw_flat_kernel cuts a weight gradient: tiles of 128 x 128 wn, the contraction's K steps into `chunks` of `spc`, a chunk's sums
-// into `sums` of `sps` steps.  Wide tiles load least per multiplication, narrow ones fill the chip where there are few K steps; every
-// partial tile is written and read once.  The fastest by this estimate of the widths and some numbers of chunks that fill the chip at
-// most once: 6 us for a block's first loads and its end, per K step 0.2 us + 0.3 us for each 128 columns of multiplication and up to 0.35 us
-// more for their loads with the whole chip at work (one term of x: less), partial tiles at 5.5 TB/s.
+// into `sums` of `sps` steps (even: the steps run in pairs).  Wide tiles load least per multiplication, narrow ones fill the chip where
+// there are few K steps; every partial tile is written and read once.  The fastest by this estimate of the widths and some numbers of
+// chunks that fill the chip at most once: 6 us for a block's first loads and its end, per K step 0.2 us + 0.3 us for each 128 columns of
+// multiplication and up to 0.35 us more for their loads with the whole chip at work (one term of x: less), partial tiles at 5.5 TB/s.
 struct DwFlatPlan {
-  int wn, m_blocks, n_blocks, chunks, spc, sums, sps;
+  int wn, m_blocks, n_blocks, chunks, spc, sums, sps;  // wn = 0: no plan
 };
 // partial tiles that a workspace holds: those of pw_dw_kernel and as many more as fill the chip with the widest tiles
 int64_t dw_partial_tiles(int64_t M, int64_t N, int64_t S) {
@@ -2050,10 +2051,27 @@ int64_t dw_partial_tiles(int64_t M, int64_t N, int64_t S) {
   const int spc = dw_samples_per_chunk(S, tiles);
   return (S + spc - 1) / spc + 768 / tiles + 1;
 }
+// K steps that a sum of 32 bits may hold, so that its error stays below that of pw_dw_kernel's sums over `quads` quads.  The error that
+// rounding leaves in a sum grows with its length times the roundings per step:
+//   * wide tiles round as that kernel does, after each product of terms: no longer than its sums;
+//   * narrow ones round the sum of the large products a third as often: 5/2 of the length; with one term of x half as often: twice
+//     the length, less a step and a half for the addition of both sums at the end (spikes, whose large products add up almost
+//     exactly, could take more, but not other values of one term; packed and dense spikes give the same bits).
+// Error against float64 / pw_dw_kernel's, 56 shapes of 29 to 400 positions: fp32 x 0.54 to 1.00, bfloat16 values in one term 0.57
+// to 1.00, spikes 0.45 to 1.00.  (Before, with 5/2 for one term, and short lengths of wide tiles rounded up to two: up to 1.42, 1.49, 1.37.)
+// With one term and sums of less than three steps so many partial tiles would be written that pw_dw_kernel is as fast, us flat / that
+// kernel: [64, 256 x 256, 49] 26.5 / 19.7, [8, 1536 x 512, 81] 28.1 / 25.4, [32, 1152 x 384, 64] 30.8 / 28.9, [64, 1024 x 256, 64]
+// 29.6 / 31.5; from three steps on it is not: [100, 1152 x 384, 32] 26.7 / 32.4.
+constexpr int64_t kDwOneTermQuads = 24;
+int64_t dw_longest_sum(int64_t quads, int wn, int x_terms) {
+  if (wn > 1) return quads / 8;
+  return x_terms == 1 ? (quads - 6) / 4 : 5 * quads / 16;
+}
 DwFlatPlan dw_flat_plan(int64_t S, int64_t M, int64_t N, int64_t L, int x_terms) {
   const int64_t steps = (S * (column_pitch(L) / 4) + 7) / 8;
   const int tiles128 = (int)(round_up(M, kTile) / kTile * (round_up(N, kTile) / kTile));
-  const int64_t longest = dw_samples_per_chunk(S, tiles128) * column_pitch(L) / kTileK;  // of pw_dw_kernel's sums
+  const int64_t quads = dw_samples_per_chunk(S, tiles128) * (column_pitch(L) / 4);  // of pw_dw_kernel's sums
+  if (x_terms == 1 && quads < kDwOneTermQuads) return {};
   const int64_t room = dw_partial_tiles(M, N, S);
   const float tile_us = (float)M * (float)N * 1.45e-6f;  // a partial tile written and read
   DwFlatPlan best = {};
@@ -2064,23 +2082,24 @@ DwFlatPlan dw_flat_plan(int64_t S, int64_t M, int64_t N, int64_t L, int x_terms)
     p.m_blocks = (int)((M + kTile - 1) / kTile);
     p.n_blocks = (int)((N + kTile * wn - 1) / (kTile * wn));
     const int64_t tiles = (int64_t)p.m_blocks * p.n_blocks;
-    const int64_t allowed = wn == 1 ? 5 * longest / 2 : longest;
+    const int64_t longest = dw_longest_sum(quads, wn, x_terms);
     const float width = (float)wn * (x_terms == 1 ? (wn == 1 ? 0.95f : 0.7f) : 1.0f);
     int64_t want = tiles >= 256 ? 1 : 256 / tiles;
     if (want > steps) want = steps;
     for (int k = 0; k < 6 && want >= 1; ++k, want = want * 5 / 8) {
       const int64_t spc = (steps + want - 1) / want, chunks = (steps + spc - 1) / spc;
-      const int64_t pairs = allowed > 3 ? allowed / 2 : 1;  // (the steps run in pairs)
-      int64_t sums = spc <= allowed ? 1 : (spc + 2 * pairs - 1) / (2 * pairs);
-      if (chunks * sums > room) {
-        if (wn != 1 || want != 1) continue;
-        sums = room / chunks;
+      int64_t sums = 1, sps = round_up(spc, 2);
+      if (spc > longest) {
+        if (longest < 2) continue;  // (a sum of its own for every step would cost more than it gains)
+        const int64_t even = longest / 2 * 2;
+        sums = (spc + even - 1) / even;
+        sps = round_up((spc + sums - 1) / sums, 2);
+        sums = (spc + sps - 1) / sps;  // (an even length may need fewer)
       }
-      const int64_t sps = ((spc + sums - 1) / sums + 1) / 2 * 2;
-      sums = (spc + sps - 1) / sps;  // (an even length may need fewer)
+      if (chunks * sums > room) continue;
       const float rounds = (float)((tiles * chunks + 255) / 256), fill = fminf(1.0f, (float)(tiles * chunks) / 256.0f);
       const float us = rounds * (6.0f + (float)spc * (0.2f + (0.3f + 0.35f * fill) * width)) + (float)(chunks * sums) * tile_us;
-      if (best.spc == 0 || us < best_us) {
+      if (best.wn == 0 || us < best_us) {
         best_us = us;
         p.chunks = (int)chunks; p.spc = (int)spc; p.sums = (int)sums; p.sps = (int)sps;
         best = p;
@@ -2250,8 +2269,10 @@ int launch_pwconv_grad_weight(const float *dy, int dy_terms, const float *dy_ama
       hipLaunchKernelGGL(dw_reduce_scalar_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, workspace, chunks, count, dw);
     return check_launch("pwconv_grad_weight(reduce)");
   };
-  if (dy_terms == (SJHIP_PW_F16 | 2) && (x_terms == 2 || x_terms == 1 || x_terms == (SJHIP_PW_F16 | 1) || x_terms == (SJHIP_PW_F16 | 2)) && dw_flat(S, M, N, L)) {
-    const DwFlatPlan plan = dw_flat_plan(S, M, N, L, x_terms & ~SJHIP_PW_F16);
+  DwFlatPlan plan = {};
+  if (dy_terms == (SJHIP_PW_F16 | 2) && (x_terms == 1 || x_terms == 2) && dw_flat(S, M, N, L))
+    plan = dw_flat_plan(S, M, N, L, x_terms);
+  if (plan.wn != 0) {
     PwDwFlatArgs f;
     f.dy = dy; f.x = x; f.partials = workspace; f.dy_amax = dy_amax; f.x_amax = x_amax;
     f.S = (int)S; f.M = (int)M; f.N = (int)N; f.L = (int)L; f.Lq = (int)column_pitch(L);
@@ -2261,7 +2282,6 @@ int launch_pwconv_grad_weight(const float *dy, int dy_terms, const float *dy_ama
     const int64_t blocks = (int64_t)plan.m_blocks * plan.n_blocks * plan.chunks;
     if (blocks > 0x7fffffffLL) return fail(SJHIP_ERR_TOO_LARGE, "pwconv_grad_weight: %lld blocks", (long long)blocks);
     ProfileScope prof(KC_PW_GRAD_WEIGHT, stream);
-    const int tb = x_terms & ~SJHIP_PW_F16;
     auto by_width = [&](auto terms, auto bits, auto ragged) {
       constexpr int TB = decltype(terms)::value;
       constexpr bool BITS = decltype(bits)::value, RAGGED = decltype(ragged)::value;
@@ -2273,7 +2293,7 @@ int launch_pwconv_grad_weight(const float *dy, int dy_terms, const float *dy_ama
     const std::integral_constant<int, 2> two;
     int rc;
     if (x_bits) rc = by_width(one, std::true_type(), std::false_type());
-    else if (tb == 1) rc = L % 4 != 0 ? by_width(one, std::false_type(), std::true_type()) : by_width(one, std::false_type(), std::false_type());
+    else if (x_terms == 1) rc = L % 4 != 0 ? by_width(one, std::false_type(), std::true_type()) : by_width(one, std::false_type(), std::false_type());
     else rc = L % 4 != 0 ? by_width(two, std::false_type(), std::true_type()) : by_width(two, std::false_type(), std::false_type());
     return rc == SJHIP_OK ? reduce(plan.chunks * plan.sums) : rc;
   }
