@@ -482,8 +482,10 @@ int sjhip_ssa_lif_backward_packed(int neuron, const sjhip_neuron_params *p, int6
  *   sjhip_pwconv_gemm           c[s][m][l] = sum_k A[m][k] b[s][k][l]: the convolution with A = weight [Cout][Cin]
  *                               (M = Cout, K = Cin), its input gradient with A = weight^T (M = Cin, K = Cout, b = dY)
  *   sjhip_pwconv_grad_weight    dw[m][n] = sum_{s,l} dy[s][m][l] x[s][n][l]; workspace of
- *                               sjhip_pwconv_grad_weight_workspace_floats(M, N, S) floats (partial sums over groups of
- *                               samples or of columns, added in a fixed order)
+ *                               sjhip_pwconv_grad_weight_workspace_floats_for(M, N, S, L, dy_terms, x_terms) floats (partial
+ *                               sums over groups of samples or of columns, added in a fixed order; dy_terms as given to the call,
+ *                               SJHIP_PW_F16 | 2 for the fp16 forms below), at most
+ *                               sjhip_pwconv_grad_weight_workspace_floats(M, N, S) for any L and terms
  */
 int64_t sjhip_pwconv_planes_elems(int64_t rows, int64_t cols);
 int sjhip_pwconv_split_weight(const float *w, int64_t rows, int64_t cols, int transpose, uint16_t *planes, void *stream);
@@ -497,6 +499,7 @@ int64_t sjhip_pwconv_gemm_stats_rows(int64_t K, int64_t S, int64_t L);
 int sjhip_pwconv_gemm_stats(const uint16_t *a_planes, int a_terms, int64_t M, int64_t K, const float *b, int b_terms, int64_t S,
                             int64_t L, float *c, float *partial, void *stream);
 int64_t sjhip_pwconv_grad_weight_workspace_floats(int64_t M, int64_t N, int64_t S);
+int64_t sjhip_pwconv_grad_weight_workspace_floats_for(int64_t M, int64_t N, int64_t S, int64_t L, int dy_terms, int x_terms);
 int sjhip_pwconv_grad_weight(const float *dy, int dy_terms, const float *x, int x_terms, int64_t S, int64_t M, int64_t N,
                              int64_t L, float *dw, float *workspace, void *stream);
 

@@ -177,7 +177,7 @@ def pw_grad_weight(dy: torch.Tensor, dy_terms: int, x: torch.Tensor, x_terms: in
     N = x.shape[1]
     dy, x = L.aligned16(dy), L.aligned16(x)
     lib = L.load()
-    ws = torch.empty(lib.sjhip_pwconv_grad_weight_workspace_floats(M, N, S), dtype=torch.float32, device=dy.device)
+    ws = torch.empty(lib.sjhip_pwconv_grad_weight_workspace_floats_for(M, N, S, Lp, dy_terms, x_terms & ~F16), dtype=torch.float32, device=dy.device)
     dw = torch.empty((M, N), dtype=torch.float32, device=dy.device)
     with torch.cuda.device(dy.device):
         if dy_terms & F16:
@@ -216,7 +216,7 @@ def pw_grad_weight_bits(dy: torch.Tensor, bits: torch.Tensor, N: int, dy_amax: O
     S, M, Lp = dy.shape
     dy = L.aligned16(dy)
     lib = L.load()
-    ws = torch.empty(lib.sjhip_pwconv_grad_weight_workspace_floats(M, N, S), dtype=torch.float32, device=dy.device)
+    ws = torch.empty(lib.sjhip_pwconv_grad_weight_workspace_floats_for(M, N, S, Lp, F16 | 2, 1), dtype=torch.float32, device=dy.device)
     dw = torch.empty((M, N), dtype=torch.float32, device=dy.device)
     if dy_amax is None:
         dy_amax = amax(dy)

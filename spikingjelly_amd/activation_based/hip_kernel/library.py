@@ -75,6 +75,7 @@ EXPORTED_SYMBOLS = (
     "sjhip_pwconv_gemm_stats_rows",
     "sjhip_pwconv_gemm_stats",
     "sjhip_pwconv_grad_weight_workspace_floats",
+    "sjhip_pwconv_grad_weight_workspace_floats_for",
     "sjhip_pwconv_grad_weight",
     "sjhip_pwconv_split_weight_f16",
     "sjhip_pwconv_amax",
@@ -275,6 +276,8 @@ def load() -> ctypes.CDLL:
                                                 c_void_p, c_void_p]
         lib.sjhip_pwconv_grad_weight_workspace_floats.restype = c_int64
         lib.sjhip_pwconv_grad_weight_workspace_floats.argtypes = [c_int64, c_int64, c_int64]
+        lib.sjhip_pwconv_grad_weight_workspace_floats_for.restype = c_int64
+        lib.sjhip_pwconv_grad_weight_workspace_floats_for.argtypes = [c_int64, c_int64, c_int64, c_int64, c_int, c_int]
         lib.sjhip_pwconv_grad_weight.restype = c_int
         lib.sjhip_pwconv_grad_weight.argtypes = [c_void_p, c_int, c_void_p, c_int, c_int64, c_int64, c_int64, c_int64,
                                                  c_void_p, c_void_p, c_void_p]

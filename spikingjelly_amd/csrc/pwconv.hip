@@ -2043,13 +2043,15 @@ int dw_samples_per_chunk(int64_t S, int tiles) {
 // chunks that fill the chip at most once: 6 us for a block's first loads and its end, per K step 0.2 us + 0.3 us for each 128 columns of
 // multiplication and up to 0.35 us more for their loads with the whole chip at work (one term of x: less), partial tiles at 5.5 TB/s.
 struct DwFlatPlan {
-  int wn, m_blocks, n_blocks, chunks, spc, sums, sps;  // wn = 0: no plan
+  int wn, m_blocks, n_blocks, chunks, spc, sums, sps;  // wn = 0: pw_dw_kernel
 };
-// partial tiles that a workspace holds: those of pw_dw_kernel and as many more as fill the chip with the widest tiles
+// partial tiles that pw_dw_kernel leaves, and the most that a plan may: as many more as fill the chip with the widest tiles
+int64_t dw_sample_chunks(int64_t M, int64_t N, int64_t S) {
+  const int spc = dw_samples_per_chunk(S, (int)(round_up(M, kTile) / kTile * (round_up(N, kTile) / kTile)));
+  return (S + spc - 1) / spc;
+}
 int64_t dw_partial_tiles(int64_t M, int64_t N, int64_t S) {
-  const int tiles = (int)(round_up(M, kTile) / kTile * (round_up(N, kTile) / kTile));
-  const int spc = dw_samples_per_chunk(S, tiles);
-  return (S + spc - 1) / spc + 768 / tiles + 1;
+  return dw_sample_chunks(M, N, S) + 768 / (round_up(M, kTile) / kTile * (round_up(N, kTile) / kTile)) + 1;
 }
 // K steps that a sum of 32 bits may hold, so that its error stays below that of pw_dw_kernel's sums over `quads` quads.  The error that
 // rounding leaves in a sum grows with its length times the roundings per step:
@@ -2067,7 +2069,8 @@ int64_t dw_longest_sum(int64_t quads, int wn, int x_terms) {
   if (wn > 1) return quads / 8;
   return x_terms == 1 ? (quads - 6) / 4 : 5 * quads / 16;
 }
-DwFlatPlan dw_flat_plan(int64_t S, int64_t M, int64_t N, int64_t L, int x_terms) {
+DwFlatPlan dw_flat_plan(int64_t S, int64_t M, int64_t N, int64_t L, int dy_terms, int x_terms) {
+  if (dy_terms != (SJHIP_PW_F16 | 2) || (x_terms != 1 && x_terms != 2) || !dw_flat(S, M, N, L)) return {};
   const int64_t steps = (S * (column_pitch(L) / 4) + 7) / 8;
   const int tiles128 = (int)(round_up(M, kTile) / kTile * (round_up(N, kTile) / kTile));
   const int64_t quads = dw_samples_per_chunk(S, tiles128) * (column_pitch(L) / 4);  // of pw_dw_kernel's sums
@@ -2236,8 +2239,11 @@ int launch_pwconv_gemm(const uint16_t *a_planes, int a_terms, int64_t M, int64_t
   return SJHIP_OK;
 }
 
-int64_t pwconv_dw_workspace_floats(int64_t M, int64_t N, int64_t S) {
-  return dw_partial_tiles(M, N, S) * M * N;
+int64_t pwconv_dw_workspace_floats(int64_t M, int64_t N, int64_t S) { return dw_partial_tiles(M, N, S) * M * N; }
+
+int64_t pwconv_dw_workspace_floats_for(int64_t M, int64_t N, int64_t S, int64_t L, int dy_terms, int x_terms) {
+  const DwFlatPlan plan = dw_flat_plan(S, M, N, L, dy_terms, x_terms);
+  return (plan.wn != 0 ? (int64_t)plan.chunks * plan.sums : dw_sample_chunks(M, N, S)) * M * N;
 }
 
 template <int TB, bool BITS, bool RAGGED, int WN> static int launch_dw_flat(const PwDwFlatArgs &a, int64_t blocks, hipStream_t stream) {
@@ -2269,9 +2275,7 @@ int launch_pwconv_grad_weight(const float *dy, int dy_terms, const float *dy_ama
       hipLaunchKernelGGL(dw_reduce_scalar_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, stream, workspace, chunks, count, dw);
     return check_launch("pwconv_grad_weight(reduce)");
   };
-  DwFlatPlan plan = {};
-  if (dy_terms == (SJHIP_PW_F16 | 2) && (x_terms == 1 || x_terms == 2) && dw_flat(S, M, N, L))
-    plan = dw_flat_plan(S, M, N, L, x_terms);
+  const DwFlatPlan plan = dw_flat_plan(S, M, N, L, dy_terms, x_terms);
   if (plan.wn != 0) {
     PwDwFlatArgs f;
     f.dy = dy; f.x = x; f.partials = workspace; f.dy_amax = dy_amax; f.x_amax = x_amax;

@@ -647,6 +647,11 @@ int64_t sjhip_pwconv_grad_weight_workspace_floats(int64_t M, int64_t N, int64_t 
   return pwconv_dw_workspace_floats(M, N, S);
 }
 
+int64_t sjhip_pwconv_grad_weight_workspace_floats_for(int64_t M, int64_t N, int64_t S, int64_t L, int dy_terms, int x_terms) {
+  if (M < 1 || N < 1 || S < 1 || L < 1 || S > (int64_t(1) << 40) / L) return 0;
+  return pwconv_dw_workspace_floats_for(M, N, S, L, dy_terms, x_terms);
+}
+
 int sjhip_pwconv_grad_weight(const float *dy, int dy_terms, const float *x, int x_terms, int64_t S, int64_t M, int64_t N,
                              int64_t L, float *dw, float *workspace, void *stream) {
   if (!dy || !x || !dw || !workspace) return fail(SJHIP_ERR_INVALID, "pwconv_grad_weight: NULL buffer");
@@ -791,7 +796,11 @@ struct ChainBackwardParts {
     partial = carve.take(B * Cout * 2);
     amax = carve.take(SJHIP_PW_AMAX_FLOATS + SJHIP_PW_AMAX_SAMPLE_WORDS * T * B);
     k_shares = carve.take(plif ? bn_lif_backward_k_workspace_floats(B, Cout, L) : 0);
-    const int64_t dw_floats = dw ? pwconv_dw_workspace_floats(Cout, Cin, T * B) : 0;
+    int64_t dw_floats = 0;  // (the activations have one or two terms)
+    for (int x_terms = 1; dw && x_terms <= 2; ++x_terms) {
+      const int64_t floats_for = pwconv_dw_workspace_floats_for(Cout, Cin, T * B, L, SJHIP_PW_F16 | 2, x_terms);
+      if (floats_for > dw_floats) dw_floats = floats_for;
+    }
     const int64_t planes_floats = dx ? (pwconv_planes_elems(Cin, Cout) + 1) / 2 : 0;
     dw_partials = carve.take(dw_floats > planes_floats ? dw_floats : planes_floats);
     planes = reinterpret_cast<uint16_t *>(dw_partials);

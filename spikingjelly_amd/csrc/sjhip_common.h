@@ -526,6 +526,7 @@ int launch_pwconv_gemm(const uint16_t *a_planes, int a_terms, int64_t M, int64_t
                        const float *b_amax, int64_t S, int64_t L, float *c, float *stats, hipStream_t stream, bool b_bits = false);
 int64_t pwconv_gemm_stats_rows(int64_t K, int64_t S, int64_t L);
 int64_t pwconv_dw_workspace_floats(int64_t M, int64_t N, int64_t S);
+int64_t pwconv_dw_workspace_floats_for(int64_t M, int64_t N, int64_t S, int64_t L, int dy_terms, int x_terms);
 int launch_pwconv_grad_weight(const float *dy, int dy_terms, const float *dy_amax, const float *x, int x_terms,
                               const float *x_amax, int64_t S, int64_t M, int64_t N, int64_t L, float *dw, float *workspace,
                               hipStream_t stream, bool x_bits = false);

@@ -276,3 +276,21 @@ def test_convolution_chain_refuses_before_its_first_launch(change, code, text):
                                        0xb0000, a["batch_stats"], 0.1, 1e-5, None, a["v_init"], a["k"], None, 0x30000, 0x40000, a["spikes"],
                                        a["bits"], a["v_last"], 0x60000, None)
     assert rc == code and text in lib.sjhip_last_error(), (rc, lib.sjhip_last_error())
+
+
+def test_weight_gradient_workspace_is_what_the_call_writes():
+    """One partial tile per chunk, not a bound over all lengths and terms: [128, 128] of one sample 196 long takes its seven K steps at
+    most, lengths and terms of the other kernel its chunks of whole samples."""
+    lib, fp16 = L.load(), 18
+    size = lib.sjhip_pwconv_grad_weight_workspace_floats_for
+    for x_terms in (1, 2):
+        assert 128 * 128 <= size(128, 128, 1, 196, fp16, x_terms) <= 7 * 128 * 128
+        assert size(128, 128, 1, 28, fp16, x_terms) == size(128, 128, 1, 196, x_terms, x_terms) == 128 * 128
+        for M, N, S, Lp in ((384, 384, 4, 196), (1152, 384, 256, 196), (1536, 512, 8, 81), (64, 64, 3000, 49), (4096, 4096, 1, 32),
+                            (5000, 1, 1, 5000), (1, 1, 1, 1), (1676, 4821, 1, 37), (745, 93, 150, 39)):
+            chunks = size(M, N, S, Lp, fp16, x_terms) // (M * N)
+            assert 1 <= chunks <= max(S, -(-S * -(-Lp // 4) // 8))
+            assert chunks * M * N == size(M, N, S, Lp, fp16, x_terms) <= lib.sjhip_pwconv_grad_weight_workspace_floats(M, N, S)
+    # the chain's backward: partial tiles instead of the planes of the transposed weights where they need more room
+    with_dw, without = (lib.sjhip_conv_bn_lif_backward_workspace_floats(1, 1, 128, 128, 196, 0, dw, 0) for dw in (1, 0))
+    assert 128 * 128 <= with_dw - without <= 7 * 128 * 128

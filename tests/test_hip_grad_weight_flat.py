@@ -117,3 +117,19 @@ def test_no_sum_is_longer_than_its_limit(S, M, N, L, x_terms):
         dy[quad // quads, torch.arange(M, device="cuda"), quad % quads * 4] = value
     got = C.pw_grad_weight(dy, C.F16 | 2, torch.ones((S, N, L), device="cuda"), C.F16 | x_terms)
     assert torch.equal(got, torch.full((M, N), 0.5, device="cuda"))
+
+
+@pytest.mark.parametrize("S, M, N, L", [(1, 128, 128, 196), (4, 384, 384, 196), (20, 1376, 480, 49), (3, 129, 127, 31), (128, 512, 512, 49), (5, 40, 24, 20)])
+@pytest.mark.parametrize("x_terms", [1, 2])
+def test_workspace_of_the_stated_size_is_enough(S, M, N, L, x_terms):
+    """(a buffer for any length, of which the part beyond the stated size keeps its contents)"""
+    from spikingjelly_amd.activation_based.hip_kernel import conv_bn_lif as C
+
+    lib = C.L.load()
+    size = lib.sjhip_pwconv_grad_weight_workspace_floats_for(M, N, S, L, C.F16 | 2, x_terms)
+    room = torch.full((lib.sjhip_pwconv_grad_weight_workspace_floats(M, N, S),), 7.0, device="cuda")
+    dy, x = seeded_randn((S, M, L), 1).cuda(), (seeded_randn((S, N, L), 2) > 0.5).float().cuda()
+    amax, dw = [C.amax(t) for t in (dy, x)], torch.empty((M, N), device="cuda")
+    assert lib.sjhip_pwconv_grad_weight_f16(dy.data_ptr(), amax[0].data_ptr(), x.data_ptr(), x_terms, amax[1].data_ptr(), S, M, N, L,
+                                            dw.data_ptr(), room.data_ptr(), C._stream(dy)) == 0
+    assert bool((room[size:] == 7.0).all()) and torch.equal(dw, C.pw_grad_weight(dy, C.F16 | 2, x, C.F16 | x_terms))
