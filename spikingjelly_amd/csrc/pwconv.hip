@@ -2056,17 +2056,18 @@ int64_t dw_partial_tiles(int64_t M, int64_t N, int64_t S) {
 // K steps that a sum of 32 bits may hold, so that its error stays below that of pw_dw_kernel's sums over `quads` quads.  The error that
 // rounding leaves in a sum grows with its length times the roundings per step:
 //   * wide tiles round as that kernel does, after each product of terms: no longer than its sums;
-//   * narrow ones round the sum of the large products a third as often: 5/2 of the length; with one term of x half as often: twice
-//     the length, less a step and a half for the addition of both sums at the end (spikes, whose large products add up almost
-//     exactly, could take more, but not other values of one term; packed and dense spikes give the same bits).
-// Error against float64 / pw_dw_kernel's, 56 shapes of 29 to 400 positions: fp32 x 0.54 to 1.00, bfloat16 values in one term 0.57
-// to 1.00, spikes 0.45 to 1.00.  (Before, with 5/2 for one term, and short lengths of wide tiles rounded up to two: up to 1.42, 1.49, 1.37.)
+//   * narrow ones round the sum of the large products a third as often: 5/2 of the length, where that is one step only (eight quads)
+//     no more than it; with one term of x half as often: twice the length, less a step and a half for the addition of both sums at
+//     the end (spikes, whose large products add up almost exactly, could take more, but not other values of one term; packed and
+//     dense spikes give the same bits).
+// Error against float64 / pw_dw_kernel's, 206 shapes of 29 to 400 positions: fp32 x 0.53 to 1.00, bfloat16 values in one term 0.50
+// to 1.00, spikes 0.35 to 1.00.  (Before, with 5/2 for one term, and short lengths of wide tiles rounded up to two: up to 1.42, 1.49, 1.37.)
 // With one term and sums of less than three steps so many partial tiles would be written that pw_dw_kernel is as fast, us flat / that
 // kernel: [64, 256 x 256, 49] 26.5 / 19.7, [8, 1536 x 512, 81] 28.1 / 25.4, [32, 1152 x 384, 64] 30.8 / 28.9, [64, 1024 x 256, 64]
 // 29.6 / 31.5; from three steps on it is not: [100, 1152 x 384, 32] 26.7 / 32.4.
 constexpr int64_t kDwOneTermQuads = 24;
 int64_t dw_longest_sum(int64_t quads, int wn, int x_terms) {
-  if (wn > 1) return quads / 8;
+  if (wn > 1 || quads < 9) return quads / 8;
   return x_terms == 1 ? (quads - 6) / 4 : 5 * quads / 16;
 }
 DwFlatPlan dw_flat_plan(int64_t S, int64_t M, int64_t N, int64_t L, int dy_terms, int x_terms) {

@@ -18,6 +18,7 @@ FORMER = [  # S, M, N, L; error of the former kernel in 1e-8: fp32 x (two terms)
     (2, 128, 384, 29, 10.14, 7.37, 6.80), (5, 130, 390, 36, 10.64, 7.82, 7.17),
     (3, 129, 127, 31, 9.95, 7.38, 6.76),
     # few samples or short rows: sums of a few steps
+    (4, 1152, 512, 32, 9.90, 7.21, 6.72), (4, 1376, 224, 30, 10.06, 7.32, 6.82),
     (31, 1536, 160, 29, 10.73, 8.16, 7.55), (38, 1152, 384, 30, 12.02, 9.13, 8.09),
     (60, 1536, 512, 32, 13.50, 10.41, 8.92), (58, 416, 416, 36, 11.84, 9.25, 8.44),
     (20, 1376, 480, 49, 11.92, 8.90, 7.80), (36, 1152, 384, 49, 12.20, 9.22, 8.17),
@@ -87,19 +88,19 @@ def test_positions_beyond_the_last_chunk_do_not_count():
 
 def _longest_sum(S, M, N, L, x_terms):
     """K steps (32 positions) that a sum of 32 bits may hold.  A chunk of whole samples that one block of the former kernel took, in
-    quads of positions; on tiles where the products of small terms have sums of their own 5 / 2 of it, with one term of x twice its
-    length less a step and a half, and from three steps on only (below, the former kernel runs)."""
+    quads of positions; on tiles where the products of small terms have sums of their own 5 / 2 of it if it is longer than a step, with
+    one term of x twice its length less a step and a half, and from three steps on only (below, the former kernel runs)."""
     tiles = -(-M // 128) * -(-N // 128)
     samples = -(-S // min(S, max(1, (1024 if tiles >= 16 else 512) // tiles)))
     quads = samples * -(-L // 4)
     if x_terms == 1:
         return (quads - 6) // 4 if quads >= 24 else -(-quads // 8)
-    return 5 * quads // 16
+    return 5 * quads // 16 if quads > 8 else 1
 
 
 @pytest.mark.parametrize("S, M, N, L", [
     (32, 1152, 384, 64), (20, 1376, 480, 49), (20, 1408, 448, 49),  # chunks whose last pieces are the tail of the loop
-    (36, 1248, 160, 49), (128, 512, 512, 49), (100, 1152, 384, 36), (58, 416, 416, 36), (41, 1472, 480, 64), (60, 1536, 512, 32),
+    (36, 1248, 160, 49), (128, 512, 512, 49), (100, 1152, 384, 36), (58, 416, 416, 36), (41, 1472, 480, 64), (60, 1536, 512, 32), (38, 1152, 384, 30),
 ])
 @pytest.mark.parametrize("x_terms", [1, 2])
 def test_no_sum_is_longer_than_its_limit(S, M, N, L, x_terms):
