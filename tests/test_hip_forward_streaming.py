@@ -30,7 +30,9 @@ def run(x, v_seq, grad):
     (torch.float32, "torch", 3, False, 0),      # at the bound: the default policy
     (torch.float16, "torch", 3, False, 5),
     (torch.float16, "fp32_state", 2, False, 8),
-    (torch.bfloat16, "torch", 64, False, 7),
+    (torch.bfloat16, "torch", 6, False, 7),
+    (torch.float16, "torch", 39, False, 3),     # the longest sequence that does not run in pieces
+    (torch.bfloat16, "torch", 64, False, 7),    # in pieces: 16 bit keeps the default policy at any size
 ])
 def test_streamed_calls_equal_their_slices(dtype, mode, T, v_seq, beside, monkeypatch):
     monkeypatch.setattr(configure, "hip_half_precision_mode", mode)
