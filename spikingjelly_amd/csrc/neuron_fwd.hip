@@ -9,8 +9,8 @@ namespace {
 
 // Whether the [T, N] tensors of a call are together a third larger than the 256 MiB cache in front of the memory: what
 // the kernel moves then passes through that cache anyway, and marking one side of it as streaming leaves the cache to
-// the other side.  Which side was measured with both policies on one machine, forward plus replaying backward, us
-// (x tensor in MB; default -> streaming):
+// the other side.  Which side was measured with both policies on one machine, forward plus replaying backward repeated on
+// the same tensors, us (x tensor in MB; default -> streaming):
 //   * fp32, stores streaming (x stays for the backward, which gains as well).  Spikes only, T = 8: 160 MB 133 -> 136,
 //     192 MB 166 -> 162, 256 MB 226 -> 211, 320 MB 283 -> 261, 536 MB 471 -> 448; T = 128: 175 MB 190 -> 201, 320 MB
 //     389 -> 363, 536 MB 580 -> 534.  With v_seq, T = 8: 110 MB 143 -> 146, 128 MB 160 -> 149, 320 MB 398 -> 365,
@@ -18,7 +18,16 @@ namespace {
 //   * 16 bit with spikes only, x loads streaming (streaming the stores: 150 -> 167 in the forward of T = 32, N = 6.4 M).
 //     fp16, T = 6: 140 MB 132 -> 131, 155 MB 144 -> 144, 170 MB 165 -> 160, 192 MB 187 -> 171, 400 MB 412 -> 410; T = 32,
 //     300 MB: 470 -> 450.  (With v_seq and every op rounded it loses from 400 MB on: 576 -> 608.)
-// Below the bound either policy costs up to 10 %: the next reader of the spikes, or the backward, finds them in the cache.
+// Inside a network less is left of it: three inputs in turn, an elementwise operation that writes x before the neuron and one that
+// reads the spikes after it, everything together, us:
+//   * fp32, T = 8, inference: 192 MB 197 -> 186, 256 MB 266 -> 262, 320 MB 327 -> 321, 536 MB 548 -> 551; training: 422 -> 422,
+//     570 -> 563, 691 -> 685, 1163 -> 1165.  With v_seq, inference 240 -> 220, 321 -> 309, 388 -> 381, 650 -> 652, training 468 -> 456,
+//     624 -> 617, 752 -> 743, 1271 -> 1271; T = 4, 128 MB 174 -> 136.  It costs at T = 4 and 5 from 160 to 192 MB (258 -> 269,
+//     206 -> 202; training 482 -> 496, 395 -> 406).
+//   * fp16, T = 8: inference 211 -> 205, 279 -> 272, 429 -> 422, training 455 -> 445, 599 -> 593, 929 -> 923.
+// A reader of the spikes finds less of them in the cache: forward and sum over T 106 -> 121 at 192 MB, 156 -> 153 at 256 MB.
+// Below the bound either policy costs up to 10 %: the next reader of the spikes, or the backward, finds them in the cache.  16-bit
+// sequences in pieces keep the default policy: neither was measured for them.
 bool beyond_cache(const FwdArgs &a, int element_bytes) {
   constexpr int64_t kBytes = (int64_t)256 * 1024 * 1024 / 3 * 4;
   const int64_t tensors = 2 + (a.v_seq != nullptr) + (a.h != nullptr);

@@ -60,6 +60,7 @@
 //   pw_dw_kernel       dW[m][n] = sum_{s,l} dY[s][m][l] X[s][n][l]
 //       both operands are contiguous along the contraction index l; a block owns a 128 x 128 tile of dW for a chunk
 //       of samples and writes its partial tile, dw_reduce_kernel adds the chunks in a fixed order.
+//   pw_dw_flat_kernel  the same on fp16 terms over rows of 29 positions and more, where dw_flat_plan finds a plan
 // Blocks that share operand tiles are numbered so that they run on the same XCD (one L2 each, blocks are dealt
 // round-robin over the eight XCDs).
 #include <cmath>
@@ -1207,10 +1208,12 @@ struct PwDwArgs {
 
 // Two LDS buffers where x has one fp16 term (spikes, 2 x 30 KiB): the next tile is split and stored while the current one is
 // multiplied, with one barrier per K step instead of two.  One buffer / two, us with the reduction, three processes of each in
-// turn on one box: (on shapes that pw_dw_flat_kernel has taken over) x as bits, dy [256, 1152, 196] and x [256, 384, 196] 146.6 / 142.0, [128, 1536, 196] and [128, 384, 196]
-// 108.6 / 105.1, [256, 384, 196] both 58.3 / 55.5; x as fp32 spikes 197.6 / 189.4, 110.1 / 110.1, 59.9 / 59.9.  With two terms of x
-// (2 x 40 KiB) two buffers measured 210.4 -> 214.0, 138.8 -> 138.4, 74.7 -> 74.5: those keep one, and every launch stays within
-// the default limit of dynamic LDS.  (The bf16 split's three planes per operand would leave one block per compute unit.)
+// turn on one box, shapes that pw_dw_flat_kernel leaves to this one: x as fp32 spikes, dy [1024, 512, 16], x [1024, 512, 16]
+// 68.8 / 65.9, [256, 1152, 16] and [256, 384, 16] 44.7 / 43.9, [64, 2048, 16] and [64, 512, 16] 37.9 / 37.5, both [128, 512, 16] 31.3 / 31.7,
+// [512, 768, 25] and [512, 256, 25] 38.6 / 38.2, both [64, 256, 49] 19.3 / 19.6; as bits 70.5 / 68.4, 44.4 / 44.4, 38.1 / 37.6, 32.5 / 32.6.
+// With two terms of x (2 x 40 KiB) two buffers measured, on shapes that pw_dw_flat_kernel has taken over, 210.4 -> 214.0, 138.8 -> 138.4,
+// 74.7 -> 74.5: those keep one, and every launch stays within the default limit of dynamic LDS.  (The bf16 split's three planes per
+// operand would leave one block per compute unit.)
 constexpr bool dw_two_buffers(bool h, int tb) { return h && tb == 1; }
 // four elements at a 16-byte or, with ANY, at a 4-byte address
 template <bool ANY> __device__ __forceinline__ f32x4 load4(const char *p) {
@@ -1488,9 +1491,10 @@ __global__ void __launch_bounds__(kPwThreads) __attribute__((amdgpu_waves_per_eu
 //   * with them 2700: the loads bound it (128 x 128 tiles move 32 KB per step and tile through a compute unit's memory path).  A block is
 //     eight wavefronts, 128 rows of dy by 128 WN of x: with WN = 3 64 KB for three tiles.  acc 96 + two tiles in flight 64 + fragments
 //     of a half step and the next one's: 246 registers, two wavefronts per SIMD, one block per compute unit.
-// Kernel and reduction, before / now, us: this shape 207 / 163, x as bits 141 / 119; dy [128, 1536, 196], x [128, 384, 196] 139 / 117;
-// both [256, 384, 196] 75 / 64; dy [64, 768, 100], x [64, 256, 100] 28.0 / 20.6; both [128, 512, 49] 43.7 / 32.9; both [16, 384, 196]
-// 21.5 / 16.5; dy [4, 1152, 196], x [4, 384, 196] 20.0 / 15.4.
+// Kernel and reduction, calls repeated on the same tensors, pw_dw_kernel / this one, us: this shape 208 / 168, x as bits 141 / 117; dy
+// [128, 1536, 196], x [128, 384, 196] 137 / 116; both [256, 384, 196] 73 / 63; both [128, 512, 49] 43.2 / 29.8; both [16, 384, 196]
+// 21.4 / 16.6; dy [4, 1152, 196], x [4, 384, 196] 19.7 / 15.3.  Inside a training step, where dy has just been written over: this shape
+// 234 / 172, its projection (384 rows of dy, x as bits) 69 / 52, dy [128, 1536, 196] 159 / 142.
 // No result is further from float64 than pw_dw_kernel's: sums of 32 bits are no longer than that kernel's chunks were (dw_longest_sum),
 // where needed a chunk leaves several partial tiles.  With WN = 1 registers are left for sums of their own for the products of small
 // terms: those of the large ones are rounded a third (one term of x: half) as often and may be longer.  Relative 2-norm of the error, before /
@@ -2042,6 +2046,10 @@ int dw_samples_per_chunk(int64_t S, int tiles) {
 // there are few K steps; every partial tile is written and read once.  The fastest by this estimate of the widths and some numbers of
 // chunks that fill the chip at most once: 6 us for a block's first loads and its end, per K step 0.2 us + 0.3 us for each 128 columns of
 // multiplication and up to 0.35 us more for their loads with the whole chip at work (one term of x: less), partial tiles at 5.5 TB/s.
+// The figures were fitted to calls repeated on the same tensors, which find in the cache in front of the memory what fits there.  Inside a
+// training step narrow tiles take a quarter longer than estimated, wide ones a twentieth: dy [128, 1536, 196], x [128, 384, 196], for which
+// the estimate prefers wn = 1 (113 us against 123), measured 138 + 7 there with wn = 1, 142 + 12 with 2, 110 + 18 with 3; dy
+// [256, 1152, 196], x [256, 384, 196] (wn = 3) 211 + 7, 200 + 13, 156 + 17.
 struct DwFlatPlan {
   int wn, m_blocks, n_blocks, chunks, spc, sums, sps;  // wn = 0: pw_dw_kernel
 };
