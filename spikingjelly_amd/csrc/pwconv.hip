@@ -1208,7 +1208,7 @@ struct PwDwArgs {
 
 // Two LDS buffers where x has one fp16 term (spikes, 2 x 30 KiB): the next tile is split and stored while the current one is
 // multiplied, with one barrier per K step instead of two.  One buffer / two, us with the reduction, three processes of each in
-// turn on one box, shapes that pw_dw_flat_kernel leaves to this one: x as fp32 spikes, dy [1024, 512, 16], x [1024, 512, 16]
+// turn on one machine, shapes that pw_dw_flat_kernel leaves to this one: x as fp32 spikes, dy [1024, 512, 16], x [1024, 512, 16]
 // 68.8 / 65.9, [256, 1152, 16] and [256, 384, 16] 44.7 / 43.9, [64, 2048, 16] and [64, 512, 16] 37.9 / 37.5, both [128, 512, 16] 31.3 / 31.7,
 // [512, 768, 25] and [512, 256, 25] 38.6 / 38.2, both [64, 256, 49] 19.3 / 19.6; as bits 70.5 / 68.4, 44.4 / 44.4, 38.1 / 37.6, 32.5 / 32.6.
 // With two terms of x (2 x 40 KiB) two buffers measured, on shapes that pw_dw_flat_kernel has taken over, 210.4 -> 214.0, 138.8 -> 138.4,
